@@ -17,8 +17,11 @@
 //                  bottom-up inside the block with LDS arrival counters, and
 //                  leaves prefix / suffix unions of the block's frontier nodes
 //   top_boxes      one wave per node above the frontier: its box from two of
-//                  those unions and the whole-block boxes between them
-// Refit runs only local (bounds phase) + top_boxes.
+//                  those unions and the whole-block boxes between them; in a
+//                  build also the nodes' places in the sibling-pair copy
+//   copies         the traversal copies of the node array: four-child records
+//                  (wide.hpp) and sibling pairs
+// Refit runs only local (bounds phase) + top_boxes + copies.
 //
 // No box crosses workgroups through a counter: every hand-off between
 // workgroups is a kernel boundary, so no agent-scope release/acquire (an L2
@@ -32,6 +35,7 @@
 // with merged keys :63-131, internal box = union of children :139-159
 // (union_aabb(left, right), src/core/aabb.cuh:113-115).
 #include "lux_runtime.hpp"
+#include "wide.hpp"
 
 namespace lux {
 namespace {
@@ -809,6 +813,25 @@ __global__ __launch_bounds__(kLocalThreads) void k_local(
     }
 }
 
+// Slots of the children of the internal node at preorder position k, whose leaf
+// range ends at `last` and whose left child's ends at `split`. In right-first
+// preorder the nodes before it are the n-1-last leaves right of its range and
+// k-(n-1-last) internal nodes, which is its internal rank r. Its children go to
+// the pair r+1: the right child (position k+1, 2 (last - split) - 1 nodes) at slot
+// 2r+2, the left child (behind it) at slot 2r+3.
+__device__ __forceinline__ void pair_slots(int n, int k, uint32_t split, uint32_t last,
+                                           uint32_t* __restrict__ pair_pos, DevInfo* info) {
+    const int node_count = 2 * n - 1;
+    const int rank = k - (n - 1 - int(last));
+    const int left = k + 2 * int(last - split);
+    if (k < 0 || rank < 0 || rank >= n - 1 || left <= k + 1 || left >= node_count) {
+        set_error(info, kErrWalkOrder);
+        return;
+    }
+    pair_pos[k + 1] = uint32_t(2 * rank + 2);
+    pair_pos[left] = uint32_t(2 * rank + 3);
+}
+
 // ---------------------------------------------------------------------------
 // 7. top boxes: one wave per node above the frontier
 // ---------------------------------------------------------------------------
@@ -819,6 +842,9 @@ __global__ __launch_bounds__(kLocalThreads) void k_local(
 // `last` (the prefix at its rightmost frontier node, a right child). The
 // blocks between are folded in contiguous runs, lane by lane, then across the
 // wave with lower lanes on the left, so the host's left-to-right order holds.
+// kLayout (build): every lane also places its node's children in the
+// sibling-pair copy; a launch of its own for that took 13 us at 2^20 leaves and
+// 5 us at 100 000.
 __device__ __forceinline__ lux_aabb shfl_down_box(const lux_aabb& b, int off) {
     lux_aabb r;
     r.p_min.x = __shfl_down(b.p_min.x, off, 64);
@@ -830,8 +856,11 @@ __device__ __forceinline__ lux_aabb shfl_down_box(const lux_aabb& b, int off) {
     return r;
 }
 
+template <bool kLayout>
 __global__ __launch_bounds__(kBlock) void k_top_boxes(int n, const uint32_t* __restrict__ first_of,
                                                       const uint32_t* __restrict__ last_of,
+                                                      const uint32_t* __restrict__ left,
+                                                      uint32_t* __restrict__ pair_pos,
                                                       const int32_t* __restrict__ pre_internal,
                                                       const lux_aabb* __restrict__ edge_boxes,
                                                       const lux_aabb* __restrict__ block_boxes,
@@ -847,6 +876,10 @@ __global__ __launch_bounds__(kBlock) void k_top_boxes(int n, const uint32_t* __r
         if (i < n - 1) {
             my_first = first_of[i];
             my_last = last_of[i];
+            if (kLayout) {
+                if (i == 0) pair_pos[0] = 0;  // the root stays at slot 0
+                pair_slots(n, pre_internal[i], left[i] & kIndexMask, my_last, pair_pos, info);
+            }
         }
         uint64_t todo = __ballot(i < n - 1 && my_first / kLocalLeaves != my_last / kLocalLeaves);
         while (todo) {
@@ -929,7 +962,7 @@ void bvh_release(BvhDev& d) {
                     d.left,      d.right,       d.parent,       d.first,      d.last,       d.leaf_parent,
                     d.edge_boxes, d.block_boxes, d.pre_internal, d.pre_leaf, d.nodes,       d.hist,
                     d.status,    d.tickets,     d.partials,     d.info,       d.counter,
-                    d.rtop_int,  d.rtop_leaf,   d.pairs,        d.pair_pos,   d.slot_pre};
+                    d.rtop_int,  d.rtop_leaf,   d.pairs,        d.pair_pos,   d.slot_pre, d.wide, d.wide_leaf};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     BvhDev empty;
@@ -940,32 +973,14 @@ void bvh_release(BvhDev& d) {
 // sibling-pair traversal copy of the node array
 // ---------------------------------------------------------------------------
 namespace {
-// Internal node i (Karras order) sits at preorder position k = pre_internal[i];
-// in right-first preorder the nodes before it are the n-1-last(i) leaves right
-// of its range and k-(n-1-last(i)) internal nodes, which is its internal rank
-// r. Its children go to the pair r+1: right child (position k+1) at slot
-// 2r+2, left child (escape of k+1) at slot 2r+3.
-__global__ __launch_bounds__(kBlock) void k_pair_layout(int n, const uint32_t* __restrict__ last,
+// Pair positions of a tree of one leaf block (larger ones: k_top_boxes).
+__global__ __launch_bounds__(kBlock) void k_pair_layout(int n, const uint32_t* __restrict__ left,
+                                                        const uint32_t* __restrict__ last,
                                                         const int32_t* __restrict__ pre_internal,
-                                                        const lux_bvh_node* __restrict__ nodes,
                                                         uint32_t* __restrict__ pair_pos, DevInfo* info) {
-    const int node_count = 2 * n - 1;
-    if (blockIdx.x == 0 && threadIdx.x == 0) pair_pos[0] = 0;  // the root (leaf or internal) stays at slot 0
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n - 1; i += gridDim.x * kBlock) {
-        const int k = pre_internal[i];
-        const int rank = k - (n - 1 - int(last[i]));
-        if (k < 0 || k + 1 >= node_count || rank < 0 || rank >= n - 1) {
-            set_error(info, kErrWalkOrder);
-            continue;
-        }
-        const int left = nodes[k + 1].escape;
-        if (left <= k + 1 || left >= node_count) {
-            set_error(info, kErrWalkOrder);
-            continue;
-        }
-        pair_pos[k + 1] = uint32_t(2 * rank + 2);
-        pair_pos[left] = uint32_t(2 * rank + 3);
-    }
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i == 0) pair_pos[0] = 0;  // the root (leaf or internal) stays at slot 0
+    if (i < n - 1) pair_slots(n, pre_internal[i], left[i] & kIndexMask, last[i], pair_pos, info);
 }
 
 // Copies every node to its slot: boxes and leaf ids as they are, internal
@@ -973,13 +988,12 @@ __global__ __launch_bounds__(kBlock) void k_pair_layout(int n, const uint32_t* _
 // Slot 1 (the root's unused sibling) gets an empty box that no walk reaches.
 // slot_pre records each slot's preorder position (the tie order of the
 // ordered walk).
-__global__ __launch_bounds__(kBlock) void k_pair_fill(int n, const lux_bvh_node* __restrict__ nodes,
-                                                      const uint32_t* __restrict__ pair_pos,
-                                                      lux_bvh_node* __restrict__ pairs,
-                                                      uint32_t* __restrict__ slot_pre, DevInfo* info) {
+__device__ __forceinline__ void fill_pairs(int n, int first, int stride, const lux_bvh_node* __restrict__ nodes,
+                                           const uint32_t* __restrict__ pair_pos, lux_bvh_node* __restrict__ pairs,
+                                           uint32_t* __restrict__ slot_pre, DevInfo* info) {
     const int node_count = 2 * n - 1;
     const int slots = 2 * n;
-    for (int k = blockIdx.x * kBlock + threadIdx.x; k < node_count; k += gridDim.x * kBlock) {
+    for (int k = first; k < node_count; k += stride) {
         lux_bvh_node nd = nodes[k];
         const uint32_t dst = pair_pos[k];
         if (dst >= uint32_t(slots)) {
@@ -1005,7 +1019,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_fill(int n, const lux_bvh_node*
         pairs[dst] = nd;
         slot_pre[dst] = uint32_t(k);
     }
-    if (n >= 2 && blockIdx.x == 0 && threadIdx.x == 0) {
+    if (n >= 2 && first == 0) {
         lux_bvh_node pad;
         pad.bounds = box_empty();
         pad.primitive_id = -1;
@@ -1015,23 +1029,115 @@ __global__ __launch_bounds__(kBlock) void k_pair_fill(int n, const lux_bvh_node*
     }
 }
 
-}  // namespace
-
-void pair_fill(BvhDev& d, hipStream_t s) {
-    if (d.n <= 0) return;
-    LUX_LAUNCH("lbvh_pair_fill", k_pair_fill, max(1, min(2048, div_up(2 * d.n - 1, kBlock))), kBlock, 0, s, d.n,
-               (const lux_bvh_node*)d.nodes, (const uint32_t*)d.pair_pos, d.pairs, d.slot_pre, d.info);
+// ---------------------------------------------------------------------------
+// four-child traversal records (wide.hpp)
+// ---------------------------------------------------------------------------
+// One thread per internal node: its two children, the larger internal one
+// opened, then the largest of the three. Its reads are gathers of positions and
+// 32-byte nodes close to each other (Karras order and preorder both follow the
+// leaves), its write one 64-byte record and 16 bytes of leaf positions.
+__device__ __forceinline__ void fill_wide(int n, int first, int stride, const uint32_t* __restrict__ left,
+                                          const uint32_t* __restrict__ right,
+                                          const int32_t* __restrict__ pre_internal,
+                                          const int32_t* __restrict__ pre_leaf,
+                                          const lux_bvh_node* __restrict__ nodes, WideNode* __restrict__ wide,
+                                          int32_t* __restrict__ wide_leaf, DevInfo* info) {
+    const int total = 2 * n - 1;
+    for (int i = first; i < n - 1; i += stride) {
+        lux_aabb box[4];
+        uint32_t ref[4];
+        int32_t pos[4];
+        float area[4] = {-1.0f, -1.0f, -1.0f, -1.0f};
+        bool bad = false;
+        auto load = [&](int k, uint32_t c) {
+            const uint32_t idx = c & kIndexMask;
+            const bool leaf = c & kLeafBit;
+            bad |= idx >= uint32_t(leaf ? n : n - 1);
+            const int p = bad ? 0 : (leaf ? pre_leaf[idx] : pre_internal[idx]);
+            bad |= uint32_t(p) >= uint32_t(total);
+            float4 a, b;
+            load_node(nodes, bad ? 0 : p, a, b);
+            box[k].p_min = lux_vec3{a.x, a.y, a.z};
+            box[k].p_max = lux_vec3{a.w, b.x, b.y};
+            pos[k] = p;
+            ref[k] = leaf ? (kLeafBit | uint32_t(__float_as_int(b.z))) : idx;
+            const float dx = a.w - a.x, dy = b.x - a.y, dz = b.y - a.z;
+            area[k] = leaf ? -1.0f : dx * dy + dy * dz + dz * dx;
+        };
+        load(0, left[i]);
+        load(1, right[i]);
+        int count = 2;
+#pragma unroll
+        for (int open = 0; open < 2; ++open) {
+            int best = -1;
+            float ba = -1.0f;
+#pragma unroll
+            for (int k = 0; k < 2 + open; ++k)
+                if (area[k] > ba) {
+                    ba = area[k];
+                    best = k;
+                }
+            if (best < 0 || bad) continue;
+            uint32_t c = 0;
+#pragma unroll
+            for (int k = 0; k < 2 + open; ++k)
+                if (k == best) c = ref[k];
+            const uint32_t cl = left[c], cr = right[c];
+#pragma unroll
+            for (int k = 0; k < 2 + open; ++k)
+                if (k == best) load(k, cl);
+            load(2 + open, cr);
+            ++count;
+        }
+        if (bad) {
+            set_error(info, kErrWalkOrder);
+            continue;
+        }
+#pragma unroll
+        for (int k = 2; k < 4; ++k)
+            if (k >= count) {
+                box[k] = box[0];
+                ref[k] = kWideEmpty;
+                pos[k] = -1;
+            }
+        WideNode w;
+        make_wide(w, box, ref, count);
+        store_wide(wide + i, w);
+        reinterpret_cast<int4*>(wide_leaf)[i] = make_int4(pos[0], pos[1], pos[2], pos[3]);
+    }
 }
 
-void pair_build(BvhDev& d, hipStream_t s) {
-    if (d.n <= 0) return;
-    if (d.n >= 2)
-        LUX_LAUNCH("lbvh_pair_layout", k_pair_layout, max(1, min(2048, div_up(d.n - 1, kBlock))), kBlock, 0, s, d.n,
-                   (const uint32_t*)d.last, (const int32_t*)d.pre_internal, (const lux_bvh_node*)d.nodes,
-                   d.pair_pos, d.info);
+// Both traversal copies of the finished node array, in one launch: the first
+// `wide_blocks` workgroups make the records, the others the sibling pairs.
+__global__ __launch_bounds__(kBlock) void k_copies(int n, int wide_blocks, const uint32_t* __restrict__ left,
+                                                   const uint32_t* __restrict__ right,
+                                                   const int32_t* __restrict__ pre_internal,
+                                                   const int32_t* __restrict__ pre_leaf,
+                                                   const lux_bvh_node* __restrict__ nodes,
+                                                   WideNode* __restrict__ wide, int32_t* __restrict__ wide_leaf,
+                                                   const uint32_t* __restrict__ pair_pos,
+                                                   lux_bvh_node* __restrict__ pairs, uint32_t* __restrict__ slot_pre,
+                                                   DevInfo* info) {
+    const int b = int(blockIdx.x);
+    if (b < wide_blocks)
+        fill_wide(n, b * kBlock + int(threadIdx.x), wide_blocks * kBlock, left, right, pre_internal, pre_leaf, nodes,
+                  wide, wide_leaf, info);
     else
-        LUX_LAUNCH("lbvh_pair_layout", k_zero_u32, 1, 64, 0, s, d.pair_pos, 1);
-    pair_fill(d, s);
+        fill_pairs(n, (b - wide_blocks) * kBlock + int(threadIdx.x), (int(gridDim.x) - wide_blocks) * kBlock, nodes,
+                   pair_pos, pairs, slot_pre, info);
+}
+
+}  // namespace
+
+// The traversal copies of the node array (build and refit).
+void fill_copies(BvhDev& d, hipStream_t s) {
+    if (d.n <= 0) return;
+    const int wide_blocks = d.n > 1 ? min(4096, div_up(d.n - 1, kBlock)) : 0;
+    const int pair_blocks = max(1, min(2048, div_up(2 * d.n - 1, kBlock)));
+    LUX_LAUNCH("lbvh_copies", k_copies, wide_blocks + pair_blocks, kBlock, 0, s, d.n, wide_blocks,
+               (const uint32_t*)d.left, (const uint32_t*)d.right, (const int32_t*)d.pre_internal,
+               (const int32_t*)d.pre_leaf, (const lux_bvh_node*)d.nodes, d.wide, d.wide_leaf,
+               (const uint32_t*)d.pair_pos, d.pairs, d.slot_pre, d.info);
 }
 
 void raysort_release(RaySortDev& r) {
@@ -1124,6 +1230,8 @@ void bvh_allocate(BvhDev& d, int n) {
     d.pairs = dalloc<lux_bvh_node>(2 * size_t(cap));
     d.pair_pos = dalloc<uint32_t>(2 * size_t(cap));
     d.slot_pre = dalloc<uint32_t>(2 * size_t(cap));
+    d.wide = dalloc<WideNode>(cap);
+    d.wide_leaf = dalloc<int32_t>(4 * size_t(cap));
     // One-time clears at allocation: look-back words (epoch 0 is never used),
     // tickets, info, frontier counts.
     hip_check(hipMemset(d.status, 0, sizeof(uint64_t) * d.status_words), "hipMemset status");
@@ -1134,10 +1242,19 @@ void bvh_allocate(BvhDev& d, int n) {
 }
 
 namespace {
+// Boxes above the leaf blocks and, in a build (kLayout), the pair positions.
+template <bool kLayout>
 void top_boxes(BvhDev& d, hipStream_t s) {
-    if (d.n <= kLocalLeaves) return;  // one leaf block: the root is local
-    LUX_LAUNCH("lbvh_top_boxes", k_top_boxes, max(1, min(2048, div_up(d.n - 1, kBlock))), kBlock, 0, s, d.n,
-               (const uint32_t*)d.first, (const uint32_t*)d.last, (const int32_t*)d.pre_internal,
+    if (d.n <= kLocalLeaves) {  // one leaf block: the root is local
+        if (kLayout)
+            LUX_LAUNCH("lbvh_pair_layout", k_pair_layout, max(1, div_up(d.n - 1, kBlock)), kBlock, 0, s, d.n,
+                       (const uint32_t*)d.left, (const uint32_t*)d.last, (const int32_t*)d.pre_internal, d.pair_pos,
+                       d.info);
+        return;
+    }
+    LUX_LAUNCH("lbvh_top_boxes", k_top_boxes<kLayout>, max(1, min(2048, div_up(d.n - 1, kBlock))), kBlock, 0, s, d.n,
+               (const uint32_t*)d.first, (const uint32_t*)d.last, (const uint32_t*)d.left, d.pair_pos,
+               (const int32_t*)d.pre_internal,
                (const lux_aabb*)d.edge_boxes, (const lux_aabb*)d.block_boxes, d.nodes, d.info);
 }
 }  // namespace
@@ -1155,7 +1272,8 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
                    (const lux_triangle*)nullptr, (const int32_t*)d.ids, d.boxes, 0, d.nodes, d.pre_leaf,
                    d.keys[0], d.vals[0], d.info, 1);
         // root box from the one leaf (the reduction result is identical)
-        pair_build(d, s);
+        top_boxes<true>(d, s);
+        fill_copies(d, s);
         return;
     }
     int mh_blocks = max(1, min(1024, div_up(n, kBlock * 16)));
@@ -1182,8 +1300,8 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
                (const uint32_t*)d.parent, (const uint32_t*)d.leaf_parent, (const uint32_t*)d.first,
                (const uint32_t*)d.last, (const uint32_t*)d.rtop_int, (const uint32_t*)d.rtop_leaf, d.nodes,
                d.pre_internal, d.pre_leaf, d.edge_boxes, d.block_boxes, d.info);
-    top_boxes(d, s);
-    pair_build(d, s);
+    top_boxes<true>(d, s);
+    fill_copies(d, s);
 }
 
 namespace {
@@ -1194,7 +1312,7 @@ void refit_launch(BvhDev& d, const lux_aabb* in_boxes, const lux_triangle* tris,
     if (n == 1) {
         LUX_LAUNCH("lbvh_single_leaf", k_single_leaf, 1, 1, 0, s, in_boxes, tris, (const int32_t*)d.ids, d.boxes,
                    wb, d.nodes, d.pre_leaf, d.keys[0], d.vals[0], d.info, 0);
-        pair_fill(d, s);
+        fill_copies(d, s);
         return;
     }
     LUX_LAUNCH(kMode == 2 ? "lbvh_local_tris" : "lbvh_local_boxes", k_local<kMode>, div_up(n, kLocalLeaves),
@@ -1202,8 +1320,8 @@ void refit_launch(BvhDev& d, const lux_aabb* in_boxes, const lux_triangle* tris,
                wb, (const uint32_t*)d.parent, (const uint32_t*)d.leaf_parent, (const uint32_t*)d.first,
                (const uint32_t*)d.last, (const uint32_t*)d.rtop_int, (const uint32_t*)d.rtop_leaf, d.nodes,
                d.pre_internal, d.pre_leaf, d.edge_boxes, d.block_boxes, d.info);
-    top_boxes(d, s);
-    pair_fill(d, s);
+    top_boxes<false>(d, s);
+    fill_copies(d, s);
 }
 }  // namespace
 

@@ -1,9 +1,9 @@
 // query.hip -- closest-hit, any-hit and AABB-overlap queries over the
 // right-first preorder stackless LBVH. Closest and any hit take the
-// near-child-first walk of ordered.hpp, which returns what the preorder walk
-// below returns; rays whose ordered stack overflows take the preorder walk.
+// near-child-first walk over four-child records (wide.hpp), which returns what
+// the preorder walk below returns; rays that it cannot settle take that walk.
 //
-// Walk rule (src/bvh/bvh_device.cuh:59-87): test node i; on a miss or after a
+// Preorder walk rule (src/bvh/bvh_device.cuh:59-87): test node i; on a miss or after a
 // leaf jump to nodes[i].escape, on an internal hit step to i+1. With the nodes in
 // right-first preorder this visits nodes in the pop order of the host stack
 // traversal (src/bvh/cpu_bvh_traversal.h:37-78), so the shrinking t_max and the
@@ -14,16 +14,15 @@
 #include <algorithm>
 
 #include "lux_runtime.hpp"
-#include "ordered.hpp"
+#include "wide.hpp"
 
 namespace lux {
 namespace {
 
-// 64 threads (one wave) per block for the ray queries: with the gathered
-// near-child-first walks the microbench step measured 822 Mrays/s at 64
-// against 802 at 128 and 791 at 256 (a workgroup's resources are freed only
-// when its last wave ends, so a finished wave's slot waits for its siblings;
-// the LDS stack is 4 KiB per block at 64).
+// 64 threads (one wave) per block for the ray queries: a workgroup's resources
+// are freed only when its last wave ends, so a finished wave's slot would wait
+// for its siblings (the gathered two-child walks measured 822 Mrays/s at 64, 802
+// at 128 and 791 at 256). The LDS stack is 5 KiB per block.
 constexpr int kBlock = 64;
 // The plain copy: 128-thread blocks, at most 4096 of them (4.8 TB/s on 1 GiB;
 // other shapes from 2048 to 16384 blocks of 256 or 512 threads measured
@@ -52,37 +51,36 @@ __device__ __forceinline__ void load_tri(const lux_triangle* tris, int i, f3& v0
     v2 = make3(p[6], p[7], p[8]);
 }
 
-// Right-first walk over the sibling-pair copy of the node array (`nodes` =
-// BvhDev::pairs, node_count = its slot count): the same node visits in the
-// same order as the preorder walk, with a node's siblings on one cache line.
+// The tree as the ray kernels read it: the right-first preorder node array and
+// the four-child records over it (wide.hpp).
+struct RayTree {
+    const lux_bvh_node* nodes;
+    const WideNode* wide;
+    const int32_t* wide_leaf;
+    int node_count;    // 2 n - 1
+    uint32_t records;  // n - 1, or 0: the preorder walk only
+};
+
+// Right-first preorder walk: the rays that the wide walk hands back, one-leaf
+// trees and trees beyond 32-bit record offsets.
 // kAny = false: closest hit; kAny = true: stop at the first accepted triangle.
 // visits/tests count node loads and triangle tests (only read by the stats kernel).
-template <bool kAny, int kMode, bool kOffset32>
-__device__ __forceinline__ int walk_impl(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                         const lux_triangle* __restrict__ tris, int tri_count, const RayIn& ray,
-                                         const SlabRay& sr, float& t_best, DevInfo* info, uint32_t& visits,
-                                         uint32_t& tests) {
-    // canonical from the start, so the loop's min/max need no per-step canonicalise
+template <bool kAny>
+__device__ __forceinline__ int walk_preorder(const lux_bvh_node* __restrict__ nodes, int node_count,
+                                          const lux_triangle* __restrict__ tris, int tri_count, const RayIn& ray,
+                                          float& t_best, DevInfo* info, uint32_t& visits, uint32_t& tests) {
+    const SlabRay sr = make_slab_ray(ray.o, ray.d, ray.t_min);
     float t_max = __builtin_canonicalizef(ray.t_max);
     int best = -1;
-    uint32_t k = 0;
-    const uint32_t nc = uint32_t(node_count);
-    int guard = node_count + 1;  // a walk visits each node at most once
-    bool bad_prim = false;
-    // The rare checks (leaf id range, step guard) are folded into lane flags and
-    // reported after the loop, keeping the loop body to one branch (the leaf's
-    // triangle test).
-    while (k < nc && --guard > 0) {
+    int k = 0;
+    bool bad_prim = false, bad_order = false;
+    while (uint32_t(k) < uint32_t(node_count)) {
         float4 a, b;
-        if (kOffset32)
-            load_node32(nodes, k, a, b);
-        else
-            load_node(nodes, int(k), a, b);
+        load_node(nodes, k, a, b);
         ++visits;
         const int prim = __float_as_int(b.z);
-        const bool pass = slab_pass<kMode>(sr, t_max, a.x, a.y, a.z, a.w, b.x, b.y);
-        // internal hit: the right child's slot; otherwise the escape
-        uint32_t next = (pass && prim < 0) ? uint32_t(~prim) : __float_as_uint(b.w);
+        const bool pass = slab_hit(sr, t_max, a.x, a.y, a.z, a.w, b.x, b.y);
+        int next = (pass && prim < 0) ? k + 1 : __float_as_int(b.w);
         bad_prim |= pass && prim >= tri_count;
         if (pass && prim >= 0 && prim < tri_count) {
             f3 v0, v1, v2;
@@ -92,287 +90,234 @@ __device__ __forceinline__ int walk_impl(const lux_bvh_node* __restrict__ nodes,
             if (tri_hit(ray.o, ray.d, ray.t_min, t_max, v0, v1, v2, t, u, v)) {
                 best = prim;
                 t_max = t;
-                if (kAny) next = 0xffffffffu;  // done
+                if (kAny) next = -1;  // done
             }
+        }
+        if (next >= 0 && next <= k) {  // preorder positions only grow
+            bad_order = true;
+            break;
         }
         k = next;
     }
     if (bad_prim) set_error(info, kErrPrimRange);
-    if (guard <= 0 && k < nc) set_error(info, kErrWalkOrder);
+    if (bad_order) set_error(info, kErrWalkOrder);
     t_best = t_max;
     return best;
 }
 
-// Any hit by the preorder walk with the triangle tests gathered across the wave.
-// A lane whose walk reaches a leaf box that passes holds that leaf and stops;
-// the wave runs the triangle tests of all held leaves together once at least
-// 1/kDeferDiv of its still-working lanes hold one (or none can step on). Each
-// lane performs the same operations in the same order as walk_impl<true>, so
-// the answer is the same; only the interleaving across lanes changes. Without
-// it, most steps of the wave carry the ~60-instruction triangle test for the
-// one or two lanes that need it. On 2^22 random rays over 2^20 triangles
-// (octant-specialised slab test): kDeferDiv 2 / 4 / 8: 4.78 / 4.67 / 4.70 ms;
-// testing each leaf at once (the plain walk), 4.93 ms before the octant
-// specialisation, against 4.87 ms with kDeferDiv 4.
-constexpr int kDeferDiv = 4;
-
-template <int kMode>
-__device__ __forceinline__ int walk_any_deferred(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                                 const lux_triangle* __restrict__ tris, int tri_count,
-                                                 const RayIn& ray, const SlabRay& sr, float& t_best,
-                                                 DevInfo* info, uint32_t& visits, uint32_t& tests) {
-    const float t_max = __builtin_canonicalizef(ray.t_max);
-    t_best = t_max;
-    const uint32_t nc = uint32_t(node_count);
-    uint32_t k = 0;
-    int held = -1, found = -1;
-    int guard = node_count;  // a walk visits each node at most once
-    bool bad_prim = false;
-    for (;;) {
-        // (& rather than &&: one mask, no nested branches)
-        if ((held < 0) & (k < nc) & (guard > 0)) {
-            --guard;
-            float4 a, b;
-            load_node32(nodes, k, a, b);
-            ++visits;
-            const int prim = __float_as_int(b.z);
-            const bool pass = slab_pass<kMode>(sr, t_max, a.x, a.y, a.z, a.w, b.x, b.y);
-            held = (pass & (prim >= 0)) ? prim : -1;
-            k = (pass & (prim < 0)) ? uint32_t(~prim) : __float_as_uint(b.w);
-        }
-        const uint64_t want = __ballot(held >= 0);
-        const uint64_t more = __ballot((held < 0) & (k < nc) & (guard > 0));
-        if (!more) {
-            if (!want) break;
-        } else if (__popcll(want) * kDeferDiv < __popcll(want | more)) {
-            continue;
-        }
-        if (held >= 0) {
-            if (held < tri_count) {
-                f3 v0, v1, v2;
-                load_tri(tris, held, v0, v1, v2);
-                ++tests;
-                float t, u, v;
-                if (tri_hit(ray.o, ray.d, ray.t_min, t_max, v0, v1, v2, t, u, v)) {
-                    found = held;
-                    t_best = t;
-                    k = 0xffffffffu;  // done
-                }
-            } else {
-                bad_prim = true;  // skipped, as the preorder walk skips it
-            }
-            held = -1;
-        }
-    }
-    if (bad_prim) set_error(info, kErrPrimRange);
-    if (guard <= 0 && k < nc) set_error(info, kErrWalkOrder);
-    return found;
-}
-
-// Any hit by the near-child-first walk with gathered triangle tests. With
-// t_max fixed, a box passes or not whatever the visit order, so the walk meets
-// the same boxes and triangles as the preorder walk until one triangle is hit;
-// near child first meets one sooner. A lane whose stack overflows takes the
-// preorder walk.
-template <int kMode>
-__device__ __forceinline__ int walk_any_ordered(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                                const lux_triangle* __restrict__ tris, int tri_count,
-                                                const RayIn& ray, const SlabRay& sr, float& t_best, uint32_t* stack,
-                                                DevInfo* info, uint32_t& visits, uint32_t& tests) {
-    const float t_max = __builtin_canonicalizef(ray.t_max);
-    OrderedBest ob(t_max);  // t_cull stays t_max: no hit is taken before the walk ends
-    int found = -1;
-    float t_found = t_max;
-    bool bad = false, bad_prim = false;
-    auto leaf = [&](uint32_t, int prim, float) {
-        if (prim >= tri_count) {
-            bad_prim = true;
-            return false;
-        }
-        f3 v0, v1, v2;
-        load_tri(tris, prim, v0, v1, v2);
-        ++tests;
-        float t, u, v;
-        if (tri_hit(ray.o, ray.d, ray.t_min, t_max, v0, v1, v2, t, u, v)) {
-            found = prim;
-            t_found = t;
-            return true;
-        }
-        return false;
-    };
-    const bool done = ordered_walk_gathered(SlabMode<kMode>{}, nodes, uint32_t(node_count), sr, ob, stack, kBlock,
-                                            visits, bad, leaf);
-    if (bad_prim) set_error(info, kErrPrimRange);
-    if (bad) set_error(info, kErrWalkOrder);
-    if (!done) return walk_any_deferred<kMode>(nodes, node_count, tris, tri_count, ray, sr, t_best, info, visits, tests);
-    t_best = t_found;
-    return found;
-}
-
-template <bool kAny>
-__device__ __forceinline__ int walk(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                    const lux_triangle* __restrict__ tris, int tri_count, const RayIn& ray,
-                                    float& t_best, DevInfo* info, uint32_t& visits, uint32_t& tests) {
-    const SlabRay sr = make_slab_ray(ray.o, ray.d, ray.t_min);
-    if (uint32_t(node_count) > kOffset32Nodes)
-        return walk_impl<kAny, kSlabParallel, false>(nodes, node_count, tris, tri_count, ray, sr, t_best, info, visits,
-                                                     tests);
-    return with_slab_mode(sr, [&](auto mode) {
-        constexpr int m = decltype(mode)::value;
-        if constexpr (kAny)
-            return walk_any_deferred<m>(nodes, node_count, tris, tri_count, ray, sr, t_best, info, visits, tests);
-        else
-            return walk_impl<false, m, true>(nodes, node_count, tris, tri_count, ray, sr, t_best, info, visits, tests);
-    });
-}
-
-// Closest hit by the near-child-first walk (ordered.hpp), equal to walk<false>.
-// stack: this lane's LDS stack (entries kBlock words apart). A ray whose stack
-// overflows, or whose walk the check of ordered.hpp flags, is walked again in
-// right-first preorder.
-template <int kMode>
-__device__ __forceinline__ int walk_ordered(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                            const uint32_t* __restrict__ slot_pre,
-                                            const lux_triangle* __restrict__ tris, int tri_count, const RayIn& ray,
-                                            const SlabRay& sr, float& t_best, uint32_t* stack, DevInfo* info,
-                                            uint32_t& visits, uint32_t& tests) {
-    OrderedBest ob(__builtin_canonicalizef(ray.t_max));
+// What one lane's walk of a ray found: a hit's primitive (-1: none), its leaf
+// child (4 * record + child) and distance (a miss: the ray's t_max), and whether
+// the ray is the preorder walk's to decide.
+struct Found {
     int best = -1;
-    uint32_t best_slot = 0;
+    uint32_t at = 0;
+    float t = 0;
+    bool failed = false;
+};
+
+// A lane's walk (wide.hpp) of the boxes met in [lo, hi] of its ray; sr.t_min =
+// lo. `group` lanes in a row (a power of two) walk one ray between them and share
+// the nearest hit (any hit: that there is one); with `skip` a lane only listens.
+template <bool kAny>
+__device__ __forceinline__ Found walk_part(const RayTree& tree, const lux_triangle* __restrict__ tris, int tri_count,
+                                           const RayIn& ray, const SlabRay& sr, float hi, int group, bool skip, uint32_t* stack,
+                                           DevInfo* info, uint32_t& visits, uint32_t& tests) {
+    Found f;
+    f.t = __builtin_canonicalizef(ray.t_max);
+    float t_cull = wide_bound(hi);
     bool bad = false, bad_prim = false;
-    auto leaf = [&](uint32_t slot, int prim, float tn) {
-        if (prim >= tri_count) {
-            bad_prim = true;
+    auto leaf = [&](uint32_t at, uint32_t ref) {
+        const uint32_t prim = ref & kIndexMask;
+        if (prim >= uint32_t(tri_count)) {
+            bad_prim |= ref != kWideEmpty;
             return false;
         }
         f3 v0, v1, v2;
-        load_tri(tris, prim, v0, v1, v2);
+        load_tri(tris, int(prim), v0, v1, v2);
         ++tests;
         float t, u, v;
-        if (tri_uvt(ray.o, ray.d, v0, v1, v2, t, u, v) && t > ray.t_min) {
-            ob.note(t, tn);
-            if (t < ob.t_max || (best >= 0 && t == ob.t_max && slot_pre[slot] < slot_pre[best_slot])) {
-                ob.take(t);
-                best = prim;
-                best_slot = slot;
-            }
+        if (!tri_uvt(ray.o, ray.d, v0, v1, v2, t, u, v) || !(t > ray.t_min)) return false;
+        if (t < f.t || (!kAny && f.best >= 0 && t == f.t && tree.wide_leaf[at] < tree.wide_leaf[f.at])) {
+            f.best = int(prim);
+            f.at = at;
+            if (kAny) return true;
+            f.t = t;
+            t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
         }
         return false;
     };
-    const bool done = ordered_walk_gathered(SlabMode<kMode>{}, nodes, uint32_t(node_count), sr, ob, stack, kBlock,
-                                            visits, bad, leaf);
+    auto share = [&]() {
+        if (group == 1) return false;
+        if (kAny) {
+            int any = f.best >= 0;
+            for (int off = 1; off < group; off <<= 1) any |= __shfl_xor(any, off, 64);
+            return any != 0;
+        }
+        float t = f.best >= 0 ? f.t : INFINITY;
+        for (int off = 1; off < group; off <<= 1) t = fminf(t, __shfl_xor(t, off, 64));
+        t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
+        return false;
+    };
+    const bool done =
+        wave_any_parallel(sr)
+            ? wide_walk<true>(tree.wide, tree.records, sr, t_cull, skip, stack, kBlock, visits, bad, leaf, share)
+            : wide_walk<false>(tree.wide, tree.records, sr, t_cull, skip, stack, kBlock, visits, bad, leaf, share);
     if (bad_prim) set_error(info, kErrPrimRange);
     if (bad) set_error(info, kErrWalkOrder);
-    if (!done || (best >= 0 && ob.ambiguous()))
-        return walk_impl<false, kMode, true>(nodes, node_count, tris, tri_count, ray, sr, t_best, info, visits,
-                                             tests);
-    t_best = ob.t_max;
-    return best;
+    f.failed = !done;
+    return f;
 }
 
-// One ray: closest hit by the near-child-first walk when `stack` is given,
-// otherwise (and for any hit) the preorder walk. Counters: nodes loaded and
-// triangle tests.
+// One ray on one lane. A ray the wide walk cannot settle is walked again in
+// preorder. With t_max fixed, whether a leaf's box passes does not depend on the
+// visit order, so an any-hit walk may end at any triangle hit in a leaf whose own
+// box passes; near child first meets one soon.
 template <bool kAny>
-__device__ __forceinline__ int trace_one(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                         const lux_triangle* __restrict__ tris, int tri_count, const RayIn& r,
-                                         float& t, DevInfo* info, uint32_t& visits, uint32_t& tests,
-                                         const uint32_t* __restrict__ slot_pre = nullptr, uint32_t* stack = nullptr) {
-    if (!kAny && stack && uint32_t(node_count) <= kOffset32Nodes && node_count > 1) {
-        const SlabRay sr = make_slab_ray(r.o, r.d, r.t_min);
-        return with_slab_mode(sr, [&](auto mode) {
-            return walk_ordered<decltype(mode)::value>(nodes, node_count, slot_pre, tris, tri_count, r, sr, t, stack,
-                                                       info, visits, tests);
-        });
+__device__ __forceinline__ int trace_one(const RayTree& tree, const lux_triangle* __restrict__ tris, int tri_count,
+                                         const RayIn& ray, float& t_best, uint32_t* stack, DevInfo* info,
+                                         uint32_t& visits, uint32_t& tests) {
+    if (tree.records != 0 && wide_takes(ray.d)) {
+        const SlabRay sr = make_slab_ray(ray.o, ray.d, ray.t_min);
+        const Found f =
+            walk_part<kAny>(tree, tris, tri_count, ray, sr, ray.t_max, 1, false, stack, info, visits, tests);
+        if (!f.failed && (f.best < 0 || wide_settled(tree.nodes, tree.wide_leaf[f.at], sr, f.t))) {
+            t_best = f.t;
+            return f.best;
+        }
     }
-    return walk<kAny>(nodes, node_count, tris, tri_count, r, t, info, visits, tests);
+    return walk_preorder<kAny>(tree.nodes, tree.node_count, tris, tri_count, ray, t_best, info, visits, tests);
 }
 
-// One ray's any hit: the near-child-first walk on this lane's LDS stack when
-// the array allows it, otherwise the preorder walk.
-__device__ __forceinline__ int trace_any_one(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                             const lux_triangle* __restrict__ tris, int tri_count, const RayIn& r,
-                                             float& t, DevInfo* info, uint32_t& visits, uint32_t& tests,
-                                             uint32_t* stack) {
-    if (stack && uint32_t(node_count) <= kOffset32Nodes && node_count > 1) {
-        const SlabRay sr = make_slab_ray(r.o, r.d, r.t_min);
-        return with_slab_mode(sr, [&](auto mode) {
-            return walk_any_ordered<decltype(mode)::value>(nodes, node_count, tris, tri_count, r, sr, t, stack, info,
-                                                           visits, tests);
-        });
+template <bool kAny>
+__device__ __forceinline__ void store_result(void* __restrict__ out, int ray, int id, float t) {
+    if (kAny) {
+        static_cast<uint8_t*>(out)[ray] = id >= 0 ? 1 : 0;
+    } else {
+        lux_hit h;
+        h.primitive_id = id;
+        h.t = id >= 0 ? t : INFINITY;
+        static_cast<lux_hit*>(out)[ray] = h;
     }
-    return trace_one<true>(nodes, node_count, tris, tri_count, r, t, info, visits, tests);
 }
 
-// Closest hit, one ray per lane in `order` (a permutation of [0, n), or input
-// order); the hit lands at the ray's own index.
-template <bool kOrdered>
-__global__ __launch_bounds__(kBlock) void k_trace_closest(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                                          const uint32_t* __restrict__ slot_pre,
-                                                          const lux_triangle* __restrict__ tris, int tri_count,
-                                                          const lux_ray* __restrict__ rays, int n,
-                                                          const uint32_t* __restrict__ order,
-                                                          lux_hit* __restrict__ hits, DevInfo* info) {
-    __shared__ uint32_t stack[kOrdered ? kOrderedStack * kBlock : 1];
+// One ray per lane in `order` (a permutation of [0, n), or input order); the
+// result lands at the ray's own index: a lux_hit, or one byte (kAny).
+// Bound by VALU issue (154 instructions a step, 26 % of the lanes busy, since a
+// wave lasts as long as its longest walk) with the texture path close behind (data
+// return 88 % busy). On 2^22 random rays through 2^20 random triangles: 4.41 ms
+// over sibling pairs (386 steps for a wave's longest ray), 3.2 ms over records
+// (192 steps). 8 waves a SIMD (64 VGPRs, 12 bytes spilled) take 3.24 ms with the
+// sort, 70 VGPRs at 7 waves 3.39 ms. Lanes refilled with new rays as theirs end
+// (from runs of 128 to 512 rays a wave, or from one pool per XCD) took 3.5 to
+// 5.2 ms: they keep more lanes busy but the wave's rays drift apart in the tree,
+// and the loads miss L1. Stack entries that carry their box's entry, to drop them
+// when a nearer hit is held, need 6 KiB a wave and took 4.3 ms.
+template <bool kAny>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_trace(
+    RayTree tree, const lux_triangle* __restrict__ tris, int tri_count, const lux_ray* __restrict__ rays, int n,
+    const uint32_t* __restrict__ order, void* __restrict__ out, DevInfo* info) {
+    __shared__ uint32_t stack[kWideStack * kBlock];
     const int i = int(xcd_block()) * kBlock + threadIdx.x;
     if (i >= n) return;
-    const int ray = order ? int(order[i]) : i;  // order is a permutation of [0, n)
-    if (uint32_t(ray) >= uint32_t(n)) {          // only if the sort itself reported an error
+    const int ray = order ? int(order[i]) : i;
+    if (uint32_t(ray) >= uint32_t(n)) {  // only if the sort itself reported an error
         set_error(info, kErrSpinLimit);
         return;
     }
-    RayIn r = load_ray(rays, ray);
+    const RayIn r = load_ray(rays, ray);
     float t;
     uint32_t visits = 0, tests = 0;
-    const int id = trace_one<false>(nodes, node_count, tris, tri_count, r, t, info, visits, tests, slot_pre,
-                                    kOrdered ? stack + threadIdx.x : nullptr);
-    lux_hit h;
-    h.primitive_id = id;
-    h.t = id >= 0 ? t : INFINITY;
-    hits[ray] = h;
+    const int id = trace_one<kAny>(tree, tris, tri_count, r, t, stack + threadIdx.x, info, visits, tests);
+    store_result<kAny>(out, ray, id, t);
 }
 
-__global__ __launch_bounds__(kBlock) void k_trace_any(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                                      const lux_triangle* __restrict__ tris, int tri_count,
-                                                      const lux_ray* __restrict__ rays, int n,
-                                                      const uint32_t* __restrict__ order,
-                                                      uint8_t* __restrict__ occluded, DevInfo* info) {
-    __shared__ uint32_t stack[kOrderedStack * kBlock];
-    const int i = int(xcd_block()) * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const int ray = order ? int(order[i]) : i;  // order is a permutation of [0, n)
-    if (uint32_t(ray) >= uint32_t(n)) {          // only if the sort itself reported an error
+// Few rays: `group` lanes (a power of two up to 64) walk one ray, each a part of
+// the interval in which it meets the root box. A call that leaves most of the
+// chip idle lasts as long as its longest walk, a chain of dependent loads; parts
+// cut the chain (2^20 random triangles, 2^14 random rays: 330 records for the
+// longest ray, 148 in 4 parts, 87 in 8) for more records in all (50, 130 and 194
+// a ray). A box met by the ray in [t_min, t_max] is met in some part, so every
+// triangle the whole walk tests is tested by some lane; the hit is the smallest
+// (t, preorder position) over the lanes, as it is over one lane's walk.
+template <bool kAny>
+__global__ __launch_bounds__(kBlock) void k_trace_parts(RayTree tree, const lux_triangle* __restrict__ tris,
+                                                        int tri_count, const lux_ray* __restrict__ rays, int n,
+                                                        const uint32_t* __restrict__ order, int group,
+                                                        void* __restrict__ out, DevInfo* info) {
+    __shared__ uint32_t stack[kWideStack * kBlock];
+    const int i = (int(xcd_block()) * kBlock + int(threadIdx.x)) / group;
+    if (i >= n) return;  // whole groups
+    const int part = int(threadIdx.x) & (group - 1);
+    const int ray = order ? int(order[i]) : i;
+    if (uint32_t(ray) >= uint32_t(n)) {
         set_error(info, kErrSpinLimit);
         return;
     }
-    RayIn r = load_ray(rays, ray);
-    float t;
+    const RayIn r = load_ray(rays, ray);
     uint32_t visits = 0, tests = 0;
-    const int id = trace_any_one(nodes, node_count, tris, tri_count, r, t, info, visits, tests, stack + threadIdx.x);
-    occluded[ray] = id >= 0 ? 1 : 0;
+    int id = -1;
+    float t = 0;
+    bool settled = false;
+    if (wide_takes(r.d)) {  // the same on every lane of the group
+        SlabRay sr = make_slab_ray(r.o, r.d, r.t_min);
+        // the root box, with a margin; an interval that is empty or not finite
+        // leaves the whole ray to the first lane
+        float4 a, b;
+        load_node(tree.nodes, 0, a, b);
+        float enter;
+        (void)slab_near<true>(sr, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, enter);
+        const float fx = (sr.neg_x ? a.x : a.w) - r.o.x, fy = (sr.neg_y ? a.y : b.x) - r.o.y,
+                    fz = (sr.neg_z ? a.z : b.y) - r.o.z;
+        float leave = r.t_max;
+        if (!sr.par_x) leave = fminf(leave, fx * sr.inv.x);
+        if (!sr.par_y) leave = fminf(leave, fy * sr.inv.y);
+        if (!sr.par_z) leave = fminf(leave, fz * sr.inv.z);
+        const float step = (leave - enter) / float(group);
+        const bool cut = step > 0.0f && step < 1e30f;
+        const float lo = enter + step * float(part), hi = enter + step * float(part + 1);
+        if (cut && part != 0) sr.t_min = lo;
+        const Found f = walk_part<kAny>(tree, tris, tri_count, r, sr, cut && part + 1 < group ? hi : r.t_max, group,
+                                        !cut && part != 0, stack + threadIdx.x, info, visits, tests);
+        sr.t_min = r.t_min;
+        // the smallest (t, position) of the group, on every lane
+        int pos = f.best >= 0 ? tree.wide_leaf[f.at] : INT32_MAX;
+        float bt = f.best >= 0 ? f.t : INFINITY;
+        int bid = f.best, fail = f.failed;
+        for (int off = 1; off < group; off <<= 1) {
+            const float ot = __shfl_xor(bt, off, 64);
+            const int op = __shfl_xor(pos, off, 64), oid = __shfl_xor(bid, off, 64);
+            fail |= __shfl_xor(fail, off, 64);
+            if (oid >= 0 && (bid < 0 || (kAny ? op < pos : (ot < bt || (ot == bt && op < pos))))) {
+                bt = ot;
+                pos = op;
+                bid = oid;
+            }
+        }
+        id = bid;
+        t = bt;
+        settled = !fail && (bid < 0 || wide_settled(tree.nodes, pos, sr, kAny ? r.t_max : bt));
+    }
+    if (part != 0) return;
+    if (!settled) id = walk_preorder<kAny>(tree.nodes, tree.node_count, tris, tri_count, r, t, info, visits, tests);
+    store_result<kAny>(out, ray, id, t);
 }
 
-// The walks of the handle, counting per ray the 32-byte nodes loaded and the
-// triangle tests (summed per wave, one atomic per wave): stats[0..2]
-// closest-hit {nodes, 0, tests}, stats[3..5] any-hit {nodes, 0, tests}. Rays
-// the near-child-first walk hands to the preorder walk count both walks. Used
-// to state the bytes a traversal actually touches.
-template <bool kOrdered>
-__global__ __launch_bounds__(kBlock) void k_trace_stats(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                                        const uint32_t* __restrict__ slot_pre,
-                                                        const lux_triangle* __restrict__ tris, int tri_count,
-                                                        const lux_ray* __restrict__ rays, int n,
+// The walks of the handle, counting per ray the 32-byte node units loaded (two
+// a record) and the triangle tests (summed per wave, one atomic per wave):
+// stats[0..2] closest-hit {nodes, 0, tests}, stats[3..5] any-hit {nodes, 0,
+// tests}. Rays handed to the preorder walk count both walks. Used to state the
+// bytes a traversal actually touches.
+__global__ __launch_bounds__(kBlock) void k_trace_stats(RayTree tree, const lux_triangle* __restrict__ tris,
+                                                        int tri_count, const lux_ray* __restrict__ rays, int n,
                                                         unsigned long long* stats, DevInfo* info) {
-    __shared__ uint32_t stack[kOrdered ? kOrderedStack * kBlock : 1];
+    __shared__ uint32_t stack[kWideStack * kBlock];
     int i = blockIdx.x * kBlock + threadIdx.x;
     uint32_t v0 = 0, t0 = 0, v1 = 0, t1 = 0;
     if (i < n) {
         RayIn r = load_ray(rays, i);
         float t;
-        trace_one<false>(nodes, node_count, tris, tri_count, r, t, info, v0, t0, slot_pre,
-                         kOrdered ? stack + threadIdx.x : nullptr);
-        trace_any_one(nodes, node_count, tris, tri_count, r, t, info, v1, t1,
-                      kOrdered ? stack + threadIdx.x : nullptr);
+        trace_one<false>(tree, tris, tri_count, r, t, stack + threadIdx.x, info, v0, t0);
+        trace_one<true>(tree, tris, tri_count, r, t, stack + threadIdx.x, info, v1, t1);
     }
     unsigned long long c[6] = {v0, 0, t0, v1, 0, t1};
 #pragma unroll
@@ -623,38 +568,62 @@ const uint32_t* closest_order(RaySortDev& r, bool sort, const BvhDev& d, const l
     return maybe_order(d, sort ? &r : nullptr, rays, n, s);
 }
 
+namespace {
+RayTree ray_tree(const BvhDev& d) {
+    RayTree t;
+    t.nodes = d.nodes;
+    t.wide = d.wide;
+    t.wide_leaf = d.wide_leaf;
+    t.node_count = d.n > 0 ? 2 * d.n - 1 : 0;
+    t.records = (d.n > 1 && uint32_t(d.n) <= kMaxWideRecords) ? uint32_t(d.n - 1) : 0u;
+    return t;
+}
+}  // namespace
+
+namespace {
+// Lanes per ray of a call of n rays (k_trace_parts): where the calls that leave
+// the chip idle end. Closest hit, 1 / 4 / 8 / 16 lanes: 2^14 rays in 2^20 random
+// triangles (with their build) 884 / 648 / 590 / 569 us, 2^15 395 / 165 / 123 /
+// 135, 2^16 in 2^18 (with the refit) 431 / 260 / 257 / 283; 2^17 in 500 000
+// 382 / 277 / 285, on a sphere mesh 133 / 119 / 122; at 2^18 one lane is the
+// best for the soup (422 / 455) and within 6 % on the sphere.
+int lanes_per_ray(const RayTree& tree, int n) {
+    if (tree.records == 0) return 1;
+    return n <= (1 << 14) ? 16 : n <= (1 << 16) ? 8 : n <= (1 << 17) ? 4 : 1;
+}
+
+template <bool kAny>
+void launch_trace(const char* name, const BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
+                  const lux_ray* rays, int n, void* out, hipStream_t s) {
+    const RayTree tree = ray_tree(d);
+    const int group = lanes_per_ray(tree, n);
+    if (group > 1)
+        LUX_LAUNCH(name, k_trace_parts<kAny>, div_up(int64_t(n) * group, kBlock), kBlock, 0, s, tree, tris, tri_count,
+                   rays, n, order, group, out, d.info);
+    else
+        LUX_LAUNCH(name, k_trace<kAny>, div_up(n, kBlock), kBlock, 0, s, tree, tris, tri_count, rays, n, order, out,
+                   d.info);
+}
+}  // namespace
+
 void trace_closest(const BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
                    const lux_ray* rays, int n, lux_hit* hits, hipStream_t s) {
     if (n <= 0) return;
-    int node_count = d.n > 1 ? 2 * d.n : (d.n > 0 ? 1 : 0);  // sibling-pair slots
-    // The near-child-first walk touches the nodes near each ray's origin first,
-    // which neighbouring rays share: tracing in ray order (octant, then origin)
-    // measured 5.12 ms against 5.60 ms in input order on 2^22 random rays over
-    // 2^20 triangles, sort included.
-    LUX_LAUNCH("trace_closest", k_trace_closest<true>, div_up(n, kBlock), kBlock, 0, s,
-               (const lux_bvh_node*)d.pairs, node_count, (const uint32_t*)d.slot_pre, tris, tri_count, rays, n,
-               order, hits, d.info);
+    launch_trace<false>("trace_closest", d, order, tris, tri_count, rays, n, hits, s);
 }
 
 void trace_any(const BvhDev& d, RaySortDev* order, const lux_triangle* tris, int tri_count, const lux_ray* rays,
                int n, uint8_t* occluded, hipStream_t s) {
     if (n <= 0) return;
-    int node_count = d.n > 1 ? 2 * d.n : (d.n > 0 ? 1 : 0);  // sibling-pair slots
-    const uint32_t* ord = maybe_order(d, order, rays, n, s);
-    // Any hit walks near child first with its triangle tests gathered across
-    // the wave: 4.52 ms against 4.66 ms for the gathered preorder walk on 2^22
-    // random rays over 2^20 triangles (ungathered, near child first had lost:
-    // 5.84 against 5.40 ms).
-    LUX_LAUNCH("trace_any", k_trace_any, div_up(n, kBlock), kBlock, 0, s, (const lux_bvh_node*)d.pairs, node_count,
-               tris, tri_count, rays, n, ord, occluded, d.info);
+    launch_trace<true>("trace_any", d, maybe_order(d, order, rays, n, s), tris, tri_count, rays, n, occluded, s);
 }
 
 void trace_stats(const BvhDev& d, const lux_triangle* tris, int tri_count, const lux_ray* rays, int n,
                  unsigned long long* d_stats, hipStream_t s) {
     LUX_LAUNCH("trace_stats_zero", k_zero_u64, 1, 64, 0, s, d_stats, 6);
     if (n <= 0 || d.n <= 0) return;
-    LUX_LAUNCH("trace_stats", k_trace_stats<true>, div_up(n, kBlock), kBlock, 0, s, (const lux_bvh_node*)d.pairs,
-               d.n > 1 ? 2 * d.n : 1, (const uint32_t*)d.slot_pre, tris, tri_count, rays, n, d_stats, d.info);
+    LUX_LAUNCH("trace_stats", k_trace_stats, div_up(n, kBlock), kBlock, 0, s, ray_tree(d), tris, tri_count, rays, n,
+               d_stats, d.info);
 }
 
 void copy_device(void* dst, const void* src, size_t bytes, hipStream_t s) {

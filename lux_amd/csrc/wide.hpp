@@ -1,0 +1,283 @@
+// wide.hpp -- four-child traversal records of an LBVH and the near-child-first
+// walk over them, with the hit the right-first preorder walk would return.
+//
+// Record i belongs to internal node i of the radix tree (Karras order; record 0
+// is the root) and holds up to four descendants whose leaf ranges make up that
+// node's: its two children, with the larger internal one (by box area) opened
+// until there are four. Every internal node has its record, so each is made
+// from the node array alone and a walk uses about half of them. A child's box
+// is kept as six bytes in the record's own frame (org + scale * byte, faces
+// moved outwards), so a record is 64 bytes: half the loads of two sibling pairs
+// with 32-byte boxes, and half the dependent steps. In a CPU model (2^20 random
+// triangles, random rays) near-first walks take 50 records (193 boxes) per ray
+// against 100 pairs (200 boxes); the byte boxes account for 2 % of them.
+//
+// Box tests are conservative: a ray that passes a leaf's own box by the
+// reference's slab test (src/core/aabb.cuh:84-109) passes every byte box above
+// it. Per axis the walk forms near = byte * (scale * inv) + (org - o) * inv.
+// With all roundings this is off the true distance by at most 2^-22 of
+// |(org - o) * inv| plus 2^-14 of |scale * inv|; the second part is covered by
+// moving each face outwards by at least 2^-10 of the scale (make_wide), the first
+// by kWideSlack in the far faces' base. An axis the reference treats as parallel
+// (|d| < 1e-12, origin inside the slab or not) compares the origin with the
+// byte faces (kPar, chosen per wave). A record with a face beyond 1e18 or not
+// finite has org = NaN, and every comparison with NaN passes. Rays with a
+// direction component beyond 1e18 (or NaN) take the preorder walk.
+//
+// Equal result. The preorder walk (src/bvh/bvh_device.cuh:59-87) accepts a
+// triangle iff its leaf box passes with entry at most the held t and t < held t,
+// in preorder, so it returns the smallest (t, preorder position) over the
+// triangles whose leaf boxes pass -- as long as no triangle's t lies below its
+// own leaf box's entry (rounded, an entry can lie a few hundred ulps above the
+// Moller-Trumbore t of a hit at a vertex or edge on the face the ray enters).
+// This walk tests every triangle of every leaf whose byte boxes pass up to
+// t_cull = t_max + |t_max| kSoftWindow, without its leaf box, and keeps the
+// smallest (t, preorder position) of all. At the end wide_settled tests the
+// winner's own leaf box the reference's way. If it passes with its entry at
+// most t, the preorder walk returns the same hit: every triangle with a smaller
+// or equal t and a smaller position would have been held here instead, so none
+// exists among the reached, and the preorder walk reaches the winner holding a
+// larger t. Otherwise (a box missed by rounding, an entry above t, a box with a
+// NaN bound) the ray is walked again in preorder. The observed gap between a
+// hit and its leaf box's entry is below 2^-14.7 relative, the window 2^-11.
+//
+// A lane whose stack is full stops and reports overflow; its caller then runs the
+// preorder walk for that ray.
+#pragma once
+
+#include "ordered.hpp"
+
+namespace lux {
+
+// Loaded as four float4: org.xyz scale.x | scale.yz lo.xy | lo.z hi.xyz | ref.
+struct alignas(64) WideNode {
+    float org[3];
+    float scale[3];
+    uint32_t lo[3];  // byte k: child k's lower face
+    uint32_t hi[3];
+    uint32_t ref[4];  // record of an internal child, kLeafBit | primitive id, kWideEmpty
+};
+static_assert(sizeof(WideNode) == 64, "wide record");
+
+constexpr uint32_t kWideEmpty = 0xffffffffu;
+// Records are loaded at base + 32-bit byte offset, so a walk takes trees of at
+// most this many leaves (4 GiB of records).
+constexpr uint32_t kMaxWideRecords = 1u << 26;
+constexpr float kWideSlack = 0x1p-20f;
+
+// Record from up to four children (boxes and refs; `count` of them). Faces are
+// rounded outwards by at least 2^-8 of the scale and org lies at least 2^-10 of
+// it below the lowest face.
+__device__ __forceinline__ void make_wide(WideNode& w, const lux_aabb* box, const uint32_t* ref, int count) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w.ref[k] = k < count ? ref[k] : kWideEmpty;
+    bool finite = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        float lo[4], hi[4], mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            lo[k] = a == 0 ? box[k].p_min.x : (a == 1 ? box[k].p_min.y : box[k].p_min.z);
+            hi[k] = a == 0 ? box[k].p_max.x : (a == 1 ? box[k].p_max.y : box[k].p_max.z);
+            if (k < count) {
+                finite = finite && fabsf(lo[k]) < 1e18f && fabsf(hi[k]) < 1e18f;
+                mn = fminf(mn, fminf(lo[k], hi[k]));
+                mx = fmaxf(mx, fmaxf(lo[k], hi[k]));
+            }
+        }
+        // the float below mn; 1e-30 below a zero or tiny one
+        const float below = fabsf(mn) > 1e-30f ? mn - fabsf(mn) * 0x1.8p-24f : mn - 1e-30f;
+        const float big = fmaxf(fabsf(mn), fabsf(mx));
+        const float s = fmaxf(fmaxf((mx - below) * (1.0f / 253.0f), big * 1e-9f), 1e-20f);
+        const float org = fminf(below, mn - s * 0x1p-10f);
+        uint32_t ql = 0, qh = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float l = floorf((lo[k] - org) / s - 0x1p-8f), h = ceilf((hi[k] - org) / s + 0x1p-8f);
+            const uint32_t bl = k < count ? uint32_t(fminf(fmaxf(l, 0.0f), 255.0f)) : 255u;
+            const uint32_t bh = k < count ? uint32_t(fminf(fmaxf(h, 0.0f), 255.0f)) : 0u;
+            ql |= bl << (8 * k);
+            qh |= bh << (8 * k);
+        }
+        w.org[a] = org;
+        w.scale[a] = s;
+        w.lo[a] = ql;
+        w.hi[a] = qh;
+    }
+    if (!finite) w.org[0] = w.org[1] = w.org[2] = NAN;
+}
+
+__device__ __forceinline__ void store_wide(WideNode* dst, const WideNode& w) {
+    float4* p = reinterpret_cast<float4*>(dst);
+    p[0] = make_float4(w.org[0], w.org[1], w.org[2], w.scale[0]);
+    p[1] = make_float4(w.scale[1], w.scale[2], __uint_as_float(w.lo[0]), __uint_as_float(w.lo[1]));
+    p[2] = make_float4(__uint_as_float(w.lo[2]), __uint_as_float(w.hi[0]), __uint_as_float(w.hi[1]),
+                       __uint_as_float(w.hi[2]));
+    p[3] = make_float4(__uint_as_float(w.ref[0]), __uint_as_float(w.ref[1]), __uint_as_float(w.ref[2]),
+                       __uint_as_float(w.ref[3]));
+}
+
+__device__ __forceinline__ void load_wide(const WideNode* nodes, uint32_t i, float4& a, float4& b, float4& c,
+                                          uint4& r) {
+    const char* p = reinterpret_cast<const char*>(nodes) + (i << 6);
+    const float4* q = reinterpret_cast<const float4*>(p);
+    a = q[0];
+    b = q[1];
+    c = q[2];
+    r = reinterpret_cast<const uint4*>(p)[3];
+}
+
+__device__ __forceinline__ float byte_of(uint32_t w, int k) { return float((w >> (8 * k)) & 0xffu); }
+
+// True when the walk below takes the ray (see above).
+__device__ __forceinline__ bool wide_takes(const f3& d) {
+    return (fabsf(d.x) < 1e18f) & (fabsf(d.y) < 1e18f) & (fabsf(d.z) < 1e18f);
+}
+
+// Where the walk's box entries end for a ray bound t (a ray's t_max).
+__device__ __forceinline__ float wide_bound(float t) { return t + fabsf(t) * kWideSlack; }
+
+// The winner (leaf node at preorder position pos, distance t): true when the
+// preorder walk returns it too (see above). An any-hit query passes the ray's
+// t_max as t: there the leaf box only has to be entered before it.
+__device__ __forceinline__ bool wide_settled(const lux_bvh_node* __restrict__ nodes, int pos, const SlabRay& sr,
+                                             float t) {
+    float4 a, b;
+    load_node(nodes, pos, a, b);
+    float tn;
+    const bool pass = slab_near<true>(sr, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, tn);
+    const bool nan = !(a.x <= INFINITY) | !(a.y <= INFINITY) | !(a.z <= INFINITY) | !(a.w <= INFINITY) |
+                     !(b.x <= INFINITY) | !(b.y <= INFINITY);
+    return pass && !(tn > t) && !nan;
+}
+
+// One axis of one child for a ray parallel to its slab: everywhere inside it,
+// or nowhere (rel = org - o).
+__device__ __forceinline__ void wide_parallel(bool par, float lo, float hi, float scale, float rel, float& tn,
+                                              float& tf) {
+    if (!par) return;
+    tn = __builtin_fmaf(lo, scale, rel) > 0.0f ? INFINITY : -INFINITY;
+    tf = __builtin_fmaf(hi, scale, rel) < 0.0f ? -INFINITY : INFINITY;
+}
+
+// Entries of a lane's LDS stack (`stride` words apart, so lanes never share a
+// bank). Of 200 000 random rays through 2^20 random triangles 23 held more than
+// 16 at once, one more than 20.
+constexpr int kWideStack = 20;
+
+// Walks the records from the root, entering boxes up to t_cull (which `leaf`
+// may lower), the nearest child first. leaf(at, ref) tests the triangle of one
+// leaf child (at = 4 * record + child); true ends the walk (any hit).
+// share() runs on every lane after each round of leaf tests; true ends the walk
+// of a lane (lanes that walk parts of one ray tell each other); a lane with `skip`
+// walks nothing and takes part in that. A lane whose step enters leaf children holds them and does not step again until they
+// are tested; the wave tests held leaves together once 1 / kGatherDiv of its
+// working lanes hold some, or none can step on. kPar: some lane of the wave has
+// an axis-parallel direction. Returns false when the stack overflowed; *bad is
+// set on a malformed array (record out of range, a record entered twice).
+template <bool kPar, typename Leaf, typename Share>
+__device__ __forceinline__ bool wide_walk(const WideNode* __restrict__ wide, uint32_t records, const SlabRay& r,
+                                          const float& t_cull, bool skip, uint32_t* stack, int stride,
+                                          uint32_t& visits, bool& bad, Leaf&& leaf, Share&& share) {
+    uint32_t c = 0, hc = 0, hmask = 0;
+    uint4 ref = make_uint4(0, 0, 0, 0);
+    int sp = 0;
+    uint32_t guard = records;  // each record is entered once
+    bool done = skip, overflow = false;
+    for (;;) {
+        if (!done & (hmask == 0)) {
+            if (c >= records || guard-- == 0) {
+                bad = true;
+                done = true;
+            } else {
+                float4 a, b, q;
+                load_wide(wide, c, a, b, q, ref);
+                visits += 2;
+                const float sx = a.w * r.inv.x, sy = b.x * r.inv.y, sz = b.y * r.inv.z;
+                const float bx = (a.x - r.o.x) * r.inv.x, by = (a.y - r.o.y) * r.inv.y, bz = (a.z - r.o.z) * r.inv.z;
+                const float ex = __builtin_fmaf(fabsf(bx), kWideSlack, bx), ey = __builtin_fmaf(fabsf(by), kWideSlack, by),
+                            ez = __builtin_fmaf(fabsf(bz), kWideSlack, bz);
+                const uint32_t lx = __float_as_uint(b.z), ly = __float_as_uint(b.w), lz = __float_as_uint(q.x),
+                               hx = __float_as_uint(q.y), hy = __float_as_uint(q.z), hz = __float_as_uint(q.w);
+                const uint32_t fx = r.neg_x ? hx : lx, gx = r.neg_x ? lx : hx, fy = r.neg_y ? hy : ly,
+                               gy = r.neg_y ? ly : hy, fz = r.neg_z ? hz : lz, gz = r.neg_z ? lz : hz;
+                float key[4];
+                uint32_t kid[4] = {ref.x, ref.y, ref.z, ref.w};
+                uint32_t mask = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float ax = __builtin_fmaf(byte_of(fx, k), sx, bx), cx = __builtin_fmaf(byte_of(gx, k), sx, ex);
+                    float ay = __builtin_fmaf(byte_of(fy, k), sy, by), cy = __builtin_fmaf(byte_of(gy, k), sy, ey);
+                    float az = __builtin_fmaf(byte_of(fz, k), sz, bz), cz = __builtin_fmaf(byte_of(gz, k), sz, ez);
+                    if (kPar) {
+                        wide_parallel(r.par_x, byte_of(lx, k), byte_of(hx, k), a.w, a.x - r.o.x, ax, cx);
+                        wide_parallel(r.par_y, byte_of(ly, k), byte_of(hy, k), b.x, a.y - r.o.y, ay, cy);
+                        wide_parallel(r.par_z, byte_of(lz, k), byte_of(hz, k), b.y, a.z - r.o.z, az, cz);
+                    }
+                    const float tn = fmaxf(fmaxf(fmaxf(ax, ay), az), r.t_min);
+                    const bool pass = !(tn > fminf(fminf(fminf(cx, cy), cz), t_cull));
+                    const bool is_leaf = int32_t(kid[k]) < 0;
+                    key[k] = (pass & !is_leaf) ? tn : INFINITY;
+                    mask |= (pass & is_leaf) ? (1u << k) : 0u;
+                }
+                hc = c;
+                hmask = mask;
+                auto order = [&](int i, int j) {
+                    const bool sw = key[j] < key[i];
+                    const float ki = sw ? key[j] : key[i], kj = sw ? key[i] : key[j];
+                    const uint32_t ri = sw ? kid[j] : kid[i], rj = sw ? kid[i] : kid[j];
+                    key[i] = ki;
+                    key[j] = kj;
+                    kid[i] = ri;
+                    kid[j] = rj;
+                };
+                order(0, 1);
+                order(2, 3);
+                order(0, 2);
+                order(1, 3);
+                order(1, 2);
+                if (key[0] < INFINITY) {
+                    c = kid[0];
+                    if (key[1] < INFINITY) {
+                        const bool p2 = key[2] < INFINITY, p3 = key[3] < INFINITY;
+                        if (sp + 1 + int(p2) + int(p3) > kWideStack) {
+                            overflow = true;
+                            done = true;
+                            hmask = 0;
+                        } else {
+                            if (p3) stack[sp++ * stride] = kid[3];
+                            if (p2) stack[sp++ * stride] = kid[2];
+                            stack[sp++ * stride] = kid[1];
+                        }
+                    }
+                } else if (sp == 0) {
+                    done = true;
+                } else {
+                    --sp;
+                    c = stack[sp * stride];
+                }
+            }
+        }
+        const bool holds = hmask != 0;
+        const uint64_t want = __ballot(holds);
+        const uint64_t more = __ballot(!done & !holds);
+        if (!more) {
+            if (!want) break;
+        } else if (__popcll(want) * kGatherDiv < __popcll(want | more)) {
+            continue;
+        }
+        while (hmask) {  // each lane's first held leaf, then its second, ...
+            const uint32_t k = uint32_t(__ffs(int(hmask))) - 1u;
+            hmask &= hmask - 1u;
+            const uint32_t r0 = (k & 1u) ? ref.y : ref.x, r1 = (k & 1u) ? ref.w : ref.z;
+            if (leaf(4u * hc + k, (k & 2u) ? r1 : r0)) {
+                done = true;
+                hmask = 0;
+            }
+        }
+        if (share()) done = true;
+    }
+    return !overflow;
+}
+
+}  // namespace lux
