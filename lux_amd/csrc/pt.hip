@@ -42,6 +42,13 @@ namespace pt {
 namespace {
 
 constexpr int kBlock = 256;
+// Batches whose trees all have fewer records walk sibling pairs. A record step
+// costs about two pair steps of instructions and pays by halving the waits for
+// memory, which a tree this small hardly has: records / pairs, Cornell box (36
+// triangles) 256 x 256 x 64 7.77 / 7.27 ms, 128 x 96 x 4 0.412 / 0.371 ms; sphere
+// of 982 triangles 256 x 256 x 16 1.00 / 1.19 ms, 128 x 128 x 4 0.40 / 0.64 ms; of
+// 32 002 1.64 / 2.16 ms; of 327 682 (1024 x 1024 x 16) 15.5 / 17.7 ms.
+constexpr uint32_t kSmallTree = 128;
 constexpr int kPlainBatch = 65536;  // RenderSettings::batch_size default (src/integrator/render_context.h:16-24)
 
 struct Queues {
@@ -66,7 +73,7 @@ struct Paths {
     float4* st;     // throughput at the vertex xyz, bits: ignored primitive
 };
 
-// Closest hit / occlusion walk over the sibling-pair copy of the right-first
+// Small trees. Closest hit / occlusion walk over the sibling-pair copy of the right-first
 // stackless LBVH (same visits and order as the preorder walk); `ignore` skips
 // one leaf's triangle test (the source primitive of a shadow ray). kParallel =
 // false drops the axis-parallel branches of the slab test (no active lane of
@@ -75,9 +82,9 @@ template <bool kParallel, bool kAny>
 __device__ __forceinline__ int closest_walk(const SceneView& sv, const f3& O, const f3& D, const SlabRay& sr,
                                             float t_min, float t_max, int ignore, float& t_hit, float& u_hit,
                                             float& v_hit) {
-    const lux_bvh_node* nodes = sv.nodes;
+    const lux_bvh_node* nodes = sv.pairs;
     const lux_triangle* soup = sv.soup;
-    const int node_count = sv.node_count, tri_count = sv.tri_count;
+    const int node_count = sv.pair_count, tri_count = sv.tri_count;
     int best = -1;
     int k = 0;
     int guard = node_count + 1;  // a walk visits each node at most once
@@ -157,7 +164,7 @@ __device__ __forceinline__ int closest_ordered(const SceneView& sv, const f3& O,
         }
         return false;
     };
-    const bool done = ordered_walk_gathered(SlabMode<kMode>{}, sv.nodes, uint32_t(sv.node_count), sr, ob, stack, stride,
+    const bool done = ordered_walk_gathered(SlabMode<kMode>{}, sv.pairs, uint32_t(sv.pair_count), sr, ob, stack, stride,
                                    visits, bad, leaf);
     if (bad) set_error(sv.info, kErrWalkOrder);
     if (!done || (best >= 0 && ob.ambiguous()))
@@ -181,7 +188,7 @@ __device__ __forceinline__ int closest(const SceneView& sv, const vec& o, const 
     const f3 O = make3(o.x, o.y, o.z), D = make3(d.x, d.y, d.z);
     const SlabRay sr = make_slab_ray(O, D, t_min);
     const bool ordered =
-        stack && !sv.preorder && sv.node_count > 1 && uint32_t(sv.node_count) <= kOffset32Nodes;
+        stack && !sv.preorder && sv.pair_count > 1 && uint32_t(sv.pair_count) <= kOffset32Nodes;
     if (ordered)
         return with_slab_mode(sr, [&](auto mode) {
             return closest_ordered<decltype(mode)::value>(sv, O, D, sr, t_min, t_max, ignore, t_hit, u_hit, v_hit,
@@ -206,29 +213,25 @@ __device__ __forceinline__ bool occluded(const SceneView& sv, const vec& o, cons
 
 // The same two queries on an instanced scene: the two-level walk (TLAS, then
 // the BLAS of each instance the ray reaches, in object space), returning the
-// scene ordinal. kTwoLevel is chosen per batch on the host, like kAnyShadow.
-// stack as for closest().
+// scene ordinal. stack as for closest().
 template <bool kTwoLevel>
 __device__ __forceinline__ int scene_closest(const SceneView& sv, const vec& o, const vec& d, float t_min,
                                              float t_max, int ignore, float& t_hit, float& u_hit, float& v_hit,
                                              uint32_t* stack, int stride) {
-    if constexpr (kTwoLevel) {
-        TwoLevelHit h;
-        const bool ordered = stack && !sv.preorder;
-        if (!ordered || !two_level_closest_ordered(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max,
-                                                   ignore, stack, stride, h))
-            h = two_level_walk<false>(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max, ignore);
-        if (h.prim >= 0) {
-            t_hit = h.t;
-            u_hit = h.u;
-            v_hit = h.v;
-        } else {
-            t_hit = t_max;
-        }
-        return h.prim;
+    if constexpr (!kTwoLevel) return closest(sv, o, d, t_min, t_max, ignore, t_hit, u_hit, v_hit, stack, stride);
+    TwoLevelHit h;
+    const bool ordered = stack && !sv.preorder;
+    if (!ordered || !two_level_closest_ordered(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max,
+                                               ignore, stack, stride, h))
+        h = two_level_walk<false>(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max, ignore);
+    if (h.prim >= 0) {
+        t_hit = h.t;
+        u_hit = h.u;
+        v_hit = h.v;
     } else {
-        return closest(sv, o, d, t_min, t_max, ignore, t_hit, u_hit, v_hit, stack, stride);
+        t_hit = t_max;
     }
+    return h.prim;
 }
 
 template <bool kTwoLevel>
@@ -238,6 +241,21 @@ __device__ __forceinline__ bool scene_occluded(const SceneView& sv, const vec& o
         return two_level_any(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max, ignore);
     else
         return occluded(sv, o, d, t_min, t_max, ignore);
+}
+
+// One ray of a one-mesh scene on `group` lanes (wide_query): the closest hit, or
+// any hit.
+__device__ __forceinline__ WideHit mesh_query(const SceneView& sv, const f3& o, const f3& d, float t_max, bool any,
+                                              int ignore, int group, int part, uint32_t* stack, int stride) {
+    uint32_t visits = 0, tests = 0;
+    WideHit h;
+    h.failed = sv.preorder != 0;
+    if (!h.failed)
+        h = wide_query(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, group, part, stack, stride,
+                       sv.info, visits, tests);
+    if (h.failed)
+        h = preorder_query(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, sv.info, visits, tests);
+    return h;
 }
 
 __device__ __forceinline__ vec xyz(const float4& f) { return mk(f.x, f.y, f.z); }
@@ -311,42 +329,97 @@ __global__ __launch_bounds__(B) void k_generate(const BatchDesc* __restrict__ de
 // material): the first hit found blocks the ray, so an any-hit walk gives the
 // same transmittance (0 or 1) as the closest-hit loop. The choice is made per
 // batch on the host; reading the scene's flag per ray instead measured slower.
+
+// One hit of the loop: true when the ray goes on behind it.
+__device__ __forceinline__ bool shadow_passes(const SceneView& sv, int prim, float t, vec& tr, f3& o, const f3& d,
+                                              float& t_max) {
+    const DevMaterial& m = sv.mats[sv.mat_id[prim]];
+    if (!passthrough(m)) {
+        tr = splat(0);
+        return false;
+    }
+    tr = tr * (m.type == kTransparent ? albedo_of(m) : splat(1));
+    if (max_component(tr) <= 0) return false;
+    const float adv = t + kEps;
+    if (adv >= t_max) return false;
+    o = make3(o.x + d.x * adv, o.y + d.y * adv, o.z + d.z * adv);
+    t_max -= adv;
+    return true;
+}
+
+// Shadow record i arrives with transmittance tr.
+__device__ __forceinline__ void shadow_arrives(const Paths& ps, uint32_t i, uint32_t path, const vec& tr) {
+    if (max_component(tr) > 0) {
+        const float4 sc = ps.sc[i], st = ps.st[i], Lq = ps.L[path];
+        const vec add = xyz(st) * (xyz(sc) * tr * ps.sd[i].w);
+        ps.L[path] = pack(xyz(Lq) + add, Lq.w);
+    }
+}
+
 template <bool kAnyShadow, bool kTwoLevel>
-__device__ __forceinline__ void shadow_ray(const BatchDesc* __restrict__ desc, const Paths& ps, uint32_t i,
-                                           uint32_t* stack, int stride) {
-    float4 so = ps.so[i], sd = ps.sd[i], sc = ps.sc[i], st = ps.st[i];
-    const uint32_t path = __float_as_uint(sc.w);
+__device__ __forceinline__ void shadow_ray(const BatchDesc* __restrict__ desc, const Paths& ps, uint32_t i) {
+    const float4 so = ps.so[i], sd = ps.sd[i];
+    const uint32_t path = __float_as_uint(ps.sc[i].w);
     const SceneView& sv = desc->seg[segment_of_path(ps, path)].sv;
-    vec o = xyz(so), d = xyz(sd);
-    float t_max = so.w, t_min = kEps;
-    int ignore = __float_as_int(st.w);
+    f3 o = make3(so.x, so.y, so.z);
+    const f3 d = make3(sd.x, sd.y, sd.z);
+    const vec D = mk(d.x, d.y, d.z);
+    float t_max = so.w;
+    int ignore = __float_as_int(ps.st[i].w);
     vec tr = splat(1);
-    if (kAnyShadow && scene_occluded<kTwoLevel>(sv, o, d, t_min, t_max, ignore)) tr = splat(0);
+    if (kAnyShadow && scene_occluded<kTwoLevel>(sv, mk(o.x, o.y, o.z), D, kEps, t_max, ignore)) tr = splat(0);
     for (int guard = 0; !kAnyShadow && guard < 1 << 16; ++guard) {
         float t = 0, u = 0, v = 0;
         // the preorder walk (no stack): with the near-child-first walk inlined a
         // second time here the one-level kernel spilled 36 VGPRs per lane
-        int prim = scene_closest<kTwoLevel>(sv, o, d, t_min, t_max, ignore, t, u, v, nullptr, 0);
-        if (prim < 0) break;
-        const DevMaterial& m = sv.mats[sv.mat_id[prim]];
-        if (!passthrough(m)) {
-            tr = splat(0);
-            break;
-        }
-        tr = tr * (m.type == kTransparent ? albedo_of(m) : splat(1));
-        if (max_component(tr) <= 0) break;
-        float adv = t + kEps;
-        if (adv >= t_max) break;
-        o = o + d * adv;
-        t_max -= adv;
-        t_min = kEps;
+        const int prim = scene_closest<kTwoLevel>(sv, mk(o.x, o.y, o.z), D, kEps, t_max, ignore, t, u, v, nullptr, 0);
+        if (prim < 0 || !shadow_passes(sv, prim, t, tr, o, d, t_max)) break;
         ignore = -1;
     }
-    if (max_component(tr) > 0) {
-        float4 Lq = ps.L[path];
-        vec add = xyz(st) * (xyz(sc) * tr * sd.w);
-        ps.L[path] = pack(xyz(Lq) + add, Lq.w);
+    shadow_arrives(ps, i, path, tr);
+}
+
+// Extension ray i (i < n_ext) or shadow record i - n_ext of a one-mesh scene, on
+// `group` lanes: one walk in the code for both, so a wave may hold both.
+template <bool kAnyShadow>
+__device__ __forceinline__ void mesh_ray(const BatchDesc* __restrict__ desc, const Paths& ps, uint32_t i,
+                                         uint32_t n_ext, const uint32_t* __restrict__ queue, int group, int part,
+                                         uint32_t* stack, int stride) {
+    const bool ext = i < n_ext;
+    const uint32_t j = i - n_ext;
+    const uint32_t path = ext ? queue[i] : __float_as_uint(ps.sc[j].w);
+    const float4 ro = ext ? ps.ro[path] : ps.so[j], rd = ext ? ps.rd[path] : ps.sd[j];
+    const SceneView& sv = desc->seg[ext ? __float_as_uint(rd.w) : segment_of_path(ps, path)].sv;
+    f3 o = make3(ro.x, ro.y, ro.z);
+    const f3 d = make3(rd.x, rd.y, rd.z);
+    float t_max = ext ? INFINITY : ro.w;
+    int ignore = ext ? -1 : __float_as_int(ps.st[j].w);
+    vec tr = splat(1);
+    WideHit h;
+    for (int guard = 0; guard < 1 << 16; ++guard) {
+        h = mesh_query(sv, o, d, t_max, kAnyShadow && !ext, ignore, group, part, stack, stride);
+        if (ext) break;
+        if (kAnyShadow) {
+            if (h.prim >= 0) tr = splat(0);
+            break;
+        }
+        if (h.prim < 0 || !shadow_passes(sv, h.prim, h.t, tr, o, d, t_max)) break;
+        ignore = -1;
     }
+    if (part != 0) return;
+    if (!ext) {
+        shadow_arrives(ps, j, path, tr);
+        return;
+    }
+    float t = INFINITY, u = 0, v = 0;
+    if (h.prim >= 0) {
+        // u, v of the winner, recomputed once rather than carried through the
+        // walk (the same operations give the same bits)
+        const float* p = reinterpret_cast<const float*>(sv.soup + h.prim);
+        (void)tri_uvt(o, d, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), t, u, v);
+        t = h.t;
+    }
+    ps.hit[path] = make_float4(__int_as_float(h.prim), t, u, v);
 }
 
 // ---- trace -----------------------------------------------------------------------
@@ -354,35 +427,52 @@ __device__ __forceinline__ void shadow_ray(const BatchDesc* __restrict__ desc, c
 // counted by counts[sh_in] (-1: none), in one grid-stride pass. Block 0 clears
 // the counters the following shade launch appends to (zero_a, zero_b; never
 // the ones read here) and adds the queue sizes to the ray totals.
-// One-level variants: at least 8 waves per SIMD (64 VGPRs, 65 uncapped). C3
-// measured 0.079 s at 8 waves against 0.096 s at 7. Two-level variants: 6
-// waves (80 VGPRs, 86 uncapped, 28-40 bytes per lane spilled); the instanced
-// field measured 91.6 ms at 6 waves, 96.7 ms at 7 and 113 ms at the natural 5.
-template <int B, bool kAnyShadow, bool kTwoLevel>
-__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kTwoLevel ? 6 : 8))) void k_trace(const BatchDesc* __restrict__ desc, Paths ps, Queues qs, int ext_in,
-                                                  int sh_in, int zero_a, int zero_b) {
+// kWalk: two-level scenes; one-mesh scenes by sibling pairs (small trees), by
+// records, or by records in parts, several lanes per ray (lanes_per_ray). A bounce of a large batch is
+// launched as kWalkMesh and kWalkParts and one of them has the work, by the
+// number of rays left; only the first clears and counts (`own`).
+// Waves per SIMD: pairs 8 (64 VGPRs); records 6 (80 VGPRs, 60 bytes per lane
+// spilled outside the walk; the 327 682-triangle frame took 17.0 / 15.5 / 17.1 /
+// 17.3 ms at 5 / 6 / 7 / 8); two-level 6 (80 VGPRs, 86 uncapped; the instanced
+// field measured 91.6 ms at 6, 96.7 ms at 7 and 113 ms at the natural 5).
+enum { kWalkTwoLevel, kWalkPairs, kWalkMesh, kWalkParts, kWalkBoth };
+template <int B, bool kAnyShadow, int kWalk>
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWalk == kWalkPairs ? 8 : 6))) void k_trace(
+    const BatchDesc* __restrict__ desc, Paths ps, Queues qs, int ext_in, int sh_in, int zero_a, int zero_b, int own,
+    int other) {
+    constexpr bool kTwoLevel = kWalk == kWalkTwoLevel;
     const uint32_t n_ext = ext_in >= 0 ? qs.counts[ext_in] : 0u;
     const uint32_t n_sh = sh_in >= 0 ? qs.counts[sh_in] : 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (own && blockIdx.x == 0 && threadIdx.x == 0) {
         if (zero_a >= 0) qs.counts[zero_a] = 0;
         if (zero_b >= 0) qs.counts[zero_b] = 0;
         qs.rays[0] += n_ext;
         qs.rays[1] += n_sh;
     }
-    // per-lane stacks of the ordered closest-hit walks
-    __shared__ uint32_t lds_stack[kOrderedStack * B];
+    // per-lane stacks
+    constexpr bool kRecords = kWalk == kWalkMesh || kWalk == kWalkParts;
+    __shared__ uint32_t lds_stack[(kRecords ? kWideStack : kOrderedStack) * B];
     uint32_t* stack = lds_stack + threadIdx.x;
     const uint32_t total = n_ext + n_sh;
+    if constexpr (kRecords) {
+        const uint32_t group = kWalk == kWalkMesh ? 1u : uint32_t(lanes_per_ray(total));
+        if (other && (total <= kPartsMaxRays) != (kWalk == kWalkParts)) return;  // the other launch's
+        const uint32_t* queue = ext_in >= 0 ? qs.q[ext_in] : nullptr;
+        for (uint32_t i = xcd_block() * B + threadIdx.x; i < total * group; i += gridDim.x * B)
+            mesh_ray<kAnyShadow>(desc, ps, kWalk == kWalkMesh ? i : i / group, n_ext, queue, int(group),
+                                 int(i & (group - 1)), stack, B);
+        return;
+    }
     for (uint32_t i = xcd_block() * B + threadIdx.x; i < total; i += gridDim.x * B) {
         if (i < n_ext) {
             const uint32_t path = qs.q[ext_in][i];
             const float4 o = ps.ro[path], d = ps.rd[path];
             const SceneView& sv = desc->seg[__float_as_uint(d.w)].sv;
             float t = INFINITY, u = 0, v = 0;
-            int prim = scene_closest<kTwoLevel>(sv, xyz(o), xyz(d), kEps, INFINITY, -1, t, u, v, stack, B);
+            const int prim = scene_closest<kTwoLevel>(sv, xyz(o), xyz(d), kEps, INFINITY, -1, t, u, v, stack, B);
             ps.hit[path] = make_float4(__int_as_float(prim), t, u, v);
         } else {
-            shadow_ray<kAnyShadow, kTwoLevel>(desc, ps, i - n_ext, stack, B);
+            shadow_ray<kAnyShadow, kTwoLevel>(desc, ps, i - n_ext);
         }
     }
 }
@@ -1143,7 +1233,7 @@ void Renderer::set_tuning(const Tuning& t) {
 void Renderer::release_graph() {
     if (graph_) (void)hipGraphExecDestroy(graph_);
     graph_ = nullptr;
-    graph_depth_ = graph_grid_ = graph_capacity_ = graph_block_ = graph_opaque_ = graph_two_level_ = graph_light_ = -1;
+    graph_depth_ = graph_grid_ = graph_capacity_ = graph_block_ = graph_opaque_ = graph_walk_ = graph_light_ = -1;
 }
 
 void Renderer::ensure_capacity(int paths) {
@@ -1217,9 +1307,12 @@ namespace {
 // a second, partial round behind the first (at block 512 it holds 128 VGPRs,
 // 2 blocks per CU: 512 blocks on 256 CUs against the tuned 768 took C3 from
 // 0.0730 to 0.0713 s and the 64-scene mix from 1.243 to 1.215 s, same films).
+// The trace kernel's grid holds the parts of a small capacity's rays
+// (lanes_per_ray).
 struct LaunchGrid {
     int grid;
     int shade;
+    int trace;
 };
 
 template <int B, int kLight>
@@ -1255,8 +1348,9 @@ int shade_resident_blocks(int block, int light) {
 
 // The wavefront launch sequence of one batch (captured or launched directly).
 // Raw launches (no probe events) when captured.
+// walk: a k_trace variant, or kWalkBoth: records, a bounce of few rays in parts.
 template <int B, bool kProbe, bool kOpaque, bool kTwoLevel, int kLight>
-void wavefront_sequence(const PathBuf& buf, int depth, LaunchGrid grid, hipStream_t stream) {
+void wavefront_sequence(const PathBuf& buf, int walk, int depth, LaunchGrid grid, hipStream_t stream) {
     const Paths ps = paths_of(buf);
     const Queues qs = queues_of(buf);
     const BatchDesc* d = buf.desc;
@@ -1269,14 +1363,30 @@ void wavefront_sequence(const PathBuf& buf, int depth, LaunchGrid grid, hipStrea
             hip_check(hipGetLastError(), NAME);                                      \
         }                                                                            \
     } while (0)
+    auto trace = [&](int ext_in, int sh_in, int zero_a, int zero_b) {
+        if constexpr (kTwoLevel) {
+            PT_LAUNCH("pt_trace", grid.grid, (k_trace<B, kOpaque, kWalkTwoLevel>), d, ps, qs, ext_in, sh_in, zero_a,
+                      zero_b, 1, 0);
+        } else {
+            const int both = walk == kWalkBoth;
+            if (walk == kWalkPairs)
+                PT_LAUNCH("pt_trace", grid.grid, (k_trace<B, kOpaque, kWalkPairs>), d, ps, qs, ext_in, sh_in, zero_a,
+                          zero_b, 1, 0);
+            if (both || walk == kWalkMesh)
+                PT_LAUNCH("pt_trace", grid.grid, (k_trace<B, kOpaque, kWalkMesh>), d, ps, qs, ext_in, sh_in, zero_a,
+                          zero_b, 1, both);
+            if (both || walk == kWalkParts)
+                PT_LAUNCH("pt_trace", grid.trace, (k_trace<B, kOpaque, kWalkParts>), d, ps, qs, ext_in, sh_in, zero_a,
+                          zero_b, int(!both), both);
+        }
+    };
     PT_LAUNCH("pt_generate", grid.grid, k_generate<B>, d, ps, qs);
     for (int b = 0; b <= depth; ++b) {
         const int in = b & 1;
-        PT_LAUNCH("pt_trace", grid.grid, (k_trace<B, kOpaque, kTwoLevel>), d, ps, qs, in,
-                  b > 0 ? 2 + ((b - 1) & 1) : -1, in ^ 1, 2 + (b & 1));
+        trace(in, b > 0 ? 2 + ((b - 1) & 1) : -1, in ^ 1, 2 + (b & 1));
         PT_LAUNCH("pt_shade", grid.shade, (k_shade<B, kLight>), d, ps, qs, in, b, -1);
     }
-    PT_LAUNCH("pt_trace", grid.grid, (k_trace<B, kOpaque, kTwoLevel>), d, ps, qs, -1, 2 + (depth & 1), -1, -1);
+    trace(-1, 2 + (depth & 1), -1, -1);
     PT_LAUNCH("pt_flush", grid.grid, k_flush<B>, d, ps);
 #undef PT_LAUNCH
 }
@@ -1284,25 +1394,26 @@ void wavefront_sequence(const PathBuf& buf, int depth, LaunchGrid grid, hipStrea
 
 namespace {
 template <bool kProbe, bool kOpaque, bool kTwoLevel, int kLight>
-void wavefront_sequence_b(int block, const PathBuf& buf, int depth, LaunchGrid grid, hipStream_t stream) {
+void wavefront_sequence_b(int block, const PathBuf& buf, int walk, int depth, LaunchGrid grid, hipStream_t stream) {
     switch (block) {
-        case 128: wavefront_sequence<128, kProbe, kOpaque, kTwoLevel, kLight>(buf, depth, grid, stream); break;
-        case 512: wavefront_sequence<512, kProbe, kOpaque, kTwoLevel, kLight>(buf, depth, grid, stream); break;
-        default: wavefront_sequence<256, kProbe, kOpaque, kTwoLevel, kLight>(buf, depth, grid, stream); break;
+        case 128: wavefront_sequence<128, kProbe, kOpaque, kTwoLevel, kLight>(buf, walk, depth, grid, stream); break;
+        case 512: wavefront_sequence<512, kProbe, kOpaque, kTwoLevel, kLight>(buf, walk, depth, grid, stream); break;
+        default: wavefront_sequence<256, kProbe, kOpaque, kTwoLevel, kLight>(buf, walk, depth, grid, stream); break;
     }
 }
 
 template <bool kProbe, bool kOpaque, bool kTwoLevel>
-void wavefront_sequence_l(int light, int block, const PathBuf& buf, int depth, LaunchGrid grid, hipStream_t stream) {
+void wavefront_sequence_l(int light, int block, const PathBuf& buf, int walk, int depth, LaunchGrid grid,
+                          hipStream_t stream) {
     switch (light) {
         case kLightUniform:
-            wavefront_sequence_b<kProbe, kOpaque, kTwoLevel, kLightUniform>(block, buf, depth, grid, stream);
+            wavefront_sequence_b<kProbe, kOpaque, kTwoLevel, kLightUniform>(block, buf, walk, depth, grid, stream);
             break;
         case kLightBvh:
-            wavefront_sequence_b<kProbe, kOpaque, kTwoLevel, kLightBvh>(block, buf, depth, grid, stream);
+            wavefront_sequence_b<kProbe, kOpaque, kTwoLevel, kLightBvh>(block, buf, walk, depth, grid, stream);
             break;
         default:
-            wavefront_sequence_b<kProbe, kOpaque, kTwoLevel, kLightPower>(block, buf, depth, grid, stream);
+            wavefront_sequence_b<kProbe, kOpaque, kTwoLevel, kLightPower>(block, buf, walk, depth, grid, stream);
             break;
     }
 }
@@ -1311,23 +1422,23 @@ void wavefront_sequence_l(int light, int block, const PathBuf& buf, int depth, L
 // scene of the batch passes light), traversal (one- or two-level) and light
 // selection are template choices made here, per batch.
 template <bool kProbe>
-void wavefront_sequence_o(bool opaque, bool two_level, int light, int block, const PathBuf& buf, int depth,
+void wavefront_sequence_o(bool opaque, int walk, int light, int block, const PathBuf& buf, int depth,
                           LaunchGrid grid, hipStream_t stream) {
-    if (two_level) {
+    if (walk == kWalkTwoLevel) {
         if (opaque)
-            wavefront_sequence_l<kProbe, true, true>(light, block, buf, depth, grid, stream);
+            wavefront_sequence_l<kProbe, true, true>(light, block, buf, walk, depth, grid, stream);
         else
-            wavefront_sequence_l<kProbe, false, true>(light, block, buf, depth, grid, stream);
+            wavefront_sequence_l<kProbe, false, true>(light, block, buf, walk, depth, grid, stream);
     } else {
         if (opaque)
-            wavefront_sequence_l<kProbe, true, false>(light, block, buf, depth, grid, stream);
+            wavefront_sequence_l<kProbe, true, false>(light, block, buf, walk, depth, grid, stream);
         else
-            wavefront_sequence_l<kProbe, false, false>(light, block, buf, depth, grid, stream);
+            wavefront_sequence_l<kProbe, false, false>(light, block, buf, walk, depth, grid, stream);
     }
 }
 }  // namespace
 
-void Renderer::launch_wavefront(int depth, bool opaque, bool two_level, int light, hipStream_t stream) {
+void Renderer::launch_wavefront(int depth, bool opaque, bool two_level, bool small, int light, hipStream_t stream) {
     const int block = tune_.block;
     const int tuned = std::max(1, std::min(tune_.grid, div_up(buf_.capacity, block)));
     if (shade_resident_block_ != block || shade_resident_light_ != light) {  // outside any capture
@@ -1335,19 +1446,24 @@ void Renderer::launch_wavefront(int depth, bool opaque, bool two_level, int ligh
         shade_resident_block_ = block;
         shade_resident_light_ = light;
     }
-    const LaunchGrid grid{tuned, std::min(tuned, shade_resident_)};
+    const int walk = two_level ? kWalkTwoLevel
+                     : small   ? kWalkPairs
+                               : (uint32_t(buf_.capacity) <= kPartsMaxRays ? kWalkParts : kWalkBoth);
+    const int64_t trace_lanes = int64_t(buf_.capacity) * lanes_per_ray(uint32_t(buf_.capacity));
+    const LaunchGrid grid{tuned, std::min(tuned, shade_resident_),
+                          std::max(1, std::min(tune_.grid, div_up(trace_lanes, block)))};
     if (!tune_.use_graph) {
-        wavefront_sequence_o<true>(opaque, two_level, light, block, buf_, depth, grid, stream);
+        wavefront_sequence_o<true>(opaque, walk, light, block, buf_, depth, grid, stream);
         return;
     }
     if (!graph_ || graph_depth_ != depth || graph_grid_ != tuned || graph_capacity_ != buf_.capacity ||
-        graph_block_ != block || graph_opaque_ != int(opaque) || graph_two_level_ != int(two_level) ||
+        graph_block_ != block || graph_opaque_ != int(opaque) || graph_walk_ != walk ||
         graph_light_ != light) {
         release_graph();
         hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         hipGraph_t g = nullptr;
         try {
-            wavefront_sequence_o<false>(opaque, two_level, light, block, buf_, depth, grid, stream);
+            wavefront_sequence_o<false>(opaque, walk, light, block, buf_, depth, grid, stream);
         } catch (...) {
             (void)hipStreamEndCapture(stream, &g);
             if (g) (void)hipGraphDestroy(g);
@@ -1362,7 +1478,7 @@ void Renderer::launch_wavefront(int depth, bool opaque, bool two_level, int ligh
         graph_capacity_ = buf_.capacity;
         graph_block_ = block;
         graph_opaque_ = int(opaque);
-        graph_two_level_ = int(two_level);
+        graph_walk_ = walk;
         graph_light_ = light;
     }
     hip_check(hipGraphLaunch(graph_, stream), "hipGraphLaunch");
@@ -1378,12 +1494,12 @@ void plain_sequence(const PathBuf& buf, int depth, uint32_t count, hipStream_t s
     LUX_LAUNCH("pt_generate", k_generate<kBlock>, grid, kBlock, 0, stream, d, ps, qs);
     for (int b = 0; b <= depth; ++b) {
         const int in = b & 1;
-        LUX_LAUNCH("pt_trace", (k_trace<kBlock, false, kTwoLevel>), grid, kBlock, 0, stream, d, ps, qs, in, -1,
-                   in ^ 1, 2 + (b & 1));
+        LUX_LAUNCH("pt_trace", (k_trace<kBlock, false, kTwoLevel ? kWalkTwoLevel : kWalkMesh>), grid, kBlock, 0, stream, d,
+                   ps, qs, in, -1, in ^ 1, 2 + (b & 1), 1, 0);
         for (int type = 0; type < kMaterialTypes; ++type)
             LUX_LAUNCH("pt_shade", (k_shade<kBlock, kLight>), grid, kBlock, 0, stream, d, ps, qs, in, b, type);
-        LUX_LAUNCH("pt_shadow", (k_trace<kBlock, false, kTwoLevel>), grid, kBlock, 0, stream, d, ps, qs, -1,
-                   2 + (b & 1), -1, -1);
+        LUX_LAUNCH("pt_shadow", (k_trace<kBlock, false, kTwoLevel ? kWalkTwoLevel : kWalkMesh>), grid, kBlock, 0, stream,
+                   d, ps, qs, -1, 2 + (b & 1), -1, -1, 1, 0);
     }
     LUX_LAUNCH("pt_flush", k_flush<kBlock>, grid, kBlock, 0, stream, d, ps);
 }
@@ -1415,6 +1531,7 @@ uint64_t Renderer::enqueue_batch(std::vector<Request*>& active, int slice_spp, i
     uint64_t used = 0;
     uint32_t nseg = 0;
     bool opaque = true;  // every scene of the batch: shadow rays may use the any-hit walk
+    bool small = true;   // every scene of the batch: the pair walk is the faster one
     // One kind per batch (traversal level and light sampler: the kernels are
     // built for one): the kind of the first request with paths left; requests
     // of another kind wait for a later batch and keep their place in `active`.
@@ -1429,6 +1546,7 @@ uint64_t Renderer::enqueue_batch(std::vector<Request*>& active, int slice_spp, i
         if (slice_spp > 0)
             take = std::min(take, uint64_t(slice_spp) * uint64_t(rq->rs.width) * uint64_t(rq->rs.height));
         opaque = opaque && rq->sv.opaque != 0;
+        small = small && rq->sv.tree.records < kSmallTree;
         slot->seg[nseg] = make_segment(*rq, rq->issued, uint32_t(used), uint32_t(take));
         slot->seg[nseg++].sv.preorder = tune_.preorder_walk;
         rq->issued += take;
@@ -1440,7 +1558,7 @@ uint64_t Renderer::enqueue_batch(std::vector<Request*>& active, int slice_spp, i
     slot->count = uint32_t(used);
     slot->nseg = nseg;
     upload(slot, stream);
-    launch_wavefront(max_depth, opaque, (kind & 1) != 0, kind >> 1, stream);
+    launch_wavefront(max_depth, opaque, (kind & 1) != 0, small, kind >> 1, stream);
     ++batch_counter_;
     return used;
 }

@@ -12,6 +12,7 @@
 #include "lux_runtime.hpp"
 #include "pt_device.hpp"
 #include "two_level.hpp"
+#include "wide.hpp"
 
 namespace lux {
 namespace pt {
@@ -112,8 +113,9 @@ struct SceneDev {
 
 // POD view of one scene handed to kernels.
 struct SceneView {
-    const lux_bvh_node* nodes;
-    const uint32_t* slot_pre;  // preorder position of each pair slot (tie order of the ordered walk)
+    RayTree tree;  // one-mesh scenes
+    const lux_bvh_node* pairs;  // the same tree's sibling pairs
+    const uint32_t* slot_pre;   // preorder position of each pair slot (tie order of the ordered walk)
     const lux_triangle* soup;
     const uint32_t* indices;
     const float* normals;
@@ -122,7 +124,7 @@ struct SceneView {
     const DevLight* lights;
     const int32_t* light_of_prim;
     DevInfo* info;
-    int32_t node_count, tri_count, mat_count, light_count;
+    int32_t pair_count, tri_count, mat_count, light_count;
     const DevLightNode* light_nodes;  // BVH light sampler: tree and leaf of each light
     const int32_t* light_leaf;
     int32_t light_node_count, light_root;  // root -1: no valid tree (power selection is used)
@@ -134,8 +136,8 @@ struct SceneView {
     const float* env_pixels;               // image texels (RGB), all images back to back
     const float* env_cdf;                  // per-texel cumulative weights
     int32_t opaque;     // 1: every hit blocks a shadow ray (no pass-through material)
-    int32_t instanced;  // 1: traverse `tl` (two-level) instead of `nodes`
-    int32_t preorder;   // 1: closest hits by the right-first preorder walk only
+    int32_t instanced;  // 1: traverse `tl` (two-level) instead of `tree`
+    int32_t preorder;   // 1: rays take the right-first preorder walk only
     DevCamera cam;
     TwoLevelView tl;
 };
@@ -241,7 +243,7 @@ private:
     void ensure_capacity(int paths);
     BatchDesc* next_slot();
     void upload(BatchDesc* slot, hipStream_t stream);
-    void launch_wavefront(int depth, bool opaque, bool two_level, int light, hipStream_t stream);
+    void launch_wavefront(int depth, bool opaque, bool two_level, bool small, int light, hipStream_t stream);
     void launch_plain(int depth, uint32_t count, bool two_level, int light, hipStream_t stream);
     void release_graph();
 
@@ -254,7 +256,7 @@ private:
     int ring_next_ = 0;
     hipGraphExec_t graph_ = nullptr;
     int graph_depth_ = -1, graph_grid_ = -1, graph_capacity_ = -1, graph_block_ = -1, graph_opaque_ = -1,
-        graph_two_level_ = -1, graph_light_ = -1;
+        graph_walk_ = -1, graph_light_ = -1;
     // k_shade blocks resident on the device for (block, light), queried outside any capture
     int shade_resident_ = 1, shade_resident_block_ = -1, shade_resident_light_ = -1;
     int64_t batch_counter_ = 0;

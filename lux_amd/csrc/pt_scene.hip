@@ -992,15 +992,13 @@ void scene_release(SceneDev& s) {
 SceneView scene_view(const SceneDev& s) {
     SceneView v{};
     if (s.instanced) {
-        v.nodes = nullptr;
-        v.slot_pre = nullptr;
-        v.node_count = 0;
         v.tl = two_level_view(s.tl);
         v.instanced = 1;
     } else {
-        v.nodes = s.bvh.pairs;  // sibling-pair traversal copy
+        v.tree = ray_tree(s.bvh);
+        v.pairs = s.bvh.pairs;
         v.slot_pre = s.bvh.slot_pre;
-        v.node_count = s.bvh.n > 1 ? 2 * s.bvh.n : (s.bvh.n > 0 ? 1 : 0);
+        v.pair_count = s.bvh.n > 1 ? 2 * s.bvh.n : (s.bvh.n > 0 ? 1 : 0);
         v.instanced = 0;
     }
     v.soup = s.soup;

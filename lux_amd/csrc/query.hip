@@ -44,158 +44,29 @@ __device__ __forceinline__ RayIn load_ray(const lux_ray* rays, int i) {
     return r;
 }
 
-__device__ __forceinline__ void load_tri(const lux_triangle* tris, int i, f3& v0, f3& v1, f3& v2) {
-    const float* p = reinterpret_cast<const float*>(tris + i);
-    v0 = make3(p[0], p[1], p[2]);
-    v1 = make3(p[3], p[4], p[5]);
-    v2 = make3(p[6], p[7], p[8]);
-}
-
-// The tree as the ray kernels read it: the right-first preorder node array and
-// the four-child records over it (wide.hpp).
-struct RayTree {
-    const lux_bvh_node* nodes;
-    const WideNode* wide;
-    const int32_t* wide_leaf;
-    int node_count;    // 2 n - 1
-    uint32_t records;  // n - 1, or 0: the preorder walk only
-};
-
-// Right-first preorder walk: the rays that the wide walk hands back, one-leaf
-// trees and trees beyond 32-bit record offsets.
-// kAny = false: closest hit; kAny = true: stop at the first accepted triangle.
-// visits/tests count node loads and triangle tests (only read by the stats kernel).
+// One ray (wide.hpp): the records' walk, or the preorder walk where it hands the
+// ray back.
 template <bool kAny>
-__device__ __forceinline__ int walk_preorder(const lux_bvh_node* __restrict__ nodes, int node_count,
-                                          const lux_triangle* __restrict__ tris, int tri_count, const RayIn& ray,
-                                          float& t_best, DevInfo* info, uint32_t& visits, uint32_t& tests) {
-    const SlabRay sr = make_slab_ray(ray.o, ray.d, ray.t_min);
-    float t_max = __builtin_canonicalizef(ray.t_max);
-    int best = -1;
-    int k = 0;
-    bool bad_prim = false, bad_order = false;
-    while (uint32_t(k) < uint32_t(node_count)) {
-        float4 a, b;
-        load_node(nodes, k, a, b);
-        ++visits;
-        const int prim = __float_as_int(b.z);
-        const bool pass = slab_hit(sr, t_max, a.x, a.y, a.z, a.w, b.x, b.y);
-        int next = (pass && prim < 0) ? k + 1 : __float_as_int(b.w);
-        bad_prim |= pass && prim >= tri_count;
-        if (pass && prim >= 0 && prim < tri_count) {
-            f3 v0, v1, v2;
-            load_tri(tris, prim, v0, v1, v2);
-            ++tests;
-            float t, u, v;
-            if (tri_hit(ray.o, ray.d, ray.t_min, t_max, v0, v1, v2, t, u, v)) {
-                best = prim;
-                t_max = t;
-                if (kAny) next = -1;  // done
-            }
-        }
-        if (next >= 0 && next <= k) {  // preorder positions only grow
-            bad_order = true;
-            break;
-        }
-        k = next;
-    }
-    if (bad_prim) set_error(info, kErrPrimRange);
-    if (bad_order) set_error(info, kErrWalkOrder);
-    t_best = t_max;
-    return best;
-}
-
-// What one lane's walk of a ray found: a hit's primitive (-1: none), its leaf
-// child (4 * record + child) and distance (a miss: the ray's t_max), and whether
-// the ray is the preorder walk's to decide.
-struct Found {
-    int best = -1;
-    uint32_t at = 0;
-    float t = 0;
-    bool failed = false;
-};
-
-// A lane's walk (wide.hpp) of the boxes met in [lo, hi] of its ray; sr.t_min =
-// lo. `group` lanes in a row (a power of two) walk one ray between them and share
-// the nearest hit (any hit: that there is one); with `skip` a lane only listens.
-template <bool kAny>
-__device__ __forceinline__ Found walk_part(const RayTree& tree, const lux_triangle* __restrict__ tris, int tri_count,
-                                           const RayIn& ray, const SlabRay& sr, float hi, int group, bool skip, uint32_t* stack,
-                                           DevInfo* info, uint32_t& visits, uint32_t& tests) {
-    Found f;
-    f.t = __builtin_canonicalizef(ray.t_max);
-    float t_cull = wide_bound(hi);
-    bool bad = false, bad_prim = false;
-    auto leaf = [&](uint32_t at, uint32_t ref) {
-        const uint32_t prim = ref & kIndexMask;
-        if (prim >= uint32_t(tri_count)) {
-            bad_prim |= ref != kWideEmpty;
-            return false;
-        }
-        f3 v0, v1, v2;
-        load_tri(tris, int(prim), v0, v1, v2);
-        ++tests;
-        float t, u, v;
-        if (!tri_uvt(ray.o, ray.d, v0, v1, v2, t, u, v) || !(t > ray.t_min)) return false;
-        if (t < f.t || (!kAny && f.best >= 0 && t == f.t && tree.wide_leaf[at] < tree.wide_leaf[f.at])) {
-            f.best = int(prim);
-            f.at = at;
-            if (kAny) return true;
-            f.t = t;
-            t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
-        }
-        return false;
-    };
-    auto share = [&]() {
-        if (group == 1) return false;
-        if (kAny) {
-            int any = f.best >= 0;
-            for (int off = 1; off < group; off <<= 1) any |= __shfl_xor(any, off, 64);
-            return any != 0;
-        }
-        float t = f.best >= 0 ? f.t : INFINITY;
-        for (int off = 1; off < group; off <<= 1) t = fminf(t, __shfl_xor(t, off, 64));
-        t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
-        return false;
-    };
-    const bool done =
-        wave_any_parallel(sr)
-            ? wide_walk<true>(tree.wide, tree.records, sr, t_cull, skip, stack, kBlock, visits, bad, leaf, share)
-            : wide_walk<false>(tree.wide, tree.records, sr, t_cull, skip, stack, kBlock, visits, bad, leaf, share);
-    if (bad_prim) set_error(info, kErrPrimRange);
-    if (bad) set_error(info, kErrWalkOrder);
-    f.failed = !done;
-    return f;
-}
-
-// One ray on one lane. A ray the wide walk cannot settle is walked again in
-// preorder. With t_max fixed, whether a leaf's box passes does not depend on the
-// visit order, so an any-hit walk may end at any triangle hit in a leaf whose own
-// box passes; near child first meets one soon.
-template <bool kAny>
-__device__ __forceinline__ int trace_one(const RayTree& tree, const lux_triangle* __restrict__ tris, int tri_count,
-                                         const RayIn& ray, float& t_best, uint32_t* stack, DevInfo* info,
-                                         uint32_t& visits, uint32_t& tests) {
-    if (tree.records != 0 && wide_takes(ray.d)) {
-        const SlabRay sr = make_slab_ray(ray.o, ray.d, ray.t_min);
-        const Found f =
-            walk_part<kAny>(tree, tris, tri_count, ray, sr, ray.t_max, 1, false, stack, info, visits, tests);
-        if (!f.failed && (f.best < 0 || wide_settled(tree.nodes, tree.wide_leaf[f.at], sr, f.t))) {
-            t_best = f.t;
-            return f.best;
-        }
-    }
-    return walk_preorder<kAny>(tree.nodes, tree.node_count, tris, tri_count, ray, t_best, info, visits, tests);
+__device__ __forceinline__ WideHit trace_one(const RayTree& tree, const lux_triangle* __restrict__ tris,
+                                             int tri_count, const RayIn& ray, int group, int part, uint32_t* stack,
+                                             DevInfo* info, uint32_t& visits, uint32_t& tests) {
+    // canonical from the start, so the loop's min/max need no per-step canonicalise
+    const float t_max = __builtin_canonicalizef(ray.t_max);
+    WideHit h = wide_query(tree, tris, tri_count, ray.o, ray.d, ray.t_min, t_max, kAny, -1, group, part, stack,
+                           kBlock, info, visits, tests);
+    if (h.failed && part == 0)
+        h = preorder_query(tree, tris, tri_count, ray.o, ray.d, ray.t_min, t_max, kAny, -1, info, visits, tests);
+    return h;
 }
 
 template <bool kAny>
-__device__ __forceinline__ void store_result(void* __restrict__ out, int ray, int id, float t) {
+__device__ __forceinline__ void store_result(void* __restrict__ out, int ray, const WideHit& found) {
     if (kAny) {
-        static_cast<uint8_t*>(out)[ray] = id >= 0 ? 1 : 0;
+        static_cast<uint8_t*>(out)[ray] = found.prim >= 0 ? 1 : 0;
     } else {
         lux_hit h;
-        h.primitive_id = id;
-        h.t = id >= 0 ? t : INFINITY;
+        h.primitive_id = found.prim;
+        h.t = found.prim >= 0 ? found.t : INFINITY;
         static_cast<lux_hit*>(out)[ray] = h;
     }
 }
@@ -224,21 +95,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
         set_error(info, kErrSpinLimit);
         return;
     }
-    const RayIn r = load_ray(rays, ray);
-    float t;
     uint32_t visits = 0, tests = 0;
-    const int id = trace_one<kAny>(tree, tris, tri_count, r, t, stack + threadIdx.x, info, visits, tests);
-    store_result<kAny>(out, ray, id, t);
+    store_result<kAny>(out, ray, trace_one<kAny>(tree, tris, tri_count, load_ray(rays, ray), 1, 0, stack + threadIdx.x, info, visits, tests));
 }
 
-// Few rays: `group` lanes (a power of two up to 64) walk one ray, each a part of
-// the interval in which it meets the root box. A call that leaves most of the
-// chip idle lasts as long as its longest walk, a chain of dependent loads; parts
-// cut the chain (2^20 random triangles, 2^14 random rays: 330 records for the
-// longest ray, 148 in 4 parts, 87 in 8) for more records in all (50, 130 and 194
-// a ray). A box met by the ray in [t_min, t_max] is met in some part, so every
-// triangle the whole walk tests is tested by some lane; the hit is the smallest
-// (t, preorder position) over the lanes, as it is over one lane's walk.
+// Few rays: `group` lanes (a power of two) walk one ray (wide_query).
 template <bool kAny>
 __global__ __launch_bounds__(kBlock) void k_trace_parts(RayTree tree, const lux_triangle* __restrict__ tris,
                                                         int tri_count, const lux_ray* __restrict__ rays, int n,
@@ -253,53 +114,9 @@ __global__ __launch_bounds__(kBlock) void k_trace_parts(RayTree tree, const lux_
         set_error(info, kErrSpinLimit);
         return;
     }
-    const RayIn r = load_ray(rays, ray);
     uint32_t visits = 0, tests = 0;
-    int id = -1;
-    float t = 0;
-    bool settled = false;
-    if (wide_takes(r.d)) {  // the same on every lane of the group
-        SlabRay sr = make_slab_ray(r.o, r.d, r.t_min);
-        // the root box, with a margin; an interval that is empty or not finite
-        // leaves the whole ray to the first lane
-        float4 a, b;
-        load_node(tree.nodes, 0, a, b);
-        float enter;
-        (void)slab_near<true>(sr, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, enter);
-        const float fx = (sr.neg_x ? a.x : a.w) - r.o.x, fy = (sr.neg_y ? a.y : b.x) - r.o.y,
-                    fz = (sr.neg_z ? a.z : b.y) - r.o.z;
-        float leave = r.t_max;
-        if (!sr.par_x) leave = fminf(leave, fx * sr.inv.x);
-        if (!sr.par_y) leave = fminf(leave, fy * sr.inv.y);
-        if (!sr.par_z) leave = fminf(leave, fz * sr.inv.z);
-        const float step = (leave - enter) / float(group);
-        const bool cut = step > 0.0f && step < 1e30f;
-        const float lo = enter + step * float(part), hi = enter + step * float(part + 1);
-        if (cut && part != 0) sr.t_min = lo;
-        const Found f = walk_part<kAny>(tree, tris, tri_count, r, sr, cut && part + 1 < group ? hi : r.t_max, group,
-                                        !cut && part != 0, stack + threadIdx.x, info, visits, tests);
-        sr.t_min = r.t_min;
-        // the smallest (t, position) of the group, on every lane
-        int pos = f.best >= 0 ? tree.wide_leaf[f.at] : INT32_MAX;
-        float bt = f.best >= 0 ? f.t : INFINITY;
-        int bid = f.best, fail = f.failed;
-        for (int off = 1; off < group; off <<= 1) {
-            const float ot = __shfl_xor(bt, off, 64);
-            const int op = __shfl_xor(pos, off, 64), oid = __shfl_xor(bid, off, 64);
-            fail |= __shfl_xor(fail, off, 64);
-            if (oid >= 0 && (bid < 0 || (kAny ? op < pos : (ot < bt || (ot == bt && op < pos))))) {
-                bt = ot;
-                pos = op;
-                bid = oid;
-            }
-        }
-        id = bid;
-        t = bt;
-        settled = !fail && (bid < 0 || wide_settled(tree.nodes, pos, sr, kAny ? r.t_max : bt));
-    }
-    if (part != 0) return;
-    if (!settled) id = walk_preorder<kAny>(tree.nodes, tree.node_count, tris, tri_count, r, t, info, visits, tests);
-    store_result<kAny>(out, ray, id, t);
+    const WideHit h = trace_one<kAny>(tree, tris, tri_count, load_ray(rays, ray), group, part, stack + threadIdx.x, info, visits, tests);
+    if (part == 0) store_result<kAny>(out, ray, h);
 }
 
 // The walks of the handle, counting per ray the 32-byte node units loaded (two
@@ -314,10 +131,9 @@ __global__ __launch_bounds__(kBlock) void k_trace_stats(RayTree tree, const lux_
     int i = blockIdx.x * kBlock + threadIdx.x;
     uint32_t v0 = 0, t0 = 0, v1 = 0, t1 = 0;
     if (i < n) {
-        RayIn r = load_ray(rays, i);
-        float t;
-        trace_one<false>(tree, tris, tri_count, r, t, stack + threadIdx.x, info, v0, t0);
-        trace_one<true>(tree, tris, tri_count, r, t, stack + threadIdx.x, info, v1, t1);
+        const RayIn r = load_ray(rays, i);
+        (void)trace_one<false>(tree, tris, tri_count, r, 1, 0, stack + threadIdx.x, info, v0, t0);
+        (void)trace_one<true>(tree, tris, tri_count, r, 1, 0, stack + threadIdx.x, info, v1, t1);
     }
     unsigned long long c[6] = {v0, 0, t0, v1, 0, t1};
 #pragma unroll
@@ -569,34 +385,11 @@ const uint32_t* closest_order(RaySortDev& r, bool sort, const BvhDev& d, const l
 }
 
 namespace {
-RayTree ray_tree(const BvhDev& d) {
-    RayTree t;
-    t.nodes = d.nodes;
-    t.wide = d.wide;
-    t.wide_leaf = d.wide_leaf;
-    t.node_count = d.n > 0 ? 2 * d.n - 1 : 0;
-    t.records = (d.n > 1 && uint32_t(d.n) <= kMaxWideRecords) ? uint32_t(d.n - 1) : 0u;
-    return t;
-}
-}  // namespace
-
-namespace {
-// Lanes per ray of a call of n rays (k_trace_parts): where the calls that leave
-// the chip idle end. Closest hit, 1 / 4 / 8 / 16 lanes: 2^14 rays in 2^20 random
-// triangles (with their build) 884 / 648 / 590 / 569 us, 2^15 395 / 165 / 123 /
-// 135, 2^16 in 2^18 (with the refit) 431 / 260 / 257 / 283; 2^17 in 500 000
-// 382 / 277 / 285, on a sphere mesh 133 / 119 / 122; at 2^18 one lane is the
-// best for the soup (422 / 455) and within 6 % on the sphere.
-int lanes_per_ray(const RayTree& tree, int n) {
-    if (tree.records == 0) return 1;
-    return n <= (1 << 14) ? 16 : n <= (1 << 16) ? 8 : n <= (1 << 17) ? 4 : 1;
-}
-
 template <bool kAny>
 void launch_trace(const char* name, const BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
                   const lux_ray* rays, int n, void* out, hipStream_t s) {
     const RayTree tree = ray_tree(d);
-    const int group = lanes_per_ray(tree, n);
+    const int group = tree.records ? lanes_per_ray(uint32_t(n)) : 1;
     if (group > 1)
         LUX_LAUNCH(name, k_trace_parts<kAny>, div_up(int64_t(n) * group, kBlock), kBlock, 0, s, tree, tris, tri_count,
                    rays, n, order, group, out, d.info);

@@ -45,6 +45,7 @@
 // preorder walk for that ray.
 #pragma once
 
+#include "lux_runtime.hpp"
 #include "ordered.hpp"
 
 namespace lux {
@@ -278,6 +279,198 @@ __device__ __forceinline__ bool wide_walk(const WideNode* __restrict__ wide, uin
         if (share()) done = true;
     }
     return !overflow;
+}
+
+// A tree as the ray kernels read it: the right-first preorder node array and the
+// four-child records over it.
+struct RayTree {
+    const lux_bvh_node* nodes;
+    const WideNode* wide;
+    const int32_t* wide_leaf;
+    int32_t node_count;  // 2 n - 1
+    uint32_t records;    // n - 1, or 0: the preorder walk only
+};
+
+inline RayTree ray_tree(const BvhDev& d) {
+    RayTree t;
+    t.nodes = d.nodes;
+    t.wide = d.wide;
+    t.wide_leaf = d.wide_leaf;
+    t.node_count = d.n > 0 ? 2 * d.n - 1 : 0;
+    t.records = (d.n > 1 && uint32_t(d.n) <= kMaxWideRecords) ? uint32_t(d.n - 1) : 0u;
+    return t;
+}
+
+// A ray's hit: primitive (-1: none), distance, its leaf's preorder position;
+// failed: the preorder walk decides.
+struct WideHit {
+    int prim = -1;
+    int pos = 0;
+    float t = 0;
+    bool failed = false;
+};
+
+// Lanes per ray of a launch over n rays whose walks leave the chip idle: where
+// the parts of wide_query pay. Closest hit, 1 / 4 / 8 / 16 lanes: 2^14 rays in
+// 2^20 random triangles (with their build) 884 / 648 / 590 / 569 us, 2^15 395 /
+// 165 / 123 / 135, 2^16 in 2^18 (with the refit) 431 / 260 / 257 / 283; 2^17 in
+// 500 000 382 / 277 / 285, on a sphere mesh 133 / 119 / 122; at 2^18 one lane is
+// the best for the soup (422 / 455) and within 6 % on the sphere.
+constexpr uint32_t kPartsMaxRays = 1u << 17;
+__host__ __device__ inline int lanes_per_ray(uint32_t n) {
+    return n <= (1u << 14) ? 16 : n <= (1u << 16) ? 8 : n <= kPartsMaxRays ? 4 : 1;
+}
+
+// One ray, on `group` lanes in a row (a power of two; 1: a lane by itself), this
+// lane walking part `part` of the interval in which the ray meets the root box.
+// Every lane of a group has the same ray and gets the group's result. any: any
+// hit in (t_min, t_max), otherwise the closest; `ignore` is a primitive to pass
+// over (-1: none).
+// A launch that leaves most of the chip idle lasts as long as its longest walk, a
+// chain of dependent loads; parts cut the chain (2^20 random triangles, 2^14
+// random rays: 330 records for the longest ray, 148 in 4 parts, 87 in 8) for more
+// records in all (50, 130 and 194 a ray). A box met by the ray in [t_min, t_max]
+// is met in some part, so every triangle the whole walk tests is tested by some
+// lane; the hit is the smallest (t, preorder position) over the lanes, as it is
+// over one lane's walk. With t_max fixed, whether a leaf's box passes does not
+// depend on the visit order, so an any-hit walk may end at any triangle hit in a
+// leaf whose own box passes; near child first meets one soon.
+__device__ __forceinline__ WideHit wide_query(const RayTree& tree, const lux_triangle* __restrict__ tris,
+                                              int tri_count, const f3& o, const f3& d, float t_min, float t_bound,
+                                              bool any, int ignore, int group, int part, uint32_t* stack, int stride,
+                                              DevInfo* info, uint32_t& visits, uint32_t& tests) {
+    WideHit hit;
+    if (tree.records == 0 || !wide_takes(d)) {
+        hit.failed = true;
+        return hit;
+    }
+    SlabRay sr = make_slab_ray(o, d, t_min);
+    float hi = t_bound;
+    bool skip = false;
+    if (group > 1) {
+        // an interval in the root box that is empty or not finite leaves the whole
+        // ray to the first lane
+        float4 a, b;
+        load_node(tree.nodes, 0, a, b);
+        float enter;
+        (void)slab_near<true>(sr, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, enter);
+        float leave = t_bound;
+        if (!sr.par_x) leave = fminf(leave, ((sr.neg_x ? a.x : a.w) - o.x) * sr.inv.x);
+        if (!sr.par_y) leave = fminf(leave, ((sr.neg_y ? a.y : b.x) - o.y) * sr.inv.y);
+        if (!sr.par_z) leave = fminf(leave, ((sr.neg_z ? a.z : b.y) - o.z) * sr.inv.z);
+        const float step = (leave - enter) / float(group);
+        const bool cut = step > 0.0f && step < 1e30f;
+        skip = !cut && part != 0;
+        if (cut && part + 1 < group) hi = enter + step * float(part + 1);
+        if (cut && part != 0) sr.t_min = enter + step * float(part);
+    }
+    float t_max = t_bound;  // the held bound
+    float t_cull = wide_bound(hi);
+    int best = -1;
+    uint32_t best_at = 0;
+    bool bad = false, bad_prim = false;
+    auto leaf = [&](uint32_t at, uint32_t ref) {
+        const uint32_t prim = ref & kIndexMask;
+        if (int(prim) == ignore) return false;
+        if (prim >= uint32_t(tri_count)) {
+            bad_prim |= ref != kWideEmpty;
+            return false;
+        }
+        const float* p = reinterpret_cast<const float*>(tris + prim);
+        ++tests;
+        float t, u, v;
+        if (!tri_uvt(o, d, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), t, u, v) ||
+            !(t > t_min))
+            return false;
+        if (t < t_max || (!any && best >= 0 && t == t_max && tree.wide_leaf[at] < tree.wide_leaf[best_at])) {
+            best = int(prim);
+            best_at = at;
+            if (any) return true;
+            t_max = t;
+            t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
+        }
+        return false;
+    };
+    auto share = [&]() {
+        if (group == 1) return false;
+        float t = best < 0 ? INFINITY : any ? -INFINITY : t_max;
+        for (int off = 1; off < group; off <<= 1) t = fminf(t, __shfl_xor(t, off, 64));
+        if (any) return t < INFINITY;
+        t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
+        return false;
+    };
+    hit.failed = wave_any_parallel(sr)
+                     ? !wide_walk<true>(tree.wide, tree.records, sr, t_cull, skip, stack, stride, visits, bad, leaf, share)
+                     : !wide_walk<false>(tree.wide, tree.records, sr, t_cull, skip, stack, stride, visits, bad, leaf, share);
+    if (bad_prim) set_error(info, kErrPrimRange);
+    if (bad) set_error(info, kErrWalkOrder);
+    hit.prim = best;
+    hit.t = t_max;
+    if (best >= 0) hit.pos = tree.wide_leaf[best_at];
+    if (group > 1) {
+        // the smallest (t, position) of the group, on every lane
+        int fail = hit.failed;
+        for (int off = 1; off < group; off <<= 1) {
+            const float ot = __shfl_xor(hit.t, off, 64);
+            const int op = __shfl_xor(hit.pos, off, 64), oid = __shfl_xor(hit.prim, off, 64);
+            fail |= __shfl_xor(fail, off, 64);
+            const bool before = (!any && ot != hit.t) ? ot < hit.t : op < hit.pos;
+            if (oid >= 0 && (hit.prim < 0 || before)) {
+                hit.t = ot;
+                hit.pos = op;
+                hit.prim = oid;
+            }
+        }
+        hit.failed = fail != 0;
+    }
+    if (!hit.failed && hit.prim >= 0) {
+        sr.t_min = t_min;
+        hit.failed = !wide_settled(tree.nodes, hit.pos, sr, hit.t);
+    }
+    return hit;
+}
+
+// Right-first preorder walk: the rays that wide_query hands back, one-leaf trees
+// and trees beyond 32-bit record offsets. any: stop at the first accepted
+// triangle. visits counts node loads, tests triangle tests.
+__device__ __forceinline__ WideHit preorder_query(const RayTree& tree, const lux_triangle* __restrict__ tris,
+                                                  int tri_count, const f3& o, const f3& d, float t_min,
+                                                  float t_bound, bool any, int ignore, DevInfo* info,
+                                                  uint32_t& visits, uint32_t& tests) {
+    const SlabRay sr = make_slab_ray(o, d, t_min);
+    WideHit hit;
+    hit.t = t_bound;
+    int k = 0;
+    bool bad_prim = false, bad_order = false;
+    while (uint32_t(k) < uint32_t(tree.node_count)) {
+        float4 a, b;
+        load_node(tree.nodes, k, a, b);
+        ++visits;
+        const int prim = __float_as_int(b.z);
+        const bool pass = slab_hit(sr, hit.t, a.x, a.y, a.z, a.w, b.x, b.y);
+        int next = (pass && prim < 0) ? k + 1 : __float_as_int(b.w);
+        const bool test = pass && prim >= 0 && prim != ignore;
+        bad_prim |= test && prim >= tri_count;
+        if (test && prim < tri_count) {
+            const float* p = reinterpret_cast<const float*>(tris + prim);
+            ++tests;
+            float t, u, v;
+            if (tri_hit(o, d, t_min, hit.t, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]),
+                        make3(p[6], p[7], p[8]), t, u, v)) {
+                hit.prim = prim;
+                hit.t = t;
+                if (any) next = -1;  // done
+            }
+        }
+        if (next >= 0 && next <= k) {  // preorder positions only grow
+            bad_order = true;
+            break;
+        }
+        k = next;
+    }
+    if (bad_prim) set_error(info, kErrPrimRange);
+    if (bad_order) set_error(info, kErrWalkOrder);
+    return hit;
 }
 
 }  // namespace lux
