@@ -63,3 +63,36 @@ def test_film_output_argument_errors(gpu, tmp_path):
     with pytest.raises(abi.LuxError) as e:
         abi.call("lux_hip_write_pfm", str(tmp_path / "x.pfm").encode(), d.ptr, -1, 1, 1)
     assert e.value.status == abi.LUX_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("size", [(1, 1), (1, 5), (7, 3), (64, 16), (37, 29)])
+def test_ppm_bytes_around_thresholds(gpu, size, offset):
+    """Values on both sides of every byte threshold, film sizes with one to three
+    values left over, buffers that are not aligned for wide loads and stores."""
+    import ctypes
+
+    print_case("ppm thresholds", size, offset)
+    w, h = size
+    t = np.zeros(255, np.float32)
+    abi.call("lux_hip_ppm_thresholds", t.ctypes.data_as(ctypes.c_void_p))
+    x = (t[:-1].astype(np.float64) / (1.0 - t[:-1].astype(np.float64))).astype(np.float32)  # c = x / (1 + x)
+    near = [x]
+    for _ in range(3):
+        near += [np.nextafter(near[-1], np.float32(np.inf)), np.nextafter(near[0] if len(near) == 1 else near[-2],
+                                                                          np.float32(0))]
+    special = np.array([0.0, -0.0, -1.0, np.nan, np.inf, -np.inf, 1e-45, 1e-38, 1e38], np.float32)
+    vals = np.concatenate(near + [special])
+    film = np.resize(np.roll(vals, -17 * w), 3 * w * h).astype(np.float32).reshape(h, w, 3)
+    d_film, d_out = lbvh.DeviceArray(4 * (3 * w * h + 1)), lbvh.DeviceArray(3 * w * h + 1)
+
+    class At:
+        def __init__(self, base, by):
+            self.ptr = ctypes.c_void_p(base.ptr.value + by)
+
+    abi.call("lux_hip_memcpy_htod", At(d_film, 4 * offset).ptr, film.ctypes.data_as(ctypes.c_void_p),
+             ctypes.c_size_t(film.nbytes))
+    F.ppm_pixels_device(At(d_film, 4 * offset), w, h, 1, At(d_out, offset))
+    lbvh.synchronize()
+    got = d_out.to_numpy(np.uint8, (3 * w * h + 1,))[offset:offset + 3 * w * h]
+    assert np.array_equal(got, oracle.film_file("ppm", film, 1)[-3 * w * h:])
