@@ -140,7 +140,7 @@ int lux_hip_bvh_refit_triangles_device(lux_hip_bvh* bvh,
                                        const lux_triangle* d_triangles, int32_t n,
                                        lux_stream stream);
 
-/* Closest-hit and any-hit calls with at least 65 536 rays trace them sorted by
+/* Closest-hit and any-hit calls with at least 2^21 rays trace them sorted by
  * direction octant, then by the Morton code of their origins (2-pass radix
  * sort of 16 key bits); hits and occlusion flags still land at each ray's own
  * index and are identical either way. On by default; enable = 0 traces in

@@ -1129,6 +1129,14 @@ __global__ __launch_bounds__(kBlock) void k_copies(int n, int wide_blocks, const
 
 }  // namespace
 
+void wide_from(const BvhDev& d, const lux_bvh_node* nodes, WideNode* wide, int32_t* wide_leaf, hipStream_t s) {
+    if (d.n < 2) return;
+    const int blocks = min(4096, div_up(d.n - 1, kBlock));
+    LUX_LAUNCH("lbvh_copies", k_copies, blocks, kBlock, 0, s, d.n, blocks, (const uint32_t*)d.left,
+               (const uint32_t*)d.right, (const int32_t*)d.pre_internal, (const int32_t*)d.pre_leaf, nodes, wide,
+               wide_leaf, (const uint32_t*)nullptr, (lux_bvh_node*)nullptr, (uint32_t*)nullptr, d.info);
+}
+
 // The traversal copies of the node array (build and refit).
 void fill_copies(BvhDev& d, hipStream_t s) {
     if (d.n <= 0) return;

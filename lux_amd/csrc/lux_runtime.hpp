@@ -165,6 +165,10 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
 void lbvh_build_triangles(BvhDev& d, const lux_triangle* tris, const lux_vec3* verts, const uint32_t* idx, int nv,
                           int n, hipStream_t s);
 
+// Enqueues the four-child records (n - 1, and 4 leaf positions each) of tree d's
+// topology over another node array of its preorder positions.
+void wide_from(const BvhDev& d, const lux_bvh_node* nodes, WideNode* wide, int32_t* wide_leaf, hipStream_t s);
+
 // Film output (film.hip): write_ppm's pixel bytes (3 per pixel, film order),
 // write_pfm's float body (rows bottom to top), both from a device film of
 // per-pixel sums; whole-file writers; the 255 gamma thresholds of the byte

@@ -176,63 +176,11 @@ __device__ __forceinline__ bool slab_near(SlabMode<kMode>, const SlabRay& r, flo
 // words apart. Returns false when the stack overflowed (the walk stopped
 // early); *bad is set on a malformed array (child slot out of range, a pair
 // entered twice).
-template <int kMode, typename Leaf>
-__device__ __forceinline__ bool ordered_walk(SlabMode<kMode> mode, const lux_bvh_node* __restrict__ nodes,
-                                             uint32_t node_count, const SlabRay& sr, OrderedBest& best,
-                                             uint32_t* stack, int stride, uint32_t& visits, bool& bad, Leaf&& leaf) {
-    float4 a, b;
-    load_node32(nodes, 0, a, b);
-    ++visits;
-    float tn;
-    if (!slab_near(mode, sr, best.t_cull, a.x, a.y, a.z, a.w, b.x, b.y, tn)) return true;
-    const int root = __float_as_int(b.z);
-    if (root >= 0) {
-        (void)leaf(0u, root, tn);
-        return true;
-    }
-    uint32_t c = ~uint32_t(root);
-    int sp = 0;
-    int guard = int(node_count / 2) + 1;  // each internal node's pair is entered once
-    const uint32_t last_pair = node_count - 1;  // a pair slot c needs c + 1 < node_count
-    const lux_bvh_node* const nodes1 = nodes + 1;  // both nodes of a pair load from one offset
-    for (;;) {
-        if (c >= last_pair || --guard < 0) {
-            bad = true;
-            return true;
-        }
-        float4 a0, b0, a1, b1;
-        load_node32(nodes, c, a0, b0);
-        load_node32(nodes1, c, a1, b1);
-        visits += 2;
-        float tn0, tn1;
-        const bool h0 = slab_near(mode, sr, best.t_cull, a0.x, a0.y, a0.z, a0.w, b0.x, b0.y, tn0);
-        const bool h1 = slab_near(mode, sr, best.t_cull, a1.x, a1.y, a1.z, a1.w, b1.x, b1.y, tn1);
-        const int p0 = __float_as_int(b0.z), p1 = __float_as_int(b1.z);
-        if (h0 && p0 >= 0 && leaf(c, p0, tn0)) return true;
-        if (h1 && p1 >= 0 && leaf(c + 1, p1, tn1)) return true;
-        const bool i0 = h0 && p0 < 0, i1 = h1 && p1 < 0;
-        if (i0 && i1) {
-            const bool far0 = tn1 < tn0;
-            if (sp == kOrderedStack) return false;
-            stack[sp * stride] = far0 ? ~uint32_t(p0) : ~uint32_t(p1);
-            ++sp;
-            c = far0 ? ~uint32_t(p1) : ~uint32_t(p0);
-        } else if (i0 || i1) {
-            c = ~uint32_t(i0 ? p0 : p1);
-        } else {
-            if (sp == 0) return true;
-            --sp;
-            c = stack[sp * stride];
-        }
-    }
-}
-
-// ordered_walk with the triangle tests gathered across the wave: a lane whose
+// The triangle tests are gathered across the wave: a lane whose
 // step passes one or both leaf children holds them and does not step again
 // until they are tested (its next slab tests depend on the t_cull they may
 // lower); the wave tests the held leaves together once a quarter of its
-// working lanes hold some, or none can step on. Each lane's sequence of box
-// tests, leaf tests and stack operations is that of ordered_walk.
+// working lanes hold some, or none can step on.
 template <int kMode, typename Leaf>
 __device__ __forceinline__ bool ordered_walk_gathered(SlabMode<kMode> mode, const lux_bvh_node* __restrict__ nodes,
                                                       uint32_t node_count, const SlabRay& sr, OrderedBest& best,

@@ -211,36 +211,15 @@ __device__ __forceinline__ bool occluded(const SceneView& sv, const vec& o, cons
     return closest_walk<false, true>(sv, O, D, sr, t_min, t_max, ignore, t, u, v) >= 0;
 }
 
-// The same two queries on an instanced scene: the two-level walk (TLAS, then
-// the BLAS of each instance the ray reaches, in object space), returning the
-// scene ordinal. stack as for closest().
-template <bool kTwoLevel>
-__device__ __forceinline__ int scene_closest(const SceneView& sv, const vec& o, const vec& d, float t_min,
-                                             float t_max, int ignore, float& t_hit, float& u_hit, float& v_hit,
-                                             uint32_t* stack, int stride) {
-    if constexpr (!kTwoLevel) return closest(sv, o, d, t_min, t_max, ignore, t_hit, u_hit, v_hit, stack, stride);
+// One ray of an instanced scene (two_level.hpp), given by world(o, d): the closest
+// hit, or any hit.
+template <typename World>
+__device__ __forceinline__ TwoLevelHit instanced_query(const SceneView& sv, World&& world, float t_max, bool any, int ignore, int group, int part,
+                                                       uint32_t* stack, int stride) {
     TwoLevelHit h;
-    const bool ordered = stack && !sv.preorder;
-    if (!ordered || !two_level_closest_ordered(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max,
-                                               ignore, stack, stride, h))
-        h = two_level_walk<false>(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max, ignore);
-    if (h.prim >= 0) {
-        t_hit = h.t;
-        u_hit = h.u;
-        v_hit = h.v;
-    } else {
-        t_hit = t_max;
-    }
-    return h.prim;
-}
-
-template <bool kTwoLevel>
-__device__ __forceinline__ bool scene_occluded(const SceneView& sv, const vec& o, const vec& d, float t_min,
-                                               float t_max, int ignore) {
-    if constexpr (kTwoLevel)
-        return two_level_any(sv.tl, make3(o.x, o.y, o.z), make3(d.x, d.y, d.z), t_min, t_max, ignore);
-    else
-        return occluded(sv, o, d, t_min, t_max, ignore);
+    if (sv.preorder || !two_level_wide<true>(sv.tl, world, kEps, t_max, any, ignore, group, part, stack, stride, h))
+        h = two_level_walk(sv.tl, world, kEps, t_max, any, ignore);
+    return h;
 }
 
 // One ray of a one-mesh scene on `group` lanes (wide_query): the closest hit, or
@@ -356,7 +335,7 @@ __device__ __forceinline__ void shadow_arrives(const Paths& ps, uint32_t i, uint
     }
 }
 
-template <bool kAnyShadow, bool kTwoLevel>
+template <bool kAnyShadow>
 __device__ __forceinline__ void shadow_ray(const BatchDesc* __restrict__ desc, const Paths& ps, uint32_t i) {
     const float4 so = ps.so[i], sd = ps.sd[i];
     const uint32_t path = __float_as_uint(ps.sc[i].w);
@@ -367,22 +346,22 @@ __device__ __forceinline__ void shadow_ray(const BatchDesc* __restrict__ desc, c
     float t_max = so.w;
     int ignore = __float_as_int(ps.st[i].w);
     vec tr = splat(1);
-    if (kAnyShadow && scene_occluded<kTwoLevel>(sv, mk(o.x, o.y, o.z), D, kEps, t_max, ignore)) tr = splat(0);
+    if (kAnyShadow && occluded(sv, mk(o.x, o.y, o.z), D, kEps, t_max, ignore)) tr = splat(0);
     for (int guard = 0; !kAnyShadow && guard < 1 << 16; ++guard) {
         float t = 0, u = 0, v = 0;
         // the preorder walk (no stack): with the near-child-first walk inlined a
         // second time here the one-level kernel spilled 36 VGPRs per lane
-        const int prim = scene_closest<kTwoLevel>(sv, mk(o.x, o.y, o.z), D, kEps, t_max, ignore, t, u, v, nullptr, 0);
+        const int prim = closest(sv, mk(o.x, o.y, o.z), D, kEps, t_max, ignore, t, u, v, nullptr, 0);
         if (prim < 0 || !shadow_passes(sv, prim, t, tr, o, d, t_max)) break;
         ignore = -1;
     }
     shadow_arrives(ps, i, path, tr);
 }
 
-// Extension ray i (i < n_ext) or shadow record i - n_ext of a one-mesh scene, on
-// `group` lanes: one walk in the code for both, so a wave may hold both.
-template <bool kAnyShadow>
-__device__ __forceinline__ void mesh_ray(const BatchDesc* __restrict__ desc, const Paths& ps, uint32_t i,
+// Extension ray i (i < n_ext) or shadow record i - n_ext, on `group` lanes (an
+// instanced scene's on one): one walk in the code for both, so a wave may hold both.
+template <bool kAnyShadow, bool kTwoLevel>
+__device__ __forceinline__ void record_ray(const BatchDesc* __restrict__ desc, const Paths& ps, uint32_t i,
                                          uint32_t n_ext, const uint32_t* __restrict__ queue, int group, int part,
                                          uint32_t* stack, int stride) {
     const bool ext = i < n_ext;
@@ -395,15 +374,25 @@ __device__ __forceinline__ void mesh_ray(const BatchDesc* __restrict__ desc, con
     float t_max = ext ? INFINITY : ro.w;
     int ignore = ext ? -1 : __float_as_int(ps.st[j].w);
     vec tr = splat(1);
-    WideHit h;
+    auto world = [&](f3& O, f3& D) {  // read again rather than held through the walk
+        const uint32_t k = ext ? path : i - n_ext;
+        const float4 a = ext ? ps.ro[k] : ps.so[k], b = ext ? ps.rd[k] : ps.sd[k];
+        O = make3(a.x, a.y, a.z);
+        D = make3(b.x, b.y, b.z);
+    };
+    typename std::conditional<kTwoLevel, TwoLevelHit, WideHit>::type h;
     for (int guard = 0; guard < 1 << 16; ++guard) {
-        h = mesh_query(sv, o, d, t_max, kAnyShadow && !ext, ignore, group, part, stack, stride);
+        if constexpr (kTwoLevel)
+            h = instanced_query(sv, world, t_max, kAnyShadow && !ext, ignore, group, part, stack, stride);
+        else
+            h = mesh_query(sv, o, d, t_max, kAnyShadow && !ext, ignore, group, part, stack, stride);
         if (ext) break;
         if (kAnyShadow) {
             if (h.prim >= 0) tr = splat(0);
             break;
         }
         if (h.prim < 0 || !shadow_passes(sv, h.prim, h.t, tr, o, d, t_max)) break;
+        if (kTwoLevel && part == 0) ps.so[j] = make_float4(o.x, o.y, o.z, t_max);
         ignore = -1;
     }
     if (part != 0) return;
@@ -413,10 +402,15 @@ __device__ __forceinline__ void mesh_ray(const BatchDesc* __restrict__ desc, con
     }
     float t = INFINITY, u = 0, v = 0;
     if (h.prim >= 0) {
-        // u, v of the winner, recomputed once rather than carried through the
-        // walk (the same operations give the same bits)
-        const float* p = reinterpret_cast<const float*>(sv.soup + h.prim);
-        (void)tri_uvt(o, d, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), t, u, v);
+        if constexpr (kTwoLevel) {
+            u = h.u;
+            v = h.v;
+        } else {
+            // u, v of the winner, recomputed once rather than carried through the
+            // walk (the same operations give the same bits)
+            const float* p = reinterpret_cast<const float*>(sv.soup + h.prim);
+            (void)tri_uvt(o, d, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), t, u, v);
+        }
         t = h.t;
     }
     ps.hit[path] = make_float4(__int_as_float(h.prim), t, u, v);
@@ -431,16 +425,15 @@ __device__ __forceinline__ void mesh_ray(const BatchDesc* __restrict__ desc, con
 // records, or by records in parts, several lanes per ray (lanes_per_ray). A bounce of a large batch is
 // launched as kWalkMesh and kWalkParts and one of them has the work, by the
 // number of rays left; only the first clears and counts (`own`).
-// Waves per SIMD: pairs 8 (64 VGPRs); records 6 (80 VGPRs, 60 bytes per lane
-// spilled outside the walk; the 327 682-triangle frame took 17.0 / 15.5 / 17.1 /
-// 17.3 ms at 5 / 6 / 7 / 8); two-level 6 (80 VGPRs, 86 uncapped; the instanced
-// field measured 91.6 ms at 6, 96.7 ms at 7 and 113 ms at the natural 5).
+// Waves per SIMD: pairs 8 (64 VGPRs); records 6 (80 VGPRs; the 327 682-triangle
+// frame took 14.6 / 15.5 / 16.6 ms at 6 / 7 / 8); two-level 6 (80 VGPRs; an instanced
+// 640 x 640 frame of 16 samples took 18.6 / 17.8 / 15.0 / 16.6 ms at 4 / 5 / 6 / 8,
+// and 20.1 ms by sibling pairs).
 enum { kWalkTwoLevel, kWalkPairs, kWalkMesh, kWalkParts, kWalkBoth };
 template <int B, bool kAnyShadow, int kWalk>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWalk == kWalkPairs ? 8 : 6))) void k_trace(
     const BatchDesc* __restrict__ desc, Paths ps, Queues qs, int ext_in, int sh_in, int zero_a, int zero_b, int own,
     int other) {
-    constexpr bool kTwoLevel = kWalk == kWalkTwoLevel;
     const uint32_t n_ext = ext_in >= 0 ? qs.counts[ext_in] : 0u;
     const uint32_t n_sh = sh_in >= 0 ? qs.counts[sh_in] : 0u;
     if (own && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -450,7 +443,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWalk == kWal
         qs.rays[1] += n_sh;
     }
     // per-lane stacks
-    constexpr bool kRecords = kWalk == kWalkMesh || kWalk == kWalkParts;
+    constexpr bool kRecords = kWalk != kWalkPairs;
     __shared__ uint32_t lds_stack[(kRecords ? kWideStack : kOrderedStack) * B];
     uint32_t* stack = lds_stack + threadIdx.x;
     const uint32_t total = n_ext + n_sh;
@@ -459,7 +452,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWalk == kWal
         if (other && (total <= kPartsMaxRays) != (kWalk == kWalkParts)) return;  // the other launch's
         const uint32_t* queue = ext_in >= 0 ? qs.q[ext_in] : nullptr;
         for (uint32_t i = xcd_block() * B + threadIdx.x; i < total * group; i += gridDim.x * B)
-            mesh_ray<kAnyShadow>(desc, ps, kWalk == kWalkMesh ? i : i / group, n_ext, queue, int(group),
+            record_ray<kAnyShadow, kWalk == kWalkTwoLevel>(desc, ps, kWalk == kWalkMesh ? i : i / group, n_ext, queue, int(group),
                                  int(i & (group - 1)), stack, B);
         return;
     }
@@ -469,10 +462,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWalk == kWal
             const float4 o = ps.ro[path], d = ps.rd[path];
             const SceneView& sv = desc->seg[__float_as_uint(d.w)].sv;
             float t = INFINITY, u = 0, v = 0;
-            const int prim = scene_closest<kTwoLevel>(sv, xyz(o), xyz(d), kEps, INFINITY, -1, t, u, v, stack, B);
+            const int prim = closest(sv, xyz(o), xyz(d), kEps, INFINITY, -1, t, u, v, stack, B);
             ps.hit[path] = make_float4(__int_as_float(prim), t, u, v);
         } else {
-            shadow_ray<kAnyShadow, kTwoLevel>(desc, ps, i - n_ext);
+            shadow_ray<kAnyShadow>(desc, ps, i - n_ext);
         }
     }
 }
@@ -1365,7 +1358,7 @@ void wavefront_sequence(const PathBuf& buf, int walk, int depth, LaunchGrid grid
     } while (0)
     auto trace = [&](int ext_in, int sh_in, int zero_a, int zero_b) {
         if constexpr (kTwoLevel) {
-            PT_LAUNCH("pt_trace", grid.grid, (k_trace<B, kOpaque, kWalkTwoLevel>), d, ps, qs, ext_in, sh_in, zero_a,
+            PT_LAUNCH("pt_trace", grid.trace, (k_trace<B, kOpaque, kWalkTwoLevel>), d, ps, qs, ext_in, sh_in, zero_a,
                       zero_b, 1, 0);
         } else {
             const int both = walk == kWalkBoth;

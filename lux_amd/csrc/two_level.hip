@@ -9,12 +9,15 @@
 namespace lux {
 namespace {
 
-// 128 threads per block: closest 20.2 -> 19.3 ms and occlusion 16.1 -> 15.7 ms
-// against 256 on 4.19 M rays over 64 instances.
 constexpr int kBlock = 128;
-// Below this many rays they are walked in input order: 2^20 random rays over 64
-// instances take 4.45 ms sorted (sort included) and 4.63 ms in input order.
-constexpr int kTwoLevelOrderMinRays = 1 << 16;
+// Rays are walked in ray order from this many rays and mesh triangles on: below,
+// the meshes' records and triangles (112 bytes each) come out of the L2s (4 MiB per
+// XCD) or the sort costs more than it gives. Closest hit over 50 or 64 instances,
+// sorted (sort included) / in input order: 262 144 triangles 1.45 / 1.27 ms at
+// 300 000 rays, 1.36 / 1.48 at 600 000, 2.04 / 2.84 at 2^20; 131 072 triangles 1.64
+// / 1.62 at 2^20 rays; 60 000 triangles 4.37 / 4.22 at 2^22.
+constexpr int kTwoLevelOrderMinRays = 1 << 19;
+constexpr int kTwoLevelOrderMinTris = 1 << 18;
 
 __device__ __forceinline__ lux_scene_hit scene_hit(const TwoLevelHit& h) {
     lux_scene_hit out;
@@ -27,44 +30,48 @@ __device__ __forceinline__ lux_scene_hit scene_hit(const TwoLevelHit& h) {
     return out;
 }
 
-// Closest hit near child first at both levels; a ray the walk cannot settle
-// (stack overflow or the check of ordered.hpp) takes the preorder walk.
+// One ray: the records' walk, or the preorder walk where it cannot settle the ray.
+template <bool kAny>
+__device__ __forceinline__ TwoLevelHit query(const TwoLevelView& s, const lux_ray* __restrict__ rays, int i,
+                                             const int32_t* __restrict__ ignore, int group, int part,
+                                             uint32_t* stack) {
+    const float t_min = rays[i].t_min, t_max = rays[i].t_max;
+    const int ign = ignore ? ignore[i] : -1;
+    auto world = [&](f3& o, f3& d) {
+        o = ld3(rays[i].origin);
+        d = ld3(rays[i].direction);
+    };
+    TwoLevelHit h;
+    if (!two_level_wide<false>(s, world, t_min, __builtin_canonicalizef(t_max), kAny, ign, group, part, stack, kBlock,
+                               h))
+        h = two_level_walk(s, world, t_min, t_max, kAny, ign);
+    return h;
+}
+
+// `group` lanes walk one ray (lanes_per_ray).
+// 7 waves per SIMD (72 VGPRs): 2^20 rays over 64 instances 2.10 / 2.02 / 2.36 ms
+// at 6 / 7 / 8.
 // `order`: the rays in ray order (a permutation of [0, n)), or null for input
-// order; a hit lands at its ray's own index.
-__global__ __launch_bounds__(kBlock) void k_two_level_closest(TwoLevelView s, const uint32_t* __restrict__ order,
-                                                              const lux_ray* __restrict__ rays,
-                                                              const int32_t* __restrict__ ignore, int n,
-                                                              lux_scene_hit* __restrict__ hits) {
-    const int j = int(xcd_block()) * kBlock + threadIdx.x;
+// order; a result lands at its ray's own index: a lux_scene_hit, or one byte (kAny).
+template <bool kAny>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7))) void k_two_level(
+    TwoLevelView s, const uint32_t* __restrict__ order, const lux_ray* __restrict__ rays,
+    const int32_t* __restrict__ ignore, int n, int group, void* __restrict__ out) {
+    const uint32_t lane = xcd_block() * kBlock + threadIdx.x;
+    const int j = int(lane / uint32_t(group)), part = int(lane & uint32_t(group - 1));
     if (j >= n) return;
-    __shared__ uint32_t stack[kOrderedStack * kBlock];
+    __shared__ uint32_t stack[kWideStack * kBlock];
     const int i = order ? int(order[j]) : j;
     if (uint32_t(i) >= uint32_t(n)) {  // only if the sort itself reported an error
         set_error(s.info, kErrSpinLimit);
         return;
     }
-    const lux_ray r = rays[i];
-    const int ign = ignore ? ignore[i] : -1;
-    TwoLevelHit h;
-    if (!two_level_closest_ordered(s, ld3(r.origin), ld3(r.direction), r.t_min, r.t_max, ign, stack + threadIdx.x,
-                                   kBlock, h))
-        h = two_level_walk<false>(s, ld3(r.origin), ld3(r.direction), r.t_min, r.t_max, ign);
-    hits[i] = scene_hit(h);
-}
-
-__global__ __launch_bounds__(kBlock) void k_two_level_occluded(TwoLevelView s, const uint32_t* __restrict__ order,
-                                                               const lux_ray* __restrict__ rays,
-                                                               const int32_t* __restrict__ ignore, int n,
-                                                               uint8_t* __restrict__ occluded) {
-    const int j = int(xcd_block()) * kBlock + threadIdx.x;
-    if (j >= n) return;
-    const int i = order ? int(order[j]) : j;
-    if (uint32_t(i) >= uint32_t(n)) {
-        set_error(s.info, kErrSpinLimit);
-        return;
-    }
-    const lux_ray r = rays[i];
-    occluded[i] = two_level_any(s, ld3(r.origin), ld3(r.direction), r.t_min, r.t_max, ignore ? ignore[i] : -1) ? 1 : 0;
+    const TwoLevelHit h = query<kAny>(s, rays, i, ignore, group, part, stack + threadIdx.x);
+    if (part != 0) return;
+    if (kAny)
+        static_cast<uint8_t*>(out)[i] = h.prim >= 0 ? 1 : 0;
+    else
+        static_cast<lux_scene_hit*>(out)[i] = scene_hit(h);
 }
 
 template <typename T>
@@ -130,19 +137,21 @@ void sync_and_check(const BvhDev& d, hipStream_t stream, const char* what) {
     if (info.error != 0) throw Error(LUX_ERR_DEVICE_CHECK, std::string("device check failed in ") + what);
 }
 
-// The culling copy of the TLAS (TwoLevelDev::tlas_cull): the same slots, each
-// leaf box the instance's world bounds intersected with the world box of its
-// mesh's bounding sphere (both widened as below), each internal box the union
-// of its two children. Every box still holds every world-space ray point that
-// can hit the geometry below it, so only the culling changes.
-void build_tlas_cull(TwoLevelDev& s, const lux_instance* instances, hipStream_t stream) {
+// The records over the TLAS with its culling boxes (TwoLevelDev::tlas_wide), and
+// each instance's leaf position: a node array of the TLAS's topology, each leaf
+// box the instance's world bounds intersected with the world box of its mesh's
+// bounding sphere (both widened as below), each internal box the union of its two
+// children. Every box still holds every world-space ray point that can hit the
+// geometry below it, so only the culling changes.
+void build_tlas_wide(TwoLevelDev& s, const lux_instance* instances, std::vector<DevInstance>& rec,
+                     hipStream_t stream) {
     const int n = s.tlas.n;
-    const int slots = n > 1 ? 2 * n : n;
-    if (s.tlas_cull) hip_check(hipFree(s.tlas_cull), "hipFree culling TLAS");
-    s.tlas_cull = nullptr;
-    if (slots <= 0) return;
-    std::vector<lux_bvh_node> nodes(static_cast<size_t>(slots));
-    hip_check(hipMemcpyAsync(nodes.data(), s.tlas.pairs, sizeof(lux_bvh_node) * slots, hipMemcpyDeviceToHost, stream),
+    const int count = n > 0 ? 2 * n - 1 : 0;
+    if (s.tlas_wide) hip_check(hipFree(s.tlas_wide), "hipFree TLAS records");
+    s.tlas_wide = nullptr;
+    if (count <= 0) return;
+    std::vector<lux_bvh_node> nodes(static_cast<size_t>(count));
+    hip_check(hipMemcpyAsync(nodes.data(), s.tlas.nodes, sizeof(lux_bvh_node) * count, hipMemcpyDeviceToHost, stream),
               "D2H TLAS");
     hip_check(hipStreamSynchronize(stream), "synchronize TLAS download");
     // A leaf box must hold every world point w(t) of a ray whose object-space
@@ -196,38 +205,34 @@ void build_tlas_cull(TwoLevelDev& s, const lux_instance* instances, hipStream_t 
                            std::nextafter(b.p_max.z, INFINITY)};
         return b;
     };
-    // post-order over the pair slots from the root: a leaf takes its
-    // instance's box, an internal node the union of its children's
-    std::vector<int> todo{0};
-    std::vector<uint8_t> expanded(static_cast<size_t>(slots), 0);
-    while (!todo.empty()) {
-        const int k = todo.back();
+    // children have larger preorder positions than their parent: the right child
+    // is the next node, the left child the right one's escape
+    for (int k = count - 1; k >= 0; --k) {
         lux_bvh_node& nd = nodes[size_t(k)];
         if (nd.primitive_id >= 0) {
-            if (nd.primitive_id < s.instance_count) nd.bounds = leaf_box(nd.primitive_id);
-            todo.pop_back();
+            if (nd.primitive_id < s.instance_count) {
+                rec[size_t(nd.primitive_id)].tlas_pos = k;
+                nd.bounds = leaf_box(nd.primitive_id);
+            }
             continue;
         }
-        const int c = ~nd.primitive_id;
-        if (c < 0 || c + 1 >= slots) throw Error(LUX_ERR_DEVICE_CHECK, "malformed TLAS slot array");
-        if (!expanded[size_t(k)]) {
-            expanded[size_t(k)] = 1;
-            todo.push_back(c);
-            todo.push_back(c + 1);
-            continue;
-        }
-        const lux_aabb& l = nodes[size_t(c)].bounds;
-        const lux_aabb& r = nodes[size_t(c) + 1].bounds;
+        const int left = k + 1 < count ? nodes[size_t(k) + 1].escape : -1;
+        if (left <= k + 1 || left >= count) throw Error(LUX_ERR_DEVICE_CHECK, "malformed TLAS node array");
+        const lux_aabb& l = nodes[size_t(left)].bounds;
+        const lux_aabb& r = nodes[size_t(k) + 1].bounds;
         nd.bounds.p_min = lux_vec3{std::min(l.p_min.x, r.p_min.x), std::min(l.p_min.y, r.p_min.y),
                                    std::min(l.p_min.z, r.p_min.z)};
         nd.bounds.p_max = lux_vec3{std::max(l.p_max.x, r.p_max.x), std::max(l.p_max.y, r.p_max.y),
                                    std::max(l.p_max.z, r.p_max.z)};
-        todo.pop_back();
     }
-    s.tlas_cull = dalloc_n<lux_bvh_node>(size_t(slots));
-    hip_check(hipMemcpyAsync(s.tlas_cull, nodes.data(), sizeof(lux_bvh_node) * slots, hipMemcpyHostToDevice, stream),
+    if (n < 2) return;
+    s.tlas_wide = static_cast<WideNode*>(static_cast<void*>(dalloc_n<uint8_t>(sizeof(WideNode) * size_t(n - 1))));
+    TempBuffer<lux_bvh_node> cull{size_t(count)};
+    TempBuffer<int32_t> leaf_pos{4 * size_t(n)};
+    hip_check(hipMemcpyAsync(cull.p, nodes.data(), sizeof(lux_bvh_node) * count, hipMemcpyHostToDevice, stream),
               "H2D culling TLAS");
-    hip_check(hipStreamSynchronize(stream), "synchronize culling TLAS upload");
+    wide_from(s.tlas, cull.p, s.tlas_wide, leaf_pos.p, stream);
+    hip_check(hipStreamSynchronize(stream), "synchronize TLAS records");
 }
 
 // TLAS over the non-empty world bounds (ids = instance ids) and the instance
@@ -246,11 +251,10 @@ void upload_instances(TwoLevelDev& s, const lux_instance* instances, int count, 
         const int64_t tri = s.mesh_tri_off[in.mesh_id + 1] - s.mesh_tri_off[in.mesh_id];
         if (cursor + tri > INT32_MAX) throw Error(LUX_ERR_INVALID_ARGUMENT, "more than 2^31 scene primitives");
         r.first = int32_t(cursor);
-        r.nodes = s.blas[in.mesh_id].pairs;
-        r.node_count = tri > 1 ? int32_t(2 * tri) : int32_t(tri);
-        r.tri_base = s.mesh_tri_off[in.mesh_id];
+        r.wide = s.blas[in.mesh_id].wide;
+        r.tris = s.soup + s.mesh_tri_off[in.mesh_id];
         r.tri_count = int32_t(tri);
-        r.pad = 0;
+        r.tlas_pos = -1;
         cursor += tri;
         if (box_is_empty(in.world_bounds)) continue;
         boxes.push_back(in.world_bounds);
@@ -260,12 +264,6 @@ void upload_instances(TwoLevelDev& s, const lux_instance* instances, int count, 
     s.instance_count = count;
     s.scene_primitives = cursor;
     s.tlas_instances = int(boxes.size());
-    if (s.instances) hip_check(hipFree(s.instances), "hipFree instances");
-    s.instances = dalloc_n<DevInstance>(rec.size());
-    if (!rec.empty())
-        hip_check(hipMemcpyAsync(s.instances, rec.data(), sizeof(DevInstance) * rec.size(), hipMemcpyHostToDevice,
-                                 stream),
-                  "H2D instances");
     const int n = int(boxes.size());
     TempBuffer<lux_aabb> d_boxes(size_t(std::max(n, 1)));
     TempBuffer<int32_t> d_ids(size_t(std::max(n, 1)));
@@ -283,14 +281,23 @@ void upload_instances(TwoLevelDev& s, const lux_instance* instances, int count, 
         limit += tri > 1 ? 2u * uint64_t(tri) : uint64_t(tri);
     }
     s.step_limit = uint32_t(std::min<uint64_t>(limit + 1, 0xffffffffu));
-    build_tlas_cull(s, instances, stream);
+    build_tlas_wide(s, instances, rec, stream);
+    if (s.instances) hip_check(hipFree(s.instances), "hipFree instances");
+    s.instances = nullptr;
+    s.instances = dalloc_n<DevInstance>(rec.size());
+    if (!rec.empty()) {
+        hip_check(hipMemcpyAsync(s.instances, rec.data(), sizeof(DevInstance) * rec.size(), hipMemcpyHostToDevice,
+                                 stream),
+                  "H2D instances");
+        hip_check(hipStreamSynchronize(stream), "synchronize instances");
+    }
 }
 
 size_t bvh_device_bytes(const BvhDev& d) {
     const size_t cap = size_t(d.capacity);
     // boxes, ids, keys/vals, tree links, slots, preorder maps, nodes, pairs
-    // and their two slot maps
-    return cap * (24 + 4 + 16 + 28 + 48 + 8 + 64 + 64 + 16);
+    // and their two slot maps, records and their leaf positions
+    return cap * (24 + 4 + 16 + 28 + 48 + 8 + 64 + 64 + 16 + 64 + 16);
 }
 
 }  // namespace
@@ -353,7 +360,7 @@ lux_aabb transform_bounds(const float* m, const lux_aabb& b) {
 void two_level_release(TwoLevelDev& s) {
     for (BvhDev& b : s.blas) bvh_release(b);
     bvh_release(s.tlas);
-    void* ptrs[] = {s.soup, s.meshes, s.instances, s.tlas_cull};
+    void* ptrs[] = {s.soup, s.meshes, s.instances, s.tlas_wide};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     s = TwoLevelDev{};
@@ -385,10 +392,10 @@ void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* of
         // the soup copied above
         lbvh_build_triangles(s.blas[m], s.soup + offsets[m], nullptr, nullptr, 0, n, stream);
         sync_and_check(s.blas[m], stream, "BLAS build");
-        meshes[m].nodes = s.blas[m].pairs;
-        meshes[m].slot_pre = s.blas[m].slot_pre;
+        meshes[m].nodes = s.blas[m].nodes;
+        meshes[m].wide_leaf = s.blas[m].wide_leaf;
         meshes[m].tris = s.soup + offsets[m];
-        meshes[m].node_count = n > 1 ? 2 * n : n;
+        meshes[m].node_count = n > 0 ? 2 * n - 1 : 0;
         meshes[m].tri_count = n;
         s.device_bytes += bvh_device_bytes(s.blas[m]);
     }
@@ -440,14 +447,13 @@ void two_level_set_instances(TwoLevelDev& s, const lux_instance* instances, int 
 
 TwoLevelView two_level_view(const TwoLevelDev& s) {
     TwoLevelView v;
-    v.tlas_nodes = s.tlas.pairs;
-    v.tlas_cull = s.tlas_cull ? s.tlas_cull : s.tlas.pairs;
-    v.tlas_slot_pre = s.tlas.slot_pre;
+    v.tlas_nodes = s.tlas.nodes;
+    v.tlas_wide = s.tlas_wide;
+    v.tlas_records = s.tlas_wide ? uint32_t(s.tlas.n - 1) : 0u;
     v.instances = s.instances;
     v.meshes = s.meshes;
-    v.soup = s.soup;
     v.info = s.tlas.info;
-    v.tlas_node_count = s.tlas.n > 1 ? 2 * s.tlas.n : s.tlas.n;
+    v.tlas_node_count = s.tlas.n > 0 ? 2 * s.tlas.n - 1 : 0;
     v.instance_count = s.instance_count;
     v.mesh_count = s.mesh_count;
     v.step_limit = s.step_limit;
@@ -455,22 +461,24 @@ TwoLevelView two_level_view(const TwoLevelDev& s) {
 }
 
 const uint32_t* two_level_order(RaySortDev& r, const TwoLevelDev& s, const lux_ray* rays, int n, hipStream_t stream) {
-    if (n < kTwoLevelOrderMinRays || s.tlas.n < 1) return nullptr;
+    if (s.tlas.n < 1 || n < kTwoLevelOrderMinRays || s.mesh_tri_off.back() < kTwoLevelOrderMinTris) return nullptr;
     return ray_order(r, s.tlas, rays, n, stream);  // origins quantised in the TLAS root box
 }
 
 void two_level_closest(const TwoLevelView& v, const uint32_t* order, const lux_ray* rays, const int32_t* ignore,
                        int n, lux_scene_hit* hits, hipStream_t stream) {
     if (n <= 0) return;
-    LUX_LAUNCH("two_level_closest", k_two_level_closest, div_up(n, kBlock), kBlock, 0, stream, v, order, rays,
-               ignore, n, hits);
+    const int group = lanes_per_ray(uint32_t(n));
+    LUX_LAUNCH("two_level_closest", k_two_level<false>, div_up(int64_t(n) * group, kBlock), kBlock, 0, stream, v, order,
+               rays, ignore, n, group, static_cast<void*>(hits));
 }
 
 void two_level_occluded(const TwoLevelView& v, const uint32_t* order, const lux_ray* rays, const int32_t* ignore,
                         int n, uint8_t* occluded, hipStream_t stream) {
     if (n <= 0) return;
-    LUX_LAUNCH("two_level_occluded", k_two_level_occluded, div_up(n, kBlock), kBlock, 0, stream, v, order, rays,
-               ignore, n, occluded);
+    const int group = lanes_per_ray(uint32_t(n));
+    LUX_LAUNCH("two_level_occluded", k_two_level<true>, div_up(int64_t(n) * group, kBlock), kBlock, 0, stream, v, order,
+               rays, ignore, n, group, static_cast<void*>(occluded));
 }
 
 }  // namespace lux

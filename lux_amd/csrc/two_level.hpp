@@ -7,48 +7,47 @@
 #include <vector>
 
 #include "lux_runtime.hpp"
-#include "ordered.hpp"
+#include "wide.hpp"
 
 namespace lux {
 
-// One mesh as the walk sees it: its BLAS (sibling-pair node copy) and its
-// triangles (object space, a slice of the scene's soup).
+// One mesh as the walks see it: its BLAS (right-first preorder nodes and the
+// four-child records' leaf positions) and its triangles (object space, a slice of
+// the scene's soup).
 struct DevMesh {
     const lux_bvh_node* nodes;
     const lux_triangle* tris;
-    const uint32_t* slot_pre;  // preorder position of each pair slot (tie order)
-    int32_t node_count;        // sibling-pair slots (0: empty mesh)
+    const int32_t* wide_leaf;  // preorder position of each leaf child (4 * record + child)
+    int32_t node_count;        // 2 n - 1 (0: empty mesh)
     int32_t tri_count;
 };
 
 // One instance: Transform::inv (row-major 4x4), the scene ordinal of its local
-// triangle 0 (GpuSceneInstance::first_primitive, src/scene/gpu_scene.h:149-172)
-// and, copied from its mesh so that entering the instance is one dependent load,
-// the mesh's BLAS (sibling-pair slots; 0 for an empty or invalid mesh) and the
-// offset of its triangles in the scene's soup.
+// triangle 0 (GpuSceneInstance::first_primitive, src/scene/gpu_scene.h:149-172),
+// the preorder position of its TLAS leaf (-1: none) and, copied from its mesh so
+// that entering the instance is one dependent load, the mesh's records and
+// triangles.
 struct DevInstance {
     float inv[16];
-    const lux_bvh_node* nodes;
-    int32_t node_count;
-    int32_t tri_base;
+    const WideNode* wide;
+    const lux_triangle* tris;
     int32_t tri_count;
     int32_t first;
     int32_t mesh;
-    int32_t pad;
+    int32_t tlas_pos;
 };
 static_assert(sizeof(DevInstance) == 96, "instance record");
 
 // What the walk kernels take by value.
 struct TwoLevelView {
-    const lux_bvh_node* tlas_nodes;  // the TLAS (sibling-pair copy) with the reference's boxes
-    const lux_bvh_node* tlas_cull;   // the same slots with tighter culling boxes (see TwoLevelDev)
-    const uint32_t* tlas_slot_pre;
+    const lux_bvh_node* tlas_nodes;  // the TLAS in right-first preorder, the reference's boxes
+    const WideNode* tlas_wide;       // its records over tighter culling boxes (see TwoLevelDev)
     const DevInstance* instances;
     const DevMesh* meshes;
-    const lux_triangle* soup;  // every mesh's object-space triangles, mesh by mesh
     DevInfo* info;
     int32_t tlas_node_count, instance_count, mesh_count;
-    uint32_t step_limit;  // TLAS slots + the BLAS slots of every instance: no walk takes more steps
+    uint32_t tlas_records;
+    uint32_t step_limit;  // TLAS nodes + the BLAS nodes of every instance: no walk takes more steps
 };
 
 // ---- device walk ------------------------------------------------------------------
@@ -67,12 +66,27 @@ __device__ __forceinline__ f3 xform_vector(const float* m, const f3& v) {
                  m[8] * v.x + m[9] * v.y + m[10] * v.z);
 }
 
+// A world ray in an instance's object space (inv: 16-byte aligned).
+__device__ __forceinline__ void xform_ray(const float* inv, const f3& WO, const f3& WD, f3& O, f3& D) {
+    float m[16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 row = reinterpret_cast<const float4*>(inv)[i];
+        m[4 * i] = row.x;
+        m[4 * i + 1] = row.y;
+        m[4 * i + 2] = row.z;
+        m[4 * i + 3] = row.w;
+    }
+    O = xform_point(m, WO);
+    D = xform_vector(m, WD);
+}
+
 struct TwoLevelHit {
     int prim = -1, instance = -1, local = -1;
     float t = 0, u = 0, v = 0;
 };
 
-// The walk is one flat loop over two levels. A lane starts in the TLAS (world
+// The preorder walk is one flat loop over two levels. A lane starts in the TLAS (world
 // ray); at an instance leaf it switches to that mesh's BLAS with the ray moved
 // to object space and keeps the TLAS escape of the leaf; when the BLAS walk
 // ends it returns to that escape with the world ray. One loop keeps the lanes
@@ -80,14 +94,14 @@ struct TwoLevelHit {
 // levels: the reference gives the BLAS walk t_max = the current hit and keeps a
 // BLAS hit only when it is nearer, which every hit the BLAS walk accepts is
 // (it only accepts t < t_max), so updating t_max at once is the same.
-// kAny stops at the first accepted triangle. `ignore` is a scene ordinal
+// `any` stops at the first accepted triangle. `ignore` is a scene ordinal
 // (should_skip_primitive) or -1.
-template <bool kAny>
-__device__ __forceinline__ TwoLevelHit two_level_walk(const TwoLevelView& s, const f3& WO, const f3& WD,
-                                                      float t_min, float t_max, int ignore) {
-    const SlabRay wsr = make_slab_ray(WO, WD, t_min);
-    SlabRay sr = wsr;
-    f3 O = WO, D = WD;
+template <typename World>
+__device__ __forceinline__ TwoLevelHit two_level_walk(const TwoLevelView& s, World&& world, float t_min, float t_max,
+                                                      bool any, int ignore) {
+    f3 O, D;
+    world(O, D);
+    SlabRay sr = make_slab_ray(O, D, t_min);
     const lux_bvh_node* nodes = s.tlas_nodes;
     uint32_t nc = uint32_t(s.tlas_node_count);
     const lux_triangle* tris = nullptr;
@@ -104,9 +118,8 @@ __device__ __forceinline__ TwoLevelHit two_level_walk(const TwoLevelView& s, con
             nodes = s.tlas_nodes;
             nc = uint32_t(s.tlas_node_count);
             k = resume;
-            sr = wsr;
-            O = WO;
-            D = WD;
+            world(O, D);
+            sr = make_slab_ray(O, D, t_min);
             continue;
         }
         if (steps-- == 0u) {
@@ -127,34 +140,25 @@ __device__ __forceinline__ TwoLevelHit two_level_walk(const TwoLevelView& s, con
             continue;
         }
         if (prim < 0) {
-            k = uint32_t(~prim);  // right child's slot
+            ++k;  // the right child
             continue;
         }
         k = esc;
         if (!in_blas) {  // instance leaf: enter its BLAS if it has one
             if (prim >= s.instance_count) continue;
             const DevInstance& in = s.instances[prim];
-            if (in.node_count <= 0 || in.first < 0) continue;
-            float inv[16];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 row = reinterpret_cast<const float4*>(in.inv)[i];
-                inv[4 * i] = row.x;
-                inv[4 * i + 1] = row.y;
-                inv[4 * i + 2] = row.z;
-                inv[4 * i + 3] = row.w;
-            }
+            if (in.tri_count <= 0 || in.first < 0) continue;
             resume = esc;
             in_blas = true;
-            nodes = in.nodes;
-            nc = uint32_t(in.node_count);
-            tris = s.soup + in.tri_base;
+            nodes = s.meshes[in.mesh].nodes;
+            nc = uint32_t(s.meshes[in.mesh].node_count);
+            tris = in.tris;
             tcount = in.tri_count;
             first = in.first;
             inst_cur = prim;
             ignore_local = (ignore >= first && ignore - first < tcount) ? ignore - first : -1;
-            O = xform_point(inv, WO);
-            D = xform_vector(inv, WD);
+            const f3 WO = O, WD = D;
+            xform_ray(in.inv, WO, WD, O, D);
             sr = make_slab_ray(O, D, t_min);
             k = 0;
             continue;
@@ -175,361 +179,279 @@ __device__ __forceinline__ TwoLevelHit two_level_walk(const TwoLevelView& s, con
             best.t = t;
             best.u = u;
             best.v = v;
-            if (kAny) break;
+            if (any) break;
         }
     }
     return best;
 }
 
-// Occlusion of the same two-level scene: two_level_walk<true>'s walk with the
-// TLAS steps culled by tlas_cull. t_max never changes and the answer is whether
-// any triangle is hit in (t_min, t_max): an instance whose culling box the
-// segment misses holds no such hit (the box holds every ray point that can
-// reach its mesh), and every other instance is walked as the reference walks
-// it. The expensive steps are gathered across the wave. A lane whose
-// walk reaches a passed leaf (an instance in the TLAS, a triangle in a BLAS)
-// holds it and stops; once a quarter of the wave's working lanes hold one (or
-// none can step on), the wave enters the held instances and tests the held
-// triangles together.
-__device__ __forceinline__ bool two_level_any(const TwoLevelView& s, const f3& WO, const f3& WD, float t_min,
-                                              float t_max, int ignore) {
-    const SlabRay wsr = make_slab_ray(WO, WD, t_min);
-    SlabRay sr = wsr;
-    f3 O = WO, D = WD;
-    const lux_bvh_node* nodes = s.tlas_cull;
-    uint32_t nc = uint32_t(s.tlas_node_count);
-    int tri_base = 0, tcount = 0, ignore_local = -1;
-    bool in_blas = false, found = false;
-    uint32_t resume = 0, k = 0;
-    uint32_t steps = s.step_limit;
-    int held = -1;
-    for (;;) {
-        // one step of the walk, for a lane that holds nothing and is not done
-        if (held < 0 && !found) {
-            if (k >= nc && in_blas) {  // back to the TLAS at the instance leaf's escape
-                in_blas = false;
-                nodes = s.tlas_cull;
-                nc = uint32_t(s.tlas_node_count);
-                k = resume;
-                sr = wsr;
-                O = WO;
-                D = WD;
-            }
-            if (k < nc) {
-                if (steps-- == 0u) {
-                    set_error(s.info, kErrWalkOrder);
-                    k = nc;
-                    in_blas = false;
-                } else {
-                    float4 a, b;
-                    load_node(nodes, int(k), a, b);
-                    const int prim = __float_as_int(b.z);
-                    const bool pass = wave_any_parallel(sr) ? slab_hit(sr, t_max, a.x, a.y, a.z, a.w, b.x, b.y)
-                                                            : slab_hit_np(sr, t_max, a.x, a.y, a.z, a.w, b.x, b.y);
-                    held = (pass && prim >= 0) ? prim : -1;
-                    k = (pass && prim < 0) ? uint32_t(~prim) : __float_as_uint(b.w);
-                }
-            }
-        }
-        const bool working = held < 0 && !found && (k < nc || in_blas);
-        const uint64_t want = __ballot(held >= 0);
-        const uint64_t more = __ballot(working);
-        if (!more) {
-            if (!want) break;
-        } else if (__popcll(want) * 4 < __popcll(want | more)) {
-            continue;
-        }
-        if (held < 0) continue;
-        if (!in_blas) {  // instance leaf: enter its BLAS if it has one (k holds the leaf's escape)
-            const int inst = held;
-            held = -1;
-            if (inst >= s.instance_count) continue;
-            const DevInstance& in = s.instances[inst];
-            if (in.node_count <= 0 || in.first < 0) continue;
-            float inv[16];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 row = reinterpret_cast<const float4*>(in.inv)[i];
-                inv[4 * i] = row.x;
-                inv[4 * i + 1] = row.y;
-                inv[4 * i + 2] = row.z;
-                inv[4 * i + 3] = row.w;
-            }
-            resume = k;
-            in_blas = true;
-            nodes = in.nodes;
-            nc = uint32_t(in.node_count);
-            tri_base = in.tri_base;
-            tcount = in.tri_count;
-            ignore_local = (ignore >= in.first && ignore - in.first < tcount) ? ignore - in.first : -1;
-            O = xform_point(inv, WO);
-            D = xform_vector(inv, WD);
-            sr = make_slab_ray(O, D, t_min);
-            k = 0;
-            continue;
-        }
-        const int prim = held;
-        held = -1;
-        if (prim == ignore_local) continue;  // should_skip_primitive
-        if (prim >= tcount) {
-            set_error(s.info, kErrPrimRange);
-            continue;
-        }
-        const float* p = reinterpret_cast<const float*>(s.soup + tri_base + prim);
-        float t, u, v;
-        if (tri_hit(O, D, t_min, t_max, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), t,
-                    u, v))
-            found = true;
-    }
-    return found;
-}
-
-// Closest hit of the same two-level scene, near child first at both levels
-// (ordered.hpp). A TLAS step tests both children of a node; each child that
-// passes is an internal node (its pair slot) or an instance leaf (its slot
-// tagged with kInstanceItem). The nearer is taken next and the other pushed on
-// the lane's LDS stack; taking an instance leaf moves the ray to object space
-// and walks that BLAS near child first on the same stack above the entry
-// depth, returning to the world ray when the stack falls back to it.
+// The same queries by the four-child records of both levels (wide.hpp), near child
+// first on one LDS stack. A TLAS step enters records and instance leaves alike, in
+// the order of their entries; taking an instance leaf moves the ray to object
+// space and walks that BLAS above the entry depth of the stack, returning to the
+// world ray when the stack falls back to it. The triangle tests and the instance
+// entries (a matrix transform and three correctly rounded quotients) are gathered
+// across the wave: a lane that holds passed leaf children or an instance waits
+// until a quarter of the working lanes hold some.
 // The preorder walk above visits triangles in the order (TLAS preorder of the
-// instance leaf, BLAS preorder of the triangle leaf) and keeps the first of
-// equal t; this walk keeps, of equal t, the one smallest in that order
-// (slot_pre of both levels, read only on an exact tie), so both return the
-// same hit. The check of ordered.hpp spans both levels: boxes of both are
-// entered up to t_cull, and a triangle's largest path entry is the larger of
-// its BLAS leaf's entry (object space) and its instance's TLAS leaf entry
-// (world space). Returns false when the stack would overflow, the arrays are
-// malformed (error bits set) or the check fires; the caller then runs
-// two_level_walk<false> for the ray.
-constexpr uint32_t kInstanceItem = 0x80000000u;
-
-__device__ __forceinline__ bool two_level_closest_ordered(const TwoLevelView& s, const f3& WO, const f3& WD,
-                                                          float t_min, float t_max0, int ignore, uint32_t* stack,
-                                                          int stride, TwoLevelHit& best) {
-    // Per-lane state is kept small (the path tracer's trace kernel holds this
-    // walk at 80 VGPRs): the world slab ray is recomputed on leaving an
-    // instance, a mesh's triangle and tie arrays are read at its leaf tests,
-    // and the winner's instance, local id, u and v are derived once at the end.
+// instance leaf, BLAS preorder of the triangle leaf) and keeps the first of equal
+// t; this walk keeps, of equal t, the one smallest in that order. The TLAS records
+// hold the culling boxes (see TwoLevelDev), every byte box only culls, and at the
+// end the winner's own boxes -- its BLAS leaf in object space and its instance's
+// TLAS leaf, the reference's box, in world space -- are tested the reference's way
+// with both entries at most t: the check of wide.hpp over both levels. An any-hit
+// query ends at its first hit and asks only that both boxes are entered before
+// t_max. world(o, d) gives the ray. Returns false when the preorder walk has to
+// decide (the check fails, the stack is full, the arrays are malformed).
+// A ray on `group` lanes: parts of it as in wide_query; an instance's culling box
+// holds its geometry at every t, so a triangle's boxes of both levels are met in
+// the same part.
+// 2^20 random rays over 64 instances of 2^16 triangles: closest 2.0 ms, occlusion
+// 1.7 ms; by sibling pairs 4.7 (near child first, one lane's entries at a time)
+// and 2.7 ms (preorder, gathered). 1000 rays over 40 instances of 5000: 105 us
+// against 422.
+// kReload: the view is in memory and read again at each use, so that its fields
+// take no registers through the walk.
+template <bool kReload, typename World>
+__device__ __forceinline__ bool two_level_wide(const TwoLevelView& view, World&& world, float t_min, float t_bound,
+                                               bool any, int ignore, int group, int part, uint32_t* stack,
+                                               int stride, TwoLevelHit& best) {
+    constexpr uint32_t kNone = 0x7fffffffu;
     best = TwoLevelHit{};
-    OrderedBest ob(t_max0);
-    float inst_tn = -INFINITY;  // entry of the current instance's TLAS leaf box
-    const uint32_t tlas_nc = uint32_t(s.tlas_node_count);
-    if (tlas_nc == 0u) return true;
-    SlabRay sr = make_slab_ray(WO, WD, t_min);
-    f3 O = WO, D = WD;
-    const lux_bvh_node* nodes = s.tlas_cull;  // TLAS steps cull with the tighter boxes
-    uint32_t nc = tlas_nc;
-    bool in_blas = false;
-    int tri_base = 0, first = -1, ignore_local = -1;
-    int best_prim = -1;
-    uint32_t inst_slot = 0, best_inst_slot = 0, best_slot = 0;
-    int sp = 0, sp0 = 0;
-    uint32_t steps = s.step_limit;
-    uint32_t item;
-    {
-        float4 a, b;
-        load_node32(nodes, 0, a, b);
-        float tn;
-        const bool par = wave_any_parallel(sr);
-        const bool hit = par ? slab_near<true>(sr, ob.t_cull, a.x, a.y, a.z, a.w, b.x, b.y, tn)
-                             : slab_near<false>(sr, ob.t_cull, a.x, a.y, a.z, a.w, b.x, b.y, tn);
-        if (!hit) return true;
-        const int p = __float_as_int(b.z);
-        item = p >= 0 ? kInstanceItem : ~uint32_t(p);
-    }
-    // Tests BLAS leaf `slot` (local triangle prim, box entry tn) of the current
-    // instance. The largest entry on the triangle's path is that of its BLAS
-    // leaf or that of the instance's TLAS leaf.
-    // A BLAS of nc slots has (nc + 1) / 2 leaves (nc = 1: a single leaf).
-    auto leaf = [&](uint32_t slot, int prim, float tn) {
-        if (prim == ignore_local) return;  // should_skip_primitive
-        if (uint32_t(prim) >= (nc + 1u) / 2u) {
-            set_error(s.info, kErrPrimRange);
-            return;
-        }
-        const float* p = reinterpret_cast<const float*>(s.soup + tri_base + prim);
-        const f3 v0 = make3(p[0], p[1], p[2]), v1 = make3(p[3], p[4], p[5]), v2 = make3(p[6], p[7], p[8]);
-        float t, u, v;
-        if (!tri_uvt(O, D, v0, v1, v2, t, u, v) || !(t > t_min)) return;
-        ob.note(t, fmaxf(tn, inst_tn));
-        bool take = t < ob.t_max;
-        if (!take && best_prim >= 0 && t == ob.t_max) {  // exact tie: the smaller (TLAS, BLAS) preorder position
-            if (inst_slot != best_inst_slot) {
-                take = s.tlas_slot_pre[inst_slot] < s.tlas_slot_pre[best_inst_slot];
-            } else {  // same instance: its mesh's BLAS preorder positions
-                float4 ta, tb;
-                load_node32(s.tlas_nodes, inst_slot, ta, tb);
-                const uint32_t* pre = s.meshes[s.instances[__float_as_int(tb.z)].mesh].slot_pre;
-                take = pre[slot] < pre[best_slot];
-            }
-        }
-        if (!take) return;
-        ob.take(t);
-        best_prim = first + prim;
-        best_inst_slot = inst_slot;
-        best_slot = slot;
+    auto fields = [&]() -> const TwoLevelView& {
+        const TwoLevelView* p = &view;
+        if (kReload) asm volatile("" : "+v"(p));
+        return *p;
     };
-    for (;;) {
-        if (steps-- == 0u) {
-            set_error(s.info, kErrWalkOrder);
+    const TwoLevelView& s = view;
+    if (s.tlas_node_count == 0) return true;
+    f3 O = make3(0, 0, 0), D = O;
+    SlabRay sr = {};
+    bool stale = true;  // sr is not the ray of the next step
+    float lo = t_min, hi = t_bound;
+    bool skip = false;
+    if (group > 1) {
+        world(O, D);
+        skip = !ray_part(s.tlas_nodes, make_slab_ray(O, D, t_min), group, part, lo, hi);
+    }
+    float t_max = t_bound;
+    float t_cull = wide_bound(hi);
+    const WideNode* wide = s.tlas_wide;
+    uint32_t records = s.tlas_records;
+    // the next record, kLeafBit | instance, or kNone: the top of the stack
+    uint32_t item = records ? 0u : kLeafBit | uint32_t(s.tlas_nodes[0].primitive_id);
+    uint32_t hc = 0, hmask = 0;
+    uint4 ref = make_uint4(0, 0, 0, 0);
+    int sp = 0, sp0 = 0;
+    const lux_triangle* tris = nullptr;
+    int inst = -1, ignore_local = -1;
+    int best_inst = -1, best_local = -1;
+    uint32_t best_at = 0;
+    uint32_t steps = s.step_limit;
+    bool in_blas = false, done = skip, failed = false;
+    auto leaf = [&](uint32_t at, uint32_t r) {
+        const uint32_t prim = r & kIndexMask;
+        if (int(prim) == ignore_local || r == kWideEmpty) return false;  // should_skip_primitive
+        if (prim > records) {  // a BLAS of `records` records has one triangle more
+            set_error(fields().info, kErrPrimRange);
             return false;
         }
-        bool descend = false;
-        if (item & kInstanceItem) {
-            // enter the instance of TLAS leaf slot `ls`, if it has a BLAS (an
-            // instance item is only taken in the TLAS, so sr is the world ray)
-            const uint32_t ls = item & ~kInstanceItem;
-            if (ls >= tlas_nc) {
-                set_error(s.info, kErrWalkOrder);
-                return false;
-            }
-            float4 a, b;
-            load_node32(s.tlas_nodes, ls, a, b);
-            const int prim = __float_as_int(b.z);
-            const DevInstance* in = (prim >= 0 && prim < s.instance_count) ? &s.instances[prim] : nullptr;
-            const bool ok = in && in->node_count > 0 && in->first >= 0;
-            if (ok && uint32_t(in->node_count) <= kOffset32Nodes) {
-                {
-                    // entry of this instance's TLAS leaf box as the reference
-                    // tests it (its own box, not the culling box): the exactness
-                    // check weighs hits against the reference walk's entries
-                    const bool wpar = wave_any_parallel(sr);
-                    (void)(wpar ? slab_near<true>(sr, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, inst_tn)
-                                : slab_near<false>(sr, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, inst_tn));
-                }
-                float inv[16];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float4 row = reinterpret_cast<const float4*>(in->inv)[i];
-                    inv[4 * i] = row.x;
-                    inv[4 * i + 1] = row.y;
-                    inv[4 * i + 2] = row.z;
-                    inv[4 * i + 3] = row.w;
-                }
-                in_blas = true;
-                sp0 = sp;
-                nodes = in->nodes;
-                nc = uint32_t(in->node_count);
-                tri_base = in->tri_base;
-                first = in->first;
-                inst_slot = ls;
-                ignore_local = (ignore >= first && ignore - first < in->tri_count) ? ignore - first : -1;
-                O = xform_point(inv, WO);
-                D = xform_vector(inv, WD);
-                sr = make_slab_ray(O, D, t_min);
-                load_node32(nodes, 0, a, b);
-                float tn;
-                const bool par = wave_any_parallel(sr);
-                const bool hit = par ? slab_near<true>(sr, ob.t_cull, a.x, a.y, a.z, a.w, b.x, b.y, tn)
-                                     : slab_near<false>(sr, ob.t_cull, a.x, a.y, a.z, a.w, b.x, b.y, tn);
-                const int root = __float_as_int(b.z);
-                if (hit && root >= 0) leaf(0u, root, tn);
-                if (hit && root < 0) {
-                    item = ~uint32_t(root);
-                    descend = true;
-                }
-            } else if (ok) {
-                return false;  // a BLAS beyond 32-bit node offsets: the preorder walk takes the ray
-            }
-        } else {
-            const uint32_t c = item;
-            if (c + 1 >= nc) {
-                set_error(s.info, kErrWalkOrder);
-                return false;
-            }
-            float4 a0, b0, a1, b1;
-            load_node32(nodes, c, a0, b0);
-            load_node32(nodes, c + 1, a1, b1);
-            float tn0, tn1;
-            const bool par = wave_any_parallel(sr);
-            const bool h0 = par ? slab_near<true>(sr, ob.t_cull, a0.x, a0.y, a0.z, a0.w, b0.x, b0.y, tn0)
-                                : slab_near<false>(sr, ob.t_cull, a0.x, a0.y, a0.z, a0.w, b0.x, b0.y, tn0);
-            const bool h1 = par ? slab_near<true>(sr, ob.t_cull, a1.x, a1.y, a1.z, a1.w, b1.x, b1.y, tn1)
-                                : slab_near<false>(sr, ob.t_cull, a1.x, a1.y, a1.z, a1.w, b1.x, b1.y, tn1);
-            const int p0 = __float_as_int(b0.z), p1 = __float_as_int(b1.z);
-            bool take0, take1;
-            uint32_t i0, i1;
-            if (in_blas) {
-                if (h0 && p0 >= 0) leaf(c, p0, tn0);
-                if (h1 && p1 >= 0) leaf(c + 1, p1, tn1);
-                take0 = h0 && p0 < 0;
-                take1 = h1 && p1 < 0;
-                i0 = ~uint32_t(p0);
-                i1 = ~uint32_t(p1);
-            } else {
-                take0 = h0;
-                take1 = h1;
-                i0 = p0 >= 0 ? (c | kInstanceItem) : ~uint32_t(p0);
-                i1 = p1 >= 0 ? ((c + 1) | kInstanceItem) : ~uint32_t(p1);
-            }
-            if (take0 && take1) {
-                if (sp == kOrderedStack) return false;
-                const bool far0 = tn1 < tn0;
-                stack[sp * stride] = far0 ? i0 : i1;
-                ++sp;
-                item = far0 ? i1 : i0;
-                descend = true;
-            } else if (take0 || take1) {
-                item = take0 ? i0 : i1;
-                descend = true;
+        const float* p = reinterpret_cast<const float*>(tris + prim);
+        float t, u, v;
+        if (!tri_uvt(O, D, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), t, u, v) ||
+            !(t > t_min))
+            return false;
+        bool take = t < t_max;
+        if (!take && !any && best_inst >= 0 && t == t_max) {  // exact tie: the smaller (TLAS, BLAS) preorder position
+            if (inst != best_inst) {
+                take = fields().instances[inst].tlas_pos < fields().instances[best_inst].tlas_pos;
+            } else if (records) {
+                const int32_t* pos = fields().meshes[fields().instances[inst].mesh].wide_leaf;
+                take = pos[at] < pos[best_at];
             }
         }
-        if (descend) continue;
-        // pop: leave the instance once its part of the stack is used up
-        if (in_blas && sp == sp0) {
-            in_blas = false;
-            nodes = s.tlas_cull;
-            nc = tlas_nc;
-            sr = make_slab_ray(WO, WD, t_min);
-            O = WO;
-            D = WD;
-        }
-        if (sp == 0) break;
-        --sp;
-        item = stack[sp * stride];
-    }
-    if (best_prim < 0) return true;
-    if (ob.ambiguous()) return false;
-    // the winner's instance, local id, u and v: the same operations on the
-    // same operands as the leaf test that took it
-    float4 a, b;
-    load_node32(s.tlas_nodes, best_inst_slot, a, b);
-    const int inst = __float_as_int(b.z);
-    const DevInstance& in = s.instances[inst];
-    float inv[16];
+        if (!take) return false;
+        best_inst = inst;
+        best_local = int(prim);
+        best_at = at;
+        if (any) return true;
+        t_max = t;
+        t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
+        return false;
+    };
+    for (;;) {
+        if (!done & (hmask == 0) & !(item & kLeafBit)) {
+            if (item == kNone) {
+                if (in_blas && sp == sp0) {  // leave the instance
+                    in_blas = false;
+                    stale = true;
+                }
+                if (sp == 0)
+                    done = true;
+                else
+                    item = stack[--sp * stride];
+            }
+            if (!done & !stale & !(item & kLeafBit)) {
+                if (item >= records || steps-- == 0u) {
+                    set_error(fields().info, kErrWalkOrder);
+                    failed = done = true;
+                } else {
+                    float4 a, b, q;
+                    load_wide(wide, item, a, b, q, ref);
+                    float key[4];
+                    bool pass[4];
+                    wide_boxes<true>(a, b, q, sr, t_cull, key, pass);
+                    uint32_t kid[4] = {ref.x, ref.y, ref.z, ref.w};
+                    uint32_t mask = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float4 row = reinterpret_cast<const float4*>(in.inv)[i];
-        inv[4 * i] = row.x;
-        inv[4 * i + 1] = row.y;
-        inv[4 * i + 2] = row.z;
-        inv[4 * i + 3] = row.w;
+                    for (int k = 0; k < 4; ++k) {
+                        const bool tri = in_blas & (int32_t(kid[k]) < 0);
+                        const bool empty = kid[k] == kWideEmpty;
+                        key[k] = (pass[k] & !tri & !empty) ? key[k] : INFINITY;
+                        mask |= (pass[k] & tri) ? (1u << k) : 0u;
+                    }
+                    hc = item;
+                    hmask = mask;
+                    item = kNone;
+                    wide_sort(key, kid);
+                    if (key[0] < INFINITY) {
+                        item = kid[0];
+                        const bool p1 = key[1] < INFINITY, p2 = key[2] < INFINITY, p3 = key[3] < INFINITY;
+                        if (sp + int(p1) + int(p2) + int(p3) > kWideStack) {
+                            failed = done = true;
+                            hmask = 0;
+                        } else {
+                            if (p3) stack[sp++ * stride] = kid[3];
+                            if (p2) stack[sp++ * stride] = kid[2];
+                            if (p1) stack[sp++ * stride] = kid[1];
+                        }
+                    }
+                }
+            }
+        }
+        const bool holds = !done & (stale | (hmask != 0) | ((item & kLeafBit) != 0));
+        const uint64_t want = __ballot(holds);
+        const uint64_t more = __ballot(!done & !holds);
+        if (!more) {
+            if (!want) break;
+        } else if (__popcll(want) * kGatherDiv < __popcll(want | more)) {
+            continue;
+        }
+        while (hmask) {
+            const uint32_t k = uint32_t(__ffs(int(hmask))) - 1u;
+            hmask &= hmask - 1u;
+            const uint32_t r0 = (k & 1u) ? ref.y : ref.x, r1 = (k & 1u) ? ref.w : ref.z;
+            if (leaf(4u * hc + k, (k & 2u) ? r1 : r0)) {
+                done = true;
+                hmask = 0;
+            }
+        }
+        if (group > 1) {  // the lanes of a ray tell each other
+            float t = best_inst < 0 ? INFINITY : any ? -INFINITY : t_max;
+            for (int off = 1; off < group; off <<= 1) t = fminf(t, __shfl_xor(t, off, 64));
+            if (any)
+                done |= t < INFINITY;
+            else
+                t_cull = fminf(t_cull, t + fabsf(t) * kSoftWindow);
+        }
+        if (!done && (stale | ((item & kLeafBit) != 0))) {  // only ever in the TLAS
+            const TwoLevelView& s = fields();
+            world(O, D);
+            wide = s.tlas_wide;
+            records = s.tlas_records;
+            stale = false;
+            const int next = item & kLeafBit ? int(item & kIndexMask) : -1;
+            if (next >= 0) {
+                item = kNone;
+                stale = true;
+            }
+            if (uint32_t(next) < uint32_t(s.instance_count)) {
+                const DevInstance& in = s.instances[next];
+                const int tri_count = in.tri_count, first = in.first;
+                if (tri_count > 0 && first >= 0) {
+                    const f3 WO = O, WD = D;
+                    xform_ray(in.inv, WO, WD, O, D);
+                    inst = next;
+                    in_blas = true;
+                    stale = false;
+                    sp0 = sp;
+                    wide = in.wide;
+                    records = uint32_t(tri_count) - 1u;
+                    tris = in.tris;
+                    ignore_local = (ignore >= first && ignore - first < tri_count) ? ignore - first : -1;
+                    if (records) {
+                        item = 0;
+                    } else {  // one triangle
+                        ref.x = kLeafBit;
+                        hc = 0;
+                        hmask = 1;
+                    }
+                }
+            }
+            sr = make_slab_ray(O, D, lo);
+            if (!wide_takes(D) || records >= kMaxWideRecords) {
+                failed = done = true;
+                hmask = 0;
+            }
+        }
     }
-    const int local = best_prim - in.first;
-    const float* p = reinterpret_cast<const float*>(s.soup + in.tri_base + local);
-    float t;
-    (void)tri_uvt(xform_point(inv, WO), xform_vector(inv, WD), make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]),
-                  make3(p[6], p[7], p[8]), t, best.u, best.v);
-    best.prim = best_prim;
-    best.instance = inst;
-    best.local = local;
-    best.t = ob.t_max;
+    int at_inst = -1, at_tri = 0;  // the winner's leaves
+    if (best_inst >= 0) {
+        const TwoLevelView& s = fields();
+        const DevInstance& in = s.instances[best_inst];
+        at_inst = in.tlas_pos;
+        at_tri = in.tri_count > 1 ? s.meshes[in.mesh].wide_leaf[best_at] : 0;
+    }
+    if (group > 1) {
+        int fail = failed;
+        for (int off = 1; off < group; off <<= 1) {
+            fail |= __shfl_xor(fail, off, 64);
+            const float t = __shfl_xor(t_max, off, 64);
+            const int i = __shfl_xor(best_inst, off, 64), l = __shfl_xor(best_local, off, 64);
+            const int ai = __shfl_xor(at_inst, off, 64), at = __shfl_xor(at_tri, off, 64);
+            const bool first = ai < at_inst || (ai == at_inst && at < at_tri);
+            if (i >= 0 && (best_inst < 0 || t < t_max || (t == t_max && first))) {
+                t_max = t;
+                best_inst = i;
+                best_local = l;
+                at_inst = ai;
+                at_tri = at;
+            }
+        }
+        failed = fail != 0;
+    }
+    if (failed) return false;
+    if (best_inst < 0) return true;
+    // the winner's boxes, and its u and v: the same operations on the same
+    // operands as the leaf test that took it
+    const TwoLevelView& v = fields();
+    const DevInstance& in = v.instances[best_inst];
+    const DevMesh& mesh = v.meshes[in.mesh];
+    world(O, D);
+    const float t_box = any ? t_bound : t_max;
+    if (!wide_settled(v.tlas_nodes, at_inst, make_slab_ray(O, D, t_min), t_box)) return false;
+    f3 o, d;
+    xform_ray(in.inv, O, D, o, d);
+    if (!wide_settled(mesh.nodes, at_tri, make_slab_ray(o, d, t_min), t_box)) return false;
+    const float* p = reinterpret_cast<const float*>(in.tris + best_local);
+    (void)tri_uvt(o, d, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), best.t, best.u,
+                  best.v);
+    best.prim = in.first + best_local;
+    best.instance = best_inst;
+    best.local = best_local;
     return true;
 }
-
 
 // ---- host side ----------------------------------------------------------------------
 struct TwoLevelDev {
     std::vector<BvhDev> blas;  // per mesh (n = 0 for an empty mesh)
     BvhDev tlas;               // over the non-empty instance world bounds, ids = instance ids
-    // The TLAS's slots again, each leaf box narrowed to its instance's world
+    // Records over the TLAS with each leaf box narrowed to its instance's world
     // bounds intersected with the world box of the mesh's bounding sphere
     // (center M c, half-extent r |row i of M| on axis i: the exact box of the
     // transformed sphere), both widened by what the instance's M inv may
     // deviate from the identity; internal boxes the unions of their children.
-    // The near-child-first closest walk and the occlusion walk cull TLAS steps
-    // with them.
-    lux_bvh_node* tlas_cull = nullptr;
+    WideNode* tlas_wide = nullptr;
     std::vector<float> mesh_sphere;  // per mesh: center xyz, radius (padded)
     lux_triangle* soup = nullptr;
     DevMesh* meshes = nullptr;

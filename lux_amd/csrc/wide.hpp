@@ -20,7 +20,7 @@
 // moving each face outwards by at least 2^-10 of the scale (make_wide), the first
 // by kWideSlack in the far faces' base. An axis the reference treats as parallel
 // (|d| < 1e-12, origin inside the slab or not) compares the origin with the
-// byte faces (kPar, chosen per wave). A record with a face beyond 1e18 or not
+// byte faces (wide_parallel; chosen per wave). A record with a face beyond 1e18 or not
 // finite has org = NaN, and every comparison with NaN passes. Rays with a
 // direction component beyond 1e18 (or NaN) take the preorder walk.
 //
@@ -152,13 +152,69 @@ __device__ __forceinline__ bool wide_settled(const lux_bvh_node* __restrict__ no
     return pass && !(tn > t) && !nan;
 }
 
-// One axis of one child for a ray parallel to its slab: everywhere inside it,
-// or nowhere (rel = org - o).
-__device__ __forceinline__ void wide_parallel(bool par, float lo, float hi, float scale, float rel, float& tn,
-                                              float& tf) {
-    if (!par) return;
-    tn = __builtin_fmaf(lo, scale, rel) > 0.0f ? INFINITY : -INFINITY;
-    tf = __builtin_fmaf(hi, scale, rel) < 0.0f ? -INFINITY : INFINITY;
+// One axis of a record for a ray parallel to it: everywhere inside a child's slab,
+// or nowhere. The origin's place in byte units, cut at 1024 either way, stands for
+// the distances, times 2^116: inside, a face is at least 2^-10 away (see above),
+// so the entry is below -2^105 and the exit beyond 2^105, more than any hit's
+// distance (coordinates below 1e18, other components above 1e-12); outside by
+// more than 2^-9, one of them is the other way round.
+__device__ __forceinline__ void wide_parallel(bool par, float org, float scale, float o, float& s, float& base) {
+    float r = (org - o) * __builtin_amdgcn_rcpf(scale);
+    r = r > 1024.0f ? 1024.0f : r;
+    r = r < -1024.0f ? -1024.0f : r;
+    s = par ? 0x1p116f : s;
+    base = par ? r * 0x1p116f : base;
+}
+
+// The four byte boxes of a record (its first three float4) against the ray: entry
+// distances and whether they are met between the ray's t_min and t_cull. kPar:
+// some axis may be parallel; its inv is 0 (no other is, see wide_takes) and signs
+// are read from inv, so that the ray's six flags need no registers.
+template <bool kPar>
+__device__ __forceinline__ void wide_boxes(const float4& a, const float4& b, const float4& q, const SlabRay& r,
+                                           float t_cull, float* key, bool* pass) {
+    float sx = a.w * r.inv.x, sy = b.x * r.inv.y, sz = b.y * r.inv.z;
+    float bx = (a.x - r.o.x) * r.inv.x, by = (a.y - r.o.y) * r.inv.y, bz = (a.z - r.o.z) * r.inv.z;
+    if (kPar) {
+        wide_parallel(r.inv.x == 0.0f, a.x, a.w, r.o.x, sx, bx);
+        wide_parallel(r.inv.y == 0.0f, a.y, b.x, r.o.y, sy, by);
+        wide_parallel(r.inv.z == 0.0f, a.z, b.y, r.o.z, sz, bz);
+    }
+    const bool nx = kPar ? r.inv.x < 0.0f : r.neg_x, ny = kPar ? r.inv.y < 0.0f : r.neg_y,
+               nz = kPar ? r.inv.z < 0.0f : r.neg_z;
+    const float ex = __builtin_fmaf(fabsf(bx), kWideSlack, bx), ey = __builtin_fmaf(fabsf(by), kWideSlack, by),
+                ez = __builtin_fmaf(fabsf(bz), kWideSlack, bz);
+    const uint32_t lx = __float_as_uint(b.z), ly = __float_as_uint(b.w), lz = __float_as_uint(q.x),
+                   hx = __float_as_uint(q.y), hy = __float_as_uint(q.z), hz = __float_as_uint(q.w);
+    const uint32_t fx = nx ? hx : lx, gx = nx ? lx : hx, fy = ny ? hy : ly, gy = ny ? ly : hy, fz = nz ? hz : lz,
+                   gz = nz ? lz : hz;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float ax = __builtin_fmaf(byte_of(fx, k), sx, bx), cx = __builtin_fmaf(byte_of(gx, k), sx, ex);
+        const float ay = __builtin_fmaf(byte_of(fy, k), sy, by), cy = __builtin_fmaf(byte_of(gy, k), sy, ey);
+        const float az = __builtin_fmaf(byte_of(fz, k), sz, bz), cz = __builtin_fmaf(byte_of(gz, k), sz, ez);
+        key[k] = fmaxf(fmaxf(fmaxf(ax, ay), az), r.t_min);
+        pass[k] = !(key[k] > fminf(fminf(fminf(cx, cy), cz), t_cull));
+    }
+}
+
+// Four children in the order of their keys.
+__device__ __forceinline__ void wide_sort(float* key, uint32_t* kid) {
+    auto order = [&](int i, int j) {
+        // loaded first: a select between array elements becomes one between their indexes
+        const float ki = key[i], kj = key[j];
+        const uint32_t ri = kid[i], rj = kid[j];
+        const bool sw = kj < ki;
+        key[i] = sw ? kj : ki;
+        key[j] = sw ? ki : kj;
+        kid[i] = sw ? rj : ri;
+        kid[j] = sw ? ri : rj;
+    };
+    order(0, 1);
+    order(2, 3);
+    order(0, 2);
+    order(1, 3);
+    order(1, 2);
 }
 
 // Entries of a lane's LDS stack (`stride` words apart, so lanes never share a
@@ -194,49 +250,20 @@ __device__ __forceinline__ bool wide_walk(const WideNode* __restrict__ wide, uin
                 float4 a, b, q;
                 load_wide(wide, c, a, b, q, ref);
                 visits += 2;
-                const float sx = a.w * r.inv.x, sy = b.x * r.inv.y, sz = b.y * r.inv.z;
-                const float bx = (a.x - r.o.x) * r.inv.x, by = (a.y - r.o.y) * r.inv.y, bz = (a.z - r.o.z) * r.inv.z;
-                const float ex = __builtin_fmaf(fabsf(bx), kWideSlack, bx), ey = __builtin_fmaf(fabsf(by), kWideSlack, by),
-                            ez = __builtin_fmaf(fabsf(bz), kWideSlack, bz);
-                const uint32_t lx = __float_as_uint(b.z), ly = __float_as_uint(b.w), lz = __float_as_uint(q.x),
-                               hx = __float_as_uint(q.y), hy = __float_as_uint(q.z), hz = __float_as_uint(q.w);
-                const uint32_t fx = r.neg_x ? hx : lx, gx = r.neg_x ? lx : hx, fy = r.neg_y ? hy : ly,
-                               gy = r.neg_y ? ly : hy, fz = r.neg_z ? hz : lz, gz = r.neg_z ? lz : hz;
                 float key[4];
+                bool pass[4];
+                wide_boxes<kPar>(a, b, q, r, t_cull, key, pass);
                 uint32_t kid[4] = {ref.x, ref.y, ref.z, ref.w};
                 uint32_t mask = 0;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    float ax = __builtin_fmaf(byte_of(fx, k), sx, bx), cx = __builtin_fmaf(byte_of(gx, k), sx, ex);
-                    float ay = __builtin_fmaf(byte_of(fy, k), sy, by), cy = __builtin_fmaf(byte_of(gy, k), sy, ey);
-                    float az = __builtin_fmaf(byte_of(fz, k), sz, bz), cz = __builtin_fmaf(byte_of(gz, k), sz, ez);
-                    if (kPar) {
-                        wide_parallel(r.par_x, byte_of(lx, k), byte_of(hx, k), a.w, a.x - r.o.x, ax, cx);
-                        wide_parallel(r.par_y, byte_of(ly, k), byte_of(hy, k), b.x, a.y - r.o.y, ay, cy);
-                        wide_parallel(r.par_z, byte_of(lz, k), byte_of(hz, k), b.y, a.z - r.o.z, az, cz);
-                    }
-                    const float tn = fmaxf(fmaxf(fmaxf(ax, ay), az), r.t_min);
-                    const bool pass = !(tn > fminf(fminf(fminf(cx, cy), cz), t_cull));
                     const bool is_leaf = int32_t(kid[k]) < 0;
-                    key[k] = (pass & !is_leaf) ? tn : INFINITY;
-                    mask |= (pass & is_leaf) ? (1u << k) : 0u;
+                    key[k] = (pass[k] & !is_leaf) ? key[k] : INFINITY;
+                    mask |= (pass[k] & is_leaf) ? (1u << k) : 0u;
                 }
                 hc = c;
                 hmask = mask;
-                auto order = [&](int i, int j) {
-                    const bool sw = key[j] < key[i];
-                    const float ki = sw ? key[j] : key[i], kj = sw ? key[i] : key[j];
-                    const uint32_t ri = sw ? kid[j] : kid[i], rj = sw ? kid[i] : kid[j];
-                    key[i] = ki;
-                    key[j] = kj;
-                    kid[i] = ri;
-                    kid[j] = rj;
-                };
-                order(0, 1);
-                order(2, 3);
-                order(0, 2);
-                order(1, 3);
-                order(1, 2);
+                wide_sort(key, kid);
                 if (key[0] < INFINITY) {
                     c = kid[0];
                     if (key[1] < INFINITY) {
@@ -321,6 +348,26 @@ __host__ __device__ inline int lanes_per_ray(uint32_t n) {
     return n <= (1u << 14) ? 16 : n <= (1u << 16) ? 8 : n <= kPartsMaxRays ? 4 : 1;
 }
 
+// Part `part` of `group` of the interval in which ray r meets the root box: lo and
+// hi (the ray's bounds before) become its ends. An interval that is empty or not
+// finite leaves the whole ray to the first lane; the others get false.
+__device__ __forceinline__ bool ray_part(const lux_bvh_node* __restrict__ nodes, const SlabRay& r, int group, int part,
+                                         float& lo, float& hi) {
+    float4 a, b;
+    load_node(nodes, 0, a, b);
+    float enter;
+    (void)slab_near<true>(r, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, enter);
+    float leave = hi;
+    if (!r.par_x) leave = fminf(leave, ((r.neg_x ? a.x : a.w) - r.o.x) * r.inv.x);
+    if (!r.par_y) leave = fminf(leave, ((r.neg_y ? a.y : b.x) - r.o.y) * r.inv.y);
+    if (!r.par_z) leave = fminf(leave, ((r.neg_z ? a.z : b.y) - r.o.z) * r.inv.z);
+    const float step = (leave - enter) / float(group);
+    const bool cut = step > 0.0f && step < 1e30f;
+    if (cut && part + 1 < group) hi = enter + step * float(part + 1);
+    if (cut && part != 0) lo = enter + step * float(part);
+    return cut || part == 0;
+}
+
 // One ray, on `group` lanes in a row (a power of two; 1: a lane by itself), this
 // lane walking part `part` of the interval in which the ray meets the root box.
 // Every lane of a group has the same ray and gets the group's result. any: any
@@ -346,24 +393,7 @@ __device__ __forceinline__ WideHit wide_query(const RayTree& tree, const lux_tri
     }
     SlabRay sr = make_slab_ray(o, d, t_min);
     float hi = t_bound;
-    bool skip = false;
-    if (group > 1) {
-        // an interval in the root box that is empty or not finite leaves the whole
-        // ray to the first lane
-        float4 a, b;
-        load_node(tree.nodes, 0, a, b);
-        float enter;
-        (void)slab_near<true>(sr, INFINITY, a.x, a.y, a.z, a.w, b.x, b.y, enter);
-        float leave = t_bound;
-        if (!sr.par_x) leave = fminf(leave, ((sr.neg_x ? a.x : a.w) - o.x) * sr.inv.x);
-        if (!sr.par_y) leave = fminf(leave, ((sr.neg_y ? a.y : b.x) - o.y) * sr.inv.y);
-        if (!sr.par_z) leave = fminf(leave, ((sr.neg_z ? a.z : b.y) - o.z) * sr.inv.z);
-        const float step = (leave - enter) / float(group);
-        const bool cut = step > 0.0f && step < 1e30f;
-        skip = !cut && part != 0;
-        if (cut && part + 1 < group) hi = enter + step * float(part + 1);
-        if (cut && part != 0) sr.t_min = enter + step * float(part);
-    }
+    const bool skip = group > 1 && !ray_part(tree.nodes, sr, group, part, sr.t_min, hi);
     float t_max = t_bound;  // the held bound
     float t_cull = wide_bound(hi);
     int best = -1;
