@@ -604,7 +604,6 @@ __global__ __launch_bounds__(kBlock) void k_top_layout(int n, const uint32_t* __
 // the nodes over an edge lie on one root path, at most 64 long (a child's
 // common key prefix is longer than its parent's, and keys have 64 bits).
 constexpr int kMaxFrontier = 128;
-constexpr int kLocalThreads = 512;
 
 struct FrontierRec {
     lux_aabb box;
@@ -619,7 +618,8 @@ __device__ __forceinline__ void store_node(lux_bvh_node* nodes, int pos, const l
     p[1] = make_float4(b.p_max.y, b.p_max.z, __int_as_float(prim), __int_as_float(esc < total ? esc : -1));
 }
 
-template <int kMode>
+// kLocalThreads: see launch_local.
+template <int kMode, int kLocalThreads>
 __global__ __launch_bounds__(kLocalThreads) void k_local(
     int n, const uint32_t* __restrict__ sorted_input, const int32_t* __restrict__ ids,
     const lux_aabb* __restrict__ src_boxes, const lux_triangle* __restrict__ src_tris,
@@ -1129,6 +1129,32 @@ __global__ __launch_bounds__(kBlock) void k_copies(int n, int wide_blocks, const
 
 }  // namespace
 
+// Few blocks: a block lasts as long as the climbs of one thread's leaves, so one
+// leaf per thread; more blocks than the CUs hold: the climbs of four leaves in
+// turn keep more of a wave's lanes at work than four waves would. Builds (with 500
+// rays) at 256 / 512 / 1024 threads: 1500 triangles 140 / 122 / 114 us, 60 000 200 /
+// 181 / 176, 131 072 212 / 197 / 201, 262 147 239 / 230 / 247, 400 000 282 / 283 / 319,
+// 2^20 522 / 538 / 631 us.
+template <int kMode>
+void launch_local(const char* name, BvhDev& d, const lux_aabb* src_boxes, const lux_triangle* src_tris, int write_back,
+                  hipStream_t s) {
+    const int blocks = div_up(d.n, kLocalLeaves);
+    auto go = [&](auto threads) {
+        constexpr int kThreads = decltype(threads)::value;
+        LUX_LAUNCH(name, (k_local<kMode, kThreads>), blocks, kThreads, 0, s, d.n, (const uint32_t*)d.vals[0],
+                   (const int32_t*)d.ids, src_boxes, src_tris, d.boxes, write_back, (const uint32_t*)d.parent,
+                   (const uint32_t*)d.leaf_parent, (const uint32_t*)d.first, (const uint32_t*)d.last,
+                   (const uint32_t*)d.rtop_int, (const uint32_t*)d.rtop_leaf, d.nodes, d.pre_internal, d.pre_leaf,
+                   d.edge_boxes, d.block_boxes, d.info);
+    };
+    if (blocks <= 96)
+        go(std::integral_constant<int, 1024>{});
+    else if (blocks <= 384)
+        go(std::integral_constant<int, 512>{});
+    else
+        go(std::integral_constant<int, 256>{});
+}
+
 void wide_from(const BvhDev& d, const lux_bvh_node* nodes, WideNode* wide, int32_t* wide_leaf, hipStream_t s) {
     if (d.n < 2) return;
     const int blocks = min(4096, div_up(d.n - 1, kBlock));
@@ -1303,11 +1329,7 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
                    (const uint32_t*)d.parent, (const uint32_t*)d.left, (const uint32_t*)d.right,
                    (const uint32_t*)d.first, (const uint32_t*)d.last, d.rtop_int, d.rtop_leaf, d.pre_internal,
                    d.info);
-    LUX_LAUNCH("lbvh_local", k_local<0>, blocks, kLocalThreads, 0, s, n, (const uint32_t*)d.vals[0],
-               (const int32_t*)d.ids, (const lux_aabb*)d.boxes, (const lux_triangle*)nullptr, d.boxes, 0,
-               (const uint32_t*)d.parent, (const uint32_t*)d.leaf_parent, (const uint32_t*)d.first,
-               (const uint32_t*)d.last, (const uint32_t*)d.rtop_int, (const uint32_t*)d.rtop_leaf, d.nodes,
-               d.pre_internal, d.pre_leaf, d.edge_boxes, d.block_boxes, d.info);
+    launch_local<0>("lbvh_local", d, d.boxes, nullptr, 0, s);
     top_boxes<true>(d, s);
     fill_copies(d, s);
 }
@@ -1323,11 +1345,7 @@ void refit_launch(BvhDev& d, const lux_aabb* in_boxes, const lux_triangle* tris,
         fill_copies(d, s);
         return;
     }
-    LUX_LAUNCH(kMode == 2 ? "lbvh_local_tris" : "lbvh_local_boxes", k_local<kMode>, div_up(n, kLocalLeaves),
-               kLocalThreads, 0, s, n, (const uint32_t*)d.vals[0], (const int32_t*)d.ids, in_boxes, tris, d.boxes,
-               wb, (const uint32_t*)d.parent, (const uint32_t*)d.leaf_parent, (const uint32_t*)d.first,
-               (const uint32_t*)d.last, (const uint32_t*)d.rtop_int, (const uint32_t*)d.rtop_leaf, d.nodes,
-               d.pre_internal, d.pre_leaf, d.edge_boxes, d.block_boxes, d.info);
+    launch_local<kMode>(kMode == 2 ? "lbvh_local_tris" : "lbvh_local_boxes", d, in_boxes, tris, wb, s);
     top_boxes<false>(d, s);
     fill_copies(d, s);
 }
