@@ -139,14 +139,14 @@ def main():
     a = ap.parse_args()
     s = summarize(a.pass_a, a.pass_b, a.fetch_scale, a.write_scale)
     print(table(s))
-    picks = {"k_trace_any": "trace_any", "k_trace_closest<true>": "trace_closest"}
+    picks = {"k_trace<true>": "trace_any", "k_trace<false>": "trace_closest"}
     if a.json:
         p = Path(a.json)
         table_ = json.loads(p.read_text()) if p.exists() else {}
         for key, e in s.items():
             name = e["kernel"]
             if name in picks and e["grid"] == a.rays:
-                table_[name.split("<")[0]] = dict(e, rays=a.rays, triangles=a.triangles, source=a.source)
+                table_["k_" + picks[name]] = dict(e, rays=a.rays, triangles=a.triangles, source=a.source)
         p.write_text(json.dumps(table_, indent=1) + "\n")
     if a.traffic:
         p = Path(a.traffic)

@@ -1134,7 +1134,8 @@ __global__ __launch_bounds__(kBlock) void k_copies(int n, int wide_blocks, const
 // turn keep more of a wave's lanes at work than four waves would. Builds (with 500
 // rays) at 256 / 512 / 1024 threads: 1500 triangles 140 / 122 / 114 us, 60 000 200 /
 // 181 / 176, 131 072 212 / 197 / 201, 262 147 239 / 230 / 247, 400 000 282 / 283 / 319,
-// 2^20 522 / 538 / 631 us.
+// 2^20 522 / 538 / 631 us. A refit has no preorder climb to share: 2^20 triangles 122
+// / 107 us for the pass at 256 / 512.
 template <int kMode>
 void launch_local(const char* name, BvhDev& d, const lux_aabb* src_boxes, const lux_triangle* src_tris, int write_back,
                   hipStream_t s) {
@@ -1149,7 +1150,7 @@ void launch_local(const char* name, BvhDev& d, const lux_aabb* src_boxes, const 
     };
     if (blocks <= 96)
         go(std::integral_constant<int, 1024>{});
-    else if (blocks <= 384)
+    else if (kMode != 0 || blocks <= 384)
         go(std::integral_constant<int, 512>{});
     else
         go(std::integral_constant<int, 256>{});

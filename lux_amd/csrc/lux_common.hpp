@@ -212,15 +212,6 @@ __device__ __forceinline__ bool wave_any_parallel(const SlabRay& r) {
 }
 
 template <int kMode>
-__device__ __forceinline__ bool slab_pass(const SlabRay& r, float t_max, float lox, float loy, float loz, float hix,
-                                          float hiy, float hiz) {
-    if constexpr (kMode == kSlabParallel)
-        return slab_hit(r, t_max, lox, loy, loz, hix, hiy, hiz);
-    else
-        return slab_hit_np<kMode>(r, t_max, lox, loy, loz, hix, hiy, hiz);
-}
-
-template <int kMode>
 using SlabMode = std::integral_constant<int, kMode>;
 
 // Calls f(SlabMode<m>{}) with the wave's slab-test mode (wave-uniform: every

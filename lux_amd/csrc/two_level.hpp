@@ -206,10 +206,9 @@ __device__ __forceinline__ TwoLevelHit two_level_walk(const TwoLevelView& s, Wor
 // A ray on `group` lanes: parts of it as in wide_query; an instance's culling box
 // holds its geometry at every t, so a triangle's boxes of both levels are met in
 // the same part.
-// 2^20 random rays over 64 instances of 2^16 triangles: closest 2.0 ms, occlusion
-// 1.7 ms; by sibling pairs 4.7 (near child first, one lane's entries at a time)
-// and 2.7 ms (preorder, gathered). 1000 rays over 40 instances of 5000: 105 us
-// against 422.
+// 2^22 rays over 64 instances of 2^16 triangles: closest 8.1 ms, occlusion 6.7 ms;
+// by sibling pairs 18.8 (near child first, one lane's entries at a time) and 11.9 ms
+// (preorder, gathered). 1000 rays over 40 instances of 5000: 105 us against 422.
 // kReload: the view is in memory and read again at each use, so that its fields
 // take no registers through the walk.
 template <bool kReload, typename World>
