@@ -82,16 +82,13 @@ void require_init() {
 
 hipStream_t pick(lux_stream s) { return s ? static_cast<hipStream_t>(s) : g_stream; }
 
-// Reads and clears the device-side check bits of a handle (caller synchronised).
-void check_device_flags(lux_hip_bvh* h) {
+// Reads and clears the device-side check bits of a handle (caller synchronised `s`).
+void check_device_flags(lux_hip_bvh* h, hipStream_t s) {
     if (!h->dev.info) return;
     DevInfo info;
     hip_check(hipMemcpy(&info, h->dev.info, sizeof(DevInfo), hipMemcpyDeviceToHost), "read device info");
     if (info.error == 0) return;
-    uint32_t zero = 0;
-    hip_check(hipMemcpy(reinterpret_cast<char*>(h->dev.info) + offsetof(DevInfo, error), &zero,
-                        sizeof(zero), hipMemcpyHostToDevice),
-              "clear device info");
+    zero_words(&h->dev.info->error, 1, s);
     std::string what;
     if (info.error & kErrNegativeId) what += " negative primitive id;";
     if (info.error & kErrPrimRange) what += " leaf primitive id outside the triangle array;";
@@ -103,8 +100,9 @@ void check_device_flags(lux_hip_bvh* h) {
 }
 
 void sync_handle(lux_hip_bvh* h) {
-    hip_check(hipStreamSynchronize(h->last_stream ? h->last_stream : g_stream), "synchronize");
-    check_device_flags(h);
+    hipStream_t s = h->last_stream ? h->last_stream : g_stream;
+    hip_check(hipStreamSynchronize(s), "synchronize");
+    check_device_flags(h, s);
 }
 
 void require_handle(lux_hip_bvh* h) {
@@ -326,7 +324,7 @@ int lux_hip_bvh_build(lux_hip_bvh* bvh, const lux_aabb* boxes, const int32_t* id
             bvh->host_ids_known = true;
             return int(LUX_OK);
         }
-        bvh_allocate(bvh->dev, n);
+        bvh_allocate(bvh->dev, n, g_stream);
         hip_check(hipMemcpyAsync(bvh->dev.boxes, boxes, sizeof(lux_aabb) * n, hipMemcpyHostToDevice, g_stream),
                   "H2D boxes");
         hip_check(hipMemcpyAsync(bvh->dev.ids, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, g_stream),
@@ -358,7 +356,7 @@ int lux_hip_bvh_build_device(lux_hip_bvh* bvh, const lux_aabb* d_boxes, const in
         hipStream_t s = pick(stream);
         if (bvh->last_stream && bvh->last_stream != s) hip_check(hipStreamSynchronize(bvh->last_stream), "synchronize");
         bvh->last_stream = s;
-        bvh_allocate(bvh->dev, n);
+        bvh_allocate(bvh->dev, n, s);
         lbvh_build(bvh->dev, d_boxes, d_ids, n, s);
         bvh->valid = true;  // negative ids are reported by lux_hip_bvh_info
         return int(LUX_OK);
@@ -685,7 +683,7 @@ static int overlap_host(lux_hip_bvh* tree, lux_hip_bvh* queries, bool self_mode,
     hip_check(hipStreamSynchronize(g_stream), "synchronize");
     int32_t copy = count < max_pairs ? count : max_pairs;
     if (copy > 0) hip_check(hipMemcpy(pairs, dp.p, sizeof(lux_pair) * copy, hipMemcpyDeviceToHost), "D2H pairs");
-    check_device_flags(tree);
+    check_device_flags(tree, g_stream);
     *found = count;
     return LUX_OK;
 }
@@ -758,16 +756,14 @@ void require_two_level(lux_hip_two_level* s) {
 
 // Waits for the scene's last stream and turns device check bits into an error.
 void sync_two_level(lux_hip_two_level* s) {
-    hip_check(hipStreamSynchronize(s->last_stream ? s->last_stream : g_stream), "synchronize");
+    hipStream_t stream = s->last_stream ? s->last_stream : g_stream;
+    hip_check(hipStreamSynchronize(stream), "synchronize");
     DevInfo* info = s->dev.tlas.info;
     if (!info) return;
     DevInfo h;
     hip_check(hipMemcpy(&h, info, sizeof(DevInfo), hipMemcpyDeviceToHost), "read device info");
     if (h.error == 0) return;
-    uint32_t zero = 0;
-    hip_check(hipMemcpy(reinterpret_cast<char*>(info) + offsetof(DevInfo, error), &zero, sizeof(zero),
-                        hipMemcpyHostToDevice),
-              "clear device info");
+    zero_words(&info->error, 1, stream);
     std::string what;
     if (h.error & kErrPrimRange) what += " leaf primitive id outside its mesh;";
     if (h.error & kErrWalkOrder) what += " two-level walk exceeded its step limit;";
@@ -1075,7 +1071,7 @@ void check_settings(const lux_render_settings* s) {
         throw lux::Error(LUX_ERR_INVALID_ARGUMENT, "unknown light sampler");
 }
 
-// Reads and clears the device check bits of a scene (caller synchronised):
+// Reads and clears the device check bits of a scene (caller synchronised g_stream):
 // the LBVH's, or the TLAS's for an instanced scene (the two-level walk
 // reports there).
 void scene_check(lux_hip_scene* sc) {
@@ -1084,10 +1080,7 @@ void scene_check(lux_hip_scene* sc) {
     lux::DevInfo info;
     lux::hip_check(hipMemcpy(&info, d, sizeof(info), hipMemcpyDeviceToHost), "read device info");
     if (info.error) {
-        uint32_t zero = 0;
-        lux::hip_check(hipMemcpy(reinterpret_cast<char*>(d) + offsetof(lux::DevInfo, error), &zero, 4,
-                                 hipMemcpyHostToDevice),
-                       "clear device info");
+        lux::zero_words(&d->error, 1, lux::g_stream);
         throw lux::Error(LUX_ERR_DEVICE_CHECK, "device check failed during render");
     }
 }

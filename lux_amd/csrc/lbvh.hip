@@ -269,6 +269,24 @@ __global__ void k_zero_u32(uint32_t* p, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
 
+// What the kernels of a new tree expect to be zero: look-back words (epoch 0 is
+// never used), tile tickets, the pair counter and the tree's info. A kernel on
+// the stream that builds the tree: hipMemset is ordered on the null stream,
+// which no stream of the library waits for, and returns before it is done
+// (16 bytes: 5 us; the fill itself came 2.6 ms later on a chip kept busy by another
+// stream). A pass that starts on another tree's tickets takes a tile out of range.
+__global__ void k_clear_tree(uint64_t* __restrict__ status, int words, uint32_t* __restrict__ tickets,
+                             int32_t* __restrict__ counter, DevInfo* __restrict__ info) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x) status[i] = 0;
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < 4) {
+            tickets[threadIdx.x] = 0;
+            counter[threadIdx.x] = 0;
+        }
+        if (threadIdx.x < sizeof(DevInfo) / 4) reinterpret_cast<uint32_t*>(info)[threadIdx.x] = 0;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // 3. one stable LSD radix pass (8-bit digit) with decoupled look-back
 // ---------------------------------------------------------------------------
@@ -1218,8 +1236,8 @@ const uint32_t* ray_order(RaySortDev& r, const BvhDev& tree, const lux_ray* rays
         r.hist = dalloc<uint32_t>(2 * kRadix);
         r.status = dalloc<uint64_t>(ray_order_status_words(n));
         r.tickets = dalloc<uint32_t>(4);
-        hip_check(hipMemset(r.status, 0, sizeof(uint64_t) * ray_order_status_words(n)), "hipMemset status");
-        hip_check(hipMemset(r.tickets, 0, sizeof(uint32_t) * 4), "hipMemset tickets");
+        zero_words(reinterpret_cast<uint32_t*>(r.status), 2 * ray_order_status_words(n), s);
+        zero_words(r.tickets, 4, s);
     }
     const RayOrderBufs b{{r.keys[0], r.keys[1]}, {r.vals[0], r.vals[1]}, r.hist, r.status, r.tickets};
     const uint32_t first = r.epoch + 1;
@@ -1227,7 +1245,7 @@ const uint32_t* ray_order(RaySortDev& r, const BvhDev& tree, const lux_ray* rays
     return ray_order_into(b, first, tree, rays, n, s);
 }
 
-void bvh_allocate(BvhDev& d, int n) {
+void bvh_allocate(BvhDev& d, int n, hipStream_t s) {
     if (n <= d.capacity && d.info) {
         d.n = n;
         return;
@@ -1267,12 +1285,8 @@ void bvh_allocate(BvhDev& d, int n) {
     d.slot_pre = dalloc<uint32_t>(2 * size_t(cap));
     d.wide = dalloc<WideNode>(cap);
     d.wide_leaf = dalloc<int32_t>(4 * size_t(cap));
-    // One-time clears at allocation: look-back words (epoch 0 is never used),
-    // tickets, info, frontier counts.
-    hip_check(hipMemset(d.status, 0, sizeof(uint64_t) * d.status_words), "hipMemset status");
-    hip_check(hipMemset(d.tickets, 0, sizeof(uint32_t) * 4), "hipMemset tickets");
-    hip_check(hipMemset(d.info, 0, sizeof(DevInfo)), "hipMemset info");
-    hip_check(hipMemset(d.counter, 0, sizeof(int32_t) * 4), "hipMemset counter");
+    LUX_LAUNCH("lbvh_clear", k_clear_tree, max(1, min(512, div_up(d.status_words, kBlock))), kBlock, 0, s, d.status,
+               d.status_words, d.tickets, d.counter, d.info);
     d.epoch = 0;
 }
 
@@ -1295,7 +1309,7 @@ void top_boxes(BvhDev& d, hipStream_t s) {
 }  // namespace
 
 void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int n, hipStream_t s) {
-    bvh_allocate(d, n);
+    bvh_allocate(d, n, s);
     if (n <= 0) return;
     int copy = (in_boxes != d.boxes || in_ids != d.ids) ? 1 : 0;
     int rb = reduce_blocks(n);
@@ -1387,7 +1401,7 @@ __global__ __launch_bounds__(kBlock) void k_tri_input(const lux_triangle* __rest
 
 void lbvh_build_triangles(BvhDev& d, const lux_triangle* tris, const lux_vec3* verts, const uint32_t* idx, int nv,
                           int n, hipStream_t s) {
-    bvh_allocate(d, n);
+    bvh_allocate(d, n, s);
     if (n <= 0) return;
     LUX_LAUNCH("lbvh_tri_input", k_tri_input, std::max(1, std::min(4096, div_up(n, kBlock))), kBlock, 0, s, tris,
                verts, idx, nv, n, d.boxes, d.ids, d.info);

@@ -112,7 +112,8 @@ struct BvhDev {
     int status_words = 0;
 };
 
-void bvh_allocate(BvhDev& d, int n);
+// Buffers for n primitives; new ones are cleared on `s`, the stream of the build.
+void bvh_allocate(BvhDev& d, int n, hipStream_t s);
 void bvh_release(BvhDev& d);
 
 // Scratch of the ray-order sort of the traversal entry points (grown on

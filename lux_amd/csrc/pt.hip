@@ -1139,6 +1139,13 @@ __global__ void k_zero_rays(unsigned long long* rays) {
     if (threadIdx.x < 2) rays[threadIdx.x] = 0;
 }
 
+// A new path buffer's counters, on the stream that uses it (a hipMemset would be
+// ordered on the null stream only).
+__global__ void k_clear_counts(uint32_t* counts, unsigned long long* rays) {
+    if (threadIdx.x < 4) counts[threadIdx.x] = 0;
+    if (threadIdx.x < 2) rays[threadIdx.x] = 0;
+}
+
 template <typename T>
 T* dalloc(size_t count) {
     void* p = nullptr;
@@ -1229,7 +1236,7 @@ void Renderer::release_graph() {
     graph_depth_ = graph_grid_ = graph_capacity_ = graph_block_ = graph_opaque_ = graph_walk_ = graph_light_ = -1;
 }
 
-void Renderer::ensure_capacity(int paths) {
+void Renderer::ensure_capacity(int paths, hipStream_t stream) {
     if (paths <= buf_.capacity) return;
     release_graph();  // the captured launches hold the old buffer addresses
     if (buf_.capacity) hip_check(hipDeviceSynchronize(), "synchronize before path buffer growth");
@@ -1242,8 +1249,7 @@ void Renderer::ensure_capacity(int paths) {
     buf_.counts = dalloc<uint32_t>(4);
     buf_.rays = dalloc<unsigned long long>(2);
     buf_.desc = static_cast<BatchDesc*>(static_cast<void*>(dalloc<uint8_t>(sizeof(BatchDesc))));
-    hip_check(hipMemset(buf_.counts, 0, 16), "hipMemset counts");
-    hip_check(hipMemset(buf_.rays, 0, 16), "hipMemset rays");
+    LUX_LAUNCH("pt_clear_counts", k_clear_counts, 1, 64, 0, stream, buf_.counts, buf_.rays);
 }
 
 namespace {
@@ -1279,7 +1285,7 @@ void Renderer::upload(BatchDesc* slot, hipStream_t stream) {
 }
 
 void Renderer::reset_ray_counts(hipStream_t stream) {
-    ensure_capacity(1);
+    ensure_capacity(1, stream);
     LUX_LAUNCH("pt_zero_rays", k_zero_rays, 1, 64, 0, stream, buf_.rays);
 }
 
@@ -1519,7 +1525,7 @@ void Renderer::launch_plain(int depth, uint32_t count, bool two_level, int light
 uint64_t Renderer::enqueue_batch(std::vector<Request*>& active, int slice_spp, int max_depth, hipStream_t stream,
                                  int64_t* batch_index) {
     const uint64_t cap = uint64_t(tune_.capacity);
-    ensure_capacity(tune_.capacity);
+    ensure_capacity(tune_.capacity, stream);
     BatchDesc* slot = next_slot();
     uint64_t used = 0;
     uint32_t nseg = 0;
@@ -1568,7 +1574,7 @@ void Renderer::render_all(std::vector<Request*>& reqs, int mode, hipStream_t str
         for (Request* rq : reqs) {
             const uint64_t npix = uint64_t(rq->rs.width) * uint64_t(rq->rs.height);
             const uint64_t B = uint64_t(rq->rs.batch_size > 0 ? rq->rs.batch_size : kPlainBatch);
-            ensure_capacity(int(std::min(B, npix)));
+            ensure_capacity(int(std::min(B, npix)), stream);
             uint32_t host_counts[4];
             for (int s = 0; s < rq->rs.spp; ++s) {
                 for (uint64_t p0 = 0; p0 < npix; p0 += B) {

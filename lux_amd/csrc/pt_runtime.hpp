@@ -240,7 +240,7 @@ public:
     int64_t batches_enqueued() const { return batch_counter_; }
 
 private:
-    void ensure_capacity(int paths);
+    void ensure_capacity(int paths, hipStream_t stream);
     BatchDesc* next_slot();
     void upload(BatchDesc* slot, hipStream_t stream);
     void launch_wavefront(int depth, bool opaque, bool two_level, bool small, int light, hipStream_t stream);

@@ -1,0 +1,141 @@
+"""Scenes of test_host_runtime.py: the library's host code stepped on the CPU over
+tests/hip_stub.cpp. Each scene runs in a process of its own (the stub's symbols
+must be there before the library is loaded):
+
+    python tests/host_runtime.py SCENE
+
+prints one JSON line. Kernels do not run; `Stub` sees every launch and does in
+host memory what a scene depends on (clears).
+"""
+
+import ctypes
+import json
+import sys
+from pathlib import Path
+
+import numpy as np
+
+ROOT = Path(__file__).resolve().parents[1]
+sys.path.insert(0, str(ROOT))
+
+STUB = Path(__file__).resolve().parent / "_build" / "libhip_stub.so"
+CALLBACK = ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p))
+
+
+class Stub:
+    def __init__(self):
+        self.lib = ctypes.CDLL(str(STUB), mode=ctypes.RTLD_GLOBAL)
+        self.lib.stub_live_bytes.restype = ctypes.c_uint64
+        self.launches = []
+        self.hooks = []  # (part of a kernel's name, function(stub, args))
+        self._cb = CALLBACK(self._launch)
+        self.lib.stub_on_launch(self._cb)
+
+    def _launch(self, name, stream, args):
+        name = name.decode()
+        self.launches.append(name)
+        if "k_zero_u32" in name:  # (uint32_t* p, int n)
+            ctypes.memset(ptr(args, 0), 0, 4 * i32(args, 1))
+        if "k_clear_tree" in name:  # (status, words, tickets, counter, info)
+            ctypes.memset(ptr(args, 0), 0, 8 * i32(args, 1))
+            for k, size in ((2, 16), (3, 16), (4, 64)):
+                ctypes.memset(ptr(args, k), 0, size)
+        if "k_clear_counts" in name:  # (counts, rays)
+            ctypes.memset(ptr(args, 0), 0, 16)
+            ctypes.memset(ptr(args, 1), 0, 16)
+        for part, fn in self.hooks:
+            if part in name:
+                fn(args)
+
+
+def ptr(args, k):
+    return ctypes.cast(args[k], ctypes.POINTER(ctypes.c_void_p))[0]
+
+
+def i32(args, k):
+    return ctypes.cast(args[k], ctypes.POINTER(ctypes.c_int32))[0]
+
+
+def words(address, count, dtype=np.uint32):
+    n = count * np.dtype(dtype).itemsize
+    return np.frombuffer((ctypes.c_uint8 * n).from_address(address), dtype)
+
+
+class SortWatch:
+    """Every radix pass must find its tile ticket at zero and, on a tree's first
+    pass, no look-back word of an earlier owner of the memory."""
+
+    def __init__(self, stub):
+        self.bad, self.passes = [], 0
+        stub.hooks.append(("k_sort_pass", self.see))
+
+    def see(self, args):
+        self.passes += 1
+        status, ticket, epoch, tiles = ptr(args, 7), ptr(args, 8), i32(args, 9), i32(args, 10)
+        if words(ticket, 1)[0] != 0:
+            self.bad.append(f"ticket {words(ticket, 1)[0]}")
+        if epoch == 1 and words(status, tiles * 256, np.uint64).any():
+            self.bad.append("look-back words of another sort")
+
+
+def sphere(k, freq=6):
+    from lux_amd import scenes
+
+    return scenes.displaced_icosphere(freq=freq + k, seed=0x4C5700 + k, width=16, height=16)
+
+
+def small_engine():
+    from lux_amd import render
+
+    render.set_tuning(capacity=4096, grid=8, block=256, use_graph=0)
+    return render
+
+
+def job(i):
+    return dict(width=16, height=16, spp=2, depth=2, seed=i)
+
+
+def tight_stream(render, scs, order, verts):
+    """The scenes served under a budget that holds two and a half of them."""
+    sizes = [sc.info()[2] for sc in scs]
+    probe = render.Server(hbm_budget=1 << 40, slice_spp=8)
+    probe.run([scs[0]], [job(0)], [0.0], want_films=False)
+    fixed = probe.stats()["peak_bytes"] - sizes[0]
+    probe.close()
+    sv = render.Server(hbm_budget=fixed + int(2.5 * max(sizes)), slice_spp=8)
+    sv.run([scs[k] for k in order], [job(i) for i in range(len(order))], [0.001 * i for i in range(len(order))],
+           vertices=verts, want_films=False)
+    st = sv.stats()
+    sv.close()
+    return st
+
+
+def clears(stub):
+    """Builds (handles, scenes, a served stream with evictions and restores) over
+    memory that holds old bytes."""
+    from lux_amd import abi, lbvh, workloads as W
+
+    watch = SortWatch(stub)
+    tris = W.soup(3000, seed=1)
+    bvh = lbvh.GpuBvh()
+    boxes = lbvh.DeviceArray.from_numpy(W.triangle_boxes(tris))
+    ids = lbvh.DeviceArray.from_numpy(np.arange(3000, dtype=np.int32))
+    bvh.build_device(boxes, ids, 3000)
+    rays = lbvh.DeviceArray(32 * ((1 << 21) + 3))
+    hits = lbvh.DeviceArray(8 * ((1 << 21) + 3))
+    d_tris = lbvh.DeviceArray.from_numpy(tris)
+    abi.call("lux_hip_trace_closest_device", bvh.handle, d_tris.ptr, 3000, rays.ptr, (1 << 21) + 3, hits.ptr,
+             None)  # sorted: the ray-order scratch
+    render = small_engine()
+    dicts = [sphere(k) for k in range(5)]
+    scs = [render.Scene(d, deferred=True) for d in dicts]
+    order = [0, 1, 2, 3, 4, 0, 2, 4, 1, 3, 0]
+    verts = [None] * len(order)
+    verts[5], verts[8] = dicts[0]["vertices"] + np.float32(1e-3), dicts[1]["vertices"] + np.float32(1e-3)
+    st = tight_stream(render, scs, order, verts)
+    return {"bad": watch.bad, "passes": watch.passes, "null_writes": stub.lib.stub_null_writes(),
+            "evictions": st["evictions"], "uploads": st["uploads"], "completed": st["completed"]}
+
+
+if __name__ == "__main__":
+    print(json.dumps(globals()[sys.argv[1]](Stub())))

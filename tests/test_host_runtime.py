@@ -1,0 +1,43 @@
+"""The library's host code over a stand-in for the HIP runtime (tests/hip_stub.cpp,
+tests/host_runtime.py): what it asks of the device, in which order, on which
+stream. On the CPU."""
+
+import json
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+
+
+@pytest.fixture(scope="session")
+def stub():
+    import shutil
+
+    include = Path("/opt/rocm/include")
+    if not (include / "hip" / "hip_runtime_api.h").exists() or shutil.which("g++") is None:
+        pytest.skip("needs g++ and the HIP headers")
+    out = HERE / "_build" / "libhip_stub.so"
+    out.parent.mkdir(exist_ok=True)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", f"-I{include}", str(HERE / "hip_stub.cpp"), "-o",
+                    str(out)], check=True)
+    return out
+
+
+def scene(stub, name):
+    r = subprocess.run([sys.executable, str(HERE / "host_runtime.py"), name], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stderr
+    return json.loads(r.stdout.splitlines()[-1])
+
+
+def test_new_trees_start_from_cleared_state_on_their_own_stream(stub):
+    """Sort tickets and look-back words are clear when the first pass of a tree (or
+    of a ray order) reads them, whatever the memory held and however late a fill
+    on the null stream comes; no device write is ordered on the null stream."""
+    r = scene(stub, "clears")
+    assert r["completed"] == 11 and r["evictions"] >= 2 and r["uploads"] >= 6 and r["passes"] > 20
+    assert r["bad"] == []
+    assert r["null_writes"] == 0
