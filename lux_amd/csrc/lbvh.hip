@@ -328,6 +328,10 @@ __global__ __launch_bounds__(kBlock) void k_sort_pass(const uint32_t* __restrict
     for (int w = tid; w < 4 * kRadix; w += kBlock) (&s_wave_cnt[0][0])[w] = 0;
     __syncthreads();
     const uint32_t tile = s_ticket;
+    if (tile >= uint32_t(num_tiles)) {  // a ticket counter that did not start at zero
+        if (tid == 0) set_error(info, kErrSpinLimit);
+        return;
+    }
     // Tickets are handed out in start order, so a tile only ever waits on tiles
     // that are already running. The last ticket resets the counter for the next
     // launch on this stream.
@@ -571,6 +575,10 @@ __global__ __launch_bounds__(kBlock) void k_top_layout(int n, const uint32_t* __
             rights += pp >> 31;
             p = pp & kIndexMask;
             ++depth;
+            if (p >= uint32_t(n - 1)) {
+                bad = true;
+                break;
+            }
         }
         const int pos = 2 * (n - 1 - int(last)) + int(rights);
         if (bad || pos < 0 || pos >= total) {
@@ -664,6 +672,7 @@ __global__ __launch_bounds__(kLocalThreads) void k_local(
     const int tid = threadIdx.x;
 
     for (int k = tid; k < kLocalLeaves / 4; k += kLocalThreads) s_arrive[k] = 0;
+    if (tid < kMaxFrontier) s_order[tid] = 0;
     if (tid == 0) s_fcount = 0;
     for (int k = tid; k < cnt; k += kLocalThreads) {
         const int i = lo + k;
@@ -746,6 +755,10 @@ __global__ __launch_bounds__(kLocalThreads) void k_local(
     for (int k = tid; k < cnt; k += kLocalThreads) {
         const int j = lo + k;
         const uint32_t in = sorted_input[j];
+        if (in >= uint32_t(n)) {  // only after a failed sort
+            set_error(info, kErrSpinLimit);
+            continue;
+        }
         lux_aabb box = kMode == 2 ? tri_box(src_tris[in]) : src_boxes[in];
         if (write_back) own_boxes[in] = box;
         int pre = s_pre_leaf[k];
@@ -818,7 +831,8 @@ __global__ __launch_bounds__(kLocalThreads) void k_local(
         for (uint32_t r = 0; r < fc; ++r) {
             const FrontierRec& f = s_fr[s_order[r]];
             acc = r ? box_join(acc, f.box) : f.box;
-            if (!(f.span >> 20)) edge_boxes[2 * size_t(lo + int((f.span >> 10) & 1023u)) + 1] = acc;
+            const int at = lo + int((f.span >> 10) & 1023u);
+            if (!(f.span >> 20) && at < n) edge_boxes[2 * size_t(at) + 1] = acc;
         }
         if (fc) block_boxes[blockIdx.x] = acc;
     } else if (tid == 64) {  // suffix unions, right to left (second wave)
@@ -826,7 +840,8 @@ __global__ __launch_bounds__(kLocalThreads) void k_local(
         for (uint32_t r = fc; r-- > 0;) {
             const FrontierRec& f = s_fr[s_order[r]];
             acc = r + 1 < fc ? box_join(f.box, acc) : f.box;
-            if (f.span >> 20) edge_boxes[2 * size_t(lo + int(f.span & 1023u))] = acc;
+            const int at = lo + int(f.span & 1023u);
+            if ((f.span >> 20) && at < n) edge_boxes[2 * size_t(at)] = acc;
         }
     }
 }
@@ -1047,84 +1062,6 @@ __device__ __forceinline__ void fill_pairs(int n, int first, int stride, const l
     }
 }
 
-// ---------------------------------------------------------------------------
-// four-child traversal records (wide.hpp)
-// ---------------------------------------------------------------------------
-// One thread per internal node: its two children, the larger internal one
-// opened, then the largest of the three. Its reads are gathers of positions and
-// 32-byte nodes close to each other (Karras order and preorder both follow the
-// leaves), its write one 64-byte record and 16 bytes of leaf positions.
-__device__ __forceinline__ void fill_wide(int n, int first, int stride, const uint32_t* __restrict__ left,
-                                          const uint32_t* __restrict__ right,
-                                          const int32_t* __restrict__ pre_internal,
-                                          const int32_t* __restrict__ pre_leaf,
-                                          const lux_bvh_node* __restrict__ nodes, WideNode* __restrict__ wide,
-                                          int32_t* __restrict__ wide_leaf, DevInfo* info) {
-    const int total = 2 * n - 1;
-    for (int i = first; i < n - 1; i += stride) {
-        lux_aabb box[4];
-        uint32_t ref[4];
-        int32_t pos[4];
-        float area[4] = {-1.0f, -1.0f, -1.0f, -1.0f};
-        bool bad = false;
-        auto load = [&](int k, uint32_t c) {
-            const uint32_t idx = c & kIndexMask;
-            const bool leaf = c & kLeafBit;
-            bad |= idx >= uint32_t(leaf ? n : n - 1);
-            const int p = bad ? 0 : (leaf ? pre_leaf[idx] : pre_internal[idx]);
-            bad |= uint32_t(p) >= uint32_t(total);
-            float4 a, b;
-            load_node(nodes, bad ? 0 : p, a, b);
-            box[k].p_min = lux_vec3{a.x, a.y, a.z};
-            box[k].p_max = lux_vec3{a.w, b.x, b.y};
-            pos[k] = p;
-            ref[k] = leaf ? (kLeafBit | uint32_t(__float_as_int(b.z))) : idx;
-            const float dx = a.w - a.x, dy = b.x - a.y, dz = b.y - a.z;
-            area[k] = leaf ? -1.0f : dx * dy + dy * dz + dz * dx;
-        };
-        load(0, left[i]);
-        load(1, right[i]);
-        int count = 2;
-#pragma unroll
-        for (int open = 0; open < 2; ++open) {
-            int best = -1;
-            float ba = -1.0f;
-#pragma unroll
-            for (int k = 0; k < 2 + open; ++k)
-                if (area[k] > ba) {
-                    ba = area[k];
-                    best = k;
-                }
-            if (best < 0 || bad) continue;
-            uint32_t c = 0;
-#pragma unroll
-            for (int k = 0; k < 2 + open; ++k)
-                if (k == best) c = ref[k];
-            const uint32_t cl = left[c], cr = right[c];
-#pragma unroll
-            for (int k = 0; k < 2 + open; ++k)
-                if (k == best) load(k, cl);
-            load(2 + open, cr);
-            ++count;
-        }
-        if (bad) {
-            set_error(info, kErrWalkOrder);
-            continue;
-        }
-#pragma unroll
-        for (int k = 2; k < 4; ++k)
-            if (k >= count) {
-                box[k] = box[0];
-                ref[k] = kWideEmpty;
-                pos[k] = -1;
-            }
-        WideNode w;
-        make_wide(w, box, ref, count);
-        store_wide(wide + i, w);
-        reinterpret_cast<int4*>(wide_leaf)[i] = make_int4(pos[0], pos[1], pos[2], pos[3]);
-    }
-}
-
 // Both traversal copies of the finished node array, in one launch: the first
 // `wide_blocks` workgroups make the records, the others the sibling pairs.
 __global__ __launch_bounds__(kBlock) void k_copies(int n, int wide_blocks, const uint32_t* __restrict__ left,
@@ -1138,8 +1075,8 @@ __global__ __launch_bounds__(kBlock) void k_copies(int n, int wide_blocks, const
                                                    DevInfo* info) {
     const int b = int(blockIdx.x);
     if (b < wide_blocks)
-        fill_wide(n, b * kBlock + int(threadIdx.x), wide_blocks * kBlock, left, right, pre_internal, pre_leaf, nodes,
-                  wide, wide_leaf, info);
+        for (int i = b * kBlock + int(threadIdx.x); i < n - 1; i += wide_blocks * kBlock)
+            fill_wide(n, i, left, right, pre_internal, pre_leaf, nodes, wide, wide_leaf, info);
     else
         fill_pairs(n, (b - wide_blocks) * kBlock + int(threadIdx.x), (int(gridDim.x) - wide_blocks) * kBlock, nodes,
                    pair_pos, pairs, slot_pre, info);

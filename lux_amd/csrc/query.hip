@@ -310,7 +310,11 @@ __global__ __launch_bounds__(kOvThreads) void k_overlap(const lux_bvh_node* __re
         bool emit = false;
         int qid = -1;
         if (tid < nql) {
-            const uint32_t src = qorder[q0 + tid];
+            uint32_t src = qorder[q0 + tid];
+            if (src >= uint32_t(nq)) {  // only after a failed sort
+                set_error(info, kErrSpinLimit);
+                src = 0;
+            }
             const lux_aabb qb = qboxes[src];
             qid = qids[src];
             sh.qb[tid] = qb;

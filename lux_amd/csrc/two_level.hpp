@@ -428,10 +428,10 @@ __device__ __forceinline__ bool two_level_wide(const TwoLevelView& view, World&&
     const DevMesh& mesh = v.meshes[in.mesh];
     world(O, D);
     const float t_box = any ? t_bound : t_max;
-    if (!wide_settled(v.tlas_nodes, at_inst, make_slab_ray(O, D, t_min), t_box)) return false;
+    if (!wide_settled(v.tlas_nodes, v.tlas_node_count, at_inst, make_slab_ray(O, D, t_min), t_box, v.info)) return false;
     f3 o, d;
     xform_ray(in.inv, O, D, o, d);
-    if (!wide_settled(mesh.nodes, at_tri, make_slab_ray(o, d, t_min), t_box)) return false;
+    if (!wide_settled(mesh.nodes, mesh.node_count, at_tri, make_slab_ray(o, d, t_min), t_box, v.info)) return false;
     const float* p = reinterpret_cast<const float*>(in.tris + best_local);
     (void)tri_uvt(o, d, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]), make3(p[6], p[7], p[8]), best.t, best.u,
                   best.v);

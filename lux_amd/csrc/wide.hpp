@@ -118,6 +118,97 @@ __device__ __forceinline__ void store_wide(WideNode* dst, const WideNode& w) {
                        __uint_as_float(w.ref[3]));
 }
 
+__device__ __forceinline__ WideNode empty_wide() {
+    WideNode w;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        w.org[a] = 0.0f;
+        w.scale[a] = 1.0f;
+        w.lo[a] = 0xffffffffu;  // an empty interval
+        w.hi[a] = 0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w.ref[k] = kWideEmpty;
+    return w;
+}
+
+// One thread per internal node: its two children, the larger internal one
+// opened, then the largest of the three. Its reads are gathers of positions and
+// 32-byte nodes close to each other (Karras order and preorder both follow the
+// leaves), its write one 64-byte record and 16 bytes of leaf positions. A node
+// whose links or positions are out of range (a damaged tree) gets a record without
+// children, never what the memory held.
+__device__ __forceinline__ void fill_wide(int n, int i, const uint32_t* __restrict__ left,
+                                          const uint32_t* __restrict__ right,
+                                          const int32_t* __restrict__ pre_internal,
+                                          const int32_t* __restrict__ pre_leaf,
+                                          const lux_bvh_node* __restrict__ nodes, WideNode* __restrict__ wide,
+                                          int32_t* __restrict__ wide_leaf, DevInfo* info) {
+    const int total = 2 * n - 1;
+    lux_aabb box[4];
+    uint32_t ref[4];
+    int32_t pos[4];
+    float area[4] = {-1.0f, -1.0f, -1.0f, -1.0f};
+    bool bad = false;
+    auto load = [&](int k, uint32_t c) {
+        const uint32_t idx = c & kIndexMask;
+        const bool leaf = c & kLeafBit;
+        bad |= idx >= uint32_t(leaf ? n : n - 1);
+        const int p = bad ? 0 : (leaf ? pre_leaf[idx] : pre_internal[idx]);
+        bad |= uint32_t(p) >= uint32_t(total);
+        float4 a, b;
+        load_node(nodes, bad ? 0 : p, a, b);
+        box[k].p_min = lux_vec3{a.x, a.y, a.z};
+        box[k].p_max = lux_vec3{a.w, b.x, b.y};
+        pos[k] = p;
+        ref[k] = leaf ? (kLeafBit | uint32_t(__float_as_int(b.z))) : idx;
+        const float dx = a.w - a.x, dy = b.x - a.y, dz = b.y - a.z;
+        area[k] = leaf ? -1.0f : dx * dy + dy * dz + dz * dx;
+    };
+    load(0, left[i]);
+    load(1, right[i]);
+    int count = 2;
+#pragma unroll
+    for (int open = 0; open < 2; ++open) {
+        int best = -1;
+        float ba = -1.0f;
+#pragma unroll
+        for (int k = 0; k < 2 + open; ++k)
+            if (area[k] > ba) {
+                ba = area[k];
+                best = k;
+            }
+        if (best < 0 || bad) continue;
+        uint32_t c = 0;
+#pragma unroll
+        for (int k = 0; k < 2 + open; ++k)
+            if (k == best) c = ref[k];
+        const uint32_t cl = left[c], cr = right[c];
+#pragma unroll
+        for (int k = 0; k < 2 + open; ++k)
+            if (k == best) load(k, cl);
+        load(2 + open, cr);
+        ++count;
+    }
+    if (bad) {
+        set_error(info, kErrWalkOrder);
+        store_wide(wide + i, empty_wide());
+        reinterpret_cast<int4*>(wide_leaf)[i] = make_int4(-1, -1, -1, -1);
+        return;
+    }
+#pragma unroll
+    for (int k = 2; k < 4; ++k)
+        if (k >= count) {
+            box[k] = box[0];
+            ref[k] = kWideEmpty;
+            pos[k] = -1;
+        }
+    WideNode w;
+    make_wide(w, box, ref, count);
+    store_wide(wide + i, w);
+    reinterpret_cast<int4*>(wide_leaf)[i] = make_int4(pos[0], pos[1], pos[2], pos[3]);
+}
+
 __device__ __forceinline__ void load_wide(const WideNode* nodes, uint32_t i, float4& a, float4& b, float4& c,
                                           uint4& r) {
     const char* p = reinterpret_cast<const char*>(nodes) + (i << 6);
@@ -140,9 +231,14 @@ __device__ __forceinline__ float wide_bound(float t) { return t + fabsf(t) * kWi
 
 // The winner (leaf node at preorder position pos, distance t): true when the
 // preorder walk returns it too (see above). An any-hit query passes the ray's
-// t_max as t: there the leaf box only has to be entered before it.
-__device__ __forceinline__ bool wide_settled(const lux_bvh_node* __restrict__ nodes, int pos, const SlabRay& sr,
-                                             float t) {
+// t_max as t: there the leaf box only has to be entered before it. A position out
+// of range (a damaged tree) is an error, and the preorder walk decides.
+__device__ __forceinline__ bool wide_settled(const lux_bvh_node* __restrict__ nodes, int node_count, int pos,
+                                             const SlabRay& sr, float t, DevInfo* info) {
+    if (uint32_t(pos) >= uint32_t(node_count)) {
+        set_error(info, kErrWalkOrder);
+        return false;
+    }
     float4 a, b;
     load_node(nodes, pos, a, b);
     float tn;
@@ -455,7 +551,7 @@ __device__ __forceinline__ WideHit wide_query(const RayTree& tree, const lux_tri
     }
     if (!hit.failed && hit.prim >= 0) {
         sr.t_min = t_min;
-        hit.failed = !wide_settled(tree.nodes, hit.pos, sr, hit.t);
+        hit.failed = !wide_settled(tree.nodes, tree.node_count, hit.pos, sr, hit.t, info);
     }
     return hit;
 }
