@@ -451,7 +451,9 @@ int lux_hip_server_submit(lux_hip_server* server, lux_hip_scene* scene, const lu
 int lux_hip_server_poll(lux_hip_server* server, int32_t block, uint64_t* done_ids, int32_t max_ids,
                         int32_t* n_done);
 /* Film sums (W*H*3, may be NULL) and arrival-to-completion latency of a
- * completed request; releases its film. */
+ * completed request; releases its film. A request whose scene could not be
+ * prepared, or whose scene's device checks failed while it rendered, returns that
+ * error here (from lux_hip_server_run: once the whole trace has ended). */
 int lux_hip_server_result(lux_hip_server* server, uint64_t request_id, float* film_sum, double* latency_s);
 int lux_hip_server_stats(lux_hip_server* server, lux_serve_stats* stats);
 /* Replays an arrival trace in real time on the server: request i arrives

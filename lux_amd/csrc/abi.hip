@@ -1071,18 +1071,10 @@ void check_settings(const lux_render_settings* s) {
         throw lux::Error(LUX_ERR_INVALID_ARGUMENT, "unknown light sampler");
 }
 
-// Reads and clears the device check bits of a scene (caller synchronised g_stream):
-// the LBVH's, or the TLAS's for an instanced scene (the two-level walk
-// reports there).
+// Device check bits of a scene as an error (caller synchronised g_stream).
 void scene_check(lux_hip_scene* sc) {
-    lux::DevInfo* d = sc->dev.instanced ? sc->dev.tl.tlas.info : sc->dev.bvh.info;
-    if (!d) return;
-    lux::DevInfo info;
-    lux::hip_check(hipMemcpy(&info, d, sizeof(info), hipMemcpyDeviceToHost), "read device info");
-    if (info.error) {
-        lux::zero_words(&d->error, 1, lux::g_stream);
+    if (lux::pt::scene_errors(sc->dev, lux::g_stream))
         throw lux::Error(LUX_ERR_DEVICE_CHECK, "device check failed during render");
-    }
 }
 
 // A scene whose device state was dropped (or never built: created deferred)
@@ -1368,7 +1360,6 @@ int lux_hip_scene_update_vertices(lux_hip_scene* sc, const lux_vec3* vertices, i
             return int(LUX_OK);
         }
         pt::scene_update_vertices(sc->dev, vertices, vertex_count, g_stream);
-        scene_check(sc);
         return int(LUX_OK);
     });
 }

@@ -284,6 +284,10 @@ void scene_upload_instanced(SceneDev& s, const lux_instanced_scene_desc& desc, h
 // shading arrays and the light table; the BLASes are kept.
 void scene_set_instances(SceneDev& s, const lux_instance* instances, int instance_count, hipStream_t stream);
 void scene_release(SceneDev& s);
+// The scene's device error bits (its LBVH's, or the TLAS's of an instanced scene,
+// where the two-level walk reports), cleared on `stream` if any is set. The caller
+// has waited for the work that may set them.
+uint32_t scene_errors(const SceneDev& s, hipStream_t stream);
 SceneView scene_view(const SceneDev& s);
 uint64_t request_paths(const lux_render_settings& rs);
 // Batch kind of a request: bit 0 two-level traversal, bits 1.. the light sampler.

@@ -638,6 +638,7 @@ void scene_upload(SceneDev& s, const lux_scene_desc& desc, hipStream_t stream) {
     LUX_LAUNCH("pt_gather_soup", k_gather_soup, std::min(div_up(nt, 256), 4096), 256, 0, stream, s.vertices,
                s.indices, nt, nv, s.soup, s.bvh.info);
     hip_check(hipStreamSynchronize(stream), "scene upload");
+    if (scene_errors(s, stream)) throw Error(LUX_ERR_DEVICE_CHECK, "device check failed during scene upload");
     s.device_bytes = scene_bytes(nt, nv, desc.normals != nullptr, nm, s.host_lights.size());
     s.resident = true;
 }
@@ -747,6 +748,7 @@ void scene_update_vertices(SceneDev& s, const lux_vec3* vertices, int vertex_cou
     upload_lights(s, stream);
     // the host arrays above are pageable: the copies complete before return
     hip_check(hipStreamSynchronize(stream), "scene update");
+    if (scene_errors(s, stream)) throw Error(LUX_ERR_DEVICE_CHECK, "device check failed during scene update");
     if (s.source) s.source->current.assign(vertices, vertices + vertex_count);
 }
 
@@ -987,6 +989,15 @@ void scene_release(SceneDev& s) {
     bvh_release(s.bvh);
     two_level_release(s.tl);
     s = SceneDev{};
+}
+
+uint32_t scene_errors(const SceneDev& s, hipStream_t stream) {
+    DevInfo* d = s.instanced ? s.tl.tlas.info : s.bvh.info;
+    if (!d) return 0;
+    uint32_t bits = 0;
+    hip_check(hipMemcpy(&bits, &d->error, sizeof(bits), hipMemcpyDeviceToHost), "read device errors");
+    if (bits) zero_words(&d->error, 1, stream);
+    return bits;
 }
 
 SceneView scene_view(const SceneDev& s) {

@@ -132,6 +132,7 @@ void Server::worker_loop() {
             scene_release(t->dead);  // hipFree waits for the device: off the scheduling thread
         } catch (...) {
             t->error = std::current_exception();
+            if (t->restore) scene_release(t->fresh);
         }
         t->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         t->done.store(true, std::memory_order_release);
@@ -147,11 +148,28 @@ void Server::finish_tasks() {
             ++it;
             continue;
         }
-        if (t->error) {
+        if (t->error && !t->scene) {
             std::exception_ptr e = t->error;
-            if (t->scene) preparing_.erase(t->scene);
             tasks_.erase(it);
             std::rethrow_exception(e);
+        }
+        if (t->error) {  // the requests that waited for the scene end with it
+            preparing_.erase(t->scene);
+            if (t->restore) {
+                resident_scene_bytes_ -= resident_[t->scene];
+                resident_.erase(t->scene);
+            }
+            for (auto w = waiting_.begin(); w != waiting_.end();) {
+                if ((*w)->scene == t->scene) {
+                    (*w)->error = t->error;
+                    complete(*w, now());
+                    w = waiting_.erase(w);
+                } else {
+                    ++w;
+                }
+            }
+            it = tasks_.erase(it);
+            continue;
         }
         freeing_bytes_ -= t->dead_bytes;
         if (t->scene) {
@@ -321,7 +339,17 @@ bool Server::enqueue_one() {
     return true;
 }
 
-void Server::retire(bool block, std::vector<uint64_t>* done) {
+void Server::complete(Job* j, double time) {
+    j->done = true;
+    j->finish = time;
+    --scene_users_[j->scene];
+    last_use_[j->scene] = ++tick_;
+    --j->scene->server_jobs;
+    ++stats_.completed;
+    finished_.push_back(j->id);
+}
+
+void Server::retire(bool block) {
     while (!inflight_.empty()) {
         Inflight f = inflight_.front();
         hipError_t q = block ? hipEventSynchronize(f.ev) : hipEventQuery(f.ev);
@@ -331,16 +359,21 @@ void Server::retire(bool block, std::vector<uint64_t>* done) {
         inflight_.pop_front();
         event_pool_.push_back(f.ev);
         double t = now();
+        auto ends = [&](const Job* j) { return j->rq.last_batch >= 0 && j->rq.last_batch <= f.batch; };
+        // a failed device check of a scene spoils the film of every request on it
+        std::vector<const SceneDev*> checked;
+        for (Job* j : active_) {
+            if (!ends(j) || std::find(checked.begin(), checked.end(), j->scene) != checked.end()) continue;
+            checked.push_back(j->scene);
+            if (!scene_errors(*j->scene, stream_)) continue;
+            for (Job* k : active_)
+                if (k->scene == j->scene)
+                    k->error = std::make_exception_ptr(
+                        Error(LUX_ERR_DEVICE_CHECK, "device check failed during render"));
+        }
         for (auto it = active_.begin(); it != active_.end();) {
-            Job* j = *it;
-            if (j->rq.last_batch >= 0 && j->rq.last_batch <= f.batch) {
-                j->done = true;
-                j->finish = t;
-                --scene_users_[j->scene];
-                last_use_[j->scene] = ++tick_;
-                --j->scene->server_jobs;
-                ++stats_.completed;
-                if (done) done->push_back(j->id);
+            if (ends(*it)) {
+                complete(*it, t);
                 it = active_.erase(it);
             } else {
                 ++it;
@@ -350,27 +383,35 @@ void Server::retire(bool block, std::vector<uint64_t>* done) {
 }
 
 void Server::progress(bool block, std::vector<uint64_t>* done) {
-    retire(false, done);
+    retire(false);
     admit();  // also takes in finished scene work
     bool enqueued = false;
     while (enqueue_one()) enqueued = true;
     if (block && !enqueued && !inflight_.empty()) {
-        retire(true, done);
+        retire(true);
         admit();
         while (enqueue_one()) {
         }
     }
+    if (done) done->insert(done->end(), finished_.begin(), finished_.end());
+    finished_.clear();
 }
 
 void Server::take_result(uint64_t id, float* host_film, double* arrival, double* admitted, double* finish) {
     auto it = jobs_.find(id);
     if (it == jobs_.end() || !it->second->done) throw Error(LUX_ERR_INVALID_ARGUMENT, "request is not complete");
     Job* j = it->second.get();
-    if (host_film)
-        hip_check(hipMemcpy(host_film, j->film, j->film_bytes, hipMemcpyDeviceToHost), "D2H film");
     if (arrival) *arrival = j->arrival;
     if (admitted) *admitted = j->admitted;
     if (finish) *finish = j->finish;
+    if (j->error) {
+        const std::exception_ptr e = j->error;
+        film_free(j->film, j->film_bytes);
+        jobs_.erase(it);
+        std::rethrow_exception(e);
+    }
+    if (host_film)
+        hip_check(hipMemcpy(host_film, j->film, j->film_bytes, hipMemcpyDeviceToHost), "D2H film");
     film_free(j->film, j->film_bytes);
     jobs_.erase(it);
 }
@@ -384,6 +425,18 @@ void run_trace(Server& sv, int n, SceneDev* const* scenes, const lux_render_sett
     std::vector<uint64_t> done;
     const double t0 = sv.now();
     int next = 0, completed = 0;
+    std::exception_ptr failed;  // a request's error: thrown once every request has ended
+    auto take = [&](uint64_t id) {
+        const int i = index_of.at(id);
+        double a = 0, ad = 0, f = 0;
+        try {
+            sv.take_result(id, films ? films[i] : nullptr, &a, &ad, &f);
+        } catch (...) {
+            if (!failed) failed = std::current_exception();
+        }
+        latency[i] = f - a;
+        ++completed;
+    };
     while (completed < n) {
         const double t = sv.now() - t0;
         while (next < n && arrival[next] <= t) {
@@ -393,13 +446,7 @@ void run_trace(Server& sv, int n, SceneDev* const* scenes, const lux_render_sett
         }
         done.clear();
         sv.progress(sv.has_inflight(), &done);
-        for (uint64_t id : done) {
-            const int i = index_of.at(id);
-            double a = 0, ad = 0, f = 0;
-            sv.take_result(id, films ? films[i] : nullptr, &a, &ad, &f);
-            latency[i] = f - a;
-            ++completed;
-        }
+        for (uint64_t id : done) take(id);
         if (!sv.has_inflight() && completed < n) {
             if (next < n) {
                 const double wait = arrival[next] - (sv.now() - t0);
@@ -412,17 +459,12 @@ void run_trace(Server& sv, int n, SceneDev* const* scenes, const lux_render_sett
                 sv.progress(false, &again);
                 if (!sv.has_inflight() && again.empty())
                     throw Error(LUX_ERR_OUT_OF_MEMORY, "a request does not fit the HBM budget on its own");
-                for (uint64_t id : again) {
-                    const int i = index_of.at(id);
-                    double a = 0, ad = 0, f = 0;
-                    sv.take_result(id, films ? films[i] : nullptr, &a, &ad, &f);
-                    latency[i] = f - a;
-                    ++completed;
-                }
+                for (uint64_t id : again) take(id);
             }
         }
     }
     if (wall) *wall = sv.now() - t0;
+    if (failed) std::rethrow_exception(failed);
 }
 
 }  // namespace pt

@@ -77,7 +77,9 @@ public:
     // Uploads, refits or frees still running on the worker.
     bool preparing() const { return !tasks_.empty(); }
 
-    // Completed request: film sums to `host_film` (nullable), times, film freed.
+    // Completed request: film sums to `host_film` (nullable), times, film freed. Throws
+    // the error of a request whose scene could not be prepared or whose scene's
+    // device checks failed while it rendered (the request is freed all the same).
     void take_result(uint64_t id, float* host_film, double* arrival, double* admitted, double* finish);
 
     ServeStats stats() const { return stats_; }
@@ -95,6 +97,7 @@ private:
         size_t film_bytes = 0;
         double arrival = 0, admitted = 0, finish = 0;
         bool done = false;
+        std::exception_ptr error;  // why its film is not to be used
     };
 
     // Work of the worker thread: a scene made resident (restore) and/or refit
@@ -112,7 +115,8 @@ private:
         double seconds = 0;
     };
 
-    void retire(bool block, std::vector<uint64_t>* done);
+    void retire(bool block);
+    void complete(Job* j, double time);
     void admit();
     void activate(Job* j);
     void finish_tasks();
@@ -155,6 +159,7 @@ private:
         int64_t batch;
         hipEvent_t ev;
     };
+    std::vector<uint64_t> finished_;  // completed, not yet reported
     std::deque<Inflight> inflight_;
     std::vector<hipEvent_t> event_pool_;
     ServeStats stats_;
@@ -163,7 +168,8 @@ private:
 // Replays an arrival trace in real time (arrival[i] seconds after the start,
 // sorted): request i renders settings[i] of scenes[i], after moving its
 // vertices to vertices[i] when that is non-null. Films (nullable) receive the
-// film sums, latency[i] = completion - arrival in seconds, wall = total time.
+// film sums, latency[i] = completion - arrival in seconds, wall = total time. A
+// failed request's error is thrown once every request has ended.
 void run_trace(Server& sv, int n, SceneDev* const* scenes, const lux_render_settings* settings, const double* arrival,
                const lux_vec3* const* vertices, const int* vertex_counts, float* const* films, double* latency,
                double* wall);

@@ -232,7 +232,7 @@ void build_tlas_wide(TwoLevelDev& s, const lux_instance* instances, std::vector<
     hip_check(hipMemcpyAsync(cull.p, nodes.data(), sizeof(lux_bvh_node) * count, hipMemcpyHostToDevice, stream),
               "H2D culling TLAS");
     wide_from(s.tlas, cull.p, s.tlas_wide, leaf_pos.p, stream);
-    hip_check(hipStreamSynchronize(stream), "synchronize TLAS records");
+    sync_and_check(s.tlas, stream, "TLAS records");
 }
 
 // TLAS over the non-empty world bounds (ids = instance ids) and the instance

@@ -137,5 +137,82 @@ def clears(stub):
             "evictions": st["evictions"], "uploads": st["uploads"], "completed": st["completed"]}
 
 
+class ErrorBits:
+    """Sets a device error bit of one tree as a launch's effect."""
+
+    def __init__(self, stub):
+        self.infos, self.build, self.render = [], None, None
+        stub.hooks.append(("k_copies", self.built))
+        stub.hooks.append(("k_flush", self.flushed))
+
+    def built(self, args):
+        info = ptr(args, 12)
+        self.infos.append(info)
+        if self.build == len(self.infos):
+            words(info + 32, 1)[0] = 2
+
+    def flushed(self, args):
+        if self.render is not None:
+            words(self.infos[self.render] + 32, 1)[0] = 2
+            self.render = None
+
+
+def status_of(fn):
+    from lux_amd.abi import LuxError
+
+    try:
+        fn()
+    except LuxError as e:
+        return e.status
+    return 0
+
+
+def errors(stub):
+    """Failed device checks of a build or a render reach the caller, and the server
+    goes on."""
+    from lux_amd import lbvh
+
+    bits = ErrorBits(stub)
+    render = small_engine()
+    out = {}
+    bits.build = 1
+    out["create"] = status_of(lambda: render.Scene(sphere(0)))
+    a = render.Scene(sphere(0))
+    bits.build = len(bits.infos) + 1
+    out["update"] = status_of(lambda: a.update_vertices(sphere(0)["vertices"]))
+    out["update_again"] = status_of(lambda: a.update_vertices(sphere(0)["vertices"]))
+    base = stub.lib.stub_live_bytes()
+    cold = render.Scene(sphere(1), deferred=True)
+    bits.build = len(bits.infos) + 1
+    out["first_use"] = status_of(lambda: cold.render(16, 16, 1, 1))
+    out["kept"] = stub.lib.stub_live_bytes() - base  # nothing of the failed build
+    sv = render.Server(slice_spp=8)
+
+    def run(scs):
+        return sv.run(scs, [job(i) for i in range(len(scs))], [0.0] * len(scs), want_films=False)
+
+    bits.build = len(bits.infos) + 1
+    out["served_upload"] = status_of(lambda: run([a, cold, a]))
+    out["served_again"] = status_of(lambda: run([a, cold, a]))
+    bits.render = bits.infos.index(bits.infos[-1])  # the scene just uploaded
+    out["served_render"] = status_of(lambda: run([a, cold, a]))
+    out["served_after"] = status_of(lambda: run([a, cold, a]))
+    # by polling: every request is reported, the failed one's result is the error
+    other = render.Scene(sphere(2), deferred=True)
+    bits.build = len(bits.infos) + 1
+    ids = [sv.submit(a, job(1)), sv.submit(other, job(2))]
+    done = []
+    for _ in range(100000):
+        done += sv.poll(block=True)
+        if len(done) == 2:
+            break
+    out["polled"] = [status_of(lambda i=i: sv.result(i)) for i in ids]
+    st = sv.stats()
+    out["open"] = st["submitted"] - st["completed"]
+    out["destroy"] = status_of(lambda: render.call("lux_hip_scene_destroy", other.handle))
+    other.handle = None
+    return out
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

@@ -41,3 +41,18 @@ def test_new_trees_start_from_cleared_state_on_their_own_stream(stub):
     assert r["completed"] == 11 and r["evictions"] >= 2 and r["uploads"] >= 6 and r["passes"] > 20
     assert r["bad"] == []
     assert r["null_writes"] == 0
+
+
+def test_failed_device_checks_reach_the_caller(stub):
+    """The error bits of a build or a walk are read after a scene's upload and when
+    the server retires a batch: the call (or the request) fails, and the next one
+    does not."""
+    from lux_amd import abi
+
+    r = scene(stub, "errors")
+    fails = abi.LUX_ERR_DEVICE_CHECK
+    for name in ("create", "update", "first_use", "served_upload", "served_render"):
+        assert r[name] == fails, name
+    for name in ("update_again", "kept", "served_again", "served_after", "open", "destroy"):
+        assert r[name] == 0, name
+    assert r["polled"] == [0, fails]
