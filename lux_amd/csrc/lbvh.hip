@@ -990,18 +990,6 @@ int sort_tiles(int n) { return max(1, div_up(n, kSortTile)); }
 
 }  // namespace
 
-void bvh_release(BvhDev& d) {
-    void* ptrs[] = {d.boxes,     d.ids,         d.keys[0],      d.keys[1],    d.vals[0],    d.vals[1],
-                    d.left,      d.right,       d.parent,       d.first,      d.last,       d.leaf_parent,
-                    d.edge_boxes, d.block_boxes, d.pre_internal, d.pre_leaf, d.nodes,       d.hist,
-                    d.status,    d.tickets,     d.partials,     d.info,       d.counter,
-                    d.rtop_int,  d.rtop_leaf,   d.pairs,        d.pair_pos,   d.slot_pre, d.wide, d.wide_leaf};
-    for (void* p : ptrs)
-        if (p) (void)hipFree(p);
-    BvhDev empty;
-    d = empty;
-}
-
 // ---------------------------------------------------------------------------
 // sibling-pair traversal copy of the node array
 // ---------------------------------------------------------------------------
@@ -1182,6 +1170,59 @@ const uint32_t* ray_order(RaySortDev& r, const BvhDev& tree, const lux_ray* rays
     return ray_order_into(b, first, tree, rays, n, s);
 }
 
+namespace {
+// Every buffer of a tree for cap primitives, with its element count.
+template <typename F>
+void bvh_buffers(BvhDev& d, int cap, F&& f) {
+    const size_t c = size_t(cap);
+    f(d.boxes, c);
+    f(d.ids, c);
+    for (int b = 0; b < 2; ++b) {
+        f(d.keys[b], c);
+        f(d.vals[b], c);
+    }
+    f(d.left, c);
+    f(d.right, c);
+    f(d.parent, c);
+    f(d.first, c);
+    f(d.last, c);
+    f(d.leaf_parent, c);
+    f(d.edge_boxes, 2 * c);
+    f(d.block_boxes, size_t(div_up(cap, kLocalLeaves)));
+    f(d.pre_internal, c);
+    f(d.pre_leaf, c);
+    f(d.nodes, 2 * c);
+    f(d.rtop_int, c);
+    f(d.rtop_leaf, c);
+    f(d.hist, size_t(kPasses * kRadix));
+    f(d.status, size_t(sort_tiles(cap)) * kRadix);
+    f(d.tickets, size_t(4));
+    f(d.partials, sizeof(BoxIds) * kReduceBlocksMax);
+    f(d.info, size_t(1));
+    f(d.counter, size_t(4));
+    f(d.pairs, 2 * c);
+    f(d.pair_pos, 2 * c);
+    f(d.slot_pre, 2 * c);
+    f(d.wide, c);
+    f(d.wide_leaf, 4 * c);
+}
+}  // namespace
+
+size_t bvh_device_bytes(int n) {
+    BvhDev d;
+    size_t bytes = 0;
+    bvh_buffers(d, max(n, 1), [&](auto*& p, size_t count) { bytes += sizeof(*p) * count; });
+    return bytes;
+}
+
+void bvh_release(BvhDev& d) {
+    bvh_buffers(d, d.capacity, [](auto*& p, size_t) {
+        if (p) (void)hipFree(p);
+    });
+    BvhDev empty;
+    d = empty;
+}
+
 void bvh_allocate(BvhDev& d, int n, hipStream_t s) {
     if (n <= d.capacity && d.info) {
         d.n = n;
@@ -1191,37 +1232,8 @@ void bvh_allocate(BvhDev& d, int n, hipStream_t s) {
     int cap = max(n, 1);
     d.capacity = cap;
     d.n = n;
-    d.boxes = dalloc<lux_aabb>(cap);
-    d.ids = dalloc<int32_t>(cap);
-    for (int b = 0; b < 2; ++b) {
-        d.keys[b] = dalloc<uint32_t>(cap);
-        d.vals[b] = dalloc<uint32_t>(cap);
-    }
-    d.left = dalloc<uint32_t>(cap);
-    d.right = dalloc<uint32_t>(cap);
-    d.parent = dalloc<uint32_t>(cap);
-    d.first = dalloc<uint32_t>(cap);
-    d.last = dalloc<uint32_t>(cap);
-    d.leaf_parent = dalloc<uint32_t>(cap);
-    d.edge_boxes = dalloc<lux_aabb>(2 * size_t(cap));
-    d.block_boxes = dalloc<lux_aabb>(div_up(cap, kLocalLeaves));
-    d.pre_internal = dalloc<int32_t>(cap);
-    d.pre_leaf = dalloc<int32_t>(cap);
-    d.nodes = dalloc<lux_bvh_node>(2 * size_t(cap));
-    d.rtop_int = dalloc<uint32_t>(cap);
-    d.rtop_leaf = dalloc<uint32_t>(cap);
-    d.hist = dalloc<uint32_t>(kPasses * kRadix);
     d.status_words = sort_tiles(cap) * kRadix;
-    d.status = dalloc<uint64_t>(d.status_words);
-    d.tickets = dalloc<uint32_t>(4);
-    d.partials = dalloc<uint8_t>(sizeof(BoxIds) * kReduceBlocksMax);
-    d.info = dalloc<DevInfo>(1);
-    d.counter = dalloc<int32_t>(4);
-    d.pairs = dalloc<lux_bvh_node>(2 * size_t(cap));
-    d.pair_pos = dalloc<uint32_t>(2 * size_t(cap));
-    d.slot_pre = dalloc<uint32_t>(2 * size_t(cap));
-    d.wide = dalloc<WideNode>(cap);
-    d.wide_leaf = dalloc<int32_t>(4 * size_t(cap));
+    bvh_buffers(d, cap, [](auto*& p, size_t count) { p = dalloc<std::remove_reference_t<decltype(*p)>>(count); });
     LUX_LAUNCH("lbvh_clear", k_clear_tree, max(1, min(512, div_up(d.status_words, kBlock))), kBlock, 0, s, d.status,
                d.status_words, d.tickets, d.counter, d.info);
     d.epoch = 0;

@@ -115,6 +115,8 @@ struct BvhDev {
 // Buffers for n primitives; new ones are cleared on `s`, the stream of the build.
 void bvh_allocate(BvhDev& d, int n, hipStream_t s);
 void bvh_release(BvhDev& d);
+// HBM that a tree over n primitives holds.
+size_t bvh_device_bytes(int n);
 
 // Scratch of the ray-order sort of the traversal entry points (grown on
 // demand; one per tree handle, used on one stream at a time).

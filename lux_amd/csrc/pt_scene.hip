@@ -535,14 +535,6 @@ void prepare_scene_lights(SceneDev& s, const lux_light* lights, int count, hipSt
                   "H2D environment weights");
     }
 }
-
-size_t bvh_bytes(int n) {
-    // boxes, ids, 2x keys/vals, 5 tree links, leaf parents, 2 edge boxes, 2
-    // layout maps, 2 node records, 2 climb words, 2 sibling-pair records with
-    // their two slot maps; block boxes and sort state
-    return size_t(std::max(n, 1)) * (24 + 4 + 16 + 20 + 4 + 48 + 8 + 64 + 8 + 64 + 16) +
-           (size_t(n) / 1024 + 1) * 24 + (size_t(n) / 2048 + 1) * 2048;
-}
 }  // namespace
 
 namespace {
@@ -565,10 +557,13 @@ void check_desc(const lux_scene_desc& desc) {
 }
 
 // HBM of a one-mesh scene: triangle soup, indices, material ids, light of each
-// triangle, vertices (and normals), materials, light records, BVH.
-size_t scene_bytes(int nt, int nv, bool normals, int nm, size_t lights) {
+// triangle, vertices (and normals), materials, light records with their tree and
+// lists, environment texels with their weights, BVH.
+size_t scene_bytes(int nt, int nv, bool normals, int nm, size_t lights, size_t texels) {
+    const size_t nl = std::max<size_t>(lights, 1);
     return size_t(nt) * (36 + 12 + 4 + 4) + size_t(nv) * (12 + (normals ? 12 : 0)) + sizeof(DevMaterial) * nm +
-           sizeof(DevLight) * std::max<size_t>(lights, 1) + bvh_bytes(nt);
+           nl * (sizeof(DevLight) + 2 * sizeof(DevLightNode) + sizeof(DevAlias) + 2 * sizeof(int32_t)) +
+           16 * std::max<size_t>(texels, 1) + bvh_device_bytes(nt);
 }
 }  // namespace
 
@@ -639,7 +634,8 @@ void scene_upload(SceneDev& s, const lux_scene_desc& desc, hipStream_t stream) {
                s.indices, nt, nv, s.soup, s.bvh.info);
     hip_check(hipStreamSynchronize(stream), "scene upload");
     if (scene_errors(s, stream)) throw Error(LUX_ERR_DEVICE_CHECK, "device check failed during scene upload");
-    s.device_bytes = scene_bytes(nt, nv, desc.normals != nullptr, nm, s.host_lights.size());
+    s.device_bytes = scene_bytes(nt, nv, desc.normals != nullptr, nm, s.host_lights.size(),
+                                 s.host_env_cdf.size());
     s.resident = true;
 }
 
@@ -675,8 +671,10 @@ void scene_create(SceneDev& s, const lux_scene_desc& desc, bool upload, hipStrea
             const lux_material& m = desc.materials[desc.material_ids[t]];
             emitters += fmaxf(m.emission.x, fmaxf(m.emission.y, m.emission.z)) > 0 ? 1 : 0;
         }
+        size_t texels = 0;
+        for (const auto& t : src->texels) texels += t.size();
         s.device_bytes = scene_bytes(int(nt), int(nv), desc.normals != nullptr, desc.material_count,
-                                     emitters + size_t(desc.light_count));
+                                     emitters + size_t(desc.light_count), texels);
         s.resident = false;
     }
     s.source = std::move(src);

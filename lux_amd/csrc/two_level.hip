@@ -293,13 +293,6 @@ void upload_instances(TwoLevelDev& s, const lux_instance* instances, int count, 
     }
 }
 
-size_t bvh_device_bytes(const BvhDev& d) {
-    const size_t cap = size_t(d.capacity);
-    // boxes, ids, keys/vals, tree links, slots, preorder maps, nodes, pairs
-    // and their two slot maps, records and their leaf positions
-    return cap * (24 + 4 + 16 + 28 + 48 + 8 + 64 + 64 + 16 + 64 + 16);
-}
-
 }  // namespace
 
 bool instance_transform_valid(const float* m16, const float* inv16) {
@@ -397,7 +390,7 @@ void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* of
         meshes[m].tris = s.soup + offsets[m];
         meshes[m].node_count = n > 0 ? 2 * n - 1 : 0;
         meshes[m].tri_count = n;
-        s.device_bytes += bvh_device_bytes(s.blas[m]);
+        s.device_bytes += bvh_device_bytes(n);
     }
     // each mesh's bounding sphere: the center of its box, the largest vertex
     // distance from it (in double, padded), radius -1 for an empty mesh
@@ -433,8 +426,7 @@ void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* of
                   "H2D meshes");
     upload_instances(s, instances, instance_count, stream);
     s.device_bytes += sizeof(lux_triangle) * size_t(total) + sizeof(DevMesh) * meshes.size() +
-                      sizeof(DevInstance) * size_t(instance_count) + bvh_device_bytes(s.tlas) +
-                      sizeof(lux_bvh_node) * 2 * size_t(std::max(instance_count, 1));
+                      sizeof(DevInstance) * size_t(instance_count) + bvh_device_bytes(s.tlas_instances) + sizeof(WideNode) * size_t(std::max(s.tlas_instances - 1, 0));
 }
 
 void two_level_set_instances(TwoLevelDev& s, const lux_instance* instances, int instance_count,

@@ -214,5 +214,25 @@ def errors(stub):
     return out
 
 
+def bytes_held(stub):
+    """Device memory a scene reports (resident, and deferred before it is built)
+    against what it allocates."""
+    render = small_engine()
+    dicts = [sphere(k, freq) for k, freq in ((0, 2), (1, 8), (2, 24))]
+    lit = dict(dicts[1])
+    lit["lights"] = [{"kind": "image_infinite", "color": (1, 1, 1), "image": np.ones((16, 32, 3), np.float32)},
+                     {"kind": "point", "vector": (0, 2, 0), "color": (1, 1, 1)}]
+    out = []
+    for d in dicts + [lit]:
+        before = stub.lib.stub_live_bytes()
+        sc = render.Scene(d)
+        deferred = render.Scene(d, deferred=True)
+        out.append([sc.info()[2], deferred.info()[2], stub.lib.stub_live_bytes() - before, len(d["indices"])])
+        deferred.close()
+        sc.close()
+        assert stub.lib.stub_live_bytes() == before
+    return {"scenes": out}
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

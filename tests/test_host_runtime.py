@@ -56,3 +56,11 @@ def test_failed_device_checks_reach_the_caller(stub):
     for name in ("update_again", "kept", "served_again", "served_after", "open", "destroy"):
         assert r[name] == 0, name
     assert r["polled"] == [0, fails]
+
+
+def test_scenes_report_the_memory_they_hold(stub):
+    """A scene's device bytes, which the server's budget counts, are those of its
+    allocations (the light tables are counted at their largest: 1 KiB here)."""
+    for resident, deferred, held, tris in scene(stub, "bytes_held")["scenes"]:
+        assert held <= resident <= held + 1024, tris
+        assert resident <= deferred <= resident + 1024, tris
