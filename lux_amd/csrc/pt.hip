@@ -358,12 +358,12 @@ __device__ __forceinline__ void shadow_ray(const BatchDesc* __restrict__ desc, c
     shadow_arrives(ps, i, path, tr);
 }
 
-// Extension ray i (i < n_ext) or shadow record i - n_ext, on `group` lanes (an
-// instanced scene's on one): one walk in the code for both, so a wave may hold both.
+// Extension ray i (i < n_ext) or shadow record i - n_ext, on `group` lanes: one
+// walk in the code for both, so a wave may hold both.
 template <bool kAnyShadow, bool kTwoLevel>
 __device__ __forceinline__ void record_ray(const BatchDesc* __restrict__ desc, const Paths& ps, uint32_t i,
-                                         uint32_t n_ext, const uint32_t* __restrict__ queue, int group, int part,
-                                         uint32_t* stack, int stride) {
+                                           uint32_t n_ext, const uint32_t* __restrict__ queue, int group, int part,
+                                           uint32_t* stack, int stride) {
     const bool ext = i < n_ext;
     const uint32_t j = i - n_ext;
     const uint32_t path = ext ? queue[i] : __float_as_uint(ps.sc[j].w);
@@ -392,7 +392,14 @@ __device__ __forceinline__ void record_ray(const BatchDesc* __restrict__ desc, c
             break;
         }
         if (h.prim < 0 || !shadow_passes(sv, h.prim, h.t, tr, o, d, t_max)) break;
-        if (kTwoLevel && part == 0) ps.so[j] = make_float4(o.x, o.y, o.z, t_max);
+        if (kTwoLevel) {
+            // the other lanes of the group read the new origin in world(): in order
+            // for one wave's memory operations, which the compiler has to be told
+            if (part == 0) ps.so[j] = make_float4(o.x, o.y, o.z, t_max);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
         ignore = -1;
     }
     if (part != 0) return;

@@ -100,6 +100,41 @@ def test_instanced_per_sample_radiance(rd, case):
     sc.close()
 
 
+def sheets_room(layers):
+    """The instanced room with a stack of tinted sheets under its ceiling light: a
+    shadow ray passes `layers` boxes, two faces each."""
+    from lux_amd import scenes
+    from lux_amd.workloads import affine
+
+    d = dict(scenes.instanced_room(64, 64))
+    m = [affine(None, (1.2, 0.01, 1.2), (0.0, 1.6 - 0.12 * k, 1.0)) for k in range(layers)]
+    d["inst_mesh"] = np.concatenate([d["inst_mesh"], np.full(layers, 2, np.int32)])
+    d["inst_m"] = np.concatenate([d["inst_m"], np.stack(m).astype(np.float32)])
+    d["inst_override"] = np.concatenate([d["inst_override"], np.full(layers, 8, np.int32)])
+    return d
+
+
+@pytest.mark.parametrize("layers", [1, 5])
+def test_shadow_rays_through_sheets_do_not_depend_on_lanes_per_ray(rd, layers):
+    """A shadow ray that goes on behind a pass-through hit starts at the same place
+    for every lane that walks it: batches of few rays (16 lanes a ray) and of more
+    than 2^17 (one lane) give the same film."""
+    print("case: shadow rays through sheets", layers, flush=True)
+    sc = rd.Scene(sheets_room(layers))
+    saved = rd.get_tuning()
+    films = []
+    try:
+        for capacity in (1 << 21, 1 << 16, 6000):
+            rd.set_tuning(capacity=capacity)
+            films.append(sc.render(64, 64, 512, 3, seed=5))
+    finally:
+        rd.set_tuning(**saved)
+    assert films[0].max() > 0
+    assert np.array_equal(bits(films[0]), bits(films[1]))
+    assert np.array_equal(bits(films[0]), bits(films[2]))
+    sc.close()
+
+
 def one_instance(d):
     """A one-mesh scene dict as an instanced scene with one identity instance."""
     n = len(d["vertices"])
