@@ -230,10 +230,11 @@ __device__ __forceinline__ WideHit mesh_query(const SceneView& sv, const f3& o, 
     WideHit h;
     h.failed = sv.preorder != 0;
     if (!h.failed)
-        h = wide_query(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, group, part, stack, stride,
-                       sv.info, visits, tests);
+        h = wide_query<true>(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, group, part, stack, stride,
+                             sv.info, visits, tests);
     if (h.failed)
-        h = preorder_query(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, sv.info, visits, tests);
+        h = preorder_query<true>(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, sv.info, visits,
+                                 tests);
     return h;
 }
 

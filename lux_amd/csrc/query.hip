@@ -101,10 +101,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
 
 // Few rays: `group` lanes (a power of two) walk one ray (wide_query).
 template <bool kAny>
-__global__ __launch_bounds__(kBlock) void k_trace_parts(RayTree tree, const lux_triangle* __restrict__ tris,
-                                                        int tri_count, const lux_ray* __restrict__ rays, int n,
-                                                        const uint32_t* __restrict__ order, int group,
-                                                        void* __restrict__ out, DevInfo* info) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAny ? 7 : 6))) void k_trace_parts(
+    RayTree tree, const lux_triangle* __restrict__ tris, int tri_count, const lux_ray* __restrict__ rays, int n,
+    const uint32_t* __restrict__ order, int group, void* __restrict__ out, DevInfo* info) {
     __shared__ uint32_t stack[kWideStack * kBlock];
     const int i = (int(xcd_block()) * kBlock + int(threadIdx.x)) / group;
     if (i >= n) return;  // whole groups

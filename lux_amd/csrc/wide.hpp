@@ -478,6 +478,8 @@ __device__ __forceinline__ bool ray_part(const lux_bvh_node* __restrict__ nodes,
 // over one lane's walk. With t_max fixed, whether a leaf's box passes does not
 // depend on the visit order, so an any-hit walk may end at any triangle hit in a
 // leaf whose own box passes; near child first meets one soon.
+// kOwnIds: see preorder_query.
+template <bool kOwnIds = false>
 __device__ __forceinline__ WideHit wide_query(const RayTree& tree, const lux_triangle* __restrict__ tris,
                                               int tri_count, const f3& o, const f3& d, float t_min, float t_bound,
                                               bool any, int ignore, int group, int part, uint32_t* stack, int stride,
@@ -498,8 +500,8 @@ __device__ __forceinline__ WideHit wide_query(const RayTree& tree, const lux_tri
     auto leaf = [&](uint32_t at, uint32_t ref) {
         const uint32_t prim = ref & kIndexMask;
         if (int(prim) == ignore) return false;
-        if (prim >= uint32_t(tri_count)) {
-            bad_prim |= ref != kWideEmpty;
+        if (prim >= uint32_t(tri_count)) {  // no child, or a leaf id out of range
+            bad_prim |= ref != kWideEmpty || (!kOwnIds && tree.wide_leaf[at] >= 0);
             return false;
         }
         const float* p = reinterpret_cast<const float*>(tris + prim);
@@ -528,8 +530,9 @@ __device__ __forceinline__ WideHit wide_query(const RayTree& tree, const lux_tri
     hit.failed = wave_any_parallel(sr)
                      ? !wide_walk<true>(tree.wide, tree.records, sr, t_cull, skip, stack, stride, visits, bad, leaf, share)
                      : !wide_walk<false>(tree.wide, tree.records, sr, t_cull, skip, stack, stride, visits, bad, leaf, share);
-    if (bad_prim) set_error(info, kErrPrimRange);
+    if (kOwnIds && bad_prim) set_error(info, kErrPrimRange);
     if (bad) set_error(info, kErrWalkOrder);
+    if (!kOwnIds) hit.failed |= bad_prim;  // the leaf's own box decides
     hit.prim = best;
     hit.t = t_max;
     if (best >= 0) hit.pos = tree.wide_leaf[best_at];
@@ -559,6 +562,11 @@ __device__ __forceinline__ WideHit wide_query(const RayTree& tree, const lux_tri
 // Right-first preorder walk: the rays that wide_query hands back, one-leaf trees
 // and trees beyond 32-bit record offsets. any: stop at the first accepted
 // triangle. visits counts node loads, tests triangle tests.
+// A leaf id at or above tri_count is an error for a ray that meets the leaf's box no
+// farther than its hit (an any-hit query: that finds none), in whatever order: a walk
+// that passed such a leaf is made again up to the hit (kOwnIds: ids the library gave
+// itself, an error at once).
+template <bool kOwnIds = false>
 __device__ __forceinline__ WideHit preorder_query(const RayTree& tree, const lux_triangle* __restrict__ tris,
                                                   int tri_count, const f3& o, const f3& d, float t_min,
                                                   float t_bound, bool any, int ignore, DevInfo* info,
@@ -566,35 +574,42 @@ __device__ __forceinline__ WideHit preorder_query(const RayTree& tree, const lux
     const SlabRay sr = make_slab_ray(o, d, t_min);
     WideHit hit;
     hit.t = t_bound;
-    int k = 0;
-    bool bad_prim = false, bad_order = false;
-    while (uint32_t(k) < uint32_t(tree.node_count)) {
-        float4 a, b;
-        load_node(tree.nodes, k, a, b);
-        ++visits;
-        const int prim = __float_as_int(b.z);
-        const bool pass = slab_hit(sr, hit.t, a.x, a.y, a.z, a.w, b.x, b.y);
-        int next = (pass && prim < 0) ? k + 1 : __float_as_int(b.w);
-        const bool test = pass && prim >= 0 && prim != ignore;
-        bad_prim |= test && prim >= tri_count;
-        if (test && prim < tri_count) {
-            const float* p = reinterpret_cast<const float*>(tris + prim);
-            ++tests;
-            float t, u, v;
-            if (tri_hit(o, d, t_min, hit.t, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]),
-                        make3(p[6], p[7], p[8]), t, u, v)) {
-                hit.prim = prim;
-                hit.t = t;
-                if (any) next = -1;  // done
+    bool bad_order = false;
+    for (bool again = false;; again = true) {
+        int k = 0;
+        bool bad_prim = false;
+        while (uint32_t(k) < uint32_t(tree.node_count)) {
+            float4 a, b;
+            load_node(tree.nodes, k, a, b);
+            ++visits;
+            const int prim = __float_as_int(b.z);
+            const bool pass = slab_hit(sr, hit.t, a.x, a.y, a.z, a.w, b.x, b.y);
+            int next = (pass && prim < 0) ? k + 1 : __float_as_int(b.w);
+            const bool test = pass && prim >= 0 && prim != ignore;
+            bad_prim |= test && prim >= tri_count;
+            if (test && prim < tri_count) {
+                const float* p = reinterpret_cast<const float*>(tris + prim);
+                ++tests;
+                float t, u, v;
+                if (tri_hit(o, d, t_min, hit.t, make3(p[0], p[1], p[2]), make3(p[3], p[4], p[5]),
+                            make3(p[6], p[7], p[8]), t, u, v)) {
+                    hit.prim = prim;
+                    hit.t = t;
+                    if (any) next = -1;  // done
+                }
             }
+            if (next >= 0 && next <= k) {  // preorder positions only grow
+                bad_order = true;
+                break;
+            }
+            k = next;
         }
-        if (next >= 0 && next <= k) {  // preorder positions only grow
-            bad_order = true;
+        if (!bad_prim || (any && hit.prim >= 0 && !kOwnIds)) break;
+        if (kOwnIds || again || hit.prim < 0) {
+            set_error(info, kErrPrimRange);
             break;
         }
-        k = next;
     }
-    if (bad_prim) set_error(info, kErrPrimRange);
     if (bad_order) set_error(info, kErrWalkOrder);
     return hit;
 }

@@ -111,6 +111,47 @@ def test_random_soup_and_axis_parallel_rays(model):
     check(model, W.triangle_boxes(tris), None, tris, rays)
 
 
+def meets(box, ray, t_max):
+    """The reference's slab test, in its own float operations."""
+    o, d = ray[0:3], ray[3:6]
+    near, far = np.float32(ray[6]), np.float32(t_max)
+    for a in range(3):
+        inv = np.float32(1) / d[a]
+        lo, hi = (box[3 + a], box[a]) if inv < 0 else (box[a], box[3 + a])
+        near, far = max(near, (lo - o[a]) * inv), min(far, (hi - o[a]) * inv)
+    return not near > far
+
+
+@pytest.mark.parametrize("bad_id", [2000, 0x7FFFFFFF])
+def test_leaf_ids_out_of_range_are_reported_where_the_leaf_box_is_met(model, bad_id):
+    """An id at or above the triangle count is an error for exactly the rays that
+    meet its leaf's own box no farther than their hit (any hit: that find none), not
+    for those that only meet the wider byte box."""
+    g = load_golden("lbvh_soup2000")
+    tris = g["tri_by_id"]
+    boxes, ids = g["boxes"].copy(), g["ids"].astype(np.int32).copy()
+    k = int(np.argmax(np.prod(boxes[:, 3:] - boxes[:, :3], axis=1)))
+    boxes[k] = [0.3, 0.3, 0.3, 0.7, 0.7, 0.7]  # a large leaf that many rays meet
+    rest = tris.copy()
+    rest[ids[k]] = 0  # what the oracle walks: never hit there
+    want = oracle.OracleBvh(boxes, ids).trace_closest(rest, g["rays"][:400])
+    ids[k] = bad_id
+    m = model(oracle.OracleBvh(boxes, ids))
+    seen = {True: 0, False: 0}
+    for i in range(400):
+        ray = g["rays"][i : i + 1]
+        hit = want["ids"][i] >= 0
+        met = meets(boxes[k], ray[0], want["t"][i] if hit else ray[0][7])
+        for group in (1, 16):
+            got, t, _, error = m.trace(tris, ray, group=group)
+            assert error == (PRIM_RANGE if met else 0), (i, group)
+            assert got[0] == want["ids"][i]
+            occ, _, _, error = m.trace(tris, ray, any_hit=True, group=group)
+            assert (occ[0] >= 0) == hit and error == (PRIM_RANGE if met and not hit else 0), (i, group)
+        seen[met] += 1
+    assert min(seen.values()) > 10
+
+
 def damaged(kind):
     """Run in a process of its own: prints the error bits."""
     g = load_golden("lbvh_soup2000")
