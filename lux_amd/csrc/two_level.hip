@@ -260,13 +260,14 @@ void upload_instances(TwoLevelDev& s, const lux_instance* instances, int count, 
         boxes.push_back(in.world_bounds);
         ids.push_back(i);
     }
-    s.host_instances.assign(instances, instances + count);
-    s.instance_count = count;
-    s.scene_primitives = cursor;
-    s.tlas_instances = int(boxes.size());
     const int n = int(boxes.size());
     TempBuffer<lux_aabb> d_boxes(size_t(std::max(n, 1)));
     TempBuffer<int32_t> d_ids(size_t(std::max(n, 1)));
+    s.whole = false;
+    s.host_instances.assign(instances, instances + count);
+    s.instance_count = count;
+    s.scene_primitives = cursor;
+    s.tlas_instances = n;
     if (n > 0) {
         hip_check(hipMemcpyAsync(d_boxes.p, boxes.data(), sizeof(lux_aabb) * n, hipMemcpyHostToDevice, stream),
                   "H2D world bounds");
@@ -291,6 +292,7 @@ void upload_instances(TwoLevelDev& s, const lux_instance* instances, int count, 
                   "H2D instances");
         hip_check(hipStreamSynchronize(stream), "synchronize instances");
     }
+    s.whole = true;
 }
 
 }  // namespace
@@ -438,6 +440,7 @@ void two_level_set_instances(TwoLevelDev& s, const lux_instance* instances, int 
 }
 
 TwoLevelView two_level_view(const TwoLevelDev& s) {
+    if (!s.whole) throw Error(LUX_ERR_INVALID_ARGUMENT, "instances were lost in a failed update: set them again");
     TwoLevelView v;
     v.tlas_nodes = s.tlas.nodes;
     v.tlas_wide = s.tlas_wide;

@@ -461,6 +461,7 @@ struct TwoLevelDev {
     int64_t scene_primitives = 0;
     uint32_t step_limit = 0;
     size_t device_bytes = 0;
+    bool whole = false;  // the instances, the TLAS and its records belong together
 };
 
 // Scene validation of one instance transform pair (src/scene/scene_validate.h:140-147,
@@ -475,7 +476,8 @@ lux_aabb transform_bounds(const float* m16, const lux_aabb& b);
 void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* mesh_offsets, int mesh_count,
                      const lux_instance* instances, int instance_count, hipStream_t stream);
 // New instance transforms / world bounds for the same meshes and instance count:
-// rebuilds the TLAS and the instance records only.
+// rebuilds the TLAS and the instance records only. If that fails half way, views of the
+// scene are refused until it succeeds.
 void two_level_set_instances(TwoLevelDev& s, const lux_instance* instances, int instance_count,
                              hipStream_t stream);
 void two_level_release(TwoLevelDev& s);

@@ -38,6 +38,7 @@ std::vector<Fill> g_pending;                  // null-stream fills not yet done
 size_t g_live_bytes = 0;
 int g_null_writes = 0;                        // device writes ordered on the null stream only
 int g_next = 1;
+int g_allocs_left = -1;  // allocations until one fails (-1: none does)
 using LaunchCb = void (*)(const char* name, void* stream, void** args);
 LaunchCb g_on_launch = nullptr;
 
@@ -72,7 +73,7 @@ extern "C" {
 void stub_on_launch(LaunchCb cb) { g_on_launch = cb; }
 uint64_t stub_live_bytes() { return g_live_bytes; }
 int stub_null_writes() { return g_null_writes; }
-int stub_is_live(const void* p) { return g_live.count(p) ? 1 : 0; }
+void stub_fail_alloc_after(int count) { g_allocs_left = count; }
 
 // ---- kernels ----
 void** __hipRegisterFatBinary(const void*) {
@@ -110,6 +111,8 @@ hipError_t hipLaunchKernel(const void* fn, dim3, dim3, void** args, size_t, hipS
 // ---- memory ----
 hipError_t hipMalloc(void** p, size_t bytes) {
     std::lock_guard<std::recursive_mutex> lk(g_mu);
+    if (g_allocs_left == 0) return hipErrorOutOfMemory;
+    if (g_allocs_left > 0) --g_allocs_left;
     *p = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
     if (!*p) return hipErrorOutOfMemory;
     // old bytes: words of 1, so that a look-back word reads as epoch 1

@@ -234,5 +234,29 @@ def bytes_held(stub):
     return {"scenes": out}
 
 
+def lost_instances(stub):
+    """set_instances that runs out of memory at each of its allocations in turn:
+    queries are refused until it has succeeded."""
+    from lux_amd import lbvh, two_level, workloads as W
+
+    lbvh.init()
+    tris = W.soup(40, seed=3).reshape(-1, 9)
+    mesh = np.array([0, 1, 0], np.int32)
+    m = np.stack([W.affine(None, (1, 1, 1), (0.5 * k, 0, 0)) for k in range(3)]).astype(np.float32)
+    offsets = np.array([0, 25, 40], np.int32)
+    inst = two_level.make_instances(mesh, m, tris, offsets)
+    sc = two_level.TwoLevelScene(tris, offsets, inst)
+    rays = W.rays(10, seed=4)
+    out = []
+    for k in range(20):
+        stub.lib.stub_fail_alloc_after(k)
+        failed = status_of(lambda: sc.set_instances(inst))
+        stub.lib.stub_fail_alloc_after(-1)
+        out.append([failed, status_of(lambda: sc.intersect(rays))])
+        if not failed:
+            break
+    return {"tries": out}
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

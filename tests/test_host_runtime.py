@@ -64,3 +64,12 @@ def test_scenes_report_the_memory_they_hold(stub):
     for resident, deferred, held, tris in scene(stub, "bytes_held")["scenes"]:
         assert held <= resident <= held + 1024, tris
         assert resident <= deferred <= resident + 1024, tris
+
+
+def test_instances_lost_in_a_failed_update_are_not_queried(stub):
+    """Between a TLAS that is rebuilt and records that are not, every ray would
+    miss: such a scene refuses queries until its instances are set."""
+    tries = scene(stub, "lost_instances")["tries"]
+    assert len(tries) > 2 and tries[-1] == [0, 0]
+    assert all(failed == 6 for failed, _ in tries[:-1])
+    assert [query for _, query in tries[:-1]] == [0, 0] + [1] * (len(tries) - 3)  # two come before any change
