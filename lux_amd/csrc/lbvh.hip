@@ -19,9 +19,10 @@
 //   top_boxes      one wave per node above the frontier: its box from two of
 //                  those unions and the whole-block boxes between them; in a
 //                  build also the nodes' places in the sibling-pair copy
-//   copies         the traversal copies of the node array: four-child records
-//                  (wide.hpp) and sibling pairs
-// Refit runs only local (bounds phase) + top_boxes + copies.
+//   copies         the traversal copies of the node array, four-child records
+//                  (wide.hpp) and sibling pairs, each before the first query that
+//                  reads it (tree_copies)
+// Refit runs only local (bounds phase) + top_boxes.
 //
 // No box crosses workgroups through a counter: every hand-off between
 // workgroups is a kernel boundary, so no agent-scope release/acquire (an L2
@@ -1107,15 +1108,48 @@ void wide_from(const BvhDev& d, const lux_bvh_node* nodes, WideNode* wide, int32
                wide_leaf, (const uint32_t*)nullptr, (lux_bvh_node*)nullptr, (uint32_t*)nullptr, d.info);
 }
 
-// The traversal copies of the node array (build and refit).
-void fill_copies(BvhDev& d, hipStream_t s) {
+namespace {
+void launch_copies(const BvhDev& d, unsigned which, hipStream_t s) {
     if (d.n <= 0) return;
-    const int wide_blocks = d.n > 1 ? min(4096, div_up(d.n - 1, kBlock)) : 0;
-    const int pair_blocks = max(1, min(2048, div_up(2 * d.n - 1, kBlock)));
+    const int wide_blocks = (which & kCopyRecords) && d.n > 1 ? min(4096, div_up(d.n - 1, kBlock)) : 0;
+    const int pair_blocks = which & kCopyPairs ? max(1, min(2048, div_up(2 * d.n - 1, kBlock))) : 0;
+    if (wide_blocks + pair_blocks == 0) return;
     LUX_LAUNCH("lbvh_copies", k_copies, wide_blocks + pair_blocks, kBlock, 0, s, d.n, wide_blocks,
                (const uint32_t*)d.left, (const uint32_t*)d.right, (const int32_t*)d.pre_internal,
                (const int32_t*)d.pre_leaf, (const lux_bvh_node*)d.nodes, d.wide, d.wide_leaf,
                (const uint32_t*)d.pair_pos, d.pairs, d.slot_pre, d.info);
+}
+
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    hip_check(hipStreamIsCapturing(s, &status), "hipStreamIsCapturing");
+    return status != hipStreamCaptureStatusNone;
+}
+
+// The node array has just been enqueued (build, refit).
+void nodes_changed(BvhDev& d, hipStream_t s) {
+    if (capturing(s)) {  // at each replay, and not yet: `stale` stays as it is
+        launch_copies(d, kCopyBoth, s);
+        return;
+    }
+    d.stale = kCopyBoth & ~d.keep;
+    launch_copies(d, d.keep, s);
+}
+}  // namespace
+
+void tree_copies(BvhDev& d, unsigned need, hipStream_t s) {
+    const unsigned missing = d.stale & need;
+    if ((d.keep & need) == need && !missing) return;
+    const bool recorded = capturing(s);
+    if (recorded) d.keep |= need;
+    if (!missing) return;
+    launch_copies(d, missing, s);
+    if (!recorded) d.stale &= ~missing;
+}
+
+void keep_copies(BvhDev& d, unsigned need, hipStream_t s) {
+    d.keep |= need;
+    tree_copies(d, need, s);
 }
 
 void raysort_release(RaySortDev& r) {
@@ -1271,7 +1305,7 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
                    d.keys[0], d.vals[0], d.info, 1);
         // root box from the one leaf (the reduction result is identical)
         top_boxes<true>(d, s);
-        fill_copies(d, s);
+        nodes_changed(d, s);
         return;
     }
     int mh_blocks = max(1, min(1024, div_up(n, kBlock * 16)));
@@ -1295,7 +1329,7 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
                    d.info);
     launch_local<0>("lbvh_local", d, d.boxes, nullptr, 0, s);
     top_boxes<true>(d, s);
-    fill_copies(d, s);
+    nodes_changed(d, s);
 }
 
 namespace {
@@ -1306,12 +1340,12 @@ void refit_launch(BvhDev& d, const lux_aabb* in_boxes, const lux_triangle* tris,
     if (n == 1) {
         LUX_LAUNCH("lbvh_single_leaf", k_single_leaf, 1, 1, 0, s, in_boxes, tris, (const int32_t*)d.ids, d.boxes,
                    wb, d.nodes, d.pre_leaf, d.keys[0], d.vals[0], d.info, 0);
-        fill_copies(d, s);
+        nodes_changed(d, s);
         return;
     }
     launch_local<kMode>(kMode == 2 ? "lbvh_local_tris" : "lbvh_local_boxes", d, in_boxes, tris, wb, s);
     top_boxes<false>(d, s);
-    fill_copies(d, s);
+    nodes_changed(d, s);
 }
 }  // namespace
 

@@ -110,6 +110,9 @@ struct BvhDev {
     int32_t* counter = nullptr;
     uint32_t epoch = 0;
     int status_words = 0;
+    // TreeCopy bits: copies behind the node array, and copies that builds and
+    // refits make at once (see tree_copies)
+    unsigned stale = 0, keep = 0;
 };
 
 // Buffers for n primitives; new ones are cleared on `s`, the stream of the build.
@@ -168,6 +171,20 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
 void lbvh_build_triangles(BvhDev& d, const lux_triangle* tris, const lux_vec3* verts, const uint32_t* idx, int nv,
                           int n, hipStream_t s);
 
+// The traversal copies of the node array: four-child records (ray queries) and
+// sibling pairs (overlap queries, small path-traced scenes).
+enum TreeCopy : unsigned { kCopyRecords = 1, kCopyPairs = 2, kCopyBoth = 3 };
+// Enqueues the copies among `need` that are stale: a build or refit leaves both so,
+// and the first query that reads one makes it, so that trees that only one kind of
+// query reads do not pay for both (2^20 triangles: refit 145 us with pairs, 227 with
+// both, 110 alone). A query that is captured into a graph may be replayed after a
+// later refit: from then on builds and refits make that copy at once. A build or
+// refit that is captured makes both at each replay.
+void tree_copies(BvhDev& d, unsigned need, hipStream_t s);
+// Makes `need` now and with every later build and refit (scenes, whose views are read
+// on other streams).
+void keep_copies(BvhDev& d, unsigned need, hipStream_t s);
+
 // Enqueues the four-child records (n - 1, and 4 leaf positions each) of tree d's
 // topology over another node array of its preorder positions.
 void wide_from(const BvhDev& d, const lux_bvh_node* nodes, WideNode* wide, int32_t* wide_leaf, hipStream_t s);
@@ -211,11 +228,11 @@ void lbvh_refit_triangles(BvhDev& d, const lux_triangle* tris, hipStream_t s);
 // kOrderMinRays (r holds the sort's buffers), else null (input order).
 const uint32_t* closest_order(RaySortDev& r, bool sort, const BvhDev& d, const lux_ray* rays, int n,
                               hipStream_t s);
-void trace_closest(const BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
+void trace_closest(BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
                    const lux_ray* rays, int n, lux_hit* hits, hipStream_t s);
-void trace_any(const BvhDev& d, RaySortDev* order, const lux_triangle* tris, int tri_count, const lux_ray* rays,
+void trace_any(BvhDev& d, RaySortDev* order, const lux_triangle* tris, int tri_count, const lux_ray* rays,
                int n, uint8_t* occluded, hipStream_t s);
-void trace_stats(const BvhDev& d, const lux_triangle* tris, int tri_count, const lux_ray* rays, int n,
+void trace_stats(BvhDev& d, const lux_triangle* tris, int tri_count, const lux_ray* rays, int n,
                  unsigned long long* d_stats, hipStream_t s);
 void copy_device(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Closest hit with the ray-order scratch in a fixed per-device array
@@ -224,9 +241,9 @@ void copy_device(void* dst, const void* src, size_t bytes, hipStream_t s);
 constexpr int kNoAllocMaxRays = 1 << 22;
 void noalloc_setup(int device);
 size_t noalloc_scratch_bytes();
-void trace_closest_noalloc(int device, const BvhDev& d, bool order_rays, const lux_triangle* tris, int tri_count,
+void trace_closest_noalloc(int device, BvhDev& d, bool order_rays, const lux_triangle* tris, int tri_count,
                            const lux_ray* rays, int n, lux_hit* hits, hipStream_t s);
-void overlap_query(const BvhDev& tree, const BvhDev& queries, bool self_mode, int max_pairs,
+void overlap_query(BvhDev& tree, const BvhDev& queries, bool self_mode, int max_pairs,
                    lux_pair* pairs, int32_t* counter, hipStream_t s);
 
 }  // namespace lux

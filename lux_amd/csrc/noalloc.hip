@@ -68,7 +68,7 @@ void noalloc_setup(int device) {
     g_scratch_ptr[device] = static_cast<uint8_t*>(ptr);
 }
 
-void trace_closest_noalloc(int device, const BvhDev& d, bool order_rays, const lux_triangle* tris, int tri_count,
+void trace_closest_noalloc(int device, BvhDev& d, bool order_rays, const lux_triangle* tris, int tri_count,
                            const lux_ray* rays, int n, lux_hit* hits, hipStream_t s) {
     if (n > kNoAllocMaxRays)
         throw Error(LUX_ERR_INVALID_ARGUMENT,

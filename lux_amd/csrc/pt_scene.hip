@@ -630,6 +630,7 @@ void scene_upload(SceneDev& s, const lux_scene_desc& desc, hipStream_t stream) {
     // BLAS over the triangle boxes (ids = triangle index), both computed on the
     // device from the indexed mesh; the soup is gathered there too
     lbvh_build_triangles(s.bvh, nullptr, s.vertices, s.indices, nv, nt, stream);
+    keep_copies(s.bvh, kCopyBoth, stream);
     LUX_LAUNCH("pt_gather_soup", k_gather_soup, std::min(div_up(nt, 256), 4096), 256, 0, stream, s.vertices,
                s.indices, nt, nv, s.soup, s.bvh.info);
     hip_check(hipStreamSynchronize(stream), "scene upload");

@@ -389,8 +389,9 @@ const uint32_t* closest_order(RaySortDev& r, bool sort, const BvhDev& d, const l
 
 namespace {
 template <bool kAny>
-void launch_trace(const char* name, const BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
+void launch_trace(const char* name, BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
                   const lux_ray* rays, int n, void* out, hipStream_t s) {
+    tree_copies(d, kCopyRecords, s);
     const RayTree tree = ray_tree(d);
     const int group = tree.records ? lanes_per_ray(uint32_t(n)) : 1;
     if (group > 1)
@@ -402,22 +403,23 @@ void launch_trace(const char* name, const BvhDev& d, const uint32_t* order, cons
 }
 }  // namespace
 
-void trace_closest(const BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
+void trace_closest(BvhDev& d, const uint32_t* order, const lux_triangle* tris, int tri_count,
                    const lux_ray* rays, int n, lux_hit* hits, hipStream_t s) {
     if (n <= 0) return;
     launch_trace<false>("trace_closest", d, order, tris, tri_count, rays, n, hits, s);
 }
 
-void trace_any(const BvhDev& d, RaySortDev* order, const lux_triangle* tris, int tri_count, const lux_ray* rays,
+void trace_any(BvhDev& d, RaySortDev* order, const lux_triangle* tris, int tri_count, const lux_ray* rays,
                int n, uint8_t* occluded, hipStream_t s) {
     if (n <= 0) return;
     launch_trace<true>("trace_any", d, maybe_order(d, order, rays, n, s), tris, tri_count, rays, n, occluded, s);
 }
 
-void trace_stats(const BvhDev& d, const lux_triangle* tris, int tri_count, const lux_ray* rays, int n,
+void trace_stats(BvhDev& d, const lux_triangle* tris, int tri_count, const lux_ray* rays, int n,
                  unsigned long long* d_stats, hipStream_t s) {
     LUX_LAUNCH("trace_stats_zero", k_zero_u64, 1, 64, 0, s, d_stats, 6);
     if (n <= 0 || d.n <= 0) return;
+    tree_copies(d, kCopyRecords, s);
     LUX_LAUNCH("trace_stats", k_trace_stats, div_up(n, kBlock), kBlock, 0, s, ray_tree(d), tris, tri_count, rays, n,
                d_stats, d.info);
 }
@@ -430,10 +432,11 @@ void copy_device(void* dst, const void* src, size_t bytes, hipStream_t s) {
                count);
 }
 
-void overlap_query(const BvhDev& tree, const BvhDev& queries, bool self_mode, int max_pairs,
+void overlap_query(BvhDev& tree, const BvhDev& queries, bool self_mode, int max_pairs,
                    lux_pair* pairs, int32_t* counter, hipStream_t s) {
     LUX_LAUNCH("overlap_zero", k_zero_counter, 1, 1, 0, s, counter);
     if (tree.n <= 0 || queries.n <= 0 || max_pairs <= 0) return;
+    tree_copies(tree, kCopyPairs, s);
     const int slots = tree.n > 1 ? 2 * tree.n : 1;  // sibling-pair array
     LUX_LAUNCH(self_mode ? "overlap_self" : "overlap_cross", k_overlap, div_up(queries.n, kOvQueries), kOvThreads,
                0, s, (const lux_bvh_node*)tree.pairs, slots, (const lux_aabb*)queries.boxes,

@@ -386,6 +386,7 @@ void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* of
         // BLAS input (triangle_bounds, local ids) computed on the device from
         // the soup copied above
         lbvh_build_triangles(s.blas[m], s.soup + offsets[m], nullptr, nullptr, 0, n, stream);
+        tree_copies(s.blas[m], kCopyRecords, stream);
         sync_and_check(s.blas[m], stream, "BLAS build");
         meshes[m].nodes = s.blas[m].nodes;
         meshes[m].wide_leaf = s.blas[m].wide_leaf;

@@ -38,6 +38,7 @@ std::vector<Fill> g_pending;                  // null-stream fills not yet done
 size_t g_live_bytes = 0;
 int g_null_writes = 0;                        // device writes ordered on the null stream only
 int g_next = 1;
+bool g_capturing = false;
 int g_allocs_left = -1;  // allocations until one fails (-1: none does)
 using LaunchCb = void (*)(const char* name, void* stream, void** args);
 LaunchCb g_on_launch = nullptr;
@@ -48,6 +49,7 @@ struct Config {
     hipStream_t stream;
 };
 thread_local Config t_cfg;
+thread_local unsigned t_grid = 0, t_block = 0;  // of the launch the callback sees
 
 template <typename T>
 T handle() {
@@ -73,6 +75,9 @@ extern "C" {
 void stub_on_launch(LaunchCb cb) { g_on_launch = cb; }
 uint64_t stub_live_bytes() { return g_live_bytes; }
 int stub_null_writes() { return g_null_writes; }
+unsigned stub_grid() { return t_grid; }
+unsigned stub_block() { return t_block; }
+void stub_capturing(int on) { g_capturing = on != 0; }
 void stub_fail_alloc_after(int count) { g_allocs_left = count; }
 
 // ---- kernels ----
@@ -97,13 +102,15 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
     *stream = t_cfg.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* fn, dim3, dim3, void** args, size_t, hipStream_t stream) {
+hipError_t hipLaunchKernel(const void* fn, dim3 grid, dim3 block, void** args, size_t, hipStream_t stream) {
     std::string name;
     {
         std::lock_guard<std::recursive_mutex> lk(g_mu);
         name = g_names.count(fn) ? g_names[fn] : "?";
         if (!stream) ++g_null_writes;
     }
+    t_grid = grid.x;
+    t_block = block.x;
     if (g_on_launch) g_on_launch(name.c_str(), stream, args);
     return hipSuccess;
 }
@@ -191,6 +198,10 @@ hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
     *ms = 0;
+    return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status) {
+    *status = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }

@@ -258,5 +258,50 @@ def lost_instances(stub):
     return {"tries": out}
 
 
+def copies(stub):
+    """Which traversal copies each call makes (r: records, p: pairs)."""
+    from lux_amd import abi, lbvh, workloads as W
+
+    made = []
+
+    def see(args):
+        wide = i32(args, 1)
+        made.append(("r" if wide else "") + ("p" if stub.lib.stub_grid() > wide else ""))
+
+    stub.hooks.append(("k_copies", see))
+    n = 5000
+    tris = W.soup(n, seed=1)
+    d_tris, rays = lbvh.DeviceArray.from_numpy(tris), lbvh.DeviceArray(36 * 64)
+    out = lbvh.DeviceArray(8 * 4096)
+    bvh = lbvh.GpuBvh()
+    calls = {
+        "build": lambda: bvh.build_triangles_device(d_tris, n),
+        "refit": lambda: bvh.refit_triangles_device(d_tris, n),
+        "trace": lambda: abi.call("lux_hip_trace_closest_device", bvh.handle, d_tris.ptr, n, rays.ptr, 64, out.ptr,
+                                  None),
+        "any": lambda: abi.call("lux_hip_trace_any_device", bvh.handle, d_tris.ptr, n, rays.ptr, 64, out.ptr, None),
+        "overlap": lambda: abi.call("lux_hip_overlap_self_device", bvh.handle, 64, out.ptr, rays.ptr, None),
+    }
+
+    def run(text):
+        got = []
+        for word in text.split():
+            made.clear()
+            stub.lib.stub_capturing(int(word.startswith("graph:")))
+            calls[word.split(":")[-1]]()
+            stub.lib.stub_capturing(0)
+            got.append("+".join(made) or "-")
+        return got
+
+    first = run("build trace any trace overlap overlap refit refit any overlap trace build overlap")
+    recorded = run("graph:refit trace overlap trace refit graph:trace trace refit trace overlap graph:build graph:trace")
+    d = sphere(0)
+    made.clear()
+    render = small_engine()
+    sc = render.Scene(d)
+    sc.update_vertices(d["vertices"])
+    return {"first": first, "recorded": recorded, "scene": list(made)}
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

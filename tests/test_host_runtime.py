@@ -73,3 +73,15 @@ def test_instances_lost_in_a_failed_update_are_not_queried(stub):
     assert len(tries) > 2 and tries[-1] == [0, 0]
     assert all(failed == 6 for failed, _ in tries[:-1])
     assert [query for _, query in tries[:-1]] == [0, 0] + [1] * (len(tries) - 3)  # two come before any change
+
+
+def test_traversal_copies_are_made_for_their_first_reader(stub):
+    """Builds and refits make no copy that nobody has asked for; a captured query
+    makes them keep its copy, since it may be replayed after them; captured builds
+    and refits make both; scenes always have both."""
+    r = scene(stub, "copies")
+    #                     build trace any trace overlap overlap refit refit any overlap trace build overlap
+    assert r["first"] == ["-", "r", "-", "-", "p", "-", "-", "-", "r", "p", "-", "-", "p"]
+    #              graph:refit trace overlap trace refit graph:trace trace refit trace overlap graph:build graph:trace
+    assert r["recorded"] == ["rp", "r", "-", "-", "-", "r", "r", "r", "-", "p", "rp", "-"]
+    assert r["scene"] == ["rp", "rp"]
