@@ -99,6 +99,28 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     store_result<kAny>(out, ray, trace_one<kAny>(tree, tris, tri_count, load_ray(rays, ray), 1, 0, stack + threadIdx.x, info, visits, tests));
 }
 
+// Trees without records (one leaf, beyond 2^26 leaves): the preorder walk alone. One
+// triangle, here / in k_trace: 1000 rays 3.6 / 3.8 us, 2^22 closest 27.8 / 28.4, any
+// hit 24.9 / 25.4 (blocks of one wave 29.0 and 25.8).
+constexpr int kPreorderBlock = 256;
+template <bool kAny>
+__global__ __launch_bounds__(kPreorderBlock) void k_trace_preorder(RayTree tree, const lux_triangle* __restrict__ tris,
+                                                           int tri_count, const lux_ray* __restrict__ rays, int n,
+                                                           const uint32_t* __restrict__ order, void* __restrict__ out,
+                                                           DevInfo* info) {
+    const int i = int(xcd_block()) * kPreorderBlock + threadIdx.x;
+    if (i >= n) return;
+    const int ray = order ? int(order[i]) : i;
+    if (uint32_t(ray) >= uint32_t(n)) {
+        set_error(info, kErrSpinLimit);
+        return;
+    }
+    uint32_t visits = 0, tests = 0;
+    const RayIn r = load_ray(rays, ray);
+    store_result<kAny>(out, ray, preorder_query(tree, tris, tri_count, r.o, r.d, r.t_min,
+                                                __builtin_canonicalizef(r.t_max), kAny, -1, info, visits, tests));
+}
+
 // Few rays: `group` lanes (a power of two) walk one ray (wide_query).
 template <bool kAny>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAny ? 7 : 6))) void k_trace_parts(
@@ -393,8 +415,11 @@ void launch_trace(const char* name, BvhDev& d, const uint32_t* order, const lux_
                   const lux_ray* rays, int n, void* out, hipStream_t s) {
     tree_copies(d, kCopyRecords, s);
     const RayTree tree = ray_tree(d);
-    const int group = tree.records ? lanes_per_ray(uint32_t(n)) : 1;
-    if (group > 1)
+    const int group = tree.records >= kPartsMinRecords ? lanes_per_ray(uint32_t(n)) : 1;
+    if (tree.records == 0)
+        LUX_LAUNCH(name, k_trace_preorder<kAny>, div_up(n, kPreorderBlock), kPreorderBlock, 0, s, tree, tris, tri_count, rays, n, order,
+                   out, d.info);
+    else if (group > 1)
         LUX_LAUNCH(name, k_trace_parts<kAny>, div_up(int64_t(n) * group, kBlock), kBlock, 0, s, tree, tris, tri_count,
                    rays, n, order, group, out, d.info);
     else

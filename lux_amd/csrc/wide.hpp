@@ -440,6 +440,10 @@ struct WideHit {
 // 500 000 382 / 277 / 285, on a sphere mesh 133 / 119 / 122; at 2^18 one lane is
 // the best for the soup (422 / 455) and within 6 % on the sphere.
 constexpr uint32_t kPartsMaxRays = 1u << 17;
+// A walk through a handful of records is no chain worth cutting: 12 triangles, parts /
+// one lane a ray, 1000 rays 3.9 / 4.0 us, 2^14 6.5 / 4.5, 2^17 8.9 / 5.5 (sibling
+// pairs before: 5.7, 6.1, 47).
+constexpr uint32_t kPartsMinRecords = 16;
 __host__ __device__ inline int lanes_per_ray(uint32_t n) {
     return n <= (1u << 14) ? 16 : n <= (1u << 16) ? 8 : n <= kPartsMaxRays ? 4 : 1;
 }

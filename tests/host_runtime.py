@@ -303,5 +303,25 @@ def copies(stub):
     return {"first": first, "recorded": recorded, "scene": list(made)}
 
 
+def query_launches(stub):
+    """The kernel and its threads for 1000 rays over trees of few triangles."""
+    from lux_amd import abi, lbvh, workloads as W
+
+    rays, hits = lbvh.DeviceArray(36 * 1000), lbvh.DeviceArray(8 * 1000)
+    seen = []
+    stub.hooks.append(("7k_trace", lambda args: seen.append(["k_trace", stub.lib.stub_grid() * stub.lib.stub_block()])))
+    stub.hooks.append(("13k_trace_parts", lambda args: seen.append(["parts", stub.lib.stub_grid() * stub.lib.stub_block()])))
+    stub.hooks.append(("16k_trace_preorder", lambda args: seen.append(["preorder", 0])))
+    out = {}
+    for n in (1, 2, 16, 17, 300):
+        d = lbvh.DeviceArray.from_numpy(W.soup(n, seed=1))
+        bvh = lbvh.GpuBvh()
+        bvh.build_triangles_device(d, n)
+        seen.clear()
+        abi.call("lux_hip_trace_closest_device", bvh.handle, d.ptr, n, rays.ptr, 1000, hits.ptr, None)
+        out[n] = seen[-1]
+    return out
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

@@ -85,3 +85,11 @@ def test_traversal_copies_are_made_for_their_first_reader(stub):
     #              graph:refit trace overlap trace refit graph:trace trace refit trace overlap graph:build graph:trace
     assert r["recorded"] == ["rp", "r", "-", "-", "-", "r", "r", "r", "-", "p", "rp", "-"]
     assert r["scene"] == ["rp", "rp"]
+
+
+def test_trees_of_few_triangles_take_one_lane_a_ray(stub):
+    """Below 16 records a ray is not cut in parts; a tree without records has the
+    preorder walk's kernel."""
+    assert scene(stub, "query_launches") == {
+        "1": ["preorder", 0], "2": ["k_trace", 1024], "16": ["k_trace", 1024], "17": ["parts", 16000],
+        "300": ["parts", 16000]}
