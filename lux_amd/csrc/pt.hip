@@ -214,8 +214,9 @@ __device__ __forceinline__ bool occluded(const SceneView& sv, const vec& o, cons
 // One ray of an instanced scene (two_level.hpp), given by world(o, d): the closest
 // hit, or any hit.
 template <typename World>
-__device__ __forceinline__ TwoLevelHit instanced_query(const SceneView& sv, World&& world, float t_max, bool any, int ignore, int group, int part,
-                                                       uint32_t* stack, int stride) {
+__device__ __forceinline__ TwoLevelHit instanced_query(const SceneView& sv, World&& world, float t_max, bool any,
+                                                       int ignore, int group, int part, uint32_t* stack,
+                                                       int stride) {
     TwoLevelHit h;
     if (sv.preorder || !two_level_wide<true>(sv.tl, world, kEps, t_max, any, ignore, group, part, stack, stride, h))
         h = two_level_walk(sv.tl, world, kEps, t_max, any, ignore);
@@ -460,8 +461,8 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWalk == kWal
         if (other && (total <= kPartsMaxRays) != (kWalk == kWalkParts)) return;  // the other launch's
         const uint32_t* queue = ext_in >= 0 ? qs.q[ext_in] : nullptr;
         for (uint32_t i = xcd_block() * B + threadIdx.x; i < total * group; i += gridDim.x * B)
-            record_ray<kAnyShadow, kWalk == kWalkTwoLevel>(desc, ps, kWalk == kWalkMesh ? i : i / group, n_ext, queue, int(group),
-                                 int(i & (group - 1)), stack, B);
+            record_ray<kAnyShadow, kWalk == kWalkTwoLevel>(desc, ps, kWalk == kWalkMesh ? i : i / group, n_ext, queue,
+                                                           int(group), int(i & (group - 1)), stack, B);
         return;
     }
     for (uint32_t i = xcd_block() * B + threadIdx.x; i < total; i += gridDim.x * B) {
@@ -1213,6 +1214,12 @@ Segment make_segment(const Request& rq, uint64_t req_begin, uint32_t slot_begin,
 
 }  // namespace
 
+namespace {
+// Rays of the scene by sibling pairs. Trees without records (one leaf, beyond 2^26
+// leaves) have only the preorder walk in the records' kernels too.
+bool small_tree(const Request& rq) { return rq.sv.tree.records < kSmallTree; }
+}  // namespace
+
 int request_kind(const Request& rq) { return (rq.sv.instanced ? 1 : 0) | (rq.rs.light_sampler << 1); }
 
 uint64_t request_paths(const lux_render_settings& rs) {
@@ -1454,8 +1461,9 @@ void Renderer::launch_wavefront(int depth, bool opaque, bool two_level, bool sma
         shade_resident_light_ = light;
     }
     const int walk = two_level ? kWalkTwoLevel
-                     : small   ? kWalkPairs
-                               : (uint32_t(buf_.capacity) <= kPartsMaxRays ? kWalkParts : kWalkBoth);
+                     : small
+                         ? kWalkPairs
+                         : (uint32_t(buf_.capacity) <= kPartsMaxRays ? kWalkParts : kWalkBoth);
     const int64_t trace_lanes = int64_t(buf_.capacity) * lanes_per_ray(uint32_t(buf_.capacity));
     const LaunchGrid grid{tuned, std::min(tuned, shade_resident_),
                           std::max(1, std::min(tune_.grid, div_up(trace_lanes, block)))};
@@ -1492,42 +1500,50 @@ void Renderer::launch_wavefront(int depth, bool opaque, bool two_level, bool sma
 }
 
 namespace {
-template <bool kTwoLevel, int kLight>
+// walk: kWalkTwoLevel, kWalkPairs or kWalkMesh. A two-level trace grid holds the
+// lanes of its rays (lanes_per_ray): 128 x 96 x 2 of an instanced room 7.0 ms with a
+// thread per path, 2.5 with a thread per lane (3.5 by sibling pairs). Small trees by
+// pairs as in the wavefront loop: Cornell box 128 x 96 x 2 1.30 / 1.17 ms.
+template <int kWalk, int kLight>
 void plain_sequence(const PathBuf& buf, int depth, uint32_t count, hipStream_t stream) {
     const Paths ps = paths_of(buf);
     const Queues qs = queues_of(buf);
     const BatchDesc* d = buf.desc;
     const int grid = std::max(1, div_up(count, kBlock));
+    const int trace_grid =
+        kWalk == kWalkTwoLevel ? std::max(1, div_up(int64_t(count) * lanes_per_ray(count), kBlock)) : grid;
     LUX_LAUNCH("pt_generate", k_generate<kBlock>, grid, kBlock, 0, stream, d, ps, qs);
     for (int b = 0; b <= depth; ++b) {
         const int in = b & 1;
-        LUX_LAUNCH("pt_trace", (k_trace<kBlock, false, kTwoLevel ? kWalkTwoLevel : kWalkMesh>), grid, kBlock, 0, stream, d,
-                   ps, qs, in, -1, in ^ 1, 2 + (b & 1), 1, 0);
+        LUX_LAUNCH("pt_trace", (k_trace<kBlock, false, kWalk>), trace_grid, kBlock, 0, stream, d, ps, qs, in, -1,
+                   in ^ 1, 2 + (b & 1), 1, 0);
         for (int type = 0; type < kMaterialTypes; ++type)
             LUX_LAUNCH("pt_shade", (k_shade<kBlock, kLight>), grid, kBlock, 0, stream, d, ps, qs, in, b, type);
-        LUX_LAUNCH("pt_shadow", (k_trace<kBlock, false, kTwoLevel ? kWalkTwoLevel : kWalkMesh>), grid, kBlock, 0, stream,
-                   d, ps, qs, -1, 2 + (b & 1), -1, -1, 1, 0);
+        LUX_LAUNCH("pt_shadow", (k_trace<kBlock, false, kWalk>), trace_grid, kBlock, 0, stream, d, ps, qs, -1,
+                   2 + (b & 1), -1, -1, 1, 0);
     }
     LUX_LAUNCH("pt_flush", k_flush<kBlock>, grid, kBlock, 0, stream, d, ps);
 }
 }  // namespace
 
 namespace {
-template <bool kTwoLevel>
+template <int kWalk>
 void plain_sequence_l(int light, const PathBuf& buf, int depth, uint32_t count, hipStream_t stream) {
     switch (light) {
-        case kLightUniform: plain_sequence<kTwoLevel, kLightUniform>(buf, depth, count, stream); break;
-        case kLightBvh: plain_sequence<kTwoLevel, kLightBvh>(buf, depth, count, stream); break;
-        default: plain_sequence<kTwoLevel, kLightPower>(buf, depth, count, stream); break;
+        case kLightUniform: plain_sequence<kWalk, kLightUniform>(buf, depth, count, stream); break;
+        case kLightBvh: plain_sequence<kWalk, kLightBvh>(buf, depth, count, stream); break;
+        default: plain_sequence<kWalk, kLightPower>(buf, depth, count, stream); break;
     }
 }
 }  // namespace
 
-void Renderer::launch_plain(int depth, uint32_t count, bool two_level, int light, hipStream_t stream) {
+void Renderer::launch_plain(int depth, uint32_t count, bool two_level, bool small, int light, hipStream_t stream) {
     if (two_level)
-        plain_sequence_l<true>(light, buf_, depth, count, stream);
+        plain_sequence_l<kWalkTwoLevel>(light, buf_, depth, count, stream);
+    else if (small)
+        plain_sequence_l<kWalkPairs>(light, buf_, depth, count, stream);
     else
-        plain_sequence_l<false>(light, buf_, depth, count, stream);
+        plain_sequence_l<kWalkMesh>(light, buf_, depth, count, stream);
 }
 
 uint64_t Renderer::enqueue_batch(std::vector<Request*>& active, int slice_spp, int max_depth, hipStream_t stream,
@@ -1553,7 +1569,7 @@ uint64_t Renderer::enqueue_batch(std::vector<Request*>& active, int slice_spp, i
         if (slice_spp > 0)
             take = std::min(take, uint64_t(slice_spp) * uint64_t(rq->rs.width) * uint64_t(rq->rs.height));
         opaque = opaque && rq->sv.opaque != 0;
-        small = small && rq->sv.tree.records < kSmallTree;
+        small = small && small_tree(*rq);
         slot->seg[nseg] = make_segment(*rq, rq->issued, uint32_t(used), uint32_t(take));
         slot->seg[nseg++].sv.preorder = tune_.preorder_walk;
         rq->issued += take;
@@ -1593,7 +1609,8 @@ void Renderer::render_all(std::vector<Request*>& reqs, int mode, hipStream_t str
                     slot->seg[0] = make_segment(*rq, uint64_t(s) * npix + p0, 0, n);
                     slot->seg[0].sv.preorder = tune_.preorder_walk;
                     upload(slot, stream);
-                    launch_plain(rq->rs.max_depth, n, rq->sv.instanced != 0, rq->rs.light_sampler, stream);
+                    launch_plain(rq->rs.max_depth, n, rq->sv.instanced != 0, small_tree(*rq), rq->rs.light_sampler,
+                                 stream);
                     hip_check(hipMemcpyAsync(host_counts, buf_.counts, sizeof(host_counts), hipMemcpyDeviceToHost,
                                              stream),
                               "D2H counts");

@@ -244,7 +244,7 @@ private:
     BatchDesc* next_slot();
     void upload(BatchDesc* slot, hipStream_t stream);
     void launch_wavefront(int depth, bool opaque, bool two_level, bool small, int light, hipStream_t stream);
-    void launch_plain(int depth, uint32_t count, bool two_level, int light, hipStream_t stream);
+    void launch_plain(int depth, uint32_t count, bool two_level, bool small, int light, hipStream_t stream);
     void release_graph();
 
     Tuning tune_;

@@ -323,5 +323,26 @@ def query_launches(stub):
     return out
 
 
+def trace_launches(stub):
+    """k_trace's walk and threads, as [walk, threads] of the first launch of each
+    render."""
+    from lux_amd import scenes
+
+    render = small_engine()
+    seen = []
+    stub.hooks.append(("7k_traceILi", lambda args: seen.append([stub.launches[-1].split("ELi")[1][0],
+                                                                stub.lib.stub_grid() * stub.lib.stub_block()])))
+    out = {}
+    made = {"room": scenes.instanced_room(64, 48), "box": scenes.cornell(64, 48),
+            "sphere": scenes.displaced_icosphere(freq=8, seed=1, width=64, height=48)}
+    for name, d in made.items():
+        sc = render.Scene(d)
+        for mode, text in ((render.PLAIN, "plain"), (render.WAVEFRONT, "wave")):
+            seen.clear()
+            sc.render(64, 48, 1, 1, mode=mode)
+            out[f"{name} {text}"] = seen[0]
+    return out
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

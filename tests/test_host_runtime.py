@@ -93,3 +93,14 @@ def test_trees_of_few_triangles_take_one_lane_a_ray(stub):
     assert scene(stub, "query_launches") == {
         "1": ["preorder", 0], "2": ["k_trace", 1024], "16": ["k_trace", 1024], "17": ["parts", 16000],
         "300": ["parts", 16000]}
+
+
+def test_trace_launches_fit_their_walk(stub):
+    """64 x 48 paths: 16 lanes a ray where a walk takes parts, so that many threads
+    (or the tuned grid of 8 x 256); trees of few triangles on the pairs' kernel, plain
+    mode included."""
+    two_level, pairs, mesh, parts = "0", "1", "2", "3"
+    paths, lanes, tuned = 64 * 48, 64 * 48 * 16, 8 * 256
+    assert scene(stub, "trace_launches") == {
+        "room plain": [two_level, lanes], "room wave": [two_level, tuned], "box plain": [pairs, paths],
+        "box wave": [pairs, tuned], "sphere plain": [mesh, paths], "sphere wave": [parts, tuned]}
