@@ -42,7 +42,9 @@ namespace pt {
 namespace {
 
 constexpr int kBlock = 256;
-// Batches whose trees all have fewer records walk sibling pairs. A record step
+// Batches whose trees all have fewer records walk sibling pairs (so does every
+// batch with the preorder walk asked for: 8 waves a SIMD hold it better than the
+// records' 6). A record step
 // costs about two pair steps of instructions and pays by halving the waits for
 // memory, which a tree this small hardly has: records / pairs, Cornell box (36
 // triangles) 256 x 256 x 64 7.77 / 7.27 ms, 128 x 96 x 4 0.412 / 0.371 ms; sphere
@@ -212,27 +214,24 @@ __device__ __forceinline__ bool occluded(const SceneView& sv, const vec& o, cons
 }
 
 // One ray of an instanced scene (two_level.hpp), given by world(o, d): the closest
-// hit, or any hit.
+// hit, or any hit; preorder: by the preorder walk.
 template <typename World>
 __device__ __forceinline__ TwoLevelHit instanced_query(const SceneView& sv, World&& world, float t_max, bool any,
-                                                       int ignore, int group, int part, uint32_t* stack,
-                                                       int stride) {
+                                                       bool preorder, int ignore, int group, int part,
+                                                       uint32_t* stack, int stride) {
     TwoLevelHit h;
-    if (sv.preorder || !two_level_wide<true>(sv.tl, world, kEps, t_max, any, ignore, group, part, stack, stride, h))
+    if (preorder || !two_level_wide<true>(sv.tl, world, kEps, t_max, any, ignore, group, part, stack, stride, h))
         h = two_level_walk(sv.tl, world, kEps, t_max, any, ignore);
     return h;
 }
 
 // One ray of a one-mesh scene on `group` lanes (wide_query): the closest hit, or
-// any hit.
+// any hit. (With the preorder walk asked for, k_trace takes the pairs' kernel.)
 __device__ __forceinline__ WideHit mesh_query(const SceneView& sv, const f3& o, const f3& d, float t_max, bool any,
                                               int ignore, int group, int part, uint32_t* stack, int stride) {
     uint32_t visits = 0, tests = 0;
-    WideHit h;
-    h.failed = sv.preorder != 0;
-    if (!h.failed)
-        h = wide_query<true>(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, group, part, stack, stride,
-                             sv.info, visits, tests);
+    WideHit h = wide_query<true>(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, group, part, stack,
+                                 stride, sv.info, visits, tests);
     if (h.failed)
         h = preorder_query<true>(sv.tree, sv.soup, sv.tri_count, o, d, kEps, t_max, any, ignore, sv.info, visits,
                                  tests);
@@ -385,7 +384,8 @@ __device__ __forceinline__ void record_ray(const BatchDesc* __restrict__ desc, c
     typename std::conditional<kTwoLevel, TwoLevelHit, WideHit>::type h;
     for (int guard = 0; guard < 1 << 16; ++guard) {
         if constexpr (kTwoLevel)
-            h = instanced_query(sv, world, t_max, kAnyShadow && !ext, ignore, group, part, stack, stride);
+            h = instanced_query(sv, world, t_max, kAnyShadow && !ext, ext && sv.preorder, ignore, group, part, stack,
+                                stride);
         else
             h = mesh_query(sv, o, d, t_max, kAnyShadow && !ext, ignore, group, part, stack, stride);
         if (ext) break;
@@ -457,7 +457,9 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(kWalk == kWal
     uint32_t* stack = lds_stack + threadIdx.x;
     const uint32_t total = n_ext + n_sh;
     if constexpr (kRecords) {
-        const uint32_t group = kWalk == kWalkMesh ? 1u : uint32_t(lanes_per_ray(total));
+        // (preorder rays are not cut in parts)
+        const bool whole = kWalk == kWalkMesh || (kWalk == kWalkTwoLevel && desc->seg[0].sv.preorder);
+        const uint32_t group = whole ? 1u : uint32_t(lanes_per_ray(total));
         if (other && (total <= kPartsMaxRays) != (kWalk == kWalkParts)) return;  // the other launch's
         const uint32_t* queue = ext_in >= 0 ? qs.q[ext_in] : nullptr;
         for (uint32_t i = xcd_block() * B + threadIdx.x; i < total * group; i += gridDim.x * B)
@@ -1461,7 +1463,7 @@ void Renderer::launch_wavefront(int depth, bool opaque, bool two_level, bool sma
         shade_resident_light_ = light;
     }
     const int walk = two_level ? kWalkTwoLevel
-                     : small
+                     : small || tune_.preorder_walk
                          ? kWalkPairs
                          : (uint32_t(buf_.capacity) <= kPartsMaxRays ? kWalkParts : kWalkBoth);
     const int64_t trace_lanes = int64_t(buf_.capacity) * lanes_per_ray(uint32_t(buf_.capacity));
@@ -1540,7 +1542,7 @@ void plain_sequence_l(int light, const PathBuf& buf, int depth, uint32_t count, 
 void Renderer::launch_plain(int depth, uint32_t count, bool two_level, bool small, int light, hipStream_t stream) {
     if (two_level)
         plain_sequence_l<kWalkTwoLevel>(light, buf_, depth, count, stream);
-    else if (small)
+    else if (small || tune_.preorder_walk)
         plain_sequence_l<kWalkPairs>(light, buf_, depth, count, stream);
     else
         plain_sequence_l<kWalkMesh>(light, buf_, depth, count, stream);

@@ -137,7 +137,7 @@ struct SceneView {
     const float* env_cdf;                  // per-texel cumulative weights
     int32_t opaque;     // 1: every hit blocks a shadow ray (no pass-through material)
     int32_t instanced;  // 1: traverse `tl` (two-level) instead of `tree`
-    int32_t preorder;   // 1: rays take the right-first preorder walk only
+    int32_t preorder;   // 1: extension rays take the right-first preorder walk only
     DevCamera cam;
     TwoLevelView tl;
 };

@@ -338,9 +338,11 @@ def trace_launches(stub):
     for name, d in made.items():
         sc = render.Scene(d)
         for mode, text in ((render.PLAIN, "plain"), (render.WAVEFRONT, "wave")):
-            seen.clear()
-            sc.render(64, 48, 1, 1, mode=mode)
-            out[f"{name} {text}"] = seen[0]
+            for preorder in (False, True):
+                render.set_tuning(preorder_walk=preorder)
+                seen.clear()
+                sc.render(64, 48, 1, 1, mode=mode)
+                out[f"{name} {text}{' preorder' if preorder else ''}"] = seen[0]
     return out
 
 

@@ -97,10 +97,15 @@ def test_trees_of_few_triangles_take_one_lane_a_ray(stub):
 
 def test_trace_launches_fit_their_walk(stub):
     """64 x 48 paths: 16 lanes a ray where a walk takes parts, so that many threads
-    (or the tuned grid of 8 x 256); trees of few triangles on the pairs' kernel, plain
-    mode included."""
+    (or the tuned grid of 8 x 256); trees of few triangles, and the preorder walk, on
+    the pairs' kernel, plain mode included."""
     two_level, pairs, mesh, parts = "0", "1", "2", "3"
     paths, lanes, tuned = 64 * 48, 64 * 48 * 16, 8 * 256
     assert scene(stub, "trace_launches") == {
-        "room plain": [two_level, lanes], "room wave": [two_level, tuned], "box plain": [pairs, paths],
-        "box wave": [pairs, tuned], "sphere plain": [mesh, paths], "sphere wave": [parts, tuned]}
+        "room plain": [two_level, lanes], "room plain preorder": [two_level, lanes],
+        "room wave": [two_level, tuned], "room wave preorder": [two_level, tuned],
+        "box plain": [pairs, paths], "box plain preorder": [pairs, paths],
+        "box wave": [pairs, tuned], "box wave preorder": [pairs, tuned],
+        "sphere plain": [mesh, paths], "sphere plain preorder": [pairs, paths],
+        "sphere wave": [parts, tuned], "sphere wave preorder": [pairs, tuned],
+    }
