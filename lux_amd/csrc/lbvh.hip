@@ -1092,12 +1092,16 @@ void launch_local(const char* name, BvhDev& d, const lux_aabb* src_boxes, const 
                    (const uint32_t*)d.rtop_int, (const uint32_t*)d.rtop_leaf, d.nodes, d.pre_internal, d.pre_leaf,
                    d.edge_boxes, d.block_boxes, d.info);
     };
-    if (blocks <= 96)
+    if (blocks <= 96) {
         go(std::integral_constant<int, 1024>{});
-    else if (kMode != 0 || blocks <= 384)
-        go(std::integral_constant<int, 512>{});
-    else
-        go(std::integral_constant<int, 256>{});
+        return;
+    }
+    if constexpr (kMode == 0)
+        if (blocks > 384) {
+            go(std::integral_constant<int, 256>{});
+            return;
+        }
+    go(std::integral_constant<int, 512>{});
 }
 
 void wide_from(const BvhDev& d, const lux_bvh_node* nodes, WideNode* wide, int32_t* wide_leaf, hipStream_t s) {
