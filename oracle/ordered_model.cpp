@@ -1,5 +1,5 @@
 // ordered_model.cpp -- CPU model of the library's near-child-first closest-hit
-// walk (lux_amd/csrc/ordered.hpp), used by the tests to show where that walk
+// walk over sibling pairs (lux_amd/csrc/ordered.hpp), used by the tests to show where that walk
 // can part from the right-first preorder walk of the host LBVH and that the
 // library's ambiguity check closes the gap.
 //

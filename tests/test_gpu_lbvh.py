@@ -233,10 +233,10 @@ def test_closest_hit_exact_ties(gpu):
 
 def test_closest_hit_deep_stack_falls_back_to_preorder(gpu):
     """2^18 parallel triangles stacked along x, every one crossing the rays'
-    line: the near-child-first walk keeps one pending sibling per level with two
-    internal children, more than its 16-entry stack holds on the way to the
-    nearest leaf, so those rays are walked again in preorder. Results equal the
-    oracle's either way."""
+    line: the walk over four-child records keeps up to three pending children per
+    record, more than its 20-entry stack holds on the way to the nearest leaf, so
+    those rays are walked again in preorder (few rays: the parts nearest the ends
+    overflow too). Results equal the oracle's either way, on one lane a ray as well."""
     print_case("closest deep stack")
     m = 1 << 18
     x = ((np.arange(m) + 0.5) / m).astype(np.float32)
@@ -255,17 +255,40 @@ def test_closest_hit_deep_stack_falls_back_to_preorder(gpu):
     hits, o = check_closest_against_oracle(gpu, tris, ids, rays)
     assert np.array_equal(hits["primitive_id"][:k], np.zeros(k, np.int32))
     assert np.array_equal(hits["primitive_id"][k:], np.full(k, m - 1, np.int32))
-    # levels with two internal children on the path to the leftmost leaf: the
-    # stack depth a +x ray reaches there
+    rng = np.random.default_rng(12)
+    many = np.repeat(rays, 1100, axis=0)  # one lane a ray
+    many[:, 1:3] = rng.uniform(0.3, 0.7, (len(many), 2))
+    hits = gpu.intersect_gpu_bvh_stackless(gpu.build_gpu_lbvh(W.triangle_boxes(tris), ids), tris, many)
+    first = np.repeat(np.arange(2 * k) < k, 1100)
+    assert len(many) > 1 << 17
+    assert np.array_equal(hits["primitive_id"], np.where(first, 0, m - 1))
+    # the entries a +x ray holds when it reaches the leftmost records: at each, the
+    # nearest internal child is next and the other internal ones are pending
     left, right = o.left.astype(np.int64), o.right.astype(np.int64)
-    node, both = 0, 0
+
+    def box(c):
+        return o.node_bounds[(c & 0x7FFFFFFF) + (m - 1 if c & 0x80000000 else 0)].astype(np.float64)
+
+    def area(c):
+        if c & 0x80000000:
+            return -1.0
+        dx, dy, dz = box(c)[3:] - box(c)[:3]
+        return dx * dy + dy * dz + dz * dx
+
+    node, held = 0, 0
     while True:
-        li, ri = (left[node] & 0x80000000) == 0, (right[node] & 0x80000000) == 0
-        both += int(li and ri)
-        if not li:
+        kids = [int(left[node]), int(right[node])]
+        for _ in range(2):
+            best = max(range(len(kids)), key=lambda i: area(kids[i]))
+            if area(kids[best]) >= 0:
+                c = kids[best]
+                kids[best : best + 1] = [int(left[c]), int(right[c])]
+        inner = sorted((c for c in kids if not c & 0x80000000), key=lambda c: box(c)[0])
+        if not inner:
             break
-        node = int(left[node])
-    assert both > 16
+        held += len(inner) - 1
+        node = inner[0]
+    assert held > 20
 
 
 def test_full_size_microbench_inputs(gpu):

@@ -134,7 +134,7 @@ def test_instanced_microbench_inputs_match_oracle(gpu):
     a 32 768-ray sample against the oracle walk; occlusion of every ray equals
     closest-found."""
     print_case("two-level microbench inputs")
-    inp = W.two_level_inputs(n_rays=1 << 18)
+    inp = W.two_level_inputs(n_rays=(1 << 19) + 1)
     tris = np.concatenate([v[i].reshape(-1, 9) for v, i in inp["meshes"]]).astype(np.float32)
     off = np.concatenate([[0], np.cumsum([len(i) for _, i in inp["meshes"]])]).astype(np.int32)
     rec = TL.make_instances(inp["inst_mesh"], inp["inst_m"], tris=tris, mesh_offsets=off)
@@ -150,9 +150,11 @@ def test_instanced_microbench_inputs_match_oracle(gpu):
     occ = s.occluded(inp["rays"])
     assert np.array_equal(occ.astype(bool), h["primitive_id"] >= 0)
     assert (h["primitive_id"] >= 0).mean() > 0.2
-    # 2^18 rays are traced in ray order (octant, then origin); chunks below the
-    # ordering threshold run in input order and must give the same bits, also
-    # with a per-ray ignored primitive
+    # 2^19 + 1 rays over 2^18 triangles are traced in ray order (octant, then origin:
+    # kTwoLevelOrderMinRays, kTwoLevelOrderMinTris); chunks below the ordering
+    # threshold run in input order and must give the same bits, also with a per-ray
+    # ignored primitive
+    assert off[-1] >= 1 << 18
     rays = inp["rays"]
     ign = np.where(h["primitive_id"] >= 0, h["primitive_id"], -1).astype(np.int32)
     h_ign, occ_ign = s.intersect(rays, ignore=ign), s.occluded(rays, ignore=ign)
@@ -251,7 +253,7 @@ def test_culling_boxes_keep_hits_of_round_meshes_and_loose_inverses(gpu):
     scene validation's 1e-4), and rays aimed at points just inside and just
     outside the spheres' silhouettes: closest hits (ids and t) equal the oracle's
     walk over the reference boxes with the same inverses, and occlusion equals
-    closest-found, through the ray-ordered path (2^17 rays)."""
+    closest-found (2^17 rays, four lanes each)."""
     from lux_amd import scenes
 
     print_case("two-level culling boxes, round meshes")

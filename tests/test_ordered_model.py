@@ -1,6 +1,7 @@
-"""The near-child-first closest-hit walk against the right-first preorder walk
-of the host LBVH, on the CPU (oracle/ordered_model.cpp models the library's
-walk). The rounding4 golden case holds a ray on which the walk without its
+"""The near-child-first closest-hit walk over sibling pairs (path-traced scenes of
+fewer than 128 records) against the right-first preorder walk of the host LBVH, on
+the CPU (oracle/ordered_model.cpp models the library's walk; test_wide_model.py runs
+the one over four-child records). The rounding4 golden case holds a ray on which the walk without its
 ambiguity check returns another triangle than the reference's host LBVH; with
 the check the ray is walked again in preorder and the hit equals the
 reference's."""

@@ -27,8 +27,9 @@ def test_noalloc_closest_equals_device_closest(gpu):
     tris = W.soup(1 << 15, seed=71)
     bvh = gpu.build_gpu_lbvh(W.triangle_boxes(tris))
     d_tris = gpu.DeviceArray.from_numpy(tris)
-    # 2^17 + 3 rays, then 70001 (both sorted through the scratch), then 1000
-    for count, seed in ((131075, 72), (70001, 73), (1000, 74)):
+    # 2^21 + 3 rays, then 2^21 (both sorted through the scratch: kOrderMinRays), then
+    # 131075 and 1000 in input order
+    for count, seed in (((1 << 21) + 3, 72), (1 << 21, 73), (131075, 76), (1000, 74)):
         print(f"case: no-alloc closest, {count} rays, seed {seed}", flush=True)
         rays = W.rays(count, seed=seed)
         ref = _closest(gpu, "lux_hip_trace_closest_device", bvh, d_tris, len(tris), rays)
