@@ -1191,14 +1191,19 @@ const uint32_t* ray_order(RaySortDev& r, const BvhDev& tree, const lux_ray* rays
     if (n > r.capacity) {
         if (r.capacity) hip_check(hipDeviceSynchronize(), "synchronize before ray-sort growth");
         raysort_release(r);
-        r.capacity = n;
-        for (int b = 0; b < 2; ++b) {
-            r.keys[b] = dalloc<uint32_t>(n);
-            r.vals[b] = dalloc<uint32_t>(n);
+        try {
+            for (int b = 0; b < 2; ++b) {
+                r.keys[b] = dalloc<uint32_t>(n);
+                r.vals[b] = dalloc<uint32_t>(n);
+            }
+            r.hist = dalloc<uint32_t>(2 * kRadix);
+            r.status = dalloc<uint64_t>(ray_order_status_words(n));
+            r.tickets = dalloc<uint32_t>(4);
+        } catch (...) {
+            raysort_release(r);
+            throw;
         }
-        r.hist = dalloc<uint32_t>(2 * kRadix);
-        r.status = dalloc<uint64_t>(ray_order_status_words(n));
-        r.tickets = dalloc<uint32_t>(4);
+        r.capacity = n;
         zero_words(reinterpret_cast<uint32_t*>(r.status), 2 * ray_order_status_words(n), s);
         zero_words(r.tickets, 4, s);
     }
@@ -1266,12 +1271,22 @@ void bvh_allocate(BvhDev& d, int n, hipStream_t s) {
         d.n = n;
         return;
     }
-    bvh_release(d);
-    int cap = max(n, 1);
+    const unsigned keep = d.keep;
+    auto release = [&] {
+        bvh_release(d);
+        d.keep = keep;
+    };
+    release();
+    const int cap = max(n, 1);
+    d.status_words = sort_tiles(cap) * kRadix;
+    try {
+        bvh_buffers(d, cap, [](auto*& p, size_t count) { p = dalloc<std::remove_reference_t<decltype(*p)>>(count); });
+    } catch (...) {  // a later build must not take the rest for allocated
+        release();
+        throw;
+    }
     d.capacity = cap;
     d.n = n;
-    d.status_words = sort_tiles(cap) * kRadix;
-    bvh_buffers(d, cap, [](auto*& p, size_t count) { p = dalloc<std::remove_reference_t<decltype(*p)>>(count); });
     LUX_LAUNCH("lbvh_clear", k_clear_tree, max(1, min(512, div_up(d.status_words, kBlock))), kBlock, 0, s, d.status,
                d.status_words, d.tickets, d.counter, d.info);
     d.epoch = 0;

@@ -1259,13 +1259,18 @@ void Renderer::ensure_capacity(int paths, hipStream_t stream) {
     if (buf_.capacity) hip_check(hipDeviceSynchronize(), "synchronize before path buffer growth");
     pathbuf_release(buf_);
     size_t P = size_t(paths);
+    try {
+        buf_.f4 = dalloc<float4>(11 * P);
+        buf_.rng = dalloc<ulonglong2>(P);
+        buf_.q = dalloc<uint32_t>(2 * P);
+        buf_.counts = dalloc<uint32_t>(4);
+        buf_.rays = dalloc<unsigned long long>(2);
+        buf_.desc = static_cast<BatchDesc*>(static_cast<void*>(dalloc<uint8_t>(sizeof(BatchDesc))));
+    } catch (...) {  // a later batch must not take the rest for allocated
+        pathbuf_release(buf_);
+        throw;
+    }
     buf_.capacity = paths;
-    buf_.f4 = dalloc<float4>(11 * P);
-    buf_.rng = dalloc<ulonglong2>(P);
-    buf_.q = dalloc<uint32_t>(2 * P);
-    buf_.counts = dalloc<uint32_t>(4);
-    buf_.rays = dalloc<unsigned long long>(2);
-    buf_.desc = static_cast<BatchDesc*>(static_cast<void*>(dalloc<uint8_t>(sizeof(BatchDesc))));
     LUX_LAUNCH("pt_clear_counts", k_clear_counts, 1, 64, 0, stream, buf_.counts, buf_.rays);
 }
 

@@ -346,5 +346,63 @@ def trace_launches(stub):
     return out
 
 
+def failed_builds(stub):
+    """A build that runs out of memory at each of its allocations in turn, then the
+    same build again with memory to spare and queries over it: the arrays its kernels
+    are given."""
+    from lux_amd import abi, lbvh, workloads as W
+
+    n = 300
+    d_tris, rays, out = lbvh.DeviceArray.from_numpy(W.soup(n, seed=1)), lbvh.DeviceArray(36), lbvh.DeviceArray(8)
+    null = []
+    want = {"k_copies": range(2, 9), "11k_sort_pass": (0, 1, 2, 3, 6, 7, 8, 11), "7k_local": (1, 2, 6, 7, 8, 9, 10)}
+    for name, ks in want.items():
+        stub.hooks.append((name, lambda args, name=name, ks=ks: null.extend([name, k] for k in ks if not ptr(args, k))))
+    base = stub.lib.stub_live_bytes()
+    tries, left = [], []
+    for k in range(60):
+        bvh = lbvh.GpuBvh()
+        stub.lib.stub_fail_alloc_after(k)
+        tries.append(status_of(lambda: bvh.build_triangles_device(d_tris, n)))
+        stub.lib.stub_fail_alloc_after(-1)
+        left.append(stub.lib.stub_live_bytes() - base if tries[-1] else 0)
+        null.clear()
+        bvh.build_triangles_device(d_tris, n - 1)
+        abi.call("lux_hip_trace_closest_device", bvh.handle, d_tris.ptr, n, rays.ptr, 1, out.ptr, None)
+        assert null == [], (k, null)
+        bvh.close()
+        if not tries[-1]:
+            break
+    # the scratch of the ray order, and a renderer's path buffer
+    m = (1 << 21) + 1
+    bvh, rays, out = lbvh.GpuBvh(), lbvh.DeviceArray(36 * m), lbvh.DeviceArray(8 * m)
+    bvh.build_triangles_device(d_tris, n)
+    render = small_engine()
+    sc = render.Scene(sphere(0))
+    film = lbvh.DeviceArray(12 * 256)
+    rs = render.settings(width=16, height=16, spp=1, depth=1)
+    stub.hooks.append(("k_generate", lambda args: null.extend(["k_generate", k] for k in range(3) if not ptr(args, k))))
+    later = {
+        "order": lambda: abi.call("lux_hip_trace_closest_device", bvh.handle, d_tris.ptr, n, rays.ptr, m, out.ptr,
+                                  None),
+        "paths": lambda: abi.call("lux_hip_render_device", sc.handle, ctypes.byref(rs), film.ptr, None),
+    }
+    counts = {}
+    for name, call in later.items():
+        base = stub.lib.stub_live_bytes()
+        for k in range(20):
+            stub.lib.stub_fail_alloc_after(k)
+            failed = status_of(call)
+            stub.lib.stub_fail_alloc_after(-1)
+            if not failed:
+                break
+            left.append(stub.lib.stub_live_bytes() - base)
+        counts[name] = k
+        null.clear()
+        call()
+        assert null == [], (name, null)
+    return {"tries": tries, "left": left, "later": counts}
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

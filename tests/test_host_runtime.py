@@ -109,3 +109,13 @@ def test_trace_launches_fit_their_walk(stub):
         "sphere plain": [mesh, paths], "sphere plain preorder": [pairs, paths],
         "sphere wave": [parts, tuned], "sphere wave preorder": [pairs, tuned],
     }
+
+
+def test_a_build_after_a_failed_one_has_all_its_arrays(stub):
+    """Out of memory in the middle of a tree's buffers (of the ray order's, of a path
+    buffer's): nothing of them stays, and the next call of no greater size does not take
+    the rest for allocated."""
+    r = scene(stub, "failed_builds")
+    assert len(r["tries"]) > 25 and r["tries"][:-1] == [6] * (len(r["tries"]) - 1) and r["tries"][-1] == 0
+    assert not any(r["left"])
+    assert r["later"] == {"order": 7, "paths": 12}  # (paths: a buffer for one, then the batch)
