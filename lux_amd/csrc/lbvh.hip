@@ -1115,6 +1115,7 @@ void wide_from(const BvhDev& d, const lux_bvh_node* nodes, WideNode* wide, int32
 namespace {
 void launch_copies(const BvhDev& d, unsigned which, hipStream_t s) {
     if (d.n <= 0) return;
+    which &= d.holds;
     const int wide_blocks = (which & kCopyRecords) && d.n > 1 ? min(4096, div_up(d.n - 1, kBlock)) : 0;
     const int pair_blocks = which & kCopyPairs ? max(1, min(2048, div_up(2 * d.n - 1, kBlock))) : 0;
     if (wide_blocks + pair_blocks == 0) return;
@@ -1243,16 +1244,21 @@ void bvh_buffers(BvhDev& d, int cap, F&& f) {
     f(d.partials, sizeof(BoxIds) * kReduceBlocksMax);
     f(d.info, size_t(1));
     f(d.counter, size_t(4));
-    f(d.pairs, 2 * c);
-    f(d.pair_pos, 2 * c);
-    f(d.slot_pre, 2 * c);
-    f(d.wide, c);
-    f(d.wide_leaf, 4 * c);
+    if (d.holds & kCopyPairs) {
+        f(d.pairs, 2 * c);
+        f(d.pair_pos, 2 * c);
+        f(d.slot_pre, 2 * c);
+    }
+    if (d.holds & kCopyRecords) {
+        f(d.wide, c);
+        f(d.wide_leaf, 4 * c);
+    }
 }
 }  // namespace
 
-size_t bvh_device_bytes(int n) {
+size_t bvh_device_bytes(int n, unsigned holds) {
     BvhDev d;
+    d.holds = holds;
     size_t bytes = 0;
     bvh_buffers(d, max(n, 1), [&](auto*& p, size_t count) { bytes += sizeof(*p) * count; });
     return bytes;
@@ -1271,9 +1277,10 @@ void bvh_allocate(BvhDev& d, int n, hipStream_t s) {
         d.n = n;
         return;
     }
-    const unsigned keep = d.keep;
+    const unsigned holds = d.holds, keep = d.keep;
     auto release = [&] {
         bvh_release(d);
+        d.holds = holds;
         d.keep = keep;
     };
     release();
@@ -1293,9 +1300,9 @@ void bvh_allocate(BvhDev& d, int n, hipStream_t s) {
 }
 
 namespace {
-// Boxes above the leaf blocks and, in a build (kLayout), the pair positions.
+// Boxes above the leaf blocks and, in a build (layout), the pair positions.
 template <bool kLayout>
-void top_boxes(BvhDev& d, hipStream_t s) {
+void launch_top_boxes(BvhDev& d, hipStream_t s) {
     if (d.n <= kLocalLeaves) {  // one leaf block: the root is local
         if (kLayout)
             LUX_LAUNCH("lbvh_pair_layout", k_pair_layout, max(1, div_up(d.n - 1, kBlock)), kBlock, 0, s, d.n,
@@ -1307,6 +1314,12 @@ void top_boxes(BvhDev& d, hipStream_t s) {
                (const uint32_t*)d.first, (const uint32_t*)d.last, (const uint32_t*)d.left, d.pair_pos,
                (const int32_t*)d.pre_internal,
                (const lux_aabb*)d.edge_boxes, (const lux_aabb*)d.block_boxes, d.nodes, d.info);
+}
+void top_boxes(BvhDev& d, bool layout, hipStream_t s) {
+    if (layout && (d.holds & kCopyPairs))
+        launch_top_boxes<true>(d, s);
+    else
+        launch_top_boxes<false>(d, s);
 }
 }  // namespace
 
@@ -1323,7 +1336,7 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
                    (const lux_triangle*)nullptr, (const int32_t*)d.ids, d.boxes, 0, d.nodes, d.pre_leaf,
                    d.keys[0], d.vals[0], d.info, 1);
         // root box from the one leaf (the reduction result is identical)
-        top_boxes<true>(d, s);
+        top_boxes(d, true, s);
         nodes_changed(d, s);
         return;
     }
@@ -1347,7 +1360,7 @@ void lbvh_build(BvhDev& d, const lux_aabb* in_boxes, const int32_t* in_ids, int 
                    (const uint32_t*)d.first, (const uint32_t*)d.last, d.rtop_int, d.rtop_leaf, d.pre_internal,
                    d.info);
     launch_local<0>("lbvh_local", d, d.boxes, nullptr, 0, s);
-    top_boxes<true>(d, s);
+    top_boxes(d, true, s);
     nodes_changed(d, s);
 }
 
@@ -1363,7 +1376,7 @@ void refit_launch(BvhDev& d, const lux_aabb* in_boxes, const lux_triangle* tris,
         return;
     }
     launch_local<kMode>(kMode == 2 ? "lbvh_local_tris" : "lbvh_local_boxes", d, in_boxes, tris, wb, s);
-    top_boxes<false>(d, s);
+    top_boxes(d, false, s);
     nodes_changed(d, s);
 }
 }  // namespace

@@ -110,16 +110,17 @@ struct BvhDev {
     int32_t* counter = nullptr;
     uint32_t epoch = 0;
     int status_words = 0;
-    // TreeCopy bits: copies behind the node array, and copies that builds and
-    // refits make at once (see tree_copies)
-    unsigned stale = 0, keep = 0;
+    // TreeCopy bits: copies the tree has arrays for (set before the first build),
+    // copies behind the node array, and copies that builds and refits make at once
+    // (see tree_copies)
+    unsigned holds = 3, stale = 0, keep = 0;
 };
 
 // Buffers for n primitives; new ones are cleared on `s`, the stream of the build.
 void bvh_allocate(BvhDev& d, int n, hipStream_t s);
 void bvh_release(BvhDev& d);
-// HBM that a tree over n primitives holds.
-size_t bvh_device_bytes(int n);
+// HBM that a tree over n primitives holds, with the copies `holds` (TreeCopy).
+size_t bvh_device_bytes(int n, unsigned holds = 3);
 
 // Scratch of the ray-order sort of the traversal entry points (grown on
 // demand; one per tree handle, used on one stream at a time).

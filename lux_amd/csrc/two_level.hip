@@ -82,17 +82,6 @@ T* dalloc_n(size_t count) {
     return static_cast<T*>(p);
 }
 
-template <typename T>
-struct TempBuffer {
-    T* p = nullptr;
-    explicit TempBuffer(size_t count) : p(dalloc_n<T>(count)) {}
-    ~TempBuffer() {
-        if (p) (void)hipFree(p);
-    }
-    TempBuffer(const TempBuffer&) = delete;
-    TempBuffer& operator=(const TempBuffer&) = delete;
-};
-
 bool box_is_empty(const lux_aabb& b) {
     return b.p_min.x > b.p_max.x || b.p_min.y > b.p_max.y || b.p_min.z > b.p_max.z;
 }
@@ -130,30 +119,29 @@ void validate_instances(const lux_instance* instances, int count, int mesh_count
 }
 
 void sync_and_check(const BvhDev& d, hipStream_t stream, const char* what) {
+    uint32_t error = 0;
+    if (d.info)
+        hip_check(hipMemcpyAsync(&error, &d.info->error, sizeof(error), hipMemcpyDeviceToHost, stream),
+                  "read device errors");
     hip_check(hipStreamSynchronize(stream), what);
-    if (!d.info) return;
-    DevInfo info;
-    hip_check(hipMemcpy(&info, d.info, sizeof(DevInfo), hipMemcpyDeviceToHost), "read device info");
-    if (info.error != 0) throw Error(LUX_ERR_DEVICE_CHECK, std::string("device check failed in ") + what);
+    if (error != 0) throw Error(LUX_ERR_DEVICE_CHECK, std::string("device check failed in ") + what);
 }
 
-// The records over the TLAS with its culling boxes (TwoLevelDev::tlas_wide), and
+// The records over the TLAS with its culling boxes (TwoLevelDev::tlas), and
 // each instance's leaf position: a node array of the TLAS's topology, each leaf
 // box the instance's world bounds intersected with the world box of its mesh's
 // bounding sphere (both widened as below), each internal box the union of its two
 // children. Every box still holds every world-space ray point that can hit the
 // geometry below it, so only the culling changes.
+// `nodes` (n > 0 instances, filled here) has to last until the stream is waited for.
 void build_tlas_wide(TwoLevelDev& s, const lux_instance* instances, std::vector<DevInstance>& rec,
-                     hipStream_t stream) {
+                     std::vector<lux_bvh_node>& nodes, hipStream_t stream) {
     const int n = s.tlas.n;
-    const int count = n > 0 ? 2 * n - 1 : 0;
-    if (s.tlas_wide) hip_check(hipFree(s.tlas_wide), "hipFree TLAS records");
-    s.tlas_wide = nullptr;
-    if (count <= 0) return;
-    std::vector<lux_bvh_node> nodes(static_cast<size_t>(count));
+    const int count = 2 * n - 1;
+    nodes.resize(static_cast<size_t>(count));
     hip_check(hipMemcpyAsync(nodes.data(), s.tlas.nodes, sizeof(lux_bvh_node) * count, hipMemcpyDeviceToHost, stream),
               "D2H TLAS");
-    hip_check(hipStreamSynchronize(stream), "synchronize TLAS download");
+    sync_and_check(s.tlas, stream, "TLAS build");
     // A leaf box must hold every world point w(t) of a ray whose object-space
     // image p(t) = inv w(t) lies in the mesh: M p(t) = (M inv) w(t) lies in the
     // transformed mesh, and M inv is the identity only to the scene
@@ -226,13 +214,16 @@ void build_tlas_wide(TwoLevelDev& s, const lux_instance* instances, std::vector<
                                    std::max(l.p_max.z, r.p_max.z)};
     }
     if (n < 2) return;
-    s.tlas_wide = static_cast<WideNode*>(static_cast<void*>(dalloc_n<uint8_t>(sizeof(WideNode) * size_t(n - 1))));
-    TempBuffer<lux_bvh_node> cull{size_t(count)};
-    TempBuffer<int32_t> leaf_pos{4 * size_t(n)};
-    hip_check(hipMemcpyAsync(cull.p, nodes.data(), sizeof(lux_bvh_node) * count, hipMemcpyHostToDevice, stream),
+    if (s.tlas_cull_capacity < count) {
+        if (s.tlas_cull) hip_check(hipFree(s.tlas_cull), "hipFree culling nodes");
+        s.tlas_cull = nullptr;
+        s.tlas_cull_capacity = 0;
+        s.tlas_cull = dalloc_n<lux_bvh_node>(size_t(count));
+        s.tlas_cull_capacity = count;
+    }
+    hip_check(hipMemcpyAsync(s.tlas_cull, nodes.data(), sizeof(lux_bvh_node) * count, hipMemcpyHostToDevice, stream),
               "H2D culling TLAS");
-    wide_from(s.tlas, cull.p, s.tlas_wide, leaf_pos.p, stream);
-    sync_and_check(s.tlas, stream, "TLAS records");
+    wide_from(s.tlas, s.tlas_cull, s.tlas.wide, s.tlas.wide_leaf, stream);
 }
 
 // TLAS over the non-empty world bounds (ids = instance ids) and the instance
@@ -261,37 +252,40 @@ void upload_instances(TwoLevelDev& s, const lux_instance* instances, int count, 
         ids.push_back(i);
     }
     const int n = int(boxes.size());
-    TempBuffer<lux_aabb> d_boxes(size_t(std::max(n, 1)));
-    TempBuffer<int32_t> d_ids(size_t(std::max(n, 1)));
     s.whole = false;
     s.host_instances.assign(instances, instances + count);
     s.instance_count = count;
     s.scene_primitives = cursor;
     s.tlas_instances = n;
+    s.tlas.holds = kCopyRecords;  // the culling records
+    bvh_allocate(s.tlas, n, stream);
     if (n > 0) {
-        hip_check(hipMemcpyAsync(d_boxes.p, boxes.data(), sizeof(lux_aabb) * n, hipMemcpyHostToDevice, stream),
+        hip_check(hipMemcpyAsync(s.tlas.boxes, boxes.data(), sizeof(lux_aabb) * n, hipMemcpyHostToDevice, stream),
                   "H2D world bounds");
-        hip_check(hipMemcpyAsync(d_ids.p, ids.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, stream),
+        hip_check(hipMemcpyAsync(s.tlas.ids, ids.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, stream),
                   "H2D instance ids");
     }
-    lbvh_build(s.tlas, d_boxes.p, d_ids.p, n, stream);
-    sync_and_check(s.tlas, stream, "TLAS build");
+    lbvh_build(s.tlas, s.tlas.boxes, s.tlas.ids, n, stream);
     uint64_t limit = n > 1 ? 2u * uint64_t(n) : uint64_t(n);
     for (int i = 0; i < count; ++i) {
         const int tri = s.mesh_tri_off[instances[i].mesh_id + 1] - s.mesh_tri_off[instances[i].mesh_id];
         limit += tri > 1 ? 2u * uint64_t(tri) : uint64_t(tri);
     }
     s.step_limit = uint32_t(std::min<uint64_t>(limit + 1, 0xffffffffu));
-    build_tlas_wide(s, instances, rec, stream);
-    if (s.instances) hip_check(hipFree(s.instances), "hipFree instances");
-    s.instances = nullptr;
-    s.instances = dalloc_n<DevInstance>(rec.size());
-    if (!rec.empty()) {
+    std::vector<lux_bvh_node> nodes;
+    if (n > 0) build_tlas_wide(s, instances, rec, nodes, stream);
+    if (s.instance_capacity < count || !s.instances) {
+        if (s.instances) hip_check(hipFree(s.instances), "hipFree instances");
+        s.instances = nullptr;
+        s.instance_capacity = 0;
+        s.instances = dalloc_n<DevInstance>(rec.size());
+        s.instance_capacity = count;
+    }
+    if (!rec.empty())
         hip_check(hipMemcpyAsync(s.instances, rec.data(), sizeof(DevInstance) * rec.size(), hipMemcpyHostToDevice,
                                  stream),
                   "H2D instances");
-        hip_check(hipStreamSynchronize(stream), "synchronize instances");
-    }
+    sync_and_check(s.tlas, stream, "TLAS records");
     s.whole = true;
 }
 
@@ -355,7 +349,7 @@ lux_aabb transform_bounds(const float* m, const lux_aabb& b) {
 void two_level_release(TwoLevelDev& s) {
     for (BvhDev& b : s.blas) bvh_release(b);
     bvh_release(s.tlas);
-    void* ptrs[] = {s.soup, s.meshes, s.instances, s.tlas_wide};
+    void* ptrs[] = {s.soup, s.meshes, s.instances, s.tlas_cull};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     s = TwoLevelDev{};
@@ -383,6 +377,7 @@ void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* of
     std::vector<DevMesh> meshes(static_cast<size_t>(mesh_count));
     for (int m = 0; m < mesh_count; ++m) {
         const int n = offsets[m + 1] - offsets[m];
+        s.blas[m].holds = kCopyRecords;
         // BLAS input (triangle_bounds, local ids) computed on the device from
         // the soup copied above
         lbvh_build_triangles(s.blas[m], s.soup + offsets[m], nullptr, nullptr, 0, n, stream);
@@ -393,7 +388,7 @@ void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* of
         meshes[m].tris = s.soup + offsets[m];
         meshes[m].node_count = n > 0 ? 2 * n - 1 : 0;
         meshes[m].tri_count = n;
-        s.device_bytes += bvh_device_bytes(n);
+        s.device_bytes += bvh_device_bytes(n, kCopyRecords);
     }
     // each mesh's bounding sphere: the center of its box, the largest vertex
     // distance from it (in double, padded), radius -1 for an empty mesh
@@ -429,7 +424,8 @@ void two_level_build(TwoLevelDev& s, const lux_triangle* tris, const int32_t* of
                   "H2D meshes");
     upload_instances(s, instances, instance_count, stream);
     s.device_bytes += sizeof(lux_triangle) * size_t(total) + sizeof(DevMesh) * meshes.size() +
-                      sizeof(DevInstance) * size_t(instance_count) + bvh_device_bytes(s.tlas_instances) + sizeof(WideNode) * size_t(std::max(s.tlas_instances - 1, 0));
+                      sizeof(DevInstance) * size_t(instance_count) + bvh_device_bytes(s.tlas_instances, kCopyRecords) +
+                      sizeof(lux_bvh_node) * size_t(std::max(2 * s.tlas_instances - 1, 0));
 }
 
 void two_level_set_instances(TwoLevelDev& s, const lux_instance* instances, int instance_count,
@@ -444,8 +440,8 @@ TwoLevelView two_level_view(const TwoLevelDev& s) {
     if (!s.whole) throw Error(LUX_ERR_INVALID_ARGUMENT, "instances were lost in a failed update: set them again");
     TwoLevelView v;
     v.tlas_nodes = s.tlas.nodes;
-    v.tlas_wide = s.tlas_wide;
-    v.tlas_records = s.tlas_wide ? uint32_t(s.tlas.n - 1) : 0u;
+    v.tlas_wide = s.tlas.wide;
+    v.tlas_records = s.tlas.n > 1 ? uint32_t(s.tlas.n - 1) : 0u;
     v.instances = s.instances;
     v.meshes = s.meshes;
     v.info = s.tlas.info;

@@ -444,13 +444,15 @@ __device__ __forceinline__ bool two_level_wide(const TwoLevelView& view, World&&
 // ---- host side ----------------------------------------------------------------------
 struct TwoLevelDev {
     std::vector<BvhDev> blas;  // per mesh (n = 0 for an empty mesh)
-    BvhDev tlas;               // over the non-empty instance world bounds, ids = instance ids
-    // Records over the TLAS with each leaf box narrowed to its instance's world
+    // Over the non-empty instance world bounds, ids = instance ids. Its records are
+    // made from culling nodes: each leaf box narrowed to its instance's world
     // bounds intersected with the world box of the mesh's bounding sphere
     // (center M c, half-extent r |row i of M| on axis i: the exact box of the
     // transformed sphere), both widened by what the instance's M inv may
     // deviate from the identity; internal boxes the unions of their children.
-    WideNode* tlas_wide = nullptr;
+    BvhDev tlas;
+    lux_bvh_node* tlas_cull = nullptr;
+    int tlas_cull_capacity = 0, instance_capacity = 0;
     std::vector<float> mesh_sphere;  // per mesh: center xyz, radius (padded)
     lux_triangle* soup = nullptr;
     DevMesh* meshes = nullptr;

@@ -235,8 +235,9 @@ def bytes_held(stub):
 
 
 def lost_instances(stub):
-    """set_instances that runs out of memory at each of its allocations in turn:
-    queries are refused until it has succeeded."""
+    """set_instances with more instances in view than before (two of three had empty
+    bounds) that runs out of memory at each of its allocations in turn: queries are
+    refused until it has succeeded."""
     from lux_amd import lbvh, two_level, workloads as W
 
     lbvh.init()
@@ -245,10 +246,12 @@ def lost_instances(stub):
     m = np.stack([W.affine(None, (1, 1, 1), (0.5 * k, 0, 0)) for k in range(3)]).astype(np.float32)
     offsets = np.array([0, 25, 40], np.int32)
     inst = two_level.make_instances(mesh, m, tris, offsets)
-    sc = two_level.TwoLevelScene(tris, offsets, inst)
+    first = inst.copy()
+    first["world_bounds"][1:] = [1, 1, 1, -1, -1, -1]
+    sc = two_level.TwoLevelScene(tris, offsets, first)
     rays = W.rays(10, seed=4)
     out = []
-    for k in range(20):
+    for k in range(60):
         stub.lib.stub_fail_alloc_after(k)
         failed = status_of(lambda: sc.set_instances(inst))
         stub.lib.stub_fail_alloc_after(-1)

@@ -70,9 +70,8 @@ def test_instances_lost_in_a_failed_update_are_not_queried(stub):
     """Between a TLAS that is rebuilt and records that are not, every ray would
     miss: such a scene refuses queries until its instances are set."""
     tries = scene(stub, "lost_instances")["tries"]
-    assert len(tries) > 2 and tries[-1] == [0, 0]
-    assert all(failed == 6 for failed, _ in tries[:-1])
-    assert [query for _, query in tries[:-1]] == [0, 0] + [1] * (len(tries) - 3)  # two come before any change
+    assert len(tries) > 10 and tries[-1] == [0, 0]
+    assert tries[:-1] == [[6, 1]] * (len(tries) - 1)  # out of memory; refused
 
 
 def test_traversal_copies_are_made_for_their_first_reader(stub):
