@@ -5,8 +5,10 @@
 
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "lux_runtime.hpp"
@@ -20,6 +22,10 @@ struct lux_hip_two_level {
 };
 
 struct lux_hip_bvh {
+    // Held from a call's look at the last stream to its last launch: two threads that
+    // query one tree on streams of their own must not meet between the copy that one
+    // of them has made (tree_copies) and its stream being the last.
+    std::mutex mu;
     lux::BvhDev dev;
     bool valid = false;              // GpuBvh::is_valid
     bool host_ids_known = false;     // host copy of the build ids is current
@@ -107,6 +113,13 @@ void sync_handle(lux_hip_bvh* h) {
 
 void require_handle(lux_hip_bvh* h) {
     if (!h) throw Error(LUX_ERR_INVALID_ARGUMENT, "null lux_hip_bvh handle");
+}
+
+// The locks of one or two handles, always taken in the order of their addresses.
+std::pair<std::unique_lock<std::mutex>, std::unique_lock<std::mutex>> lock_both(lux_hip_bvh* a, lux_hip_bvh* b) {
+    if (std::less<>()(b, a)) std::swap(a, b);
+    std::unique_lock<std::mutex> first(a->mu);
+    return {std::move(first), a == b ? std::unique_lock<std::mutex>() : std::unique_lock<std::mutex>(b->mu)};
 }
 
 template <typename T>
@@ -302,6 +315,7 @@ int lux_hip_bvh_destroy(lux_hip_bvh* bvh) {
 int lux_hip_bvh_set_ray_order(lux_hip_bvh* bvh, int32_t enable) {
     return guarded([&] {
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         bvh->order_rays = enable != 0;
         return int(LUX_OK);
     });
@@ -311,6 +325,7 @@ int lux_hip_bvh_build(lux_hip_bvh* bvh, const lux_aabb* boxes, const int32_t* id
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative primitive count");
         if (n > 0 && (!boxes || !ids)) throw Error(LUX_ERR_INVALID_ARGUMENT, "null input arrays");
         if (n >= (1 << 29)) throw Error(LUX_ERR_INVALID_ARGUMENT, "primitive count exceeds 2^29");
@@ -344,6 +359,7 @@ int lux_hip_bvh_build_device(lux_hip_bvh* bvh, const lux_aabb* d_boxes, const in
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative primitive count");
         if (n > 0 && (!d_boxes || !d_ids)) throw Error(LUX_ERR_INVALID_ARGUMENT, "null input arrays");
         if (n >= (1 << 29)) throw Error(LUX_ERR_INVALID_ARGUMENT, "primitive count exceeds 2^29");
@@ -367,6 +383,7 @@ int lux_hip_bvh_build_triangles_device(lux_hip_bvh* bvh, const lux_triangle* d_t
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative primitive count");
         if (n > 0 && !d_tris) throw Error(LUX_ERR_INVALID_ARGUMENT, "null triangle array");
         if (n >= (1 << 29)) throw Error(LUX_ERR_INVALID_ARGUMENT, "primitive count exceeds 2^29");
@@ -389,6 +406,7 @@ int lux_hip_bvh_refit(lux_hip_bvh* bvh, const lux_aabb* boxes, const int32_t* id
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0 || (n > 0 && (!boxes || !ids))) throw Error(LUX_ERR_INVALID_ARGUMENT, "bad refit input");
         if (n != (bvh->valid ? bvh->dev.n : 0))
             throw Error(LUX_ERR_MISMATCH, "refit primitive count does not match the built BVH");
@@ -417,6 +435,7 @@ int lux_hip_bvh_refit_device(lux_hip_bvh* bvh, const lux_aabb* d_boxes, int32_t 
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n != (bvh->valid ? bvh->dev.n : 0))
             throw Error(LUX_ERR_MISMATCH, "refit primitive count does not match the built BVH");
         if (!bvh->valid) return int(LUX_OK);
@@ -434,6 +453,7 @@ int lux_hip_bvh_refit_triangles_device(lux_hip_bvh* bvh, const lux_triangle* d_t
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n != (bvh->valid ? bvh->dev.n : 0))
             throw Error(LUX_ERR_MISMATCH, "refit primitive count does not match the built BVH");
         if (!bvh->valid) return int(LUX_OK);
@@ -450,6 +470,7 @@ int lux_hip_bvh_info(lux_hip_bvh* bvh, int32_t* valid, int32_t* count, lux_aabb*
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (bvh->valid) sync_handle(bvh);
         if (valid) *valid = bvh->valid ? 1 : 0;
         if (count) *count = bvh->valid ? bvh->dev.n : 0;
@@ -469,6 +490,7 @@ int lux_hip_bvh_view(lux_hip_bvh* bvh, lux_bvh_view* out) {
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (!out) throw Error(LUX_ERR_INVALID_ARGUMENT, "null output");
         lux_bvh_view v;
         std::memset(&v, 0, sizeof(v));
@@ -488,6 +510,7 @@ int lux_hip_bvh_download_nodes(lux_hip_bvh* bvh, lux_bvh_node* nodes, int32_t ca
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (!bvh->valid) return int(LUX_OK);
         int total = 2 * bvh->dev.n - 1;
         if (!nodes || capacity < total) throw Error(LUX_ERR_INVALID_ARGUMENT, "node buffer too small");
@@ -503,6 +526,7 @@ int lux_hip_bvh_download_topology(lux_hip_bvh* bvh, uint32_t* morton_sorted, uin
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (!bvh->valid) return int(LUX_OK);
         sync_handle(bvh);
         const BvhDev& d = bvh->dev;
@@ -538,6 +562,7 @@ int lux_hip_bvh_download_input(lux_hip_bvh* bvh, lux_aabb* boxes, int32_t* primi
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (!bvh->valid) return int(LUX_OK);
         sync_handle(bvh);
         const size_t n = size_t(bvh->dev.n);
@@ -552,6 +577,7 @@ int lux_hip_bvh_device_arrays(lux_hip_bvh* bvh, const lux_aabb** d_input_bounds,
                               const uint32_t** d_sorted_indices) {
     return guarded([&] {
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         const bool v = bvh->valid;
         if (d_input_bounds) *d_input_bounds = v ? bvh->dev.boxes : nullptr;
         if (d_primitive_ids) *d_primitive_ids = v ? bvh->dev.ids : nullptr;
@@ -565,6 +591,7 @@ int lux_hip_trace_closest(lux_hip_bvh* bvh, const lux_triangle* tris, int32_t tr
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::unique_lock<std::mutex> lock(bvh->mu);
         if (n < 0 || tri_count < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative count");
         if (n > 0 && (!rays || !hits)) throw Error(LUX_ERR_INVALID_ARGUMENT, "null ray/hit arrays");
         for (int32_t i = 0; i < n; ++i) {
@@ -582,6 +609,7 @@ int lux_hip_trace_closest(lux_hip_bvh* bvh, const lux_triangle* tris, int32_t tr
         bvh->last_stream = g_stream;
         trace_closest(bvh->dev, closest_order(bvh->order, bvh->order_rays, bvh->dev, dr.p, n, g_stream), dt.p, tri_count,
                       dr.p, n, dh.p, g_stream);
+        lock.unlock();
         hip_check(hipMemcpyAsync(hits, dh.p, sizeof(lux_hit) * n, hipMemcpyDeviceToHost, g_stream), "D2H hits");
         sync_handle(bvh);
         return int(LUX_OK);
@@ -593,6 +621,7 @@ int lux_hip_trace_closest_device(lux_hip_bvh* bvh, const lux_triangle* d_tris, i
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0 || tri_count < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative count");
         if (n > 0 && (!d_rays || !d_hits)) throw Error(LUX_ERR_INVALID_ARGUMENT, "null ray/hit arrays");
         if (!bvh->valid) throw Error(LUX_ERR_INVALID_ARGUMENT, "BVH is not valid");
@@ -610,6 +639,7 @@ int lux_hip_trace_closest_device_noalloc(lux_hip_bvh* bvh, const lux_triangle* d
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0 || tri_count < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative count");
         if (n > kNoAllocMaxRays)
             throw Error(LUX_ERR_INVALID_ARGUMENT,
@@ -629,6 +659,7 @@ int lux_hip_trace_any(lux_hip_bvh* bvh, const lux_triangle* tris, int32_t tri_co
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::unique_lock<std::mutex> lock(bvh->mu);
         if (n < 0 || tri_count < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative count");
         if (n > 0 && (!rays || !occluded)) throw Error(LUX_ERR_INVALID_ARGUMENT, "null ray/output arrays");
         std::memset(occluded, 0, size_t(n));
@@ -642,6 +673,7 @@ int lux_hip_trace_any(lux_hip_bvh* bvh, const lux_triangle* tris, int32_t tri_co
         hip_check(hipMemcpyAsync(dr.p, rays, sizeof(lux_ray) * n, hipMemcpyHostToDevice, g_stream), "H2D rays");
         bvh->last_stream = g_stream;
         trace_any(bvh->dev, bvh->order_rays ? &bvh->order : nullptr, dt.p, tri_count, dr.p, n, dh.p, g_stream);
+        lock.unlock();
         hip_check(hipMemcpyAsync(occluded, dh.p, size_t(n), hipMemcpyDeviceToHost, g_stream), "D2H occluded");
         sync_handle(bvh);
         return int(LUX_OK);
@@ -653,6 +685,7 @@ int lux_hip_trace_any_device(lux_hip_bvh* bvh, const lux_triangle* d_tris, int32
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0 || tri_count < 0) throw Error(LUX_ERR_INVALID_ARGUMENT, "negative count");
         if (n > 0 && (!d_rays || !d_occluded)) throw Error(LUX_ERR_INVALID_ARGUMENT, "null ray/output arrays");
         if (!bvh->valid) throw Error(LUX_ERR_INVALID_ARGUMENT, "BVH is not valid");
@@ -669,6 +702,7 @@ static int overlap_host(lux_hip_bvh* tree, lux_hip_bvh* queries, bool self_mode,
     require_init();
     require_handle(tree);
     require_handle(queries);
+    const auto locks = lock_both(tree, queries);
     if (!found) throw Error(LUX_ERR_INVALID_ARGUMENT, "null found_count");
     *found = 0;
     if (!tree->valid || !queries->valid || max_pairs <= 0) return LUX_OK;
@@ -702,6 +736,7 @@ static int overlap_device(lux_hip_bvh* tree, lux_hip_bvh* queries, bool self_mod
     require_init();
     require_handle(tree);
     require_handle(queries);
+    const auto locks = lock_both(tree, queries);
     if (!d_found) throw Error(LUX_ERR_INVALID_ARGUMENT, "null found_count");
     if (max_pairs > 0 && !d_pairs) throw Error(LUX_ERR_INVALID_ARGUMENT, "null pair buffer");
     hipStream_t s = pick(stream);
@@ -730,6 +765,7 @@ int lux_hip_trace_stats_device(lux_hip_bvh* bvh, const lux_triangle* d_tris, int
     return guarded([&] {
         require_init();
         require_handle(bvh);
+        std::lock_guard<std::mutex> lock(bvh->mu);
         if (n < 0 || tri_count < 0 || !stats) throw Error(LUX_ERR_INVALID_ARGUMENT, "bad stats arguments");
         if (n > 0 && !d_rays) throw Error(LUX_ERR_INVALID_ARGUMENT, "null rays");
         constexpr int kStats = 6;  // {closest, any-hit} x {node units, visits, triangle tests}

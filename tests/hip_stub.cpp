@@ -34,6 +34,7 @@ std::map<const void*, std::string> g_names;   // kernel -> mangled name
 std::map<const void*, size_t> g_live;         // device allocations
 std::map<const void*, void*> g_symbols;       // __device__ variables
 std::map<const void*, size_t> g_symbol_bytes;
+std::map<void*, long> g_launches, g_waited;   // per stream: launches so far, and when it was last waited for
 std::vector<Fill> g_pending;                  // null-stream fills not yet done
 size_t g_live_bytes = 0;
 int g_null_writes = 0;                        // device writes ordered on the null stream only
@@ -75,6 +76,14 @@ extern "C" {
 void stub_on_launch(LaunchCb cb) { g_on_launch = cb; }
 uint64_t stub_live_bytes() { return g_live_bytes; }
 int stub_null_writes() { return g_null_writes; }
+long stub_launches(void* s) {
+    std::lock_guard<std::recursive_mutex> lk(g_mu);
+    return g_launches[s];
+}
+long stub_waited(void* s) {
+    std::lock_guard<std::recursive_mutex> lk(g_mu);
+    return g_waited[s];
+}
 unsigned stub_grid() { return t_grid; }
 unsigned stub_block() { return t_block; }
 void stub_capturing(int on) { g_capturing = on != 0; }
@@ -108,6 +117,7 @@ hipError_t hipLaunchKernel(const void* fn, dim3 grid, dim3 block, void** args, s
         std::lock_guard<std::recursive_mutex> lk(g_mu);
         name = g_names.count(fn) ? g_names[fn] : "?";
         if (!stream) ++g_null_writes;
+        ++g_launches[stream];
     }
     t_grid = grid.x;
     t_block = block.x;
@@ -181,10 +191,15 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned flags) {
     return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }  // that stream's work; fills stay pending
+hipError_t hipStreamSynchronize(hipStream_t s) {  // that stream's work; fills stay pending
+    std::lock_guard<std::recursive_mutex> lk(g_mu);
+    g_waited[s] = g_launches[s];
+    return hipSuccess;
+}
 hipError_t hipDeviceSynchronize() {
     std::lock_guard<std::recursive_mutex> lk(g_mu);
     finish_fills();
+    g_waited = g_launches;
     return hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t* e) {

@@ -34,6 +34,7 @@ class Stub:
     def _launch(self, name, stream, args):
         name = name.decode()
         self.launches.append(name)
+        self.stream = stream or 0
         if "k_zero_u32" in name:  # (uint32_t* p, int n)
             ctypes.memset(ptr(args, 0), 0, 4 * i32(args, 1))
         if "k_clear_tree" in name:  # (status, words, tickets, counter, info)
@@ -405,6 +406,52 @@ def failed_builds(stub):
         call()
         assert null == [], (name, null)
     return {"tries": tries, "left": left, "later": counts}
+
+
+def two_threads(stub):
+    """Two threads that query one tree on streams of their own right after a refit:
+    every walk must be ordered behind the launch that made its records."""
+    import threading
+
+    from lux_amd import abi, lbvh, workloads as W
+
+    for fn in (stub.lib.stub_launches, stub.lib.stub_waited):
+        fn.restype, fn.argtypes = ctypes.c_long, [ctypes.c_void_p]
+    n = 300
+    d_tris, rays, out = lbvh.DeviceArray.from_numpy(W.soup(n, seed=1)), lbvh.DeviceArray(36), lbvh.DeviceArray(8)
+    bvh = lbvh.GpuBvh()
+    bvh.build_triangles_device(d_tris, n)
+    streams = [ctypes.c_void_p(0xA000), ctypes.c_void_p(0xB000)]
+    here = threading.local()
+    made, late, walks = {}, [], [0]
+
+    def see(name, stream):  # in the launching thread
+        if "k_copies" in name:
+            made[0] = (stream, stub.lib.stub_launches(stream))
+        elif "13k_trace_parts" in name:
+            walks[0] += 1
+            s, index = made[0]
+            if s != stream and stub.lib.stub_waited(s) < index:
+                late.append(walks[0])
+
+    cb = CALLBACK(lambda name, stream, args: see(name.decode(), stream or 0))
+    stub.lib.stub_on_launch(cb)
+    start, stop = threading.Barrier(2), threading.Barrier(2)
+
+    def work(k):
+        for _ in range(400):
+            if k == 0:
+                bvh.refit_triangles_device(d_tris, n, stream=streams[0])
+            start.wait()
+            abi.call("lux_hip_trace_closest_device", bvh.handle, d_tris.ptr, n, rays.ptr, 1, out.ptr, streams[k])
+            stop.wait()
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    return {"walks": walks[0], "late": len(late)}
 
 
 if __name__ == "__main__":

@@ -118,3 +118,8 @@ def test_a_build_after_a_failed_one_has_all_its_arrays(stub):
     assert len(r["tries"]) > 25 and r["tries"][:-1] == [6] * (len(r["tries"]) - 1) and r["tries"][-1] == 0
     assert not any(r["left"])
     assert r["later"] == {"order": 7, "paths": 12}  # (paths: a buffer for one, then the batch)
+
+
+def test_two_threads_on_one_tree_wait_for_its_copies(stub):
+    r = scene(stub, "two_threads")
+    assert r["walks"] == 800 and r["late"] == 0
