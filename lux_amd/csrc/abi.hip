@@ -611,7 +611,8 @@ int lux_hip_trace_closest(lux_hip_bvh* bvh, const lux_triangle* tris, int32_t tr
                       dr.p, n, dh.p, g_stream);
         lock.unlock();
         hip_check(hipMemcpyAsync(hits, dh.p, sizeof(lux_hit) * n, hipMemcpyDeviceToHost, g_stream), "D2H hits");
-        sync_handle(bvh);
+        hip_check(hipStreamSynchronize(g_stream), "synchronize");  // another call's stream may be the last
+        check_device_flags(bvh, g_stream);
         return int(LUX_OK);
     });
 }
@@ -675,7 +676,8 @@ int lux_hip_trace_any(lux_hip_bvh* bvh, const lux_triangle* tris, int32_t tri_co
         trace_any(bvh->dev, bvh->order_rays ? &bvh->order : nullptr, dt.p, tri_count, dr.p, n, dh.p, g_stream);
         lock.unlock();
         hip_check(hipMemcpyAsync(occluded, dh.p, size_t(n), hipMemcpyDeviceToHost, g_stream), "D2H occluded");
-        sync_handle(bvh);
+        hip_check(hipStreamSynchronize(g_stream), "synchronize");  // another call's stream may be the last
+        check_device_flags(bvh, g_stream);
         return int(LUX_OK);
     });
 }

@@ -34,7 +34,7 @@ std::map<const void*, std::string> g_names;   // kernel -> mangled name
 std::map<const void*, size_t> g_live;         // device allocations
 std::map<const void*, void*> g_symbols;       // __device__ variables
 std::map<const void*, size_t> g_symbol_bytes;
-std::map<void*, long> g_launches, g_waited;   // per stream: launches so far, and when it was last waited for
+std::map<void*, long> g_launches, g_waited;   // per stream: launches and copies so far, and when it was last waited for
 std::vector<Fill> g_pending;                  // null-stream fills not yet done
 size_t g_live_bytes = 0;
 int g_null_writes = 0;                        // device writes ordered on the null stream only
@@ -43,6 +43,8 @@ bool g_capturing = false;
 int g_allocs_left = -1;  // allocations until one fails (-1: none does)
 using LaunchCb = void (*)(const char* name, void* stream, void** args);
 LaunchCb g_on_launch = nullptr;
+using DownloadCb = void (*)(void* stream);
+DownloadCb g_on_download = nullptr;  // before each asynchronous copy to the host
 
 struct Config {
     dim3 grid, block;
@@ -74,6 +76,7 @@ void drop_fills(const void* p, size_t bytes) {
 extern "C" {
 
 void stub_on_launch(LaunchCb cb) { g_on_launch = cb; }
+void stub_on_download(DownloadCb cb) { g_on_download = cb; }
 uint64_t stub_live_bytes() { return g_live_bytes; }
 int stub_null_writes() { return g_null_writes; }
 long stub_launches(void* s) {
@@ -171,7 +174,9 @@ hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind kin
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+    if (kind == hipMemcpyDeviceToHost && g_on_download) g_on_download(s);
     std::lock_guard<std::recursive_mutex> lk(g_mu);
+    ++g_launches[s];
     if (!s && kind != hipMemcpyDeviceToHost) ++g_null_writes;
     std::memcpy(dst, src, bytes);
     return hipSuccess;

@@ -454,5 +454,40 @@ def two_threads(stub):
     return {"walks": walks[0], "late": len(late)}
 
 
+def host_queries(stub):
+    """Queries from and to host arrays, with another thread's call on a stream of its
+    own between their walk and the copy of their results: launches and copies of their
+    own stream that they did not wait for."""
+    import threading
+
+    from lux_amd import abi, lbvh, workloads as W
+
+    for fn in (stub.lib.stub_launches, stub.lib.stub_waited):
+        fn.restype, fn.argtypes = ctypes.c_long, [ctypes.c_void_p]
+    n = 300
+    soup, host_rays = W.soup(n, seed=1), W.rays(10, seed=4)
+    d_tris, rays, out = lbvh.DeviceArray.from_numpy(soup), lbvh.DeviceArray(36), lbvh.DeviceArray(8)
+    bvh = lbvh.GpuBvh()
+    bvh.build_triangles_device(d_tris, n)
+    own = stub.stream
+    calls = [0]
+
+    def other(stream):
+        calls[0] += 1
+        t = threading.Thread(target=abi.call, args=("lux_hip_trace_closest_device", bvh.handle, d_tris.ptr, n, rays.ptr, 1,
+                                                    out.ptr, ctypes.c_void_p(0xA000)))
+        t.start()
+        t.join()
+
+    cb = ctypes.CFUNCTYPE(None, ctypes.c_void_p)(other)
+    stub.lib.stub_on_download(cb)
+    open_work = []
+    for query in (lbvh.intersect_gpu_bvh_stackless, lbvh.trace_any):
+        query(bvh, soup, host_rays)
+        open_work.append(stub.lib.stub_launches(own) - stub.lib.stub_waited(own))
+    stub.lib.stub_on_download(None)
+    return {"calls": calls[0], "open": open_work}
+
+
 if __name__ == "__main__":
     print(json.dumps(globals()[sys.argv[1]](Stub())))

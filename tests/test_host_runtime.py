@@ -123,3 +123,8 @@ def test_a_build_after_a_failed_one_has_all_its_arrays(stub):
 def test_two_threads_on_one_tree_wait_for_its_copies(stub):
     r = scene(stub, "two_threads")
     assert r["walks"] == 800 and r["late"] == 0
+
+
+def test_host_queries_wait_for_their_own_results(stub):
+    """Whatever stream another thread's call has made the tree's last one."""
+    assert scene(stub, "host_queries") == {"calls": 2, "open": [0, 0]}
